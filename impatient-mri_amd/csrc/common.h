@@ -74,6 +74,8 @@ enum WsSlot {
     WS_STACK,      // stacked-trajectory detection flags
     WS_QSTACK,     // stacked Q: one partition's 2D planes and the z factor
     WS_GRID,       // gridding: binned samples, grids and line-transform tables
+    WS_NU_GEO,     // separable NUDFT: geometry scan
+    WS_NU,         // separable NUDFT: tables and grids
     WS_COUNT
 };
 

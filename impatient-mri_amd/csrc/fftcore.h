@@ -20,70 +20,72 @@
 namespace imp {
 namespace fftc {
 
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-    return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+// The butterflies are written once for float2 and double2 lines (the Toeplitz
+// passes and the NUDFT's wide-kernel transforms).
+template <class C2>
+struct scalar_of;
+template <>
+struct scalar_of<float2> { using type = float; };
+template <>
+struct scalar_of<double2> { using type = double; };
+
+template <class C2>
+__device__ __forceinline__ C2 mk(typename scalar_of<C2>::type x, typename scalar_of<C2>::type y) {
+    C2 r;
+    r.x = x;
+    r.y = y;
+    return r;
 }
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+template <class C2>
+__device__ __forceinline__ C2 cmul(C2 a, C2 b) {
+    return mk<C2>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+template <class C2>
+__device__ __forceinline__ C2 cadd(C2 a, C2 b) { return mk<C2>(a.x + b.x, a.y + b.y); }
+template <class C2>
+__device__ __forceinline__ C2 csub(C2 a, C2 b) { return mk<C2>(a.x - b.x, a.y - b.y); }
 // multiply by -i (forward) or +i (inverse)
-template <bool INV>
-__device__ __forceinline__ float2 rot90(float2 a) {
-    return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
+template <bool INV, class C2>
+__device__ __forceinline__ C2 rot90(C2 a) {
+    return INV ? mk<C2>(-a.y, a.x) : mk<C2>(a.y, -a.x);
 }
 // multiply by e^(-+ i pi / 4) (forward / inverse)
-template <bool INV>
-__device__ __forceinline__ float2 rot45(float2 a) {
-    constexpr float h = 0.70710678118654752f;
-    return INV ? make_float2(h * (a.x - a.y), h * (a.x + a.y))
-               : make_float2(h * (a.x + a.y), h * (a.y - a.x));
+template <bool INV, class C2>
+__device__ __forceinline__ C2 rot45(C2 a) {
+    using F = typename scalar_of<C2>::type;
+    constexpr F h = (F)0.70710678118654752440;
+    return INV ? mk<C2>(h * (a.x - a.y), h * (a.x + a.y)) : mk<C2>(h * (a.x + a.y), h * (a.y - a.x));
 }
-template <bool INV>
-__device__ __forceinline__ float2 rot135(float2 a) {  // e^(-+ 3 i pi / 4)
-    constexpr float h = 0.70710678118654752f;
-    return INV ? make_float2(-h * (a.x + a.y), h * (a.x - a.y))
-               : make_float2(h * (a.y - a.x), -h * (a.x + a.y));
+template <bool INV, class C2>
+__device__ __forceinline__ C2 rot135(C2 a) {  // e^(-+ 3 i pi / 4)
+    using F = typename scalar_of<C2>::type;
+    constexpr F h = (F)0.70710678118654752440;
+    return INV ? mk<C2>(-h * (a.x + a.y), h * (a.x - a.y))
+               : mk<C2>(h * (a.y - a.x), -h * (a.x + a.y));
 }
 
-// In-register DFT of size R in natural order: v[k] <- sum_n v[n] w^(nk),
-// w = e^(-2 pi i / R) (forward) or e^(+2 pi i / R) (inverse).
-template <int R, bool INV>
-__device__ __forceinline__ void dft(float2 *v);
-
-template <>
-__device__ __forceinline__ void dft<1, false>(float2 *) {}
-template <>
-__device__ __forceinline__ void dft<1, true>(float2 *) {}
-
-template <bool INV>
-__device__ __forceinline__ void dft2(float2 *v) {
-    const float2 a = v[0], b = v[1];
+template <bool INV, class C2>
+__device__ __forceinline__ void dft2(C2 *v) {
+    const C2 a = v[0], b = v[1];
     v[0] = cadd(a, b);
     v[1] = csub(a, b);
 }
-template <>
-__device__ __forceinline__ void dft<2, false>(float2 *v) { dft2<false>(v); }
-template <>
-__device__ __forceinline__ void dft<2, true>(float2 *v) { dft2<true>(v); }
 
-template <bool INV>
-__device__ __forceinline__ void dft4(float2 *v) {
-    const float2 s02 = cadd(v[0], v[2]), d02 = csub(v[0], v[2]);
-    const float2 s13 = cadd(v[1], v[3]), d13 = rot90<INV>(csub(v[1], v[3]));
+template <bool INV, class C2>
+__device__ __forceinline__ void dft4(C2 *v) {
+    const C2 s02 = cadd(v[0], v[2]), d02 = csub(v[0], v[2]);
+    const C2 s13 = cadd(v[1], v[3]), d13 = rot90<INV>(csub(v[1], v[3]));
     v[0] = cadd(s02, s13);
     v[2] = csub(s02, s13);
     v[1] = cadd(d02, d13);
     v[3] = csub(d02, d13);
 }
-template <>
-__device__ __forceinline__ void dft<4, false>(float2 *v) { dft4<false>(v); }
-template <>
-__device__ __forceinline__ void dft<4, true>(float2 *v) { dft4<true>(v); }
 
 // radix-2 decimation in time: X[k] = E[k] + w^k O[k], X[k + R/2] = E[k] - w^k O[k]
-template <bool INV>
-__device__ __forceinline__ void dft8(float2 *v) {
-    float2 e[4] = {v[0], v[2], v[4], v[6]};
-    float2 o[4] = {v[1], v[3], v[5], v[7]};
+template <bool INV, class C2>
+__device__ __forceinline__ void dft8(C2 *v) {
+    C2 e[4] = {v[0], v[2], v[4], v[6]};
+    C2 o[4] = {v[1], v[3], v[5], v[7]};
     dft4<INV>(e);
     dft4<INV>(o);
     o[1] = rot45<INV>(o[1]);
@@ -95,15 +97,12 @@ __device__ __forceinline__ void dft8(float2 *v) {
         v[k + 4] = csub(e[k], o[k]);
     }
 }
-template <>
-__device__ __forceinline__ void dft<8, false>(float2 *v) { dft8<false>(v); }
-template <>
-__device__ __forceinline__ void dft<8, true>(float2 *v) { dft8<true>(v); }
 
-template <bool INV>
-__device__ __forceinline__ void dft16(float2 *v) {
+template <bool INV, class C2>
+__device__ __forceinline__ void dft16(C2 *v) {
+    using F = typename scalar_of<C2>::type;
     // 16 = 4 x 4: DFT-4 over n = a + 4 c (c), twiddle w16^(a k1), DFT-4 over a
-    float2 x[4][4];
+    C2 x[4][4];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
 #pragma unroll
@@ -112,10 +111,9 @@ __device__ __forceinline__ void dft16(float2 *v) {
     }
     // twiddles w16^(a k1) for a, k1 in 1..3 (exponents 1, 2, 3, 4, 6, 9);
     // w16^m = cos(pi m / 8) -+ i sin(pi m / 8)
-    constexpr float c1 = 0.92387953251128676f, s1 = 0.38268343236508977f;
-    constexpr float sg = INV ? 1.f : -1.f;
-    const float2 w1 = make_float2(c1, sg * s1), w3 = make_float2(s1, sg * c1),
-                 w9 = make_float2(-c1, -sg * s1);
+    constexpr F c1 = (F)0.92387953251128675613, s1 = (F)0.38268343236508977173;
+    constexpr F sg = INV ? (F)1 : (F)-1;
+    const C2 w1 = mk<C2>(c1, sg * s1), w3 = mk<C2>(s1, sg * c1), w9 = mk<C2>(-c1, -sg * s1);
     x[1][1] = cmul(x[1][1], w1);
     x[1][2] = rot45<INV>(x[1][2]);
     x[1][3] = cmul(x[1][3], w3);
@@ -127,37 +125,31 @@ __device__ __forceinline__ void dft16(float2 *v) {
     x[3][3] = cmul(x[3][3], w9);
 #pragma unroll
     for (int k1 = 0; k1 < 4; ++k1) {
-        float2 y[4] = {x[0][k1], x[1][k1], x[2][k1], x[3][k1]};
+        C2 y[4] = {x[0][k1], x[1][k1], x[2][k1], x[3][k1]};
         dft4<INV>(y);
 #pragma unroll
         for (int k2 = 0; k2 < 4; ++k2) v[k1 + 4 * k2] = y[k2];
     }
 }
-template <>
-__device__ __forceinline__ void dft<16, false>(float2 *v) { dft16<false>(v); }
-template <>
-__device__ __forceinline__ void dft<16, true>(float2 *v) { dft16<true>(v); }
 
-template <bool INV>
-__device__ __forceinline__ void dft3(float2 *v) {
-    constexpr float r3 = 0.86602540378443865f;  // sqrt(3) / 2
-    const float2 s = cadd(v[1], v[2]);
-    const float2 d = rot90<INV>(csub(v[1], v[2]));
-    const float2 t = make_float2(v[0].x - 0.5f * s.x, v[0].y - 0.5f * s.y);
+template <bool INV, class C2>
+__device__ __forceinline__ void dft3(C2 *v) {
+    using F = typename scalar_of<C2>::type;
+    constexpr F r3 = (F)0.86602540378443864676;  // sqrt(3) / 2
+    const C2 s = cadd(v[1], v[2]);
+    const C2 d = rot90<INV>(csub(v[1], v[2]));
+    const C2 t = mk<C2>(v[0].x - (F)0.5 * s.x, v[0].y - (F)0.5 * s.y);
     v[0] = cadd(v[0], s);
-    v[1] = make_float2(t.x + r3 * d.x, t.y + r3 * d.y);
-    v[2] = make_float2(t.x - r3 * d.x, t.y - r3 * d.y);
+    v[1] = mk<C2>(t.x + r3 * d.x, t.y + r3 * d.y);
+    v[2] = mk<C2>(t.x - r3 * d.x, t.y - r3 * d.y);
 }
-template <>
-__device__ __forceinline__ void dft<3, false>(float2 *v) { dft3<false>(v); }
-template <>
-__device__ __forceinline__ void dft<3, true>(float2 *v) { dft3<true>(v); }
 
-template <bool INV>
-__device__ __forceinline__ void dft12(float2 *v) {
+template <bool INV, class C2>
+__device__ __forceinline__ void dft12(C2 *v) {
+    using F = typename scalar_of<C2>::type;
     // 12 = 4 x 3: DFT-3 over n = a + 4 c (c), twiddle w12^(a k1), DFT-4 over a;
     // output k = k1 + 3 k2
-    float2 x[4][3];
+    C2 x[4][3];
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
 #pragma unroll
@@ -165,28 +157,36 @@ __device__ __forceinline__ void dft12(float2 *v) {
         dft3<INV>(x[a]);
     }
     // w12^m = cos(pi m / 6) -+ i sin(pi m / 6), m = a k1 in {1, 2, 2, 4, 3, 6}
-    constexpr float r3 = 0.86602540378443865f;
-    constexpr float sg = INV ? 1.f : -1.f;
-    const float2 w1 = make_float2(r3, sg * 0.5f), w2 = make_float2(0.5f, sg * r3),
-                 w4 = make_float2(-0.5f, sg * r3);
+    constexpr F r3 = (F)0.86602540378443864676;
+    constexpr F sg = INV ? (F)1 : (F)-1, hf = (F)0.5;
+    const C2 w1 = mk<C2>(r3, sg * hf), w2 = mk<C2>(hf, sg * r3), w4 = mk<C2>(-hf, sg * r3);
     x[1][1] = cmul(x[1][1], w1);
     x[1][2] = cmul(x[1][2], w2);
     x[2][1] = cmul(x[2][1], w2);
     x[2][2] = cmul(x[2][2], w4);
     x[3][1] = rot90<INV>(x[3][1]);
-    x[3][2] = make_float2(-x[3][2].x, -x[3][2].y);
+    x[3][2] = mk<C2>(-x[3][2].x, -x[3][2].y);
 #pragma unroll
     for (int k1 = 0; k1 < 3; ++k1) {
-        float2 y[4] = {x[0][k1], x[1][k1], x[2][k1], x[3][k1]};
+        C2 y[4] = {x[0][k1], x[1][k1], x[2][k1], x[3][k1]};
         dft4<INV>(y);
 #pragma unroll
         for (int k2 = 0; k2 < 4; ++k2) v[k1 + 3 * k2] = y[k2];
     }
 }
-template <>
-__device__ __forceinline__ void dft<12, false>(float2 *v) { dft12<false>(v); }
-template <>
-__device__ __forceinline__ void dft<12, true>(float2 *v) { dft12<true>(v); }
+
+// In-register DFT of size R in natural order: v[k] <- sum_n v[n] w^(nk),
+// w = e^(-2 pi i / R) (forward) or e^(+2 pi i / R) (inverse).
+template <int R, bool INV, class C2>
+__device__ __forceinline__ void dft(C2 *v) {
+    static_assert(R == 1 || R == 2 || R == 3 || R == 4 || R == 8 || R == 12 || R == 16, "radix");
+    if constexpr (R == 2) dft2<INV>(v);
+    if constexpr (R == 3) dft3<INV>(v);
+    if constexpr (R == 4) dft4<INV>(v);
+    if constexpr (R == 8) dft8<INV>(v);
+    if constexpr (R == 12) dft12<INV>(v);
+    if constexpr (R == 16) dft16<INV>(v);
+}
 
 // ------------------------------------------------------------------ plans
 // Supported lengths: 2^k (2..4096) and 3 * 2^k (12..3072).

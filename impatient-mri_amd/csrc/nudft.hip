@@ -35,6 +35,7 @@
 // Sample sums are blocked and folded into compensated (two-sum) totals;
 // chunk partials are reduced in FP64.
 #include "common.h"
+#include "nufft.h"
 
 #include <algorithm>
 #include <cmath>
@@ -1252,6 +1253,61 @@ size_t adjoint_fixed_bytes(int num_k, int num_x, int ncoils, bool d3) {
 
 }  // namespace
 
+// ---- direct sum or separable evaluation (nufft.hip) -------------------------
+// Times of both in microseconds on an MI355X, fitted to single calls over
+// 48^2..512^2 voxels x 2e3..4e5 samples x 1..32 coils (within 30%).  The
+// direct kernels cost the same for every geometry; the separable form pays per
+// sample and time term for the spread, and per grid column for the
+// transforms, behind a fixed part (geometry read-back, sort, ~20 launches).
+constexpr double NUFFT_MIN_PAIRS = 6e8;   // below: the direct kernels win at every size measured
+
+double direct_us(double pairs, int ncoils) {
+    return 60.0 + pairs * (ncoils <= 1 ? 7.9e-4 : ncoils == 2 ? 8.4e-4
+                           : ncoils <= MF_COLS ? 5.6e-4 : 8.1e-4);
+}
+
+// The separable form evaluates 2D problems of as many coils as one direct
+// launch takes; refusals and everything else stay with the direct path.
+// G->ok tells whether it is to be used.  A stream under capture stays direct
+// (the geometry is read back).
+int choose_separable(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *kx,
+                     const float *ky, const float *t, const float *x, const float *y,
+                     const float *fm, NuGeometry *G) {
+    G->ok = false;
+    const double pairs = (double)num_k * num_x;
+    if (pairs < NUFFT_MIN_PAIRS || ncoils > 2 * MF_COLS) return IMP_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    IMP_HIP(hipStreamIsCapturing(ctx->stream, &cap));
+    if (cap != hipStreamCaptureStatusNone) return IMP_OK;
+    IMP_TRY(nufft_geometry(ctx, num_k, num_x, kx, ky, t, x, y, fm, G));
+    if (G->ok && nufft_adjoint_us(*G, num_k, ncoils) >= direct_us(pairs, ncoils)) G->ok = false;
+    return IMP_OK;
+}
+
+// Workspaces of the direct adjoint of this size, so that a call captured into
+// a graph after calls that took the separable form finds them allocated.
+int reserve_direct(imp_ctx *ctx, int num_k, int num_x, int ncoils) {
+    void *p = nullptr;
+    IMP_TRY(workspace(ctx, WS_SPOS, spos_bytes(num_k, false), &p));
+    IMP_TRY(workspace(ctx, WS_LANES, (size_t)num_x * sizeof(float4), &p));
+    IMP_TRY(workspace(ctx, WS_W, (size_t)num_k * ncoils * sizeof(float2), &p));
+    if (ncoils >= MFMA_MIN_RHS) {
+        const int tiles = ceil_div(ncoils, MF_COLS), n_steps = ceil_div(num_k, MF_K);
+        const long wgs = ceil_div(num_x, MF_WAVE_PTS * (NU_THREADS / 64));
+        const int chunks = pick_chunks(ctx, wgs, n_steps, 4 * MF_FOLD);
+        IMP_TRY(workspace(ctx, WS_MAXBITS, 256, &p));
+        IMP_TRY(workspace(ctx, WS_BPACK,
+                          (size_t)(n_steps + MF_BPAD) * tiles * 64 * sizeof(BPair), &p));
+        IMP_TRY(workspace(ctx, WS_PARTIAL, (size_t)chunks * tiles * 32 * num_x * sizeof(float),
+                          &p));
+    } else {
+        const int chunks = pick_chunks(ctx, ceil_div(num_x, NU_THREADS), num_k, 4 * NU_BLK);
+        IMP_TRY(workspace(ctx, WS_BPACK, (size_t)num_k * 2 * ncoils * sizeof(float), &p));
+        IMP_TRY(workspace(ctx, WS_PARTIAL, (size_t)chunks * num_x * sizeof(float2), &p));
+    }
+    return IMP_OK;
+}
+
 int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *kx,
                   const float *ky, const float *kz, const float *t, const float *x,
                   const float *y, const float *z, const float *fm,
@@ -1261,6 +1317,15 @@ int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
     if (!adjoint_args_ok(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, phi_r, phi_i, d_r, d_i,
                          s_r, s_i, out_r, out_i))
         return fail(IMP_EINVAL, "nudft_adjoint: bad arguments");
+    if (!(kz && z)) {
+        NuGeometry G;
+        IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, &G));
+        if (G.ok) {
+            IMP_TRY(reserve_direct(ctx, num_k, num_x, ncoils));
+            return nufft_adjoint(ctx, G, num_k, num_x, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
+                                 d_r, d_i, s_r, s_i, out_r, out_i);
+        }
+    }
     Scratch S{ctx};
     return adjoint_impl(ctx, S, true, num_k, num_x, ncoils, kx, ky, kz, t, x, y, z, fm, phi_r,
                         phi_i, d_r, d_i, s_r, s_i, out_r, out_i);

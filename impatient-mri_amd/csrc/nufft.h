@@ -1,0 +1,50 @@
+// Separable evaluation of the NUDFT on image grids (nufft.hip).
+#pragma once
+
+#include "common.h"
+
+#include <vector>
+
+namespace imp {
+
+// One image axis against the sample coordinate k it pairs with.
+struct NuAxis {
+    int n;            // image points
+    int L;            // transform length
+    int nf;           // spread-grid points (every sample's window fits)
+    int uniform;      // points are c0 + i d: read the bins, else interpolate
+    int flip;         // d < 0
+    int shift;        // grid point of bin 0, mod L
+    double kc;        // centre of k
+    double xc;        // centre of the points
+    double inv_d;     // grid cells per unit of k
+    double j0;        // grid point of kc
+};
+
+struct NuGeometry {
+    bool ok = false;
+    bool a_is_y = false;      // axis A (fastest in the voxel index) is y
+    NuAxis A{}, B{};
+    double tc = 0, th = 0;    // centre and half width of t, and of w
+    double wc = 0, wh = 0;
+    int nt = 0, nleg = 0;     // terms of e^{iwt}, Legendre coefficients of each
+    std::vector<double> coef, mul;
+};
+
+bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double> &mul, int *nt,
+                    int *nleg);
+
+int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                   const float *x, const float *y, const float *fm, NuGeometry *G);
+
+// Predicted time of nufft_adjoint in microseconds (for the choice against
+// the direct kernels).
+double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils);
+
+int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int n, int ncoils, const float *kx,
+                  const float *ky, const float *t, const float *x, const float *y,
+                  const float *fm, const float *phi_r, const float *phi_i, const float *d_r,
+                  const float *d_i, const float *s_r, const float *s_i, float *out_r,
+                  float *out_i);
+
+}  // namespace imp

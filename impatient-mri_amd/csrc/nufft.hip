@@ -1,0 +1,1732 @@
+// F^H d on image grids by wide-kernel spreading and FP64 line transforms.
+//
+//     out(r) = sum_c conj(S_c(r)) sum_k conj(phi_c(k)) d_c(k) e^{i(2pi k.r + w(r) t_k)}
+//
+// evaluated to rounding level without visiting every (sample, voxel) pair.
+// Three separations, each exact to about 1e-8 of the largest term (the
+// hardware sine of the direct kernel is good to 1.2e-7):
+//   time    e^{i w t} = sum_l mu_l psi_l(w) psi_l(t), psi_l the prolate
+//           spheroidal wave functions of the (w, t) rectangle the operands
+//           span (Slepian and Pollak 1961; computed in a Legendre basis as in
+//           Xiao, Rokhlin and Yarvin, Inverse Problems 17, 2001): the shortest
+//           such sum, nt terms, real factors;
+//   space   each sample is spread over NW x NW cells of a regular k grid with
+//           the Kaiser-Bessel kernel at 1.5x oversampling, the grid is summed
+//           onto the image axes one axis at a time and the kernel's transform
+//           divided out (nonuniform FFT of types 1 and 3: Dutt and Rokhlin
+//           1993, Greengard and Lee 2004, Lee and Greengard 2005);
+//   axes    the image points must form a tensor grid (checked on the device,
+//           bit for bit).  Uniform axes read the FFT's bins; others (for
+//           example (i - N/2)/N rounded to float with N no power of two)
+//           interpolate in the transformed line with the same kernel.
+// All sums, grids and transforms are FP64 (half the FP32 rate here), so the
+// result carries the rounding of its final FP32 store only.
+//
+// Layout.  Columns q = (l, c), l time term and c coil, are innermost in every
+// grid: grid[gB][gA][q] -> mid[ia][gB][q] -> image.  A is the image axis that
+// varies fastest in the voxel index.  Rows gB go through the spread and the
+// A transform in blocks, so the spread grid stays small.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <vector>
+
+#include "common.h"
+#include "fftcore.h"
+#include "nufft.h"
+
+namespace imp {
+
+namespace {
+
+using fftc::cmul;
+
+constexpr int NW = 12;           // kernel width in cells
+constexpr double NU_SIGMA = 1.5; // oversampling of both grids
+// KB shape for width 12 at 1.5x: pi NW (1 - 1/(2 sigma)), 1% lower (smallest
+// worst-case error over the band, 5e-9, by a scan of the factor)
+constexpr double NU_BETA = 0.99 * M_PI * NW * (1.0 - 1.0 / (2.0 * NU_SIGMA));
+constexpr double NU_TIME_TOL = 1e-8;   // largest error of the time expansion
+constexpr int NU_MAX_TERMS = 48;       // time terms above which the direct kernel runs
+                                       // (16 per lane, 3 groups of a 4-group wave)
+constexpr int NU_MAX_LEG = 160;        // Legendre coefficients per prolate function
+
+// ------------------------------------------------------------------ geometry
+// Words of the scan result (device and host).
+enum {
+    G_MIN = 0,        // kx, ky, t, x, y, w: smallest, as ordered integers
+    G_MAX = 6,        // largest
+    G_FCX = 12,       // first index where x / y differs from index 0
+    G_FCY,
+    G_FLAGS,          // 1: a voxel value is not finite, 2: not a tensor grid
+    G_DEVA,           // largest distance of an axis from uniform spacing (float bits)
+    G_DEVB,
+    G_A0, G_A1, G_B0, G_B1,   // first and last coordinate of each axis (float bits)
+    G_KFLAG,          // a sample value is not finite
+    G_WORDS = 32
+};
+
+__host__ __device__ inline unsigned enc_f(unsigned u) {
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+inline float dec_f(unsigned e) {
+    const unsigned u = (e & 0x80000000u) ? (e & 0x7fffffffu) : ~e;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
+inline float bits_f(unsigned u) {
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
+}
+
+// One block range scans the samples, the other the voxels; block results
+// [block][GB_WORDS] are reduced by k_geo_final (atomics on the few shared
+// words cost 0.2 ms at 512^2 x 393216).
+constexpr int GB_WORDS = 9;   // 3 min, 3 max, first change of a and b, flags
+
+__global__ __launch_bounds__(256) void k_geo_scan(int m, const float *kx, const float *ky,
+                                                  const float *t, int n, const float *x,
+                                                  const float *y, const float *fm, int kblocks,
+                                                  unsigned *part) {
+    const bool ks = (int)blockIdx.x < kblocks;
+    const float *a = ks ? kx : x, *b = ks ? ky : y, *c = ks ? t : fm;
+    const int cnt = ks ? m : n;
+    const int nb = ks ? kblocks : (int)gridDim.x - kblocks;
+    const int bi = ks ? blockIdx.x : blockIdx.x - kblocks;
+    unsigned w[GB_WORDS] = {~0u, ~0u, ~0u, 0u, 0u, 0u, (unsigned)cnt, (unsigned)cnt, 0u};
+    const float a0 = a[0], b0 = b[0];
+    for (int i = bi * 256 + threadIdx.x; i < cnt; i += nb * 256) {
+        const float v[3] = {a[i], b[i], c ? c[i] : 0.f};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (!isfinite(v[q])) w[8] = 1u;
+            const unsigned e = enc_f(__float_as_uint(v[q]));
+            w[q] = min(w[q], e);
+            w[3 + q] = max(w[3 + q], e);
+        }
+        if (v[0] != a0) w[6] = min(w[6], (unsigned)i);
+        if (v[1] != b0) w[7] = min(w[7], (unsigned)i);
+    }
+    __shared__ unsigned sm[4][GB_WORDS];
+#pragma unroll
+    for (int q = 0; q < GB_WORDS; ++q) {
+        const bool mx = (q >= 3 && q < 6) || q == 8;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned o = (unsigned)__shfl_xor((int)w[q], off, 64);
+            w[q] = mx ? max(w[q], o) : min(w[q], o);
+        }
+        if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6][q] = w[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < GB_WORDS) {
+        const int q = threadIdx.x;
+        const bool mx = (q >= 3 && q < 6) || q == 8;
+        unsigned v = sm[0][q];
+        for (int u = 1; u < 4; ++u) v = mx ? max(v, sm[u][q]) : min(v, sm[u][q]);
+        part[blockIdx.x * GB_WORDS + q] = v;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, const unsigned *part,
+                                                   unsigned *geo) {
+    // one wave per result word and block range
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int r = wave; r < 2 * GB_WORDS; r += 4) {
+        const int q = r % GB_WORDS;
+        const bool ks = r < GB_WORDS, mx = (q >= 3 && q < 6) || q == 8;
+        unsigned v = mx ? 0u : ~0u;
+        const int b0 = ks ? 0 : kblocks, nb = ks ? kblocks : xblocks;
+        for (int b = lane; b < nb; b += 64) {
+            const unsigned o = part[(b0 + b) * GB_WORDS + q];
+            v = mx ? max(v, o) : min(v, o);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned o = (unsigned)__shfl_xor((int)v, off, 64);
+            v = mx ? max(v, o) : min(v, o);
+        }
+        if (lane == 0) {
+            if (q < 3) geo[G_MIN + (ks ? 0 : 3) + q] = v;
+            else if (q < 6) geo[G_MAX + (ks ? 0 : 3) + q - 3] = v;
+            else if (q == 8) geo[ks ? G_KFLAG : G_FLAGS] = v;
+            else if (!ks) geo[q == 6 ? G_FCX : G_FCY] = v;
+        }
+    }
+    if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = 0u;
+}
+
+// Axis structure implied by the first changes: the coordinate that changes
+// first is axis A, its period nA.  false: none.
+__host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool *a_is_y,
+                                         int *nA) {
+    *a_is_y = false;
+    *nA = 0;
+    if (fcx == 1 && fcy > 1) {
+        *nA = (int)fcy;
+    } else if (fcy == 1 && fcx > 1) {
+        *a_is_y = true;
+        *nA = (int)fcx;
+    } else {
+        return false;
+    }
+    return n % *nA == 0;
+}
+
+__global__ void k_geo_check(int n, const float *x, const float *y, unsigned *geo) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    bool a_is_y;
+    int nA;
+    if (!geo_axes(geo[G_FCX], geo[G_FCY], n, &a_is_y, &nA)) {
+        if (i == 0) atomicOr(&geo[G_FLAGS], 2u);
+        return;
+    }
+    const float *a = a_is_y ? y : x, *b = a_is_y ? x : y;
+    const int ia = i % nA, nB = n / nA;
+    const bool ok = a[i] == a[ia] && b[i] == b[i - ia];
+    if (__ballot(!ok) && !ok) atomicOr(&geo[G_FLAGS], 2u);
+    if (i < nA) {
+        const double a0 = a[0], d = nA > 1 ? ((double)a[nA - 1] - a0) / (nA - 1) : 0.0;
+        const float dev = (float)(fabs((double)a[i] - (a0 + i * d)) * 1.000001);
+        if (dev > 0.f) atomicMax(&geo[G_DEVA], __float_as_uint(dev));
+    }
+    if (ia == 0) {
+        const int ib = i / nA;
+        const double b0 = b[0], d = nB > 1 ? ((double)b[(size_t)(nB - 1) * nA] - b0) / (nB - 1) : 0.0;
+        const float dev = (float)(fabs((double)b[i] - (b0 + ib * d)) * 1.000001);
+        if (dev > 0.f) atomicMax(&geo[G_DEVB], __float_as_uint(dev));
+    }
+    if (i == 0) {
+        geo[G_A0] = __float_as_uint(a[0]);
+        geo[G_A1] = __float_as_uint(a[nA - 1]);
+        geo[G_B0] = __float_as_uint(b[0]);
+        geo[G_B1] = __float_as_uint(b[(size_t)(nB - 1) * nA]);
+    }
+}
+
+// ------------------------------------------------------- prolate expansion
+// Eigenvectors of a symmetric tridiagonal matrix (diagonal d, off-diagonal
+// e[i] between i and i + 1) by implicit QL with Wilkinson shifts; z gets one
+// row per component.  Sorted ascending.
+bool tridiag_eig(std::vector<double> &d, std::vector<double> e, std::vector<double> &z) {
+    const int n = (int)d.size();
+    z.assign((size_t)n * n, 0.0);
+    for (int i = 0; i < n; ++i) z[(size_t)i * n + i] = 1.0;
+    e.resize(n, 0.0);
+    for (int l = 0; l < n; ++l) {
+        for (int it = 0;; ++it) {
+            int m = l;
+            while (m + 1 < n &&
+                   std::fabs(e[m]) > 1e-17 * (std::fabs(d[m]) + std::fabs(d[m + 1])))
+                ++m;
+            if (m == l) break;
+            if (it > 60) return false;
+            double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
+            double r = std::hypot(g, 1.0);
+            g = d[m] - d[l] + e[l] / (g + std::copysign(r, g));
+            double s = 1.0, c = 1.0, p = 0.0;
+            bool split = false;
+            for (int i = m - 1; i >= l; --i) {
+                double f = s * e[i];
+                const double b = c * e[i];
+                r = std::hypot(f, g);
+                e[i + 1] = r;
+                if (r == 0.0) {   // the matrix splits here
+                    d[i + 1] -= p;
+                    e[m] = 0.0;
+                    split = true;
+                    break;
+                }
+                s = f / r;
+                c = g / r;
+                g = d[i + 1] - p;
+                r = (d[i] - g) * s + 2.0 * c * b;
+                p = s * r;
+                d[i + 1] = g + p;
+                g = c * r - b;
+                for (int k = 0; k < n; ++k) {
+                    f = z[(size_t)k * n + i + 1];
+                    z[(size_t)k * n + i + 1] = s * z[(size_t)k * n + i] + c * f;
+                    z[(size_t)k * n + i] = c * z[(size_t)k * n + i] - s * f;
+                }
+            }
+            if (split) continue;
+            d[l] -= p;
+            e[l] = g;
+            e[m] = 0.0;
+        }
+    }
+    std::vector<int> o(n);
+    for (int i = 0; i < n; ++i) o[i] = i;
+    std::sort(o.begin(), o.end(), [&](int a, int b) { return d[a] < d[b]; });
+    std::vector<double> d2(n), z2((size_t)n * n);
+    for (int i = 0; i < n; ++i) {
+        d2[i] = d[o[i]];
+        for (int k = 0; k < n; ++k) z2[(size_t)k * n + i] = z[(size_t)k * n + o[i]];
+    }
+    d.swap(d2);
+    z.swap(z2);
+    return true;
+}
+
+}  // namespace
+
+// e^{i theta s u} = sum_l i^(l mod 2) m_l psi_l(s) psi_l(u) on [-1, 1]^2 (m_l
+// real, sign included; i for odd l), psi_l = sum_k coef[l][k] P_(2k + l%2);
+// the recurrence constants of prolate() follow the coefficients.
+// False when more than NU_MAX_TERMS terms are needed.
+bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double> &mul, int *nt,
+                    int *nleg) {
+    if (!(theta >= 0.0) || theta > 0.5 * M_PI * NU_MAX_TERMS) return false;
+    const int K = 2 * (((int)(0.75 * theta) + 36) / 2);   // Legendre degrees, both parities
+    const int H = K / 2;
+    if (K > NU_MAX_LEG) return false;
+    std::vector<double> z[2];
+    const double c2 = theta * theta;
+    for (int par = 0; par < 2; ++par) {
+        std::vector<double> d(H), e(H, 0.0);
+        for (int i = 0; i < H; ++i) {
+            const double k = 2 * i + par;
+            d[i] = k * (k + 1) + (2 * k * (k + 1) - 1) / ((2 * k + 3) * (2 * k - 1)) * c2;
+            e[i] = (k + 2) * (k + 1) / ((2 * k + 3) * std::sqrt((2 * k + 1) * (2 * k + 5))) * c2;
+        }
+        e[H - 1] = 0.0;
+        if (!tridiag_eig(d, e, z[par])) return false;
+    }
+    const int nmax = std::min(NU_MAX_TERMS + 1, K - 8);
+    std::vector<double> m(nmax), at1(nmax);
+    std::vector<double> c((size_t)nmax * H);
+    for (int l = 0; l < nmax; ++l) {
+        const int par = l & 1, col = l / 2;
+        double s1 = 0.0, v0 = 0.0, p = 1.0;
+        // P_k(0) for even k and P_k'(0) for odd k, by their recurrences:
+        // P_(k+2)(0) = -(k+1)/(k+2) P_k(0); P_(k+2)'(0) = -(k+2)/(k+1) P_k'(0)
+        for (int i = 0; i < H; ++i) {
+            const double k = 2 * i + par;
+            const double a = z[par][(size_t)i * H + col] * std::sqrt(k + 0.5);
+            c[(size_t)l * H + i] = a;
+            s1 += a;
+            v0 += a * p;
+            p *= par ? -(k + 2) / (k + 1) : -(k + 1) / (k + 2);
+        }
+        at1[l] = s1;
+        // int e^{i theta s u} psi(s) ds = mu psi(u), at u = 0 (its derivative
+        // for odd l); only the Legendre degree 0 (1) of psi integrates
+        const double a0 = c[(size_t)l * H];
+        if (par == 0)
+            m[l] = 2.0 * a0 / v0;
+        else
+            m[l] = theta * (2.0 / 3.0) * a0 / v0;
+    }
+    // tail beyond the kept terms, at the corner where it is largest
+    int keep = nmax;
+    double tail = 0.0;
+    while (keep > 1) {
+        const double next = tail + std::fabs(m[keep - 1]) * at1[keep - 1] * at1[keep - 1];
+        if (!(next < NU_TIME_TOL)) break;
+        tail = next;
+        --keep;
+    }
+    if (keep >= nmax) return false;
+    *nt = keep;
+    *nleg = H;
+    coef.assign(c.begin(), c.begin() + (size_t)keep * H);
+    // (k+1) P_(k+1) = (2k+1) u P_k - k P_(k-1) for the degrees 2i + 2, 2i + 3
+    for (int i = 0; i < H; ++i) {
+        const double k = 2 * i;
+        coef.push_back((2 * k + 3) / (k + 2));
+        coef.push_back((k + 1) / (k + 2));
+        coef.push_back((2 * k + 5) / (k + 3));
+        coef.push_back((k + 2) / (k + 3));
+    }
+    mul.assign(m.begin(), m.begin() + keep);
+    return true;
+}
+
+namespace {
+
+// -------------------------------------------------------------- device maths
+__device__ __forceinline__ double kb(double z) {
+    const double a = 1.0 - z * z * (4.0 / (NW * NW));
+    return a >= 0.0 ? cyl_bessel_i0(NU_BETA * sqrt(a)) : 0.0;
+}
+// kb on one cell of a window as a polynomial: a point NW/2 - 1 + g behind the
+// window's last whole cell, g in [0, 1], is NW/2 - 1 + g - c from cell c, and
+// kb there is a polynomial in x = 2 g - 1 (degree KB_DEG, fitted on the host
+// at Chebyshev nodes to 1e-14 of kb(0)).  An eighth of the work of I0.
+constexpr int KB_DEG = 12;
+constexpr int KB_WORDS = NW * (KB_DEG + 1);
+__device__ __forceinline__ double kb_cell(const double *poly, int cell, double x) {
+    const double *c = poly + cell * (KB_DEG + 1);
+    double v = c[KB_DEG];
+#pragma unroll
+    for (int d = KB_DEG - 1; d >= 0; --d) v = fma(v, x, c[d]);
+    return v;
+}
+
+const double *kb_poly_table() {
+    static const std::vector<double> table = [] {
+        std::vector<double> t(KB_WORDS);
+        constexpr int n = KB_DEG + 1;
+        for (int cell = 0; cell < NW; ++cell) {
+            double f[n], cheb[n], mono[n] = {}, tp[n] = {}, tc[n] = {};
+            for (int i = 0; i < n; ++i) {
+                const double z = 0.5 * NW - 1 + 0.5 * (std::cos(M_PI * (i + 0.5) / n) + 1) - cell;
+                f[i] = std::cyl_bessel_i(0.0, NU_BETA * std::sqrt(std::max(0.0, 1 - z * z * 4.0 / (NW * NW))));
+            }
+            for (int k = 0; k < n; ++k) {
+                double v = 0.0;
+                for (int i = 0; i < n; ++i) v += f[i] * std::cos(M_PI * k * (i + 0.5) / n);
+                cheb[k] = v * (k ? 2.0 : 1.0) / n;
+            }
+            // sum cheb[k] T_k in powers of x, T_(k+1) = 2 x T_k - T_(k-1)
+            tp[0] = 1.0;
+            tc[1] = 1.0;
+            for (int d = 0; d < n; ++d) mono[d] = cheb[0] * tp[d] + cheb[1] * tc[d];
+            for (int k = 2; k < n; ++k) {
+                double tn[n] = {};
+                for (int d = 0; d < n; ++d) tn[d] = (d ? 2.0 * tc[d - 1] : 0.0) - tp[d];
+                for (int d = 0; d < n; ++d) {
+                    mono[d] += cheb[k] * tn[d];
+                    tp[d] = tc[d];
+                    tc[d] = tn[d];
+                }
+            }
+            for (int d = 0; d < n; ++d) t[cell * n + d] = mono[d];
+        }
+        return t;
+    }();
+    return table.data();
+}
+
+// Fourier transform of kb at u cycles per cell; pi NW |u| < NU_BETA for
+// |u| <= 1/(2 sigma)
+__device__ __forceinline__ double kb_hat(double u) {
+    const double s = sqrt(NU_BETA * NU_BETA - (M_PI * NW * u) * (M_PI * NW * u));
+    return NW * sinh(s) / s;
+}
+
+// psi_l(u): Legendre sum over one parity.  rec holds, per pair of degrees,
+// the constants of P_(k+1) = a u P_k - b P_(k-1) (two steps).
+__device__ __forceinline__ double prolate(const double *coef, const double *rec, int nleg, int par,
+                                          double u) {
+    double p0 = 1.0, p1 = u, s = 0.0;   // P_k, P_(k+1), k = 2 i
+    for (int i = 0; i < nleg; ++i) {
+        s = fma(coef[i], par ? p1 : p0, s);
+        const double p2 = rec[4 * i] * (u * p1) - rec[4 * i + 1] * p0;
+        p1 = rec[4 * i + 2] * (u * p2) - rec[4 * i + 3] * p1;
+        p0 = p2;
+    }
+    return s;
+}
+
+__device__ __forceinline__ double clamp1(double u) { return fmin(1.0, fmax(-1.0, u)); }
+
+// first cell of a sample's window on one axis, and its position in cells
+__device__ __forceinline__ int window(const NuAxis &X, float k, double *s) {
+    *s = ((double)k - X.kc) * X.inv_d + X.j0;
+    const int b = (int)ceil(*s - 0.5 * NW);
+    return min(max(b, 0), X.nf - NW);
+}
+
+// ------------------------------------------------------------ sort by cell
+__global__ void k_nu_keys(int m, const float *kA, const float *kB, NuAxis A, NuAxis B, int *key,
+                          int *val) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= m) return;
+    double s;
+    const int a = window(A, kA[j], &s), b = window(B, kB[j], &s);
+    key[j] = b * (A.nf - NW + 1) + a;
+    val[j] = j;
+}
+
+// Stable LSD radix sort of (cell, sample), 8-bit digits: each wave owns
+// RX_WAVE consecutive elements, so ranks need no order between waves beyond
+// their histograms, and equal cells keep the sample order (every run sums in
+// the same order).
+constexpr int RX_BINS = 256, RX_WAVES = 4, RX_ROUNDS = 8;
+constexpr int RX_WAVE = 64 * RX_ROUNDS, RX_BLOCK = RX_WAVES * RX_WAVE;
+
+__global__ __launch_bounds__(256) void k_rx_count(const int *__restrict__ key, int m, int shift,
+                                                  int *__restrict__ hist) {
+    __shared__ int cnt[RX_BINS];
+    cnt[threadIdx.x] = 0;
+    __syncthreads();
+    for (int r = 0; r < RX_BLOCK / 256; ++r) {
+        const int i = blockIdx.x * RX_BLOCK + r * 256 + threadIdx.x;
+        if (i < m) atomicAdd(&cnt[(key[i] >> shift) & (RX_BINS - 1)], 1);
+    }
+    __syncthreads();
+    hist[blockIdx.x * RX_BINS + threadIdx.x] = cnt[threadIdx.x];
+}
+
+__global__ __launch_bounds__(256) void k_rx_scatter(const int *__restrict__ key,
+                                                    const int *__restrict__ val, int m, int shift,
+                                                    int nblk, const int *__restrict__ hist,
+                                                    int *__restrict__ key_out,
+                                                    int *__restrict__ val_out) {
+    __shared__ int cnt[RX_WAVES][RX_BINS];
+    __shared__ int wsum[RX_WAVES];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // first output position of this block's elements with digit threadIdx.x:
+    // all smaller digits, then the same digit in earlier blocks
+    int first = 0;
+    {
+        int total = 0, before = 0;
+#pragma unroll 16
+        for (int b = 0; b < nblk; ++b) {
+            const int c = hist[b * RX_BINS + threadIdx.x];
+            total += c;
+            before += b < (int)blockIdx.x ? c : 0;
+        }
+        int inc = total;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) wsum[wave] = inc;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) first += wsum[w];
+        first += inc - total + before;
+    }
+    for (int i = threadIdx.x; i < RX_WAVES * RX_BINS; i += 256) cnt[i / RX_BINS][i % RX_BINS] = 0;
+    __syncthreads();
+    const int base = blockIdx.x * RX_BLOCK + wave * RX_WAVE;
+    int k[RX_ROUNDS];
+#pragma unroll
+    for (int r = 0; r < RX_ROUNDS; ++r) {
+        const int i = base + r * 64 + lane;
+        k[r] = i < m ? key[i] : 0;
+        if (i < m) atomicAdd(&cnt[wave][(k[r] >> shift) & (RX_BINS - 1)], 1);
+    }
+    __syncthreads();
+    {   // per wave and bin: first output position
+        int run = first;
+#pragma unroll
+        for (int w = 0; w < RX_WAVES; ++w) {
+            const int c = cnt[w][threadIdx.x];
+            cnt[w][threadIdx.x] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll
+    for (int r = 0; r < RX_ROUNDS; ++r) {
+        const int i = base + r * 64 + lane;
+        const bool ok = i < m;
+        const int d = (k[r] >> shift) & (RX_BINS - 1);
+        unsigned long long same = __ballot(ok);   // lanes with this lane's digit
+#pragma unroll
+        for (int b = 0; b < 8; ++b) {
+            const unsigned long long set = __ballot((d >> b) & 1);
+            same &= ((d >> b) & 1) ? set : ~set;
+        }
+        int pos = 0;
+        if (ok) pos = cnt[wave][d] + __popcll(same & lt);
+        __builtin_amdgcn_wave_barrier();
+        if (ok) {
+            key_out[pos] = k[r];
+            val_out[pos] = val[i];
+            if ((same >> lane) == 1ull) cnt[wave][d] = pos + 1;   // the last lane of the digit
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// start[c] = first sorted sample whose cell is >= c, c = 0..ncells
+__global__ void k_nu_starts(int m, const int *key, int ncells, int *start) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c > ncells) return;
+    int lo = 0, hi = m;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (key[mid] < c) lo = mid + 1;
+        else hi = mid;
+    }
+    start[c] = lo;
+}
+
+// Per sorted sample: window start on A, kernel weights on both axes (zeros on
+// either side so a tile may read past the window), time factors.  A workgroup
+// fills PREP_S samples, one thread per table entry (coalesced stores).
+constexpr int PREP_S = 32;
+__global__ __launch_bounds__(256) void k_nu_prep(int m, const int *perm, const float *kA,
+                                                 const float *kB, const float *t, NuAxis A,
+                                                 NuAxis B, double tc, double tinv,
+                                                 const double *coef, const double *poly, int nt,
+                                                 int ntp, int nleg, int padA, int padB, int *bx,
+                                                 double *wx, double *wy, double *u) {
+    __shared__ double px[PREP_S], py[PREP_S], pt[PREP_S], pl[KB_WORDS];
+    const int s0 = blockIdx.x * PREP_S, ns = min(PREP_S, m - s0);
+    for (int i = threadIdx.x; i < KB_WORDS; i += 256) pl[i] = poly[i];
+    if ((int)threadIdx.x < ns) {
+        const int i = threadIdx.x, j = perm[s0 + i];
+        double p;
+        const int a = window(A, kA[j], &p);
+        px[i] = 2.0 * (p - a - (0.5 * NW - 1)) - 1.0;
+        bx[s0 + i] = a;
+        const int b = window(B, kB[j], &p);
+        py[i] = 2.0 * (p - b - (0.5 * NW - 1)) - 1.0;
+        pt[i] = clamp1(((double)t[j] - tc) * tinv);
+    }
+    __syncthreads();
+    const int nx = NW + 2 * padA, ny = NW + 2 * padB;
+    for (int e = threadIdx.x; e < ns * nx; e += 256) {
+        const int s = e / nx, g = e - s * nx - padA;
+        wx[(size_t)s0 * nx + e] = g >= 0 && g < NW ? kb_cell(pl, g, px[s]) : 0.0;
+    }
+    for (int e = threadIdx.x; e < ns * ny; e += 256) {
+        const int s = e / ny, g = e - s * ny - padB;
+        wy[(size_t)s0 * ny + e] = g >= 0 && g < NW ? kb_cell(pl, g, py[s]) : 0.0;
+    }
+    for (int e = threadIdx.x; e < ns * ntp; e += 256) {
+        const int s = e / ntp, l = e - s * ntp;
+        u[(size_t)s0 * ntp + e] =
+            l < nt ? prolate(coef + (size_t)l * nleg, coef + (size_t)nt * nleg, nleg, l & 1, pt[s])
+                   : 0.0;
+    }
+}
+
+// Sample weights conj(phi) d e^{i(2pi (kA - kcA) xcA + ... + wc (t - tc))},
+// [sample][coil slot] FP64 pairs, zero in the slots beyond the group.
+constexpr int WD_S = 64;
+__global__ __launch_bounds__(256) void k_nu_data(int m, int c0, int nc, int slots,
+                                                 const float *kA, const float *kB,
+                                                 const float *t, NuAxis A, NuAxis B, double tc,
+                                                 double wc_cyc, const float *phi_r,
+                                                 const float *phi_i, const float *d_r,
+                                                 const float *d_i, double2 *wd) {
+    __shared__ double2 rot[WD_S];
+    __shared__ double2 tile[8][WD_S + 1];
+    const int j0 = blockIdx.x * WD_S, tj = threadIdx.x & (WD_S - 1), tc4 = threadIdx.x / WD_S;
+    if (threadIdx.x < WD_S) {
+        const int j = min(j0 + (int)threadIdx.x, m - 1);
+        const double rev = ((double)kA[j] - A.kc) * A.xc + ((double)kB[j] - B.kc) * B.xc +
+                           ((double)t[j] - tc) * wc_cyc;
+        double s, c;
+        sincospi(2.0 * (rev - rint(rev)), &s, &c);
+        rot[threadIdx.x] = make_double2(c, s);
+    }
+    __syncthreads();
+    for (int cb = 0; cb < slots; cb += 8) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int c = cb + tc4 + 4 * h, j = j0 + tj;
+            double2 v = make_double2(0.0, 0.0);
+            if (c < nc && j < m) {
+                const size_t o = (size_t)(c0 + c) * m + j;
+                double re = d_r[o], im = d_i[o];
+                if (phi_r) {
+                    const double pr = phi_r[o], pi = phi_i[o], x = pr * re + pi * im;
+                    im = pr * im - pi * re;
+                    re = x;
+                }
+                v = cmul(make_double2(re, im), rot[tj]);
+            }
+            tile[tc4 + 4 * h][tj] = v;
+        }
+        __syncthreads();
+        const int nw = min(8, slots - cb);
+        for (int e = threadIdx.x; e < WD_S * nw; e += 256) {
+            const int j = e / nw, c = e % nw;
+            if (j0 + j < m) wd[(size_t)(j0 + j) * slots + cb + c] = tile[c][j];
+        }
+        __syncthreads();
+    }
+}
+
+// ------------------------------------------------------------------- spread
+// Tile: `T` cells along A on `yg` rows of one row block.  Work entries split
+// a tile's visits (sample, row) into runs of at most the chunk length the
+// count pass settled on; a tile with several runs sums them from slots.
+constexpr int SP_CH0 = 128;        // shortest chunk, visits
+constexpr int SP_LEVELS = 12;      // chunk lengths SP_CH0 << level
+constexpr int SP_SLOTS = 8192;     // partial tiles a row block may use
+
+struct SpEntry {
+    int tile, v0, v1, slot;
+};
+struct SpMulti {
+    int tile, slot, n, pad;
+};
+// Per row block counters: entries, slots, multi-run tiles, slot demand per level
+struct SpCount {
+    int entries, slots, multis, pad;
+    int need[SP_LEVELS];
+};
+
+struct SpGeom {
+    int T, yg, rb;          // tile cells, rows, rows per block (multiple of yg)
+    int ntx, nty;           // tiles along A, tile rows per block
+    int ncA, ncB;           // cells (window starts) per axis
+    int nfA, nfB;
+    int entry_cap;          // per row block
+};
+
+__device__ __forceinline__ int row_range(const SpGeom &G, const int *start, int gy0, int gx0,
+                                         int row, int *s0) {
+    const int by = gy0 - (NW - 1) + row;
+    *s0 = 0;
+    if (by < 0 || by >= G.ncB || gy0 >= G.nfB) return 0;
+    const int lo = max(0, gx0 - (NW - 1)), hi = min(G.ncA - 1, gx0 + G.T - 1);
+    if (lo > hi) return 0;
+    *s0 = start[by * G.ncA + lo];
+    return start[by * G.ncA + hi + 1] - *s0;
+}
+
+__device__ __forceinline__ int tile_visits(const SpGeom &G, const int *start, int block,
+                                           int tile) {
+    const int gy0 = block * G.rb + (tile / G.ntx) * G.yg, gx0 = (tile % G.ntx) * G.T;
+    int n = 0, s0;
+    for (int r = 0; r < NW + G.yg - 1; ++r) n += row_range(G, start, gy0, gx0, r, &s0);
+    return n;
+}
+
+__global__ void k_sp_zero(int *v, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) v[i] = 0;
+}
+
+__global__ __launch_bounds__(256) void k_sp_count(SpGeom G, const int *start, int *visits,
+                                                  SpCount *cnt) {
+    __shared__ int need[SP_LEVELS];
+    if (threadIdx.x < SP_LEVELS) need[threadIdx.x] = 0;
+    __syncthreads();
+    const int tile = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
+    const int ntile = G.ntx * G.nty;
+    if (tile < ntile) {
+        const int n = tile_visits(G, start, block, tile);
+        visits[(size_t)block * ntile + tile] = n;
+        if (n > SP_CH0) {
+#pragma unroll
+            for (int k = 0; k < SP_LEVELS; ++k) {
+                const int ch = SP_CH0 << k;
+                if (n > ch) atomicAdd(&need[k], (n + ch - 1) / ch);
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < SP_LEVELS && need[threadIdx.x])
+        atomicAdd(&cnt[block].need[threadIdx.x], need[threadIdx.x]);
+}
+
+// The chunk length is the shortest whose slot demand fits, so it depends on
+// the operands only; which slot a run gets does not change what is summed.
+__global__ __launch_bounds__(256) void k_sp_list(SpGeom G, const int *visits, SpCount *cnt,
+                                                 SpEntry *entries, SpMulti *multis) {
+    const int tile = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
+    const int ntile = G.ntx * G.nty;
+    if (tile >= ntile) return;
+    SpCount &C = cnt[block];
+    int level = 0;
+    while (level < SP_LEVELS && C.need[level] > SP_SLOTS) ++level;
+    const int n = visits[(size_t)block * ntile + tile];
+    const int ch = level < SP_LEVELS ? SP_CH0 << level : 0x7fffffff;
+    const int runs = n > ch ? (n + ch - 1) / ch : 1;
+    const int e0 = atomicAdd(&C.entries, runs);
+    SpEntry *E = entries + (size_t)block * G.entry_cap + e0;
+    if (runs == 1) {
+        E[0] = SpEntry{tile, 0, n, -1};
+        return;
+    }
+    const int s0 = atomicAdd(&C.slots, runs);
+    const int m0 = atomicAdd(&C.multis, 1);
+    multis[(size_t)block * SP_SLOTS + m0] = SpMulti{tile, s0, runs, 0};
+    for (int r = 0; r < runs; ++r) E[r] = SpEntry{tile, r * ch, min(n, (r + 1) * ch), s0 + r};
+}
+
+typedef const __attribute__((address_space(4))) double *cdbl;
+typedef const __attribute__((address_space(4))) int *cint;
+
+struct SpArgs {
+    SpGeom G;
+    int r0, block;             // first grid row of the block, its index
+    int nt, ntp, nc;           // time terms, padded, coils
+    int lc, ll;                // log2 of coil slots and time groups in a wave
+    const int *start, *perm, *bx;
+    const double *wx, *wy, *u;
+    const double *wd;          // [sample][2 slots]
+    const SpCount *cnt;
+    const SpEntry *entries;
+    const SpMulti *multis;
+    double *part;              // [slot][NL * T][64]
+    double *grid;              // [row in block][nfA][nt * nc][2]
+};
+
+template <int NL, int T>
+__device__ __forceinline__ void sp_store(const SpArgs &P, int tile, int lane,
+                                         const double (&acc)[NL][T]) {
+    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
+    const int lg = (lane >> (1 + P.lc)) & ((1 << P.ll) - 1), yg = lane >> (1 + P.lc + P.ll);
+    const int row = (tile / P.G.ntx) * P.G.yg + yg, gx0 = (tile % P.G.ntx) * T;
+    if (c >= P.nc || row >= P.G.rb || P.r0 + row >= P.G.nfB) return;
+    double *out = P.grid + (((size_t)row * P.G.nfA + gx0) * P.nt * P.nc + c) * 2 + part;
+    const size_t sx = (size_t)P.nt * P.nc * 2, sl = (size_t)P.nc * 2;
+#pragma unroll
+    for (int i = 0; i < T; ++i) {
+#pragma unroll
+        for (int k = 0; k < NL; ++k) {
+            const int l = lg * NL + k;
+            if (gx0 + i < P.G.nfA && l < P.nt) out[i * sx + l * sl] = acc[k][i];
+        }
+    }
+}
+
+// One wave sums one entry.  Lanes are (re/im, coil, time group, row); each
+// holds NL time terms x T cells in FP64 registers, so a visit costs NL + 1
+// products and NL T FMAs per lane against one weight load per lane and one
+// set of wave-uniform kernel weights (scalar registers).  Visits are listed
+// 64 at a time (lane v finds its row and sample), then run two at a time from
+// alternating register sets: a set is loaded while the other is consumed.
+// All scalar loads of a set are waited for before the next set's are issued,
+// since scalar loads return in any order.
+template <int NL, int T, bool UNI>
+struct SpSet {
+    double wx[T], wy, w;
+    double u[NL];
+};
+
+template <int NL, int T, bool UNI>
+__global__ __launch_bounds__(64) void k_spread(SpArgs P) {
+    const int lane = threadIdx.x;
+    const int wave = blockIdx.x, nwaves = gridDim.x;
+    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
+    const int lg = UNI ? 0 : (lane >> (1 + P.lc)) & ((1 << P.ll) - 1);
+    const int yl = UNI ? 0 : lane >> (1 + P.lc + P.ll);
+    const int slots2 = 2 << P.lc, wdo = 2 * c + part;
+    const int nx = NW + 2 * (T - 1), ny = NW + 2 * (P.G.yg - 1);
+    const int rows = NW + P.G.yg - 1;
+    const int ne = ((cint)(const int *)&P.cnt[P.block])[0];
+    using Set = SpSet<NL, T, UNI>;
+    for (int e = wave; e < ne; e += nwaves) {
+        const cint ep = (cint)(const int *)(P.entries + (size_t)P.block * P.G.entry_cap + e);
+        const int tile = ep[0], v0 = ep[1], v1 = ep[2], slot = ep[3];
+        const int gy0 = P.r0 + (tile / P.G.ntx) * P.G.yg, gx0 = (tile % P.G.ntx) * T;
+        double acc[NL][T];
+#pragma unroll
+        for (int k = 0; k < NL; ++k)
+#pragma unroll
+            for (int i = 0; i < T; ++i) acc[k][i] = 0.0;
+        // lane r holds the sample range of row r
+        int rs = 0, rn = 0;
+        if (lane < rows) rn = row_range(P.G, P.start, gy0, gx0, lane, &rs);
+        for (int vb = v0; vb < v1; vb += 64) {
+            const int nb = min(64, v1 - vb);
+            // visit vb + lane: its row and sample
+            int row = 0, smp = -1, base = 0;
+            for (int r = 0; r < rows; ++r) {
+                const int n = __builtin_amdgcn_readlane(rn, r);
+                const int o = vb + lane - base;
+                if (o >= 0 && o < n) {
+                    row = r;
+                    smp = __builtin_amdgcn_readlane(rs, r) + o;
+                }
+                base += n;
+            }
+            int va = 0, vj = 0;
+            smp = max(smp, 0);
+            if (lane < nb) {
+                va = P.bx[smp];
+                vj = P.perm[smp];
+            }
+            // offset of the tile's first cell in the sample's padded window
+            const int vx = gx0 - va + T - 1;
+            auto load = [&](int i, Set &S) {
+                const int s = __builtin_amdgcn_readlane(smp, i);
+                const int j = __builtin_amdgcn_readlane(vj, i);
+                const int ox = __builtin_amdgcn_readlane(vx, i);
+                // row by = gy0 - (NW - 1) + r: this lane's row takes weight
+                // gy0 + yl - by of the window
+                const int iy = NW - 1 - __builtin_amdgcn_readlane(row, i) + P.G.yg - 1;
+                S.w = P.wd[(size_t)j * slots2 + wdo];
+                const cdbl px = (cdbl)P.wx + ((size_t)s * nx + ox);
+#pragma unroll
+                for (int q = 0; q < T; ++q) S.wx[q] = px[q];
+                if constexpr (UNI) {
+                    S.wy = ((cdbl)P.wy)[(size_t)s * ny + iy];
+#pragma unroll
+                    for (int k = 0; k < NL; ++k) S.u[k] = ((cdbl)P.u)[(size_t)s * P.ntp + k];
+                } else {
+                    S.wy = P.wy[(size_t)s * ny + iy + yl];
+                    const double *pu = P.u + ((size_t)s * P.ntp + lg * NL);
+#pragma unroll
+                    for (int k = 0; k < NL; ++k) S.u[k] = pu[k];
+                }
+            };
+            auto use = [&](const Set &S) {
+                const double v = S.w * S.wy;
+#pragma unroll
+                for (int k = 0; k < NL; ++k) {
+                    const double vu = v * S.u[k];
+#pragma unroll
+                    for (int q = 0; q < T; ++q) acc[k][q] = fma(vu, S.wx[q], acc[k][q]);
+                }
+            };
+            // scalar loads issued so far have arrived
+            auto arrived = [] {
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            Set s0, s1;
+            load(0, s0);
+            // an odd count runs its last visit again with weight zero: one
+            // loop and no copies of the accumulators
+            for (int i = 0; i < nb; i += 2) {
+                arrived();
+                load(min(i + 1, nb - 1), s1);
+                __builtin_amdgcn_sched_barrier(0);
+                use(s0);
+                arrived();
+                if (i + 1 >= nb) s1.wy = 0.0;
+                load(min(i + 2, nb - 1), s0);
+                __builtin_amdgcn_sched_barrier(0);
+                use(s1);
+            }
+        }
+        if (slot < 0) {
+            sp_store<NL, T>(P, tile, lane, acc);
+        } else {
+            double *o = P.part + (size_t)slot * NL * T * 64 + lane;
+#pragma unroll
+            for (int k = 0; k < NL; ++k)
+#pragma unroll
+                for (int i = 0; i < T; ++i) o[(k * T + i) * 64] = acc[k][i];
+        }
+    }
+}
+
+// tiles summed in several runs: one wave per (tile, time term) adds the runs
+// in order
+template <int NL, int T>
+__global__ __launch_bounds__(256) void k_spread_multi(SpArgs P) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
+    const int lg = (lane >> (1 + P.lc)) & ((1 << P.ll) - 1), yg = lane >> (1 + P.lc + P.ll);
+    const int n = P.cnt[P.block].multis * NL;
+    for (int e = wave; e < n; e += gridDim.x * 4) {
+        const SpMulti M = P.multis[(size_t)P.block * SP_SLOTS + e / NL];
+        const int k = e % NL;
+        double acc[T];
+#pragma unroll
+        for (int i = 0; i < T; ++i) acc[i] = 0.0;
+        const double *o = P.part + ((size_t)M.slot * NL + k) * T * 64 + lane;
+#pragma unroll 2
+        for (int r = 0; r < M.n; ++r, o += NL * T * 64)
+#pragma unroll
+            for (int i = 0; i < T; ++i) acc[i] += o[i * 64];
+        const int row = (M.tile / P.G.ntx) * P.G.yg + yg, gx0 = (M.tile % P.G.ntx) * T;
+        const int l = lg * NL + k;
+        if (c >= P.nc || row >= P.G.rb || P.r0 + row >= P.G.nfB || l >= P.nt) continue;
+        double *g = P.grid +
+                    ((((size_t)row * P.G.nfA + gx0) * P.nt + l) * P.nc + c) * 2 + part;
+#pragma unroll
+        for (int i = 0; i < T; ++i)
+            if (gx0 + i < P.G.nfA) g[(size_t)i * P.nt * P.nc * 2] = acc[i];
+    }
+}
+
+// tile shape for nl time terms per lane: about 48 FP64 accumulators
+constexpr int sp_cells(int nl) { return nl >= 13 ? 3 : nl >= 10 ? 4 : nl >= 8 ? 6 : nl == 7 ? 7
+                                        : nl == 6 ? 8 : nl == 5 ? 10 : nl == 4 ? 12 : 16; }
+
+using SpFn = void (*)(SpArgs);
+template <int NL>
+SpFn sp_pick1(bool uni) {
+    return uni ? (SpFn)k_spread<NL, sp_cells(NL), true> : (SpFn)k_spread<NL, sp_cells(NL), false>;
+}
+template <int NL>
+SpFn sp_multi1() { return (SpFn)k_spread_multi<NL, sp_cells(NL)>; }
+
+template <class F>
+auto sp_switch(int nl, F f) {
+    switch (nl) {
+        case 1: return f(std::integral_constant<int, 1>{});
+        case 2: return f(std::integral_constant<int, 2>{});
+        case 3: return f(std::integral_constant<int, 3>{});
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 5: return f(std::integral_constant<int, 5>{});
+        case 6: return f(std::integral_constant<int, 6>{});
+        case 7: return f(std::integral_constant<int, 7>{});
+        case 8: return f(std::integral_constant<int, 8>{});
+        case 9: return f(std::integral_constant<int, 9>{});
+        case 10: return f(std::integral_constant<int, 10>{});
+        case 11: return f(std::integral_constant<int, 11>{});
+        case 12: return f(std::integral_constant<int, 12>{});
+        case 13: return f(std::integral_constant<int, 13>{});
+        case 14: return f(std::integral_constant<int, 14>{});
+        case 15: return f(std::integral_constant<int, 15>{});
+        default: return f(std::integral_constant<int, 16>{});
+    }
+}
+constexpr int SP_MAX_NL = 16;
+
+// ---------------------------------------------------------- line transforms
+// FP64 Stockham lines: E values per thread, lines interleaved in LDS
+// [position][line] (columns q are contiguous in memory, so a wave's loads of
+// one element cover LINES x 16 bytes), re and im exchanged in turn to halve
+// the LDS.
+namespace ln {
+__host__ __device__ constexpr bool has3(int L) { return L % 3 == 0; }
+__host__ __device__ constexpr int vals(int L) { return has3(L) ? 12 : 8; }
+__host__ __device__ constexpr int threads(int L) { return L / vals(L); }
+// lines of a workgroup of up to wg threads
+__host__ __device__ constexpr int lines(int L, int wg) {
+    int n = 64;
+    while (n > 1 && n * threads(L) > wg) n /= 2;
+    return n;
+}
+__host__ __device__ constexpr int bits(int n) { return n <= 1 ? 0 : 1 + bits(n / 2); }
+__host__ __device__ constexpr int stages(int L) {
+    return has3(L) ? 1 + (bits(L / 12) + 1) / 2 : (bits(L) + 2) / 3;
+}
+__host__ __device__ constexpr int radix(int L, int s) {
+    return has3(L) ? (s == 0 ? 12 : (bits(L / 12) - 2 * (s - 1) >= 2 ? 4 : 2))
+                   : (bits(L) - 3 * s >= 3 ? 8 : 1 << (bits(L) - 3 * s));
+}
+__host__ __device__ constexpr int span(int L, int s) {
+    return s == 0 ? 1 : span(L, s - 1) * radix(L, s - 1);
+}
+__host__ __device__ constexpr int pad(int L, int i) { return i + i / vals(L); }
+__host__ __device__ constexpr int words(int L, int P) { return (L + L / vals(L)) * P; }
+
+// element index of register (b, r) before / after stage S
+template <int L, int S>
+__device__ __forceinline__ int in_idx(int t, int b, int r) {
+    return t + threads(L) * b + r * (L / radix(L, S));
+}
+template <int L, int S>
+__device__ __forceinline__ int out_idx(int t, int b, int r) {
+    constexpr int R = radix(L, S), NS = span(L, S);
+    const int j = t + threads(L) * b, k = NS > 1 ? j % NS : 0;
+    return (j - k) * R + k + r * NS;
+}
+
+template <int L, int S>
+__device__ __forceinline__ void butterflies(double2 (&v)[vals(L)], int t, const double2 *tw) {
+    constexpr int R = radix(L, S), NS = span(L, S), NB = vals(L) / R;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if constexpr (NS > 1) {
+            const int k = (t + threads(L) * b) % NS, step = (L / (NS * R)) * k;
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[b * R + r] = cmul(v[b * R + r], tw[r * step]);
+        }
+        fftc::dft<R, true>(&v[b * R]);
+    }
+}
+
+template <int L, int S, int P>
+__device__ __forceinline__ void exchange(double2 (&v)[vals(L)], int t, int c, double *buf) {
+    constexpr int R = radix(L, S), NB = vals(L) / R;
+    constexpr int R2 = radix(L, S + 1), NB2 = vals(L) / R2;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                buf[pad(L, out_idx<L, S>(t, b, r)) * P + c] = h ? v[b * R + r].y : v[b * R + r].x;
+        __syncthreads();
+        double x[vals(L)];
+#pragma unroll
+        for (int b = 0; b < NB2; ++b)
+#pragma unroll
+            for (int r = 0; r < R2; ++r) x[b * R2 + r] = buf[pad(L, in_idx<L, S + 1>(t, b, r)) * P + c];
+#pragma unroll
+        for (int i = 0; i < vals(L); ++i) {
+            if (h) v[i].y = x[i];
+            else v[i].x = x[i];
+        }
+    }
+}
+
+// inverse DFT (e^{+i}) of a line held as in_idx<L, 0>; tw[m] = e^{+2 pi i m / L}
+template <int L, int P, int S = 0>
+__device__ __forceinline__ void transform(double2 (&v)[vals(L)], int t, int c, double *buf,
+                                          const double2 *tw) {
+    butterflies<L, S>(v, t, tw);
+    if constexpr (S + 1 < stages(L)) {
+        exchange<L, S, P>(v, t, c, buf);
+        transform<L, P, S + 1>(v, t, c, buf, tw);
+    }
+}
+}  // namespace ln
+
+// One axis' tables: twiddles [L], input scale [nf] (nonuniform axes) and
+// output weights: [n] (uniform) or [n][NW] with window starts base[n].
+__global__ void k_nu_axis(NuAxis X, const float *coord, int cstride, double2 *tw, double *inw,
+                          double *outw, int *base) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < X.L) {
+        double s, c;
+        sincospi(2.0 * i / X.L, &s, &c);
+        tw[i] = make_double2(c, s);
+    }
+    if (!X.uniform && i < X.nf) inw[i] = 1.0 / kb_hat((i - X.j0) / X.L);
+    if (i < X.n) {
+        if (X.uniform) {
+            outw[i] = 1.0 / kb_hat((double)(i - X.n / 2) / X.L);
+        } else {
+            const double u = ((double)coord[(size_t)i * cstride] - X.xc) / X.inv_d;  // cycles/cell
+            const double p = u * X.L, h = kb_hat(u);
+            const int b = (int)ceil(p - 0.5 * NW);
+            base[i] = b;
+            for (int k = 0; k < NW; ++k) outw[(size_t)i * NW + k] = kb(p - (b + k)) / h;
+        }
+    }
+}
+
+// threads per workgroup: whole 128-byte row segments for the storing pass;
+// the combining pass, whose accumulators leave 3 waves per SIMD, runs
+// smaller ones so that several share a CU
+constexpr int ST_WG = 256, CO_WG = 256;
+
+struct LineArgs {
+    const double2 *in;          // element j of line x, column q: in[x in_line + j in_el + q]
+    size_t in_line;
+    unsigned in_el;
+    int nq, nlines;             // columns, lines
+    NuAxis X;
+    const double2 *tw;
+    const double *inw, *outw;
+    const int *base;
+};
+
+// Loads element i (mod L) of a line: grid points j = i + j0 mod L, folded on
+// uniform axes (there the grid is L-periodic exactly) and scaled on others.
+// base is wave-uniform and the lane offsets are 32 bits wide (a line's
+// elements span far less than 4 GB): one address register per element.
+template <bool UNI>
+__device__ __forceinline__ double2 line_load(const LineArgs &P, const double2 *base, unsigned c,
+                                             int L, int i) {
+    double2 s = make_double2(0.0, 0.0);
+    int j = i + P.X.shift;
+    if (j >= L) j -= L;
+    if constexpr (UNI) {
+        for (; j < P.X.nf; j += L) {
+            const double2 v = base[(unsigned)j * P.in_el + c];
+            s.x += v.x;
+            s.y += v.y;
+        }
+    } else if (j < P.X.nf) {
+        const double2 v = base[(unsigned)j * P.in_el + c];
+        const double w = P.inw[j];
+        s = make_double2(v.x * w, v.y * w);
+    }
+    return s;
+}
+
+// bin of an L-point transform -> image index on a uniform axis (or >= n)
+__device__ __forceinline__ unsigned bin_index(const NuAxis &X, int L, int i) {
+    const int f = i < L / 2 ? i : i - L;
+    return (unsigned)((X.flip ? -f : f) + X.n / 2);
+}
+
+// Interpolated values of the thread's outputs o = t + T m (nonuniform axes).
+template <int L, int W>
+__device__ __forceinline__ void line_interp(const LineArgs &P, double2 (&v)[ln::vals(L)], int t,
+                                            int c, double *buf, double2 (&o)[ln::vals(L)]) {
+    constexpr int E = ln::vals(L), T = ln::threads(L), S = ln::stages(L) - 1;
+    constexpr int R = ln::radix(L, S), NB = E / R;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        __syncthreads();
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                buf[ln::pad(L, ln::out_idx<L, S>(t, b, r)) * W + c] =
+                    h ? v[b * R + r].y : v[b * R + r].x;
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < E; ++m) {
+            const int i = t + T * m;
+            double s = 0.0;
+            if (i < P.X.n) {
+                const int b = P.base[i];
+                const double *w = P.outw + (size_t)i * NW;
+#pragma unroll 2
+                for (int k = 0; k < NW; ++k) {
+                    int p = b + k;
+                    p += p < 0 ? L : 0;
+                    s = fma(w[k], buf[ln::pad(L, p) * W + c], s);
+                }
+            }
+            if (h) o[m].y = s;
+            else o[m].x = s;
+        }
+    }
+}
+
+// One axis of a grid: out[i out_el + line out_line + q].
+template <int L, bool UNI>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG)) void k_line_store(
+    LineArgs P, double2 *out, size_t out_line, size_t out_el) {
+    constexpr int E = ln::vals(L), W = ln::lines(L, ST_WG), T = ln::threads(L);
+    __shared__ double buf[ln::words(L, W)];
+    const int c = threadIdx.x % W, t = threadIdx.x / W;
+    const int np = (P.nq + W - 1) / W;
+    // workgroups go round the 8 XCDs: b and b + 8 (one XCD) take adjacent
+    // panels, which share 128-byte rows in that XCD's L2
+    const int b = (blockIdx.x & ~15) | ((blockIdx.x & 7) << 1) | ((blockIdx.x >> 3) & 1);
+    const int line = b / np, q = (b % np) * W + c;
+    if (line >= P.nlines) return;
+    const bool ok = q < P.nq;
+    const double2 *base = P.in + (size_t)line * P.in_line + (q - c);
+    double2 v[E];
+    constexpr int R0 = ln::radix(L, 0);
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        v[i] = ok ? line_load<UNI>(P, base, c, L, ln::in_idx<L, 0>(t, i / R0, i % R0)) : make_double2(0., 0.);
+    ln::transform<L, W>(v, t, c, buf, P.tw);
+    double2 *o = out + (size_t)line * out_line + q;
+    if constexpr (UNI) {
+        constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(t, i / R, i % R));
+            if (ok && x < (unsigned)P.X.n) {
+                const double w = P.outw[x];
+                o[x * out_el] = make_double2(v[i].x * w, v[i].y * w);
+            }
+        }
+    } else {
+        double2 x[E];
+        line_interp<L, W>(P, v, t, c, buf, x);
+#pragma unroll
+        for (int m = 0; m < E; ++m) {
+            const int i = t + T * m;
+            if (ok && i < P.X.n) o[i * out_el] = x[m];
+        }
+    }
+}
+
+// Last axis with the time and coil sums: line = ia, out over ib.
+// partial[split][ia][ib] = sum over the split's columns of
+// i^(l mod 2) vt[l] conj(S_c) P_(l,c).
+template <int L, bool UNI>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_line_combine(
+    LineArgs P, int ncg, int splits, const double *vt, const float2 *sens, unsigned nvox,
+    double2 *partial) {
+    constexpr int E = ln::vals(L), W = ln::lines(L, CO_WG), T = ln::threads(L);
+    __shared__ double buf[ln::words(L, W)];
+    const int c = threadIdx.x % W, t = threadIdx.x / W;
+    const int np = (P.nq + W - 1) / W;
+    const int line = blockIdx.x / splits, split = blockIdx.x % splits;
+    const int p0 = (int)((long)np * split / splits), p1 = (int)((long)np * (split + 1) / splits);
+    constexpr int R0 = ln::radix(L, 0), S = ln::stages(L) - 1, R = ln::radix(L, S);
+    double2 acc[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) acc[i] = make_double2(0.0, 0.0);
+    const double *vline = vt + (size_t)line * P.X.n;
+    const float2 *sline = sens ? sens + (size_t)line * P.X.n : nullptr;
+    // offsets within vt and sens stay below 2^32 bytes (checked at launch)
+    auto add = [&](int i, unsigned x, double2 p, unsigned vo, unsigned so, bool odd) {
+        if (sens) {
+            const float2 s = sline[so + x];
+            p = make_double2(p.x * s.x + p.y * s.y, p.y * s.x - p.x * s.y);
+        }
+        const double f = vline[vo + x];
+        acc[i].x = fma(f, odd ? -p.y : p.x, acc[i].x);
+        acc[i].y = fma(f, odd ? p.x : p.y, acc[i].y);
+    };
+    for (int p = p0; p < p1; ++p) {
+        // opaque to the optimizer: the LDS and element indices are recomputed
+        // per panel instead of being held in registers across panels (spills)
+        int tp = t;
+        asm volatile("" : "+v"(tp));
+        const int q = p * W + c;
+        const bool ok = q < P.nq;
+        const int l = ok ? q / ncg : 0, cc = ok ? q - l * ncg : 0;
+        const double2 *base = P.in + (size_t)line * P.in_line + p * W;
+        double2 v[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+            v[i] = ok ? line_load<UNI>(P, base, c, L, ln::in_idx<L, 0>(tp, i / R0, i % R0))
+                      : make_double2(0., 0.);
+        ln::transform<L, W>(v, tp, c, buf, P.tw);
+        const unsigned vo = (unsigned)l * nvox, so = (unsigned)cc * nvox;
+        if constexpr (UNI) {
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(tp, i / R, i % R));
+                if (ok && x < (unsigned)P.X.n) add(i, x, v[i], vo, so, l & 1);
+            }
+        } else {
+            double2 o[E];
+            line_interp<L, W>(P, v, tp, c, buf, o);
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+                if (ok && tp + T * m < P.X.n) add(m, tp + T * m, o[m], vo, so, l & 1);
+        }
+    }
+    double2 *out = partial + (size_t)split * nvox + (size_t)line * P.X.n;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        double2 a = acc[i];
+#pragma unroll
+        for (int off = W / 2; off > 0; off >>= 1) {
+            a.x += __shfl_xor(a.x, off, 64);
+            a.y += __shfl_xor(a.y, off, 64);
+        }
+        if (c != 0) continue;
+        if constexpr (UNI) {
+            const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(t, i / R, i % R));
+            if (x < (unsigned)P.X.n) {
+                const double w = P.outw[x];
+                out[x] = make_double2(a.x * w, a.y * w);
+            }
+        } else {
+            if (t + T * i < P.X.n) out[t + T * i] = a;
+        }
+    }
+}
+
+// vt[l][ia][ib] = m_l psi_l(w), in (A, B) order; one thread per value
+__global__ __launch_bounds__(256) void k_nu_vt(int nA, int nB, const float *fm, double wc,
+                                               double winv, int nt, const double *coef,
+                                               const double *mul, int nleg, double *vt) {
+    const int x = blockIdx.x * 256 + threadIdx.x, l = blockIdx.y;
+    if (x >= nA * nB) return;
+    const int ia = x / nB, ib = x % nB;
+    const double s = clamp1(((fm ? (double)fm[(size_t)ib * nA + ia] : 0.0) - wc) * winv);
+    vt[(size_t)l * nA * nB + x] =
+        mul[l] * prolate(coef + (size_t)l * nleg, coef + (size_t)nt * nleg, nleg, l & 1, s);
+}
+
+// S_c [ib][ia] split -> [ia][ib] pairs, 32 x 32 tiles
+__global__ __launch_bounds__(256) void k_nu_sens(int nA, int nB, const float *s_r,
+                                                 const float *s_i, float2 *out) {
+    __shared__ float2 tile[32][33];
+    const size_t o = (size_t)blockIdx.z * nA * nB;
+    const int a0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    for (int r = ty; r < 32; r += 8) {
+        const int ib = b0 + r, ia = a0 + tx;
+        if (ib < nB && ia < nA) {
+            const size_t i = o + (size_t)ib * nA + ia;
+            tile[r][tx] = make_float2(s_r[i], s_i[i]);
+        }
+    }
+    __syncthreads();
+    for (int r = ty; r < 32; r += 8) {
+        const int ia = a0 + r, ib = b0 + tx;
+        if (ib < nB && ia < nA) out[o + (size_t)ia * nB + ib] = tile[tx][r];
+    }
+}
+
+// out[ib][ia] = e^{i(2pi kc.r + w tc)} sum_s partial[s][ia][ib]
+__global__ __launch_bounds__(256) void k_nu_out(int nA, int nB, int splits,
+                                                const double2 *partial, const float *cA,
+                                                const float *cB, const float *fm, double kcA,
+                                                double kcB, double tc_2pi, float *out_r,
+                                                float *out_i) {
+    __shared__ double2 tile[16][17];
+    const int a0 = blockIdx.x * 16, b0 = blockIdx.y * 16;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    {
+        const int ia = a0 + ty, ib = b0 + tx;
+        double2 s = make_double2(0.0, 0.0);
+        if (ia < nA && ib < nB)
+            for (int q = 0; q < splits; ++q) {
+                const double2 v = partial[(size_t)q * nA * nB + (size_t)ia * nB + ib];
+                s.x += v.x;
+                s.y += v.y;
+            }
+        tile[ty][tx] = s;
+    }
+    __syncthreads();
+    const int ia = a0 + tx, ib = b0 + ty;
+    if (ia >= nA || ib >= nB) return;
+    const size_t i = (size_t)ib * nA + ia;
+    const double rev = kcA * cA[i] + kcB * cB[i] + (fm ? tc_2pi * fm[i] : 0.0);
+    double s, c;
+    sincospi(2.0 * (rev - rint(rev)), &s, &c);
+    const double2 v = cmul(tile[tx][ty], make_double2(c, s));
+    out_r[i] = (float)v.x;
+    out_i[i] = (float)v.y;
+}
+
+// --------------------------------------------------------------- dispatching
+constexpr int NU_LENGTHS[] = {96, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096};
+
+int pick_length(double want) {
+    for (int L : NU_LENGTHS)
+        if (L >= want) return L;
+    return 0;
+}
+
+template <class F>
+int line_switch(int L, F f) {
+    switch (L) {
+        case 96: return f(std::integral_constant<int, 96>{});
+        case 128: return f(std::integral_constant<int, 128>{});
+        case 192: return f(std::integral_constant<int, 192>{});
+        case 256: return f(std::integral_constant<int, 256>{});
+        case 384: return f(std::integral_constant<int, 384>{});
+        case 512: return f(std::integral_constant<int, 512>{});
+        case 768: return f(std::integral_constant<int, 768>{});
+        case 1024: return f(std::integral_constant<int, 1024>{});
+        case 1536: return f(std::integral_constant<int, 1536>{});
+        case 2048: return f(std::integral_constant<int, 2048>{});
+        case 3072: return f(std::integral_constant<int, 3072>{});
+        case 4096: return f(std::integral_constant<int, 4096>{});
+        default: return fail(IMP_EINVAL, "NUDFT: line length %d", L);
+    }
+}
+
+int line_store(imp_ctx *ctx, LineArgs P, int nlines, double2 *out, size_t out_line,
+               size_t out_el) {
+    P.nlines = nlines;
+    return line_switch(P.X.L, [&](auto len) -> int {
+        constexpr int L = decltype(len)::value;
+        // a multiple of 16 for the panel order
+        const long wgs = ((long)nlines * ceil_div(P.nq, ln::lines(L, ST_WG)) + 15) & ~15L;
+        hipLaunchKernelGGL((P.X.uniform ? k_line_store<L, true> : k_line_store<L, false>), dim3((unsigned)wgs),
+                           dim3(ln::threads(L) * ln::lines(L, ST_WG)), 0, ctx->stream, P, out, out_line,
+                           out_el);
+        IMP_CHECK_LAUNCH();
+        return IMP_OK;
+    });
+}
+
+int line_combine(imp_ctx *ctx, const LineArgs &P, int nlines, int ncg, int splits,
+                 const double *vt, const float2 *sens, size_t nvox, double2 *partial) {
+    return line_switch(P.X.L, [&](auto len) -> int {
+        constexpr int L = decltype(len)::value;
+        hipLaunchKernelGGL((P.X.uniform ? k_line_combine<L, true> : k_line_combine<L, false>), dim3((unsigned)(nlines * splits)),
+                           dim3(ln::threads(L) * ln::lines(L, CO_WG)), 0, ctx->stream, P, ncg, splits,
+                           vt, sens, nvox, partial);
+        IMP_CHECK_LAUNCH();
+        return IMP_OK;
+    });
+}
+
+// Axis of n coordinates from c0 to c1 (dev: largest distance from uniform)
+// against frequencies [klo, khi].  False: the transform lengths do not fit.
+bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, float klo, float khi,
+               NuAxis *X) {
+    if (n < 2) return false;
+    X->n = n;
+    X->kc = 0.5 * ((double)klo + khi);
+    const double Kh = 0.5 * ((double)khi - klo);
+    const double d = ((double)c1 - c0) / (n - 1);
+    // a coordinate off by dev turns the phase by at most 2 pi Kh dev
+    X->uniform = d != 0.0 && Kh * dev < 1e-10;
+    if (X->uniform) {
+        X->L = pick_length(NU_SIGMA * n);
+        if (!X->L) return false;
+        X->xc = c0 + (n / 2) * d;
+        X->flip = d < 0.0;
+        X->inv_d = X->L * std::fabs(d);
+    } else {
+        X->xc = 0.5 * ((double)cmin + cmax);
+        const double Xh = 0.5 * ((double)cmax - cmin);
+        if (!(Xh > 0.0)) return false;
+        X->flip = 0;
+        X->inv_d = 2.0 * NU_SIGMA * Xh;
+    }
+    const double cells = Kh * X->inv_d;
+    if (!(cells < 4096.0)) return false;
+    X->j0 = std::ceil(cells + 0.5 * NW) + 1;
+    X->nf = 2 * (int)X->j0 + 1;
+    if (!X->uniform) {
+        // at least n: every thread interpolates at most vals(L) outputs
+        X->L = pick_length(std::max<double>(NU_SIGMA * X->nf, n));
+        if (!X->L) return false;
+    }
+    X->shift = (int)X->j0 % X->L;
+    return true;
+}
+
+}  // namespace
+
+// Geometry of a 2D problem: axes and time expansion, or ok = false when the
+// separable evaluation does not apply.  Synchronises (one small read-back).
+int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                   const float *x, const float *y, const float *fm, NuGeometry *G) {
+    G->ok = false;
+    const hipStream_t st = ctx->stream;
+    void *w = nullptr;
+    IMP_TRY(workspace(ctx, WS_NU_GEO, (G_WORDS + 512 * GB_WORDS) * sizeof(unsigned), &w));
+    unsigned *geo = (unsigned *)w, *part = geo + G_WORDS;
+    const int kb = std::min(256, ceil_div(m, 1024)), xb = std::min(256, ceil_div(n, 1024));
+    hipLaunchKernelGGL(k_geo_scan, dim3(kb + xb), dim3(256), 0, st, m, kx, ky, t, n, x, y, fm, kb,
+                       part);
+    hipLaunchKernelGGL(k_geo_final, dim3(1), dim3(256), 0, st, kb, xb, (const unsigned *)part,
+                       geo);
+    hipLaunchKernelGGL(k_geo_check, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, x, y, geo);
+    IMP_CHECK_LAUNCH();
+    unsigned h[G_WORDS];
+    IMP_HIP(hipMemcpyAsync(h, geo, sizeof(h), hipMemcpyDeviceToHost, st));
+    IMP_HIP(hipStreamSynchronize(st));
+    int nA = 0;
+    bool a_is_y = false;
+    if (h[G_FLAGS] || h[G_KFLAG] || !geo_axes(h[G_FCX], h[G_FCY], n, &a_is_y, &nA)) return IMP_OK;
+    const int nB = n / nA;
+    auto lo = [&](int i) { return dec_f(h[G_MIN + i]); };
+    auto hi = [&](int i) { return dec_f(h[G_MAX + i]); };
+    const int a = a_is_y ? 1 : 0, b = 1 - a;
+    if (!plan_axis(nA, bits_f(h[G_A0]), bits_f(h[G_A1]), bits_f(h[G_DEVA]), lo(3 + a), hi(3 + a),
+                   lo(a), hi(a), &G->A) ||
+        !plan_axis(nB, bits_f(h[G_B0]), bits_f(h[G_B1]), bits_f(h[G_DEVB]), lo(3 + b), hi(3 + b),
+                   lo(b), hi(b), &G->B))
+        return IMP_OK;
+    const double tlo = lo(2), thi = hi(2), wlo = fm ? lo(5) : 0.0, whi = fm ? hi(5) : 0.0;
+    G->tc = 0.5 * (tlo + thi);
+    G->th = 0.5 * (thi - tlo);
+    G->wc = 0.5 * (wlo + whi);
+    G->wh = 0.5 * (whi - wlo);
+    if (!prolate_expand(G->wh * G->th, G->coef, G->mul, &G->nt, &G->nleg)) return IMP_OK;
+    G->a_is_y = a_is_y;
+    G->ok = true;
+    return IMP_OK;
+}
+
+namespace {
+
+struct Carver {
+    size_t off = 0;
+    size_t take(size_t bytes) {
+        const size_t o = off;
+        off += (bytes + 255) & ~(size_t)255;
+        return o;
+    }
+};
+
+// largest spread-grid block and A-transformed grid (bytes): coils go in
+// groups so the second stays below its limit, rows in blocks for the first
+constexpr size_t NU_BLOCK_BYTES = (size_t)512 << 20;
+constexpr size_t NU_MID_BYTES = (size_t)3 << 30;
+
+int log2i(int n) {
+    int b = 0;
+    while ((1 << b) < n) ++b;
+    return b;
+}
+
+}  // namespace
+
+double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils) {
+    const double cols = (double)G.nt * (1 << log2i(ncoils));
+    const double grid = (double)G.A.nf * G.B.nf + (double)G.A.n * G.B.nf;
+    return 250.0 + 3.0e-5 * m * cols + 1.0e-5 * grid * cols;
+}
+
+int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int n, int ncoils, const float *kx,
+                  const float *ky, const float *t, const float *x, const float *y,
+                  const float *fm, const float *phi_r, const float *phi_i, const float *d_r,
+                  const float *d_i, const float *s_r, const float *s_i, float *out_r,
+                  float *out_i) {
+    const hipStream_t st = ctx->stream;
+    const NuAxis &A = G.A, &B = G.B;
+    const float *kA = G.a_is_y ? ky : kx, *kB = G.a_is_y ? kx : ky;
+    const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
+    const int nA = A.n, nB = B.n, nt = G.nt;
+    const size_t nvox = (size_t)nA * nB;
+    // coils per group: a power of two up to 32 whose A-transformed grid fits
+    int cg = std::min(32, 1 << log2i(ncoils));
+    while (cg > 1 && (size_t)nA * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
+    // wave layout: coil slots x time groups x rows = 32 lane pairs; fewer
+    // coils when the time terms need more groups
+    while (cg > 1 && ceil_div(nt, 32 / cg) > SP_MAX_NL) cg /= 2;
+    const int groups = ceil_div(ncoils, cg);
+    const int lc = log2i(cg), ll = std::min(5 - lc, log2i(nt));
+    const int nl = ceil_div(nt, 1 << ll);
+    const int yg = 1 << (5 - lc - ll);
+    const bool uni = lc == 5;
+    const int T = sp_switch(nl, [](auto k) { return sp_cells(decltype(k)::value); });
+    const int ntp = nl << ll;
+    // spread geometry
+    SpGeom S{};
+    S.T = T;
+    S.yg = yg;
+    S.ncA = A.nf - NW + 1;
+    S.ncB = B.nf - NW + 1;
+    S.nfA = A.nf;
+    S.nfB = B.nf;
+    S.ntx = ceil_div(A.nf, T);
+    const int nc0 = std::min(cg, ncoils);
+    const size_t row_bytes = (size_t)A.nf * nt * nc0 * sizeof(double2);
+    int rb = (int)std::max<size_t>(1, NU_BLOCK_BYTES / row_bytes);
+    rb = std::min(ceil_div(B.nf, yg) * yg, std::max(yg, rb / yg * yg));
+    const int blocks = ceil_div(B.nf, rb);
+    rb = ceil_div(ceil_div(B.nf, blocks), yg) * yg;   // even blocks
+    S.rb = rb;
+    S.nty = rb / yg;
+    const int ntile = S.ntx * S.nty;
+    S.entry_cap = ntile + SP_SLOTS;
+    const int ncells = S.ncA * S.ncB;
+    const int nblk = ceil_div(m, RX_BLOCK);
+    const int splits_max = 8;
+    // --- workspace: tables, then grids
+    Carver W;
+    const size_t o_key0 = W.take((size_t)m * 4), o_key1 = W.take((size_t)m * 4);
+    const size_t o_val0 = W.take((size_t)m * 4), o_val1 = W.take((size_t)m * 4);
+    const size_t o_hist = W.take((size_t)RX_BINS * nblk * 4);
+    const size_t o_start = W.take(((size_t)ncells + 1) * 4);
+    const size_t o_bx = W.take((size_t)m * 4);
+    const size_t o_wx = W.take((size_t)m * (NW + 2 * (T - 1)) * 8);
+    const size_t o_wy = W.take((size_t)m * (NW + 2 * (yg - 1)) * 8);
+    const size_t o_u = W.take((size_t)m * ntp * 8);
+    const size_t o_wd = W.take((size_t)m * (1 << lc) * sizeof(double2));
+    const size_t o_vis = W.take((size_t)blocks * ntile * 4);
+    const size_t o_cnt = W.take((size_t)blocks * sizeof(SpCount));
+    const size_t o_ent = W.take((size_t)blocks * S.entry_cap * sizeof(SpEntry));
+    const size_t o_mul = W.take((size_t)blocks * SP_SLOTS * sizeof(SpMulti));
+    const size_t o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * 8);
+    const size_t o_coef = W.take(G.coef.size() * 8);
+    const size_t o_mu = W.take(G.mul.size() * 8);
+    const size_t o_poly = W.take(KB_WORDS * 8);
+    size_t o_tw[2], o_in[2], o_ow[2], o_ob[2];
+    for (int a = 0; a < 2; ++a) {
+        const NuAxis &X = a ? B : A;
+        o_tw[a] = W.take((size_t)X.L * sizeof(double2));
+        o_in[a] = W.take((size_t)X.nf * 8);
+        o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
+        o_ob[a] = W.take((size_t)X.n * 4);
+    }
+    const size_t o_vt = W.take((size_t)nt * nvox * 8);
+    const size_t o_sens = W.take(s_r ? (size_t)ncoils * nvox * sizeof(float2) : 0);
+    const size_t o_img = W.take((size_t)groups * splits_max * nvox * sizeof(double2));
+    const size_t o_grid = W.take((size_t)rb * row_bytes);
+    const size_t o_mid = W.take((size_t)nA * B.nf * nt * nc0 * sizeof(double2));
+    void *wsp = nullptr;
+    IMP_TRY(workspace(ctx, WS_NU, W.off, &wsp));
+    char *ws = (char *)wsp;
+    int *key0 = (int *)(ws + o_key0), *key1 = (int *)(ws + o_key1);
+    int *val0 = (int *)(ws + o_val0), *val1 = (int *)(ws + o_val1);
+    int *hist = (int *)(ws + o_hist), *start = (int *)(ws + o_start);
+    SpCount *cnt = (SpCount *)(ws + o_cnt);
+    double *coef = (double *)(ws + o_coef), *mul = (double *)(ws + o_mu);
+    double *poly = (double *)(ws + o_poly);
+    const int rec = prof_begin(ctx, "nufft_adjoint");
+    IMP_HIP(hipMemcpyAsync(coef, G.coef.data(), G.coef.size() * 8, hipMemcpyHostToDevice, st));
+    IMP_HIP(hipMemcpyAsync(poly, kb_poly_table(), KB_WORDS * 8, hipMemcpyHostToDevice, st));
+    IMP_HIP(hipMemcpyAsync(mul, G.mul.data(), G.mul.size() * 8, hipMemcpyHostToDevice, st));
+    // --- samples sorted by window start
+    const dim3 gm(ceil_div(m, 256)), b256(256);
+    hipLaunchKernelGGL(k_nu_keys, gm, b256, 0, st, m, kA, kB, A, B, key0, val0);
+    for (int shift = 0; shift == 0 || (ncells - 1) >> shift; shift += 8) {
+        hipLaunchKernelGGL(k_rx_count, dim3(nblk), b256, 0, st, (const int *)key0, m, shift,
+                           hist);
+        hipLaunchKernelGGL(k_rx_scatter, dim3(nblk), b256, 0, st, (const int *)key0,
+                           (const int *)val0, m, shift, nblk, (const int *)hist, key1, val1);
+        std::swap(key0, key1);
+        std::swap(val0, val1);
+    }
+    IMP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m,
+                       (const int *)key0, ncells, start);
+    hipLaunchKernelGGL(k_nu_prep, dim3(ceil_div(m, PREP_S)), b256, 0, st, m, (const int *)val0, kA,
+                       kB, t, A, B, G.tc, G.th > 0.0 ? 1.0 / G.th : 0.0, (const double *)coef,
+                       (const double *)poly, nt, ntp, G.nleg, T - 1, yg - 1, (int *)(ws + o_bx),
+                       (double *)(ws + o_wx), (double *)(ws + o_wy), (double *)(ws + o_u));
+    // --- spread work lists, image-side tables
+    hipLaunchKernelGGL(k_sp_zero, dim3(ceil_div((long)(blocks * sizeof(SpCount) / 4), 256)), b256,
+                       0, st, (int *)cnt, (int)(blocks * sizeof(SpCount) / 4));
+    hipLaunchKernelGGL(k_sp_count, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
+                       (const int *)start, (int *)(ws + o_vis), cnt);
+    hipLaunchKernelGGL(k_sp_list, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
+                       (const int *)(ws + o_vis), cnt, (SpEntry *)(ws + o_ent),
+                       (SpMulti *)(ws + o_mul));
+    for (int a = 0; a < 2; ++a) {
+        const NuAxis &X = a ? B : A;
+        const int len = std::max(std::max(X.L, X.nf), X.n);
+        hipLaunchKernelGGL(k_nu_axis, dim3(ceil_div(len, 256)), b256, 0, st, X, a ? cB : cA,
+                           a ? nA : 1, (double2 *)(ws + o_tw[a]), (double *)(ws + o_in[a]),
+                           (double *)(ws + o_ow[a]), (int *)(ws + o_ob[a]));
+    }
+    hipLaunchKernelGGL(k_nu_vt, dim3(ceil_div((long)nvox, 256), nt), b256, 0, st, nA, nB, fm, G.wc,
+                       G.wh > 0.0 ? 1.0 / G.wh : 0.0, nt, (const double *)coef,
+                       (const double *)mul, G.nleg, (double *)(ws + o_vt));
+    if (s_r)
+        hipLaunchKernelGGL(k_nu_sens, dim3(ceil_div(nA, 32), ceil_div(nB, 32), ncoils), b256, 0,
+                           st, nA, nB, s_r, s_i, (float2 *)(ws + o_sens));
+    IMP_CHECK_LAUNCH();
+    // --- per coil group: spread and transform row blocks, then the B axis
+    SpFn spread = sp_switch(nl, [&](auto k) { return sp_pick1<decltype(k)::value>(uni); });
+    SpFn multi = sp_switch(nl, [](auto k) { return sp_multi1<decltype(k)::value>(); });
+    LineArgs LA{}, LB{};
+    LA.X = A;
+    LB.X = B;
+    LineArgs *LX[2] = {&LA, &LB};
+    for (int a = 0; a < 2; ++a) {
+        LX[a]->tw = (const double2 *)(ws + o_tw[a]);
+        LX[a]->inw = (const double *)(ws + o_in[a]);
+        LX[a]->outw = (const double *)(ws + o_ow[a]);
+        LX[a]->base = (const int *)(ws + o_ob[a]);
+    }
+    int parts = 0;
+    for (int g = 0; g < groups; ++g) {
+        const int c0 = g * cg, nc = std::min(cg, ncoils - c0), nq = nt * nc;
+        hipLaunchKernelGGL(k_nu_data, dim3(ceil_div(m, WD_S)), b256, 0, st, m, c0, nc, 1 << lc, kA,
+                           kB, t, A, B, G.tc, G.wc / (2.0 * M_PI), phi_r, phi_i, d_r, d_i,
+                           (double2 *)(ws + o_wd));
+        SpArgs P{};
+        P.G = S;
+        P.nt = nt;
+        P.ntp = ntp;
+        P.nc = nc;
+        P.lc = lc;
+        P.ll = ll;
+        P.start = start;
+        P.perm = val0;
+        P.bx = (const int *)(ws + o_bx);
+        P.wx = (const double *)(ws + o_wx);
+        P.wy = (const double *)(ws + o_wy);
+        P.u = (const double *)(ws + o_u);
+        P.wd = (const double *)(ws + o_wd);
+        P.cnt = cnt;
+        P.entries = (const SpEntry *)(ws + o_ent);
+        P.multis = (const SpMulti *)(ws + o_mul);
+        P.part = (double *)(ws + o_part);
+        P.grid = (double *)(ws + o_grid);
+        for (int b = 0; b < blocks; ++b) {
+            P.r0 = b * rb;
+            P.block = b;
+            // one-wave workgroups: a wave that ends makes room at once
+            hipLaunchKernelGGL(spread, dim3(std::min(S.entry_cap, 64 * ctx->num_cus)), dim3(64),
+                               0, st, P);
+            hipLaunchKernelGGL(multi, dim3(4 * ctx->num_cus), b256, 0, st, P);
+            IMP_CHECK_LAUNCH();
+            LA.in = (const double2 *)(ws + o_grid);
+            LA.in_line = (size_t)A.nf * nq;
+            LA.in_el = nq;
+            LA.nq = nq;
+            // mid[ia][gB][q]
+            IMP_TRY(line_store(ctx, LA, std::min(rb, B.nf - b * rb),
+                               (double2 *)(ws + o_mid) + (size_t)b * rb * nq, nq,
+                               (size_t)B.nf * nq));
+        }
+        LB.in = (const double2 *)(ws + o_mid);
+        LB.in_line = (size_t)B.nf * nq;
+        LB.in_el = nq;
+        LB.nq = nq;
+        const int panels = line_switch(B.L, [&](auto len) -> int {
+            return ceil_div(nq, ln::lines(decltype(len)::value, CO_WG));
+        });
+        const int splits =
+            std::max(1, std::min(std::min(splits_max, panels), 12 * ctx->num_cus / nA));
+        IMP_TRY(line_combine(ctx, LB, nA, nc, splits, (const double *)(ws + o_vt),
+                             s_r ? (const float2 *)(ws + o_sens) + (size_t)c0 * nvox : nullptr,
+                             nvox, (double2 *)(ws + o_img) + (size_t)parts * nvox));
+        parts += splits;
+    }
+    hipLaunchKernelGGL(k_nu_out, dim3(ceil_div(nA, 16), ceil_div(nB, 16)), b256, 0, st, nA, nB,
+                       parts, (const double2 *)(ws + o_img), cA, cB, fm, A.kc, B.kc,
+                       G.tc / (2.0 * M_PI), out_r, out_i);
+    prof_end(ctx, rec);
+    IMP_CHECK_LAUNCH();
+    return IMP_OK;
+}
+
+}  // namespace imp

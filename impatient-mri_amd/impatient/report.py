@@ -141,17 +141,21 @@ def main(argv=None):
     ops.nudft_adjoint(ctx, p.kx, p.ky, p.kz, p.t, p.x, p.y, p.z, p.fm, d, p.sens)
     timer_on()
     b = ops.nudft_adjoint(ctx, p.kx, p.ky, p.kz, p.t, p.x, p.y, p.z, p.fm, d, p.sens)
-    # direct kernels, or the stacked path's group launches and its reduction
+    # direct kernels, the stacked path's group launches and its reduction, or
+    # the separable evaluation (which visits no pairs)
     parts = {k: kernel_ms(k) for k in ("k_nudft_mfma", "k_nudft_valu", "k_nudft_stack",
-                                       "k_reduce_stack")}
+                                       "k_reduce_stack", "nufft_adjoint")}
     fhd_ms = sum(v[0] for v in parts.values())
     stacked = parts["k_nudft_stack"][1] > 0
-    path = "stacked (z-separable)" if stacked else "direct"
+    separable = parts["nufft_adjoint"][1] > 0
+    path = "separable" if separable else "stacked (z-separable)" if stacked else "direct"
     pairs = float(nc) * nk * nv
     # (sample, voxel) pairs whose phase and sin/cos were evaluated: once per
     # pair for all coils on the direct path; on the stacked path once per
     # pair of one partition and group launch of 32 coil-partition columns
-    if stacked:
+    if separable:
+        evaluated = 0.0
+    elif stacked:
         K = nk // p.Nz
         evaluated = float(parts["k_nudft_stack"][1]) * K * nv
     else:

@@ -1,0 +1,161 @@
+"""The separable F^H d of large 2D problems (csrc/nufft.hip) against the FP64
+oracle and against the direct kernels.
+
+Tolerance: 2e-7 relative L2.  The separable form sums in FP64 and rounds once
+to FP32 (at most 6e-8 per value); its time expansion and its two kernel
+separations are each good to 1e-8 of the largest term.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-7
+DIRECT_TOL = 2e-6   # the direct kernels' own tolerance (test_gpu_nudft.py)
+
+
+def _timer(ctx, fn, *names):
+    from impatient._lib import call
+    call("imp_profile_enable", ctx.h, C.c_int(1))
+    call("imp_profile_reset", ctx.h)
+    r = fn()
+    counts = []
+    for name in names:
+        tot, n = C.c_double(), C.c_int()
+        call("imp_profile_read", ctx.h, name.encode(), C.byref(tot), C.byref(n))
+        counts.append(n.value)
+    call("imp_profile_enable", ctx.h, C.c_int(0))
+    return r, counts
+
+
+def _problem(Nx, Ny, nc, M, seed=3, kscale=1.0, max_hz=120.0, t_read=8e-3, clump=False):
+    rng = np.random.default_rng(seed)
+    f = lambda a: np.ascontiguousarray(a, np.float32)
+    if clump:   # every sample within half a cycle: a handful of grid cells
+        kx, ky = rng.uniform(-0.4, 0.4, (2, M))
+    else:       # dense centre, ragged edge
+        r = 0.5 * rng.uniform(0, 1, M) ** 1.3 * kscale
+        th = rng.uniform(0, 2 * np.pi, M)
+        kx, ky = Nx * r * np.cos(th) + 0.3, Ny * r * np.sin(th) - 0.2
+    t = rng.uniform(0, t_read, M) + 1e-3
+    Y, X = np.meshgrid((np.arange(Ny) - Ny // 2) / Ny, (np.arange(Nx) - Nx // 2) / Nx,
+                       indexing="ij")
+    fm = 2 * np.pi * max_hz * (np.exp(-((X - .1) ** 2 + Y ** 2) / .05) - 0.3 * X)
+    d = rng.standard_normal((nc, M)) + 1j * rng.standard_normal((nc, M))
+    s = rng.standard_normal((nc, Nx * Ny)) + 1j * rng.standard_normal((nc, Nx * Ny))
+    return dict(kx=f(kx), ky=f(ky), t=f(t), x=f(X).reshape(-1), y=f(Y).reshape(-1),
+                fm=f(fm).reshape(-1), d=d.astype(np.complex64), s=s.astype(np.complex64))
+
+
+def _check(ctx, p, separable=True, sens=True, phi=None, tol=TOL):
+    from impatient import ops
+    from oracle import oracle as orc
+    s = p["s"] if sens else None
+    got, (n,) = _timer(ctx, lambda: ops.nudft_adjoint(
+        ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"], p["d"], s, phi),
+        "nufft_adjoint")
+    assert (n > 0) == separable
+    idx = np.unique(np.concatenate([[0, len(p["x"]) - 1],
+                                    np.random.default_rng(1).integers(0, len(p["x"]), 60)]))
+    ref = orc.nudft_adjoint(p["kx"], p["ky"], None, p["t"], p["x"][idx], p["y"][idx], None,
+                            None if p["fm"] is None else p["fm"][idx], p["d"],
+                            None if s is None else s[:, idx], phi)
+    err = rel_l2(got[idx], ref)
+    print(f"rel_l2 {err:.2e}")
+    assert err < tol
+    return got
+
+
+# sizes: uniform axes at exact and rounded line lengths, rounded coordinates,
+# odd and unequal axes; coil counts on both sides of every wave layout
+@pytest.mark.parametrize("Nx,Ny,nc,M", [
+    (128, 128, 1, 60001), (160, 128, 2, 50000), (150, 131, 3, 70001), (192, 97, 5, 80000),
+    (129, 256, 8, 65537), (144, 144, 9, 90000), (128, 256, 16, 70000), (200, 187, 17, 60013),
+    (160, 160, 31, 80000), (128, 200, 32, 70001)])
+def test_adjoint_separable(ctx, Nx, Ny, nc, M):
+    _check(ctx, _problem(Nx, Ny, nc, M))
+
+
+@pytest.mark.parametrize("what", ["x_outer", "x_falling", "y_falling", "no_field_map",
+                                  "no_sens", "phi", "beyond_nyquist", "wide_time", "clump",
+                                  "axis_shuffled"])
+def test_adjoint_separable_forms(ctx, what):
+    """Voxel orders, axis directions and spacings, optional operands, samples
+    beyond the band, many time terms, all samples in a few cells."""
+    N, nc, M = 160, 4, 60000
+    kw = dict(beyond_nyquist=dict(kscale=1.7), wide_time=dict(max_hz=900.0, t_read=10e-3),
+              clump=dict(clump=True)).get(what, {})
+    p = _problem(N, N, nc, M, **kw)
+    grid = lambda a: a.reshape(N, N)
+    if what == "x_outer":
+        for k in ("x", "y", "fm"):
+            p[k] = np.ascontiguousarray(grid(p[k]).T).reshape(-1)
+    if what in ("x_falling", "y_falling"):
+        p[what[0]] = -p[what[0]]
+    if what == "axis_shuffled":
+        o = np.random.default_rng(9).permutation(N)
+        p["x"] = np.ascontiguousarray(grid(p["x"])[:, o]).reshape(-1)
+    if what == "no_field_map":
+        p["fm"] = None
+    phi = None
+    if what == "phi":
+        r = np.random.default_rng(5)
+        phi = (1 + 0.3 * r.standard_normal((nc, M)) + 0.2j * r.standard_normal((nc, M))).astype(
+            np.complex64)
+    if what == "no_sens":
+        p["d"] = p["d"][:1]
+    _check(ctx, p, sens=what != "no_sens", phi=phi)
+
+
+@pytest.mark.parametrize("what", ["points", "nan_point", "inf_time", "one_row_moved"])
+def test_adjoint_other_points_stay_direct(ctx, what):
+    """Points that form no tensor grid, and operands that are not finite, take
+    the direct kernels as before."""
+    p = _problem(160, 160, 4, 40000)
+    if what == "points":
+        r = np.random.default_rng(2)
+        p["x"] = (p["x"] + r.uniform(-1e-3, 1e-3, len(p["x"]))).astype(np.float32)
+    if what == "one_row_moved":
+        p["x"] = p["x"].copy()
+        p["x"][160 * 71 + 5] += np.float32(1e-4)
+    if what in ("points", "one_row_moved"):
+        _check(ctx, p, separable=False, tol=DIRECT_TOL)
+        return
+    from impatient import ops
+    if what == "nan_point":
+        p["x"] = p["x"].copy()
+        p["x"][77] = np.nan
+    else:
+        p["t"] = p["t"].copy()
+        p["t"][77] = np.inf
+    got, n = _timer(ctx, lambda: ops.nudft_adjoint(
+        ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"], p["d"], p["s"]),
+        "nufft_adjoint", "k_nudft_mfma")
+    assert n == [0, 1]
+    assert np.isnan(got[77])
+
+
+def test_adjoint_separable_repeats_bits_and_matches_direct(ctx):
+    """Repeated calls give the same bits (no atomics on the grid), and the
+    allocation-free entry point (always direct) the same image."""
+    from impatient import ops
+    from impatient._lib import call, ptr
+    p = _problem(128, 128, 8, 40000)
+    run = lambda: ops.nudft_adjoint(ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None,
+                                    p["fm"], p["d"], p["s"])
+    (a, (n,)) = _timer(ctx, run, "nufft_adjoint")
+    assert n > 0
+    assert np.array_equal(a, run())
+    up = lambda v: ctx.to_device(np.ascontiguousarray(v, np.float32).reshape(-1))
+    dev = [up(p[k]) for k in ("kx", "ky", "t", "x", "y", "fm")]
+    dr, di, sr, si = (up(v) for v in (p["d"].real, p["d"].imag, p["s"].real, p["s"].imag))
+    o = [ctx.alloc((len(p["x"]),)) for _ in range(2)]
+    call("imp_nudft_adjoint_noalloc", ctx.h, C.c_int(40000), C.c_int(128 * 128), C.c_int(8),
+         ptr(dev[0]), ptr(dev[1]), None, ptr(dev[2]), ptr(dev[3]), ptr(dev[4]), None, ptr(dev[5]),
+         None, None, ptr(dr), ptr(di), ptr(sr), ptr(si), ptr(o[0]), ptr(o[1]))
+    ctx.synchronize()
+    assert rel_l2(a, o[0].get() + 1j * o[1].get()) < DIRECT_TOL

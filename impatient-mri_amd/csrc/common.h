@@ -13,6 +13,8 @@
 
 namespace imp {
 
+constexpr size_t HOST_TABLE_WORDS = 4096;   // of imp_ctx::host_tables()
+
 // ---------------------------------------------------------------- errors
 // Thread-local last error; every C entry point records its failure here.
 void set_error(const std::string &msg);
@@ -75,6 +77,7 @@ enum WsSlot {
     WS_QSTACK,     // stacked Q: one partition's 2D planes and the z factor
     WS_GRID,       // gridding: binned samples, grids and line-transform tables
     WS_NU_GEO,     // separable NUDFT: geometry scan
+    WS_NU_SORT,    // separable NUDFT: samples sorted by window
     WS_NU,         // separable NUDFT: tables and grids
     WS_COUNT
 };
@@ -92,6 +95,10 @@ struct imp_ctx {
     size_t dscratch_n = 0;
     // pinned host words for scalar readback
     double *host_scalars = nullptr;
+    // pinned host words for the separable NUDFT's tables (uploads from it may
+    // still be running when the call that filled it returns; the next such
+    // call synchronises the stream before it writes)
+    double *host_tables() const { return host_scalars + 64; }
     // FFT twiddle tables: table for length L at offset L (L = 2..2048)
     float2 *twiddle = nullptr;
     // live Toeplitz operators created on this context

@@ -1279,7 +1279,7 @@ int choose_separable(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     IMP_HIP(hipStreamIsCapturing(ctx->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return IMP_OK;
-    IMP_TRY(nufft_geometry(ctx, num_k, num_x, kx, ky, t, x, y, fm, G));
+    IMP_TRY(nufft_geometry(ctx, num_k, num_x, kx, ky, t, x, y, nullptr, fm, G));
     if (G->ok && nufft_adjoint_us(*G, num_k, ncoils) >= direct_us(pairs, ncoils)) G->ok = false;
     return IMP_OK;
 }
@@ -1322,7 +1322,7 @@ int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
         IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, &G));
         if (G.ok) {
             IMP_TRY(reserve_direct(ctx, num_k, num_x, ncoils));
-            return nufft_adjoint(ctx, G, num_k, num_x, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
+            return nufft_adjoint(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
                                  d_r, d_i, s_r, s_i, out_r, out_i);
         }
     }
@@ -2436,6 +2436,14 @@ int toeplitz_q(imp_ctx *ctx, int num_k, const float *kx, const float *ky,
     const float t0 = t_host_first_last[0];
     const float tlast = t_host_first_last[1];
     const float tau = ntime_segs > 0 ? (tlast - t0) / (float)ntime_segs : (tlast - t0);
+    if (std_grid && !d3 && !(flags & IMP_Q_DIRECT) && tau > 0.f && std::isfinite(tau) &&
+        std::isfinite(t0)) {
+        NuGeometry G;
+        IMP_TRY(nufft_q_geometry(ctx, num_k, kx, ky, t, Nx, Ny, nseg, &G));
+        if (G.ok)
+            return nufft_q(ctx, G, num_k, kx, ky, t, phi_r, phi_i, Nx, Ny, nseg, tau, t0,
+                           (flags & IMP_Q_CUMULATIVE) != 0, q_r, q_i);
+    }
     const double *spos = nullptr;
     IMP_TRY(build_spos(ctx, num_k, kx, ky, d3 ? kz : nullptr, nullptr, 0.0, &spos));
     void *lanes = nullptr, *W = nullptr;
@@ -2445,7 +2453,7 @@ int toeplitz_q(imp_ctx *ctx, int num_k, const float *kx, const float *ky,
     IMP_CHECK_LAUNCH();
     const Out mode = (flags & IMP_Q_CUMULATIVE) ? Out::PerRhsCumulative : Out::PerRhs;
     // Standard grid (main_mri.cu:461-500; y outer, x, z inner, r = (x/Nx,
-    // y/Ny, z/Nz)): the separable GEMM unless the direct kernel is asked for
+    // y/Ny, z/Nz)), 3D or beyond the 2D transforms: the separable GEMM unless the direct kernel is asked for
     // (or tau is degenerate); the direct kernel evaluates the half grid and
     // fills the rest by Hermitian symmetry.
     if (std_grid && !(flags & IMP_Q_DIRECT) && tau > 0.f && std::isfinite(tau) &&

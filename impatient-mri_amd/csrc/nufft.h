@@ -23,28 +23,32 @@ struct NuAxis {
 
 struct NuGeometry {
     bool ok = false;
-    bool a_is_y = false;      // axis A (fastest in the voxel index) is y
+    bool a_is_y = false;      // axis A (fastest in the voxel index after z) is y
     NuAxis A{}, B{};
+    int nz = 1;               // z planes (z fastest)
     double tc = 0, th = 0;    // centre and half width of t, and of w
     double wc = 0, wh = 0;
-    int nt = 0, nleg = 0;     // terms of e^{iwt}, Legendre coefficients of each
-    std::vector<double> coef, mul;
 };
 
 bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double> &mul, int *nt,
                     int *nleg);
 
 int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
-                   const float *x, const float *y, const float *fm, NuGeometry *G);
-
+                   const float *x, const float *y, const float *z, const float *fm,
+                   NuGeometry *G);
 // Predicted time of nufft_adjoint in microseconds (for the choice against
 // the direct kernels).
 double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils);
-
-int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int n, int ncoils, const float *kx,
+int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
                   const float *ky, const float *t, const float *x, const float *y,
                   const float *fm, const float *phi_r, const float *phi_i, const float *d_r,
                   const float *d_i, const float *s_r, const float *s_i, float *out_r,
                   float *out_i);
+
+int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
+                     int Ny, int nseg, NuGeometry *G);
+int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const float *ky,
+            const float *t, const float *phi_r, const float *phi_i, int Nx, int Ny, int nseg,
+            float tau, float t0, bool cumulative, float *q_r, float *q_i);
 
 }  // namespace imp

@@ -49,6 +49,7 @@ constexpr double NU_BETA = 0.99 * M_PI * NW * (1.0 - 1.0 / (2.0 * NU_SIGMA));
 constexpr double NU_TIME_TOL = 1e-8;   // largest error of the time expansion
 constexpr int NU_MAX_TERMS = 48;       // time terms above which the direct kernel runs
                                        // (16 per lane, 3 groups of a 4-group wave)
+constexpr double NU_MAX_THETA = 40.0;  // half widths of t and w multiplied: 44 terms
 constexpr int NU_MAX_LEG = 160;        // Legendre coefficients per prolate function
 
 // ------------------------------------------------------------------ geometry
@@ -96,7 +97,7 @@ __global__ __launch_bounds__(256) void k_geo_scan(int m, const float *kx, const 
     const int nb = ks ? kblocks : (int)gridDim.x - kblocks;
     const int bi = ks ? blockIdx.x : blockIdx.x - kblocks;
     unsigned w[GB_WORDS] = {~0u, ~0u, ~0u, 0u, 0u, 0u, (unsigned)cnt, (unsigned)cnt, 0u};
-    const float a0 = a[0], b0 = b[0];
+    const float a0 = cnt ? a[0] : 0.f, b0 = cnt ? b[0] : 0.f;
     for (int i = bi * 256 + threadIdx.x; i < cnt; i += nb * 256) {
         const float v[3] = {a[i], b[i], c ? c[i] : 0.f};
 #pragma unroll
@@ -158,52 +159,54 @@ __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, con
     if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = 0u;
 }
 
-// Axis structure implied by the first changes: the coordinate that changes
-// first is axis A, its period nA.  false: none.
-__host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool *a_is_y,
-                                         int *nA) {
-    *a_is_y = false;
-    *nA = 0;
-    if (fcx == 1 && fcy > 1) {
-        *nA = (int)fcy;
-    } else if (fcy == 1 && fcx > 1) {
-        *a_is_y = true;
-        *nA = (int)fcx;
-    } else {
-        return false;
-    }
-    return n % *nA == 0;
+// Axis structure implied by the first changes.  In 3D (nz_known = 0) z runs
+// fastest and its period is where x or y first changes; then the coordinate
+// that changes first is axis A, of nA points.  false: none.
+__host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool d3, bool *a_is_y,
+                                         int *nA, int *nz) {
+    const unsigned f = fcx < fcy ? fcx : fcy;
+    *a_is_y = fcy < fcx;
+    *nz = d3 ? (int)f : 1;
+    const unsigned slow = *a_is_y ? fcx : fcy;
+    *nA = (int)(slow / (unsigned)*nz);
+    return (d3 || f == 1) && fcx != fcy && slow % (unsigned)*nz == 0 &&
+           (unsigned)n % slow == 0;
 }
 
-__global__ void k_geo_check(int n, const float *x, const float *y, unsigned *geo) {
+__global__ void k_geo_check(int n, const float *x, const float *y, const float *z,
+                            unsigned *geo) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     bool a_is_y;
-    int nA;
-    if (!geo_axes(geo[G_FCX], geo[G_FCY], n, &a_is_y, &nA)) {
+    int nA, nz;
+    if (!geo_axes(geo[G_FCX], geo[G_FCY], n, z != nullptr, &a_is_y, &nA, &nz)) {
         if (i == 0) atomicOr(&geo[G_FLAGS], 2u);
         return;
     }
     const float *a = a_is_y ? y : x, *b = a_is_y ? x : y;
-    const int ia = i % nA, nB = n / nA;
-    const bool ok = a[i] == a[ia] && b[i] == b[i - ia];
+    const int sa = nz, sb = nz * nA, nB = n / sb;
+    const int ia = (i / sa) % nA, ib = i / sb;
+    bool ok = a[i] == a[(size_t)ia * sa] && b[i] == b[(size_t)ib * sb];
+    if (z) ok = ok && z[i] == z[i % nz] && isfinite(z[i]);
     if (__ballot(!ok) && !ok) atomicOr(&geo[G_FLAGS], 2u);
-    if (i < nA) {
-        const double a0 = a[0], d = nA > 1 ? ((double)a[nA - 1] - a0) / (nA - 1) : 0.0;
-        const float dev = (float)(fabs((double)a[i] - (a0 + i * d)) * 1.000001);
+    if (i % sa) return;
+    if (i < sb) {
+        const double a0 = a[0],
+                     d = nA > 1 ? ((double)a[(size_t)(nA - 1) * sa] - a0) / (nA - 1) : 0.0;
+        const float dev = (float)(fabs((double)a[i] - (a0 + ia * d)) * 1.000001);
         if (dev > 0.f) atomicMax(&geo[G_DEVA], __float_as_uint(dev));
     }
-    if (ia == 0) {
-        const int ib = i / nA;
-        const double b0 = b[0], d = nB > 1 ? ((double)b[(size_t)(nB - 1) * nA] - b0) / (nB - 1) : 0.0;
+    if (i % sb == 0) {
+        const double b0 = b[0],
+                     d = nB > 1 ? ((double)b[(size_t)(nB - 1) * sb] - b0) / (nB - 1) : 0.0;
         const float dev = (float)(fabs((double)b[i] - (b0 + ib * d)) * 1.000001);
         if (dev > 0.f) atomicMax(&geo[G_DEVB], __float_as_uint(dev));
     }
     if (i == 0) {
         geo[G_A0] = __float_as_uint(a[0]);
-        geo[G_A1] = __float_as_uint(a[nA - 1]);
+        geo[G_A1] = __float_as_uint(a[(size_t)(nA - 1) * sa]);
         geo[G_B0] = __float_as_uint(b[0]);
-        geo[G_B1] = __float_as_uint(b[(size_t)(nB - 1) * nA]);
+        geo[G_B1] = __float_as_uint(b[(size_t)(nB - 1) * sb]);
     }
 }
 
@@ -280,7 +283,13 @@ bool tridiag_eig(std::vector<double> &d, std::vector<double> e, std::vector<doub
 // False when more than NU_MAX_TERMS terms are needed.
 bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double> &mul, int *nt,
                     int *nleg) {
-    if (!(theta >= 0.0) || theta > 0.5 * M_PI * NU_MAX_TERMS) return false;
+    if (!(theta >= 0.0) || theta > NU_MAX_THETA) return false;
+    if (theta == 0.0) {   // one constant term
+        coef.assign({1.0, 0.0, 0.0, 0.0, 0.0});
+        mul.assign(1, 1.0);
+        *nt = *nleg = 1;
+        return true;
+    }
     const int K = 2 * (((int)(0.75 * theta) + 36) / 2);   // Legendre degrees, both parities
     const int H = K / 2;
     if (K > NU_MAX_LEG) return false;
@@ -539,8 +548,10 @@ __global__ __launch_bounds__(256) void k_rx_scatter(const int *__restrict__ key,
 }
 
 // start[c] = first sorted sample whose cell is >= c, c = 0..ncells
-__global__ void k_nu_starts(int m, const int *key, int ncells, int *start) {
+// (clears the work-list counters on the way)
+__global__ void k_nu_starts(int m, const int *key, int ncells, int *start, int *zero, int nzero) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < nzero) zero[c] = 0;
     if (c > ncells) return;
     int lo = 0, hi = m;
     while (lo < hi) {
@@ -685,11 +696,6 @@ __device__ __forceinline__ int tile_visits(const SpGeom &G, const int *start, in
     int n = 0, s0;
     for (int r = 0; r < NW + G.yg - 1; ++r) n += row_range(G, start, gy0, gx0, r, &s0);
     return n;
-}
-
-__global__ void k_sp_zero(int *v, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) v[i] = 0;
 }
 
 __global__ __launch_bounds__(256) void k_sp_count(SpGeom G, const int *start, int *visits,
@@ -1062,25 +1068,35 @@ __device__ __forceinline__ void transform(double2 (&v)[vals(L)], int t, int c, d
 
 // One axis' tables: twiddles [L], input scale [nf] (nonuniform axes) and
 // output weights: [n] (uniform) or [n][NW] with window starts base[n].
-__global__ void k_nu_axis(NuAxis X, const float *coord, int cstride, double2 *tw, double *inw,
-                          double *outw, int *base) {
+struct AxisTab {
+    NuAxis X;
+    const float *coord;
+    int stride;
+    double2 *tw;
+    double *inw, *outw;
+    int *base;
+};
+
+__global__ void k_nu_axis(AxisTab ta, AxisTab tb) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const AxisTab &P = blockIdx.y ? tb : ta;
+    const NuAxis &X = P.X;
     if (i < X.L) {
         double s, c;
         sincospi(2.0 * i / X.L, &s, &c);
-        tw[i] = make_double2(c, s);
+        P.tw[i] = make_double2(c, s);
     }
-    if (!X.uniform && i < X.nf) inw[i] = 1.0 / kb_hat((i - X.j0) / X.L);
-    if (i < X.n) {
-        if (X.uniform) {
-            outw[i] = 1.0 / kb_hat((double)(i - X.n / 2) / X.L);
-        } else {
-            const double u = ((double)coord[(size_t)i * cstride] - X.xc) / X.inv_d;  // cycles/cell
-            const double p = u * X.L, h = kb_hat(u);
-            const int b = (int)ceil(p - 0.5 * NW);
-            base[i] = b;
-            for (int k = 0; k < NW; ++k) outw[(size_t)i * NW + k] = kb(p - (b + k)) / h;
-        }
+    if (!X.uniform && i < X.nf) P.inw[i] = 1.0 / kb_hat((i - X.j0) / X.L);
+    if (i >= X.n) return;
+    if (X.uniform) {
+        P.outw[i] = 1.0 / kb_hat((double)(i - X.n / 2) / X.L);
+    } else {
+        // cycles per cell, and the position in the transformed line
+        const double u = ((double)P.coord[(size_t)i * P.stride] - X.xc) / X.inv_d;
+        const double p = u * X.L, h = kb_hat(u);
+        const int b = (int)ceil(p - 0.5 * NW);
+        P.base[i] = b;
+        for (int k = 0; k < NW; ++k) P.outw[(size_t)i * NW + k] = kb(p - (b + k)) / h;
     }
 }
 
@@ -1422,7 +1438,7 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
     // a coordinate off by dev turns the phase by at most 2 pi Kh dev
     X->uniform = d != 0.0 && Kh * dev < 1e-10;
     if (X->uniform) {
-        X->L = pick_length(NU_SIGMA * n);
+        X->L = pick_length(2.0 * NU_SIGMA * (n / 2));   // bins up to n / 2
         if (!X->L) return false;
         X->xc = c0 + (n / 2) * d;
         X->flip = d < 0.0;
@@ -1449,11 +1465,11 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
 
 }  // namespace
 
-// Geometry of a 2D problem: axes and time expansion, or ok = false when the
-// separable evaluation does not apply.  Synchronises (one small read-back).
-int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
-                   const float *x, const float *y, const float *fm, NuGeometry *G) {
-    G->ok = false;
+// Scan of the operands: value ranges, tensor structure of the voxels.  n = 0
+// scans the samples alone.
+static int geo_scan(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                    const float *x, const float *y, const float *z, const float *fm,
+                    unsigned (&h)[G_WORDS]) {
     const hipStream_t st = ctx->stream;
     void *w = nullptr;
     IMP_TRY(workspace(ctx, WS_NU_GEO, (G_WORDS + 512 * GB_WORDS) * sizeof(unsigned), &w));
@@ -1463,15 +1479,29 @@ int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky,
                        part);
     hipLaunchKernelGGL(k_geo_final, dim3(1), dim3(256), 0, st, kb, xb, (const unsigned *)part,
                        geo);
-    hipLaunchKernelGGL(k_geo_check, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, x, y, geo);
+    if (n)
+        hipLaunchKernelGGL(k_geo_check, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, x, y, z, geo);
     IMP_CHECK_LAUNCH();
-    unsigned h[G_WORDS];
     IMP_HIP(hipMemcpyAsync(h, geo, sizeof(h), hipMemcpyDeviceToHost, st));
     IMP_HIP(hipStreamSynchronize(st));
-    int nA = 0;
+    return IMP_OK;
+}
+
+// Geometry of an image problem (z null: 2D; else z fastest): axes A and B and
+// the ranges of t and w, or ok = false when the separable evaluation does not
+// apply.  Synchronises (one small read-back).
+int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                   const float *x, const float *y, const float *z, const float *fm,
+                   NuGeometry *G) {
+    G->ok = false;
+    unsigned h[G_WORDS];
+    IMP_TRY(geo_scan(ctx, m, n, kx, ky, t, x, y, z, fm, h));
+    int nA = 0, nz = 0;
     bool a_is_y = false;
-    if (h[G_FLAGS] || h[G_KFLAG] || !geo_axes(h[G_FCX], h[G_FCY], n, &a_is_y, &nA)) return IMP_OK;
-    const int nB = n / nA;
+    if (h[G_FLAGS] || h[G_KFLAG] ||
+        !geo_axes(h[G_FCX], h[G_FCY], n, z != nullptr, &a_is_y, &nA, &nz))
+        return IMP_OK;
+    const int nB = n / (nA * nz);
     auto lo = [&](int i) { return dec_f(h[G_MIN + i]); };
     auto hi = [&](int i) { return dec_f(h[G_MAX + i]); };
     const int a = a_is_y ? 1 : 0, b = 1 - a;
@@ -1481,13 +1511,13 @@ int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky,
                    lo(b), hi(b), &G->B))
         return IMP_OK;
     const double tlo = lo(2), thi = hi(2), wlo = fm ? lo(5) : 0.0, whi = fm ? hi(5) : 0.0;
+    G->nz = nz;
     G->tc = 0.5 * (tlo + thi);
     G->th = 0.5 * (thi - tlo);
     G->wc = 0.5 * (wlo + whi);
     G->wh = 0.5 * (whi - wlo);
-    if (!prolate_expand(G->wh * G->th, G->coef, G->mul, &G->nt, &G->nleg)) return IMP_OK;
     G->a_is_y = a_is_y;
-    G->ok = true;
+    G->ok = G->wh * G->th <= NU_MAX_THETA;
     return IMP_OK;
 }
 
@@ -1502,7 +1532,7 @@ struct Carver {
     }
 };
 
-// largest spread-grid block and A-transformed grid (bytes): coils go in
+// largest spread-grid block and A-transformed grid (bytes): columns go in
 // groups so the second stays below its limit, rows in blocks for the first
 constexpr size_t NU_BLOCK_BYTES = (size_t)512 << 20;
 constexpr size_t NU_MID_BYTES = (size_t)3 << 30;
@@ -1513,164 +1543,200 @@ int log2i(int n) {
     return b;
 }
 
-}  // namespace
-
-double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils) {
-    const double cols = (double)G.nt * (1 << log2i(ncoils));
-    const double grid = (double)G.A.nf * G.B.nf + (double)G.A.n * G.B.nf;
-    return 250.0 + 3.0e-5 * m * cols + 1.0e-5 * grid * cols;
+// time terms as the predicted times use them (the exact count follows from
+// prolate_expand; within 2)
+double terms_estimate(const NuGeometry &G) {
+    const double th = G.wh * G.th;
+    return th > 0.0 ? 8.0 + 1.2 * std::pow(th, 0.9) : 1.0;
 }
 
-int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int n, int ncoils, const float *kx,
-                  const float *ky, const float *t, const float *x, const float *y,
-                  const float *fm, const float *phi_r, const float *phi_i, const float *d_r,
-                  const float *d_i, const float *s_r, const float *s_i, float *out_r,
-                  float *out_i) {
-    const hipStream_t st = ctx->stream;
-    const NuAxis &A = G.A, &B = G.B;
-    const float *kA = G.a_is_y ? ky : kx, *kB = G.a_is_y ? kx : ky;
-    const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
-    const int nA = A.n, nB = B.n, nt = G.nt;
-    const size_t nvox = (size_t)nA * nB;
-    // coils per group: a power of two up to 32 whose A-transformed grid fits
-    int cg = std::min(32, 1 << log2i(ncoils));
-    while (cg > 1 && (size_t)nA * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
-    // wave layout: coil slots x time groups x rows = 32 lane pairs; fewer
-    // coils when the time terms need more groups
-    while (cg > 1 && ceil_div(nt, 32 / cg) > SP_MAX_NL) cg /= 2;
-    const int groups = ceil_div(ncoils, cg);
-    const int lc = log2i(cg), ll = std::min(5 - lc, log2i(nt));
-    const int nl = ceil_div(nt, 1 << ll);
-    const int yg = 1 << (5 - lc - ll);
-    const bool uni = lc == 5;
-    const int T = sp_switch(nl, [](auto k) { return sp_cells(decltype(k)::value); });
-    const int ntp = nl << ll;
-    // spread geometry
+// The stages shared by the separable operators: samples sorted by window,
+// tables, work lists; then per group of columns, weights -> spread grid ->
+// mid[ia][gB][q].
+struct NuPass {
+    imp_ctx *ctx;
+    const NuGeometry &G;
+    int m;                         // samples
+    const float *kA, *kB, *t;
+    int nt = 1, nleg = 1;          // time terms
+    std::vector<double> tab;       // coefficients, recurrence, mul, KB polynomials
+    size_t tab_mul = 0, tab_poly = 0;
+    int cg = 1, groups = 1, lc = 0, ll = 0, nl = 1, yg = 1, T = 1, ntp = 1, blocks = 1;
+    bool uni = false;
     SpGeom S{};
-    S.T = T;
-    S.yg = yg;
-    S.ncA = A.nf - NW + 1;
-    S.ncB = B.nf - NW + 1;
-    S.nfA = A.nf;
-    S.nfB = B.nf;
-    S.ntx = ceil_div(A.nf, T);
-    const int nc0 = std::min(cg, ncoils);
-    const size_t row_bytes = (size_t)A.nf * nt * nc0 * sizeof(double2);
-    int rb = (int)std::max<size_t>(1, NU_BLOCK_BYTES / row_bytes);
-    rb = std::min(ceil_div(B.nf, yg) * yg, std::max(yg, rb / yg * yg));
-    const int blocks = ceil_div(B.nf, rb);
-    rb = ceil_div(ceil_div(B.nf, blocks), yg) * yg;   // even blocks
-    S.rb = rb;
-    S.nty = rb / yg;
-    const int ntile = S.ntx * S.nty;
-    S.entry_cap = ntile + SP_SLOTS;
-    const int ncells = S.ncA * S.ncB;
-    const int nblk = ceil_div(m, RX_BLOCK);
-    const int splits_max = 8;
-    // --- workspace: tables, then grids
     Carver W;
-    const size_t o_key0 = W.take((size_t)m * 4), o_key1 = W.take((size_t)m * 4);
-    const size_t o_val0 = W.take((size_t)m * 4), o_val1 = W.take((size_t)m * 4);
-    const size_t o_hist = W.take((size_t)RX_BINS * nblk * 4);
-    const size_t o_start = W.take(((size_t)ncells + 1) * 4);
-    const size_t o_bx = W.take((size_t)m * 4);
-    const size_t o_wx = W.take((size_t)m * (NW + 2 * (T - 1)) * 8);
-    const size_t o_wy = W.take((size_t)m * (NW + 2 * (yg - 1)) * 8);
-    const size_t o_u = W.take((size_t)m * ntp * 8);
-    const size_t o_wd = W.take((size_t)m * (1 << lc) * sizeof(double2));
-    const size_t o_vis = W.take((size_t)blocks * ntile * 4);
-    const size_t o_cnt = W.take((size_t)blocks * sizeof(SpCount));
-    const size_t o_ent = W.take((size_t)blocks * S.entry_cap * sizeof(SpEntry));
-    const size_t o_mul = W.take((size_t)blocks * SP_SLOTS * sizeof(SpMulti));
-    const size_t o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * 8);
-    const size_t o_coef = W.take(G.coef.size() * 8);
-    const size_t o_mu = W.take(G.mul.size() * 8);
-    const size_t o_poly = W.take(KB_WORDS * 8);
-    size_t o_tw[2], o_in[2], o_ow[2], o_ob[2];
-    for (int a = 0; a < 2; ++a) {
-        const NuAxis &X = a ? B : A;
-        o_tw[a] = W.take((size_t)X.L * sizeof(double2));
-        o_in[a] = W.take((size_t)X.nf * 8);
-        o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
-        o_ob[a] = W.take((size_t)X.n * 4);
+    size_t o_bx, o_wx, o_wy, o_u, o_wd, o_vis, o_cnt, o_ent, o_mul, o_part, o_tab, o_start,
+        o_grid, o_mid, o_tw[2], o_in[2], o_ow[2], o_ob[2];
+    char *ws = nullptr;
+    const int *perm = nullptr, *key = nullptr;
+
+    NuPass(imp_ctx *c, const NuGeometry &g, int m_, const float *kx, const float *ky,
+           const float *t_)
+        : ctx(c), G(g), m(m_), kA(g.a_is_y ? ky : kx), kB(g.a_is_y ? kx : ky), t(t_) {}
+
+    // samples sorted by window start (launched before the time expansion is
+    // computed on the host)
+    int sort() {
+        const hipStream_t st = ctx->stream;
+        const int ncells = (G.A.nf - NW + 1) * (G.B.nf - NW + 1), nblk = ceil_div(m, RX_BLOCK);
+        Carver c;
+        const size_t k0 = c.take((size_t)m * 4), k1 = c.take((size_t)m * 4);
+        const size_t v0 = c.take((size_t)m * 4), v1 = c.take((size_t)m * 4);
+        const size_t hi = c.take((size_t)RX_BINS * nblk * 4);
+        void *p = nullptr;
+        IMP_TRY(workspace(ctx, WS_NU_SORT, c.off, &p));
+        char *b = (char *)p;
+        int *key0 = (int *)(b + k0), *key1 = (int *)(b + k1);
+        int *val0 = (int *)(b + v0), *val1 = (int *)(b + v1), *hist = (int *)(b + hi);
+        hipLaunchKernelGGL(k_nu_keys, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, kA, kB, G.A,
+                           G.B, key0, val0);
+        for (int shift = 0; shift == 0 || (ncells - 1) >> shift; shift += 8) {
+            hipLaunchKernelGGL(k_rx_count, dim3(nblk), dim3(256), 0, st, (const int *)key0, m,
+                               shift, hist);
+            hipLaunchKernelGGL(k_rx_scatter, dim3(nblk), dim3(256), 0, st, (const int *)key0,
+                               (const int *)val0, m, shift, nblk, (const int *)hist, key1, val1);
+            std::swap(key0, key1);
+            std::swap(val0, val1);
+        }
+        IMP_CHECK_LAUNCH();
+        key = key0;
+        perm = val0;
+        return IMP_OK;
     }
-    const size_t o_vt = W.take((size_t)nt * nvox * 8);
-    const size_t o_sens = W.take(s_r ? (size_t)ncoils * nvox * sizeof(float2) : 0);
-    const size_t o_img = W.take((size_t)groups * splits_max * nvox * sizeof(double2));
-    const size_t o_grid = W.take((size_t)rb * row_bytes);
-    const size_t o_mid = W.take((size_t)nA * B.nf * nt * nc0 * sizeof(double2));
-    void *wsp = nullptr;
-    IMP_TRY(workspace(ctx, WS_NU, W.off, &wsp));
-    char *ws = (char *)wsp;
-    int *key0 = (int *)(ws + o_key0), *key1 = (int *)(ws + o_key1);
-    int *val0 = (int *)(ws + o_val0), *val1 = (int *)(ws + o_val1);
-    int *hist = (int *)(ws + o_hist), *start = (int *)(ws + o_start);
-    SpCount *cnt = (SpCount *)(ws + o_cnt);
-    double *coef = (double *)(ws + o_coef), *mul = (double *)(ws + o_mu);
-    double *poly = (double *)(ws + o_poly);
-    const int rec = prof_begin(ctx, "nufft_adjoint");
-    IMP_HIP(hipMemcpyAsync(coef, G.coef.data(), G.coef.size() * 8, hipMemcpyHostToDevice, st));
-    IMP_HIP(hipMemcpyAsync(poly, kb_poly_table(), KB_WORDS * 8, hipMemcpyHostToDevice, st));
-    IMP_HIP(hipMemcpyAsync(mul, G.mul.data(), G.mul.size() * 8, hipMemcpyHostToDevice, st));
-    // --- samples sorted by window start
-    const dim3 gm(ceil_div(m, 256)), b256(256);
-    hipLaunchKernelGGL(k_nu_keys, gm, b256, 0, st, m, kA, kB, A, B, key0, val0);
-    for (int shift = 0; shift == 0 || (ncells - 1) >> shift; shift += 8) {
-        hipLaunchKernelGGL(k_rx_count, dim3(nblk), b256, 0, st, (const int *)key0, m, shift,
-                           hist);
-        hipLaunchKernelGGL(k_rx_scatter, dim3(nblk), b256, 0, st, (const int *)key0,
-                           (const int *)val0, m, shift, nblk, (const int *)hist, key1, val1);
-        std::swap(key0, key1);
-        std::swap(val0, val1);
+
+    // sizes for ncols columns of coils (or other right-hand sides) and the
+    // time expansion; the caller then takes its own regions from W
+    int layout(int ncols) {
+        std::vector<double> mul;
+        if (!prolate_expand(G.wh * G.th, tab, mul, &nt, &nleg))
+            return fail(IMP_EINVAL, "NUDFT: time expansion of %g", G.wh * G.th);
+        tab_mul = tab.size();
+        tab.insert(tab.end(), mul.begin(), mul.end());
+        tab_poly = tab.size();
+        tab.insert(tab.end(), kb_poly_table(), kb_poly_table() + KB_WORDS);
+        const NuAxis &A = G.A, &B = G.B;
+        cg = std::min(32, 1 << log2i(ncols));
+        while (cg > 1 && (size_t)A.n * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
+        // wave layout: column slots x time groups x rows = 32 lane pairs;
+        // fewer columns when the time terms need more groups
+        while (cg > 1 && ceil_div(nt, 32 / cg) > SP_MAX_NL) cg /= 2;
+        groups = ceil_div(ncols, cg);
+        lc = log2i(cg);
+        ll = std::min(5 - lc, log2i(nt));
+        nl = ceil_div(nt, 1 << ll);
+        yg = 1 << (5 - lc - ll);
+        uni = lc == 5;
+        T = sp_switch(nl, [](auto k) { return sp_cells(decltype(k)::value); });
+        ntp = nl << ll;
+        S.T = T;
+        S.yg = yg;
+        S.ncA = A.nf - NW + 1;
+        S.ncB = B.nf - NW + 1;
+        S.nfA = A.nf;
+        S.nfB = B.nf;
+        S.ntx = ceil_div(A.nf, T);
+        const int nc0 = std::min(cg, ncols);
+        const size_t row_bytes = (size_t)A.nf * nt * nc0 * sizeof(double2);
+        int rb = (int)std::max<size_t>(1, NU_BLOCK_BYTES / row_bytes);
+        rb = std::min(ceil_div(B.nf, yg) * yg, std::max(yg, rb / yg * yg));
+        blocks = ceil_div(B.nf, rb);
+        rb = ceil_div(ceil_div(B.nf, blocks), yg) * yg;   // even blocks
+        blocks = ceil_div(B.nf, rb);
+        S.rb = rb;
+        S.nty = rb / yg;
+        S.entry_cap = S.ntx * S.nty + SP_SLOTS;
+        const int ncells = S.ncA * S.ncB;
+        o_start = W.take(((size_t)ncells + 1) * 4);
+        o_bx = W.take((size_t)m * 4);
+        o_wx = W.take((size_t)m * (NW + 2 * (T - 1)) * 8);
+        o_wy = W.take((size_t)m * (NW + 2 * (yg - 1)) * 8);
+        o_u = W.take((size_t)m * ntp * 8);
+        o_wd = W.take((size_t)m * (1 << lc) * sizeof(double2));
+        o_vis = W.take((size_t)blocks * S.ntx * S.nty * 4);
+        o_cnt = W.take((size_t)blocks * sizeof(SpCount));
+        o_ent = W.take((size_t)blocks * S.entry_cap * sizeof(SpEntry));
+        o_mul = W.take((size_t)blocks * SP_SLOTS * sizeof(SpMulti));
+        o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * 8);
+        o_tab = W.take(tab.size() * 8);
+        for (int a = 0; a < 2; ++a) {
+            const NuAxis &X = a ? B : A;
+            o_tw[a] = W.take((size_t)X.L * sizeof(double2));
+            o_in[a] = W.take((size_t)X.nf * 8);
+            o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
+            o_ob[a] = W.take((size_t)X.n * 4);
+        }
+        o_grid = W.take((size_t)rb * row_bytes);
+        o_mid = W.take((size_t)A.n * B.nf * nt * nc0 * sizeof(double2));
+        return IMP_OK;
     }
-    IMP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m,
-                       (const int *)key0, ncells, start);
-    hipLaunchKernelGGL(k_nu_prep, dim3(ceil_div(m, PREP_S)), b256, 0, st, m, (const int *)val0, kA,
-                       kB, t, A, B, G.tc, G.th > 0.0 ? 1.0 / G.th : 0.0, (const double *)coef,
-                       (const double *)poly, nt, ntp, G.nleg, T - 1, yg - 1, (int *)(ws + o_bx),
-                       (double *)(ws + o_wx), (double *)(ws + o_wy), (double *)(ws + o_u));
-    // --- spread work lists, image-side tables
-    hipLaunchKernelGGL(k_sp_zero, dim3(ceil_div((long)(blocks * sizeof(SpCount) / 4), 256)), b256,
-                       0, st, (int *)cnt, (int)(blocks * sizeof(SpCount) / 4));
-    hipLaunchKernelGGL(k_sp_count, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
-                       (const int *)start, (int *)(ws + o_vis), cnt);
-    hipLaunchKernelGGL(k_sp_list, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
-                       (const int *)(ws + o_vis), cnt, (SpEntry *)(ws + o_ent),
-                       (SpMulti *)(ws + o_mul));
-    for (int a = 0; a < 2; ++a) {
-        const NuAxis &X = a ? B : A;
-        const int len = std::max(std::max(X.L, X.nf), X.n);
-        hipLaunchKernelGGL(k_nu_axis, dim3(ceil_div(len, 256)), b256, 0, st, X, a ? cB : cA,
-                           a ? nA : 1, (double2 *)(ws + o_tw[a]), (double *)(ws + o_in[a]),
-                           (double *)(ws + o_ow[a]), (int *)(ws + o_ob[a]));
+
+    template <class P>
+    P at(size_t o) const { return (P)(ws + o); }
+    const double *coef() const { return at<const double *>(o_tab); }
+    const double *mul() const { return coef() + tab_mul; }
+
+    // Allocates everything taken from W and fills the tables.  cA, cB: axis
+    // coordinates, sA and sB elements apart (read on nonuniform axes).
+    int build(const float *cA, int sA, const float *cB, int sB) {
+        const hipStream_t st = ctx->stream;
+        const dim3 b256(256);
+        void *p = nullptr;
+        IMP_TRY(workspace(ctx, WS_NU, W.off, &p));
+        ws = (char *)p;
+        // staged in pinned memory: free, since the geometry read-back of this
+        // call waited for every earlier upload
+        if (tab.size() > HOST_TABLE_WORDS)
+            return fail(IMP_EINVAL, "NUDFT: %zu table words", tab.size());
+        std::copy(tab.begin(), tab.end(), ctx->host_tables());
+        IMP_HIP(hipMemcpyAsync(ws + o_tab, ctx->host_tables(), tab.size() * 8,
+                               hipMemcpyHostToDevice, st));
+        const int ncells = S.ncA * S.ncB, ntile = S.ntx * S.nty;
+        SpCount *cnt = at<SpCount *>(o_cnt);
+        hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m, key,
+                           ncells, at<int *>(o_start), (int *)cnt,
+                           (int)(blocks * sizeof(SpCount) / 4));
+        hipLaunchKernelGGL(k_nu_prep, dim3(ceil_div(m, PREP_S)), b256, 0, st, m, perm, kA, kB, t,
+                           G.A, G.B, G.tc, G.th > 0.0 ? 1.0 / G.th : 0.0, coef(),
+                           coef() + tab_poly, nt, ntp, nleg, T - 1, yg - 1, at<int *>(o_bx),
+                           at<double *>(o_wx), at<double *>(o_wy), at<double *>(o_u));
+        hipLaunchKernelGGL(k_sp_count, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
+                           at<const int *>(o_start), at<int *>(o_vis), cnt);
+        hipLaunchKernelGGL(k_sp_list, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
+                           at<const int *>(o_vis), cnt, at<SpEntry *>(o_ent),
+                           at<SpMulti *>(o_mul));
+        AxisTab ta[2];
+        int len = 0;
+        for (int a = 0; a < 2; ++a) {
+            const NuAxis &X = a ? G.B : G.A;
+            len = std::max(len, std::max(std::max(X.L, X.nf), X.n));
+            ta[a] = AxisTab{X, a ? cB : cA, a ? sB : sA, at<double2 *>(o_tw[a]),
+                            at<double *>(o_in[a]), at<double *>(o_ow[a]), at<int *>(o_ob[a])};
+        }
+        hipLaunchKernelGGL(k_nu_axis, dim3(ceil_div(len, 256), 2), b256, 0, st, ta[0], ta[1]);
+        IMP_CHECK_LAUNCH();
+        return IMP_OK;
     }
-    hipLaunchKernelGGL(k_nu_vt, dim3(ceil_div((long)nvox, 256), nt), b256, 0, st, nA, nB, fm, G.wc,
-                       G.wh > 0.0 ? 1.0 / G.wh : 0.0, nt, (const double *)coef,
-                       (const double *)mul, G.nleg, (double *)(ws + o_vt));
-    if (s_r)
-        hipLaunchKernelGGL(k_nu_sens, dim3(ceil_div(nA, 32), ceil_div(nB, 32), ncoils), b256, 0,
-                           st, nA, nB, s_r, s_i, (float2 *)(ws + o_sens));
-    IMP_CHECK_LAUNCH();
-    // --- per coil group: spread and transform row blocks, then the B axis
-    SpFn spread = sp_switch(nl, [&](auto k) { return sp_pick1<decltype(k)::value>(uni); });
-    SpFn multi = sp_switch(nl, [](auto k) { return sp_multi1<decltype(k)::value>(); });
-    LineArgs LA{}, LB{};
-    LA.X = A;
-    LB.X = B;
-    LineArgs *LX[2] = {&LA, &LB};
-    for (int a = 0; a < 2; ++a) {
-        LX[a]->tw = (const double2 *)(ws + o_tw[a]);
-        LX[a]->inw = (const double *)(ws + o_in[a]);
-        LX[a]->outw = (const double *)(ws + o_ow[a]);
-        LX[a]->base = (const int *)(ws + o_ob[a]);
+
+    LineArgs line(int axis, const void *in, size_t in_line, unsigned in_el, int nq) const {
+        LineArgs P{};
+        P.in = (const double2 *)in;
+        P.in_line = in_line;
+        P.in_el = in_el;
+        P.nq = nq;
+        P.X = axis ? G.B : G.A;
+        P.tw = at<const double2 *>(o_tw[axis]);
+        P.inw = at<const double *>(o_in[axis]);
+        P.outw = at<const double *>(o_ow[axis]);
+        P.base = at<const int *>(o_ob[axis]);
+        return P;
     }
-    int parts = 0;
-    for (int g = 0; g < groups; ++g) {
-        const int c0 = g * cg, nc = std::min(cg, ncoils - c0), nq = nt * nc;
-        hipLaunchKernelGGL(k_nu_data, dim3(ceil_div(m, WD_S)), b256, 0, st, m, c0, nc, 1 << lc, kA,
-                           kB, t, A, B, G.tc, G.wc / (2.0 * M_PI), phi_r, phi_i, d_r, d_i,
-                           (double2 *)(ws + o_wd));
+
+    // weights of nc columns (in wd) -> mid[ia][gB][l nc + c]
+    int to_mid(int nc) {
+        const hipStream_t st = ctx->stream;
+        const int nq = nt * nc;
+        SpFn spread = sp_switch(nl, [&](auto k) { return sp_pick1<decltype(k)::value>(uni); });
+        SpFn multi = sp_switch(nl, [](auto k) { return sp_multi1<decltype(k)::value>(); });
         SpArgs P{};
         P.G = S;
         P.nt = nt;
@@ -1678,52 +1744,219 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int n, int ncoils, c
         P.nc = nc;
         P.lc = lc;
         P.ll = ll;
-        P.start = start;
-        P.perm = val0;
-        P.bx = (const int *)(ws + o_bx);
-        P.wx = (const double *)(ws + o_wx);
-        P.wy = (const double *)(ws + o_wy);
-        P.u = (const double *)(ws + o_u);
-        P.wd = (const double *)(ws + o_wd);
-        P.cnt = cnt;
-        P.entries = (const SpEntry *)(ws + o_ent);
-        P.multis = (const SpMulti *)(ws + o_mul);
-        P.part = (double *)(ws + o_part);
-        P.grid = (double *)(ws + o_grid);
+        P.start = at<const int *>(o_start);
+        P.perm = perm;
+        P.bx = at<const int *>(o_bx);
+        P.wx = at<const double *>(o_wx);
+        P.wy = at<const double *>(o_wy);
+        P.u = at<const double *>(o_u);
+        P.wd = at<const double *>(o_wd);
+        P.cnt = at<const SpCount *>(o_cnt);
+        P.entries = at<const SpEntry *>(o_ent);
+        P.multis = at<const SpMulti *>(o_mul);
+        P.part = at<double *>(o_part);
+        P.grid = at<double *>(o_grid);
+        LineArgs LA = line(0, ws + o_grid, (size_t)G.A.nf * nq, nq, nq);
         for (int b = 0; b < blocks; ++b) {
-            P.r0 = b * rb;
+            P.r0 = b * S.rb;
             P.block = b;
             // one-wave workgroups: a wave that ends makes room at once
+            const int rec = prof_begin(ctx, "k_spread");
             hipLaunchKernelGGL(spread, dim3(std::min(S.entry_cap, 64 * ctx->num_cus)), dim3(64),
                                0, st, P);
-            hipLaunchKernelGGL(multi, dim3(4 * ctx->num_cus), b256, 0, st, P);
+            prof_end(ctx, rec);
+            hipLaunchKernelGGL(multi, dim3(4 * ctx->num_cus), dim3(256), 0, st, P);
             IMP_CHECK_LAUNCH();
-            LA.in = (const double2 *)(ws + o_grid);
-            LA.in_line = (size_t)A.nf * nq;
-            LA.in_el = nq;
-            LA.nq = nq;
-            // mid[ia][gB][q]
-            IMP_TRY(line_store(ctx, LA, std::min(rb, B.nf - b * rb),
-                               (double2 *)(ws + o_mid) + (size_t)b * rb * nq, nq,
-                               (size_t)B.nf * nq));
+            IMP_TRY(line_store(ctx, LA, std::min(S.rb, G.B.nf - b * S.rb),
+                               at<double2 *>(o_mid) + (size_t)b * S.rb * nq, nq,
+                               (size_t)G.B.nf * nq));
         }
-        LB.in = (const double2 *)(ws + o_mid);
-        LB.in_line = (size_t)B.nf * nq;
-        LB.in_el = nq;
-        LB.nq = nq;
-        const int panels = line_switch(B.L, [&](auto len) -> int {
-            return ceil_div(nq, ln::lines(decltype(len)::value, CO_WG));
+        return IMP_OK;
+    }
+    LineArgs lines_b(int nc) const {
+        return line(1, ws + o_mid, (size_t)G.B.nf * nt * nc, nt * nc, nt * nc);
+    }
+};
+
+}  // namespace
+
+// predicted microseconds of the spread and transforms of ncols columns of nt
+// time terms, without the fixed part
+static double separable_us(const NuAxis &A, const NuAxis &B, int m, double cols) {
+    return 3.0e-5 * m * cols + 1.0e-5 * ((double)A.nf * B.nf + (double)A.n * B.nf) * cols;
+}
+
+double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils) {
+    return 250.0 + separable_us(G.A, G.B, m, terms_estimate(G) * (1 << log2i(ncoils)));
+}
+
+int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
+                  const float *ky, const float *t, const float *x, const float *y,
+                  const float *fm, const float *phi_r, const float *phi_i, const float *d_r,
+                  const float *d_i, const float *s_r, const float *s_i, float *out_r,
+                  float *out_i) {
+    const hipStream_t st = ctx->stream;
+    const dim3 b256(256);
+    const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
+    const int nA = G.A.n, nB = G.B.n;
+    const size_t nvox = (size_t)nA * nB;
+    const int rec = prof_begin(ctx, "nufft_adjoint");
+    NuPass N(ctx, G, m, kx, ky, t);
+    IMP_TRY(N.sort());
+    IMP_TRY(N.layout(ncoils));
+    constexpr int splits_max = 8;
+    const size_t o_vt = N.W.take((size_t)N.nt * nvox * 8);
+    const size_t o_sens = N.W.take(s_r ? (size_t)ncoils * nvox * sizeof(float2) : 0);
+    const size_t o_img = N.W.take((size_t)N.groups * splits_max * nvox * sizeof(double2));
+    IMP_TRY(N.build(cA, 1, cB, nA));
+    hipLaunchKernelGGL(k_nu_vt, dim3(ceil_div((long)nvox, 256), N.nt), b256, 0, st, nA, nB, fm,
+                       G.wc, G.wh > 0.0 ? 1.0 / G.wh : 0.0, N.nt, N.coef(), N.mul(), N.nleg,
+                       N.at<double *>(o_vt));
+    if (s_r)
+        hipLaunchKernelGGL(k_nu_sens, dim3(ceil_div(nA, 32), ceil_div(nB, 32), ncoils), b256, 0,
+                           st, nA, nB, s_r, s_i, N.at<float2 *>(o_sens));
+    IMP_CHECK_LAUNCH();
+    int parts = 0;
+    for (int g = 0; g < N.groups; ++g) {
+        const int c0 = g * N.cg, nc = std::min(N.cg, ncoils - c0);
+        hipLaunchKernelGGL(k_nu_data, dim3(ceil_div(m, WD_S)), b256, 0, st, m, c0, nc, 1 << N.lc,
+                           N.kA, N.kB, t, G.A, G.B, G.tc, G.wc / (2.0 * M_PI), phi_r, phi_i, d_r,
+                           d_i, N.at<double2 *>(N.o_wd));
+        IMP_TRY(N.to_mid(nc));
+        const LineArgs LB = N.lines_b(nc);
+        const int panels = line_switch(G.B.L, [&](auto len) -> int {
+            return ceil_div(LB.nq, ln::lines(decltype(len)::value, CO_WG));
         });
         const int splits =
             std::max(1, std::min(std::min(splits_max, panels), 12 * ctx->num_cus / nA));
-        IMP_TRY(line_combine(ctx, LB, nA, nc, splits, (const double *)(ws + o_vt),
-                             s_r ? (const float2 *)(ws + o_sens) + (size_t)c0 * nvox : nullptr,
-                             nvox, (double2 *)(ws + o_img) + (size_t)parts * nvox));
+        IMP_TRY(line_combine(ctx, LB, nA, nc, splits, N.at<const double *>(o_vt),
+                             s_r ? N.at<const float2 *>(o_sens) + (size_t)c0 * nvox : nullptr,
+                             nvox, N.at<double2 *>(o_img) + (size_t)parts * nvox));
         parts += splits;
     }
     hipLaunchKernelGGL(k_nu_out, dim3(ceil_div(nA, 16), ceil_div(nB, 16)), b256, 0, st, nA, nB,
-                       parts, (const double2 *)(ws + o_img), cA, cB, fm, A.kc, B.kc,
+                       parts, N.at<const double2 *>(o_img), cA, cB, fm, G.A.kc, G.B.kc,
                        G.tc / (2.0 * M_PI), out_r, out_i);
+    prof_end(ctx, rec);
+    IMP_CHECK_LAUNCH();
+    return IMP_OK;
+}
+
+// ------------------------------------------------------------------------ Q_l
+// Q_l(r) = sum_k a_l(t_k) |phi_k|^2 e^{i 2pi k.r} on the standard grid
+// r = (ix/Nx, iy/Ny), |ix| <= Nx, |iy| <= Ny.  The weights are real, so
+// segments 2c and 2c + 1 share a column: with w = a_2c + i a_(2c+1) the
+// column's sum is P = Q_2c + i Q_(2c+1), and Q_l(-r) = conj(Q_l(r)) gives
+// Q_2c = (P(r) + conj(P(-r))) / 2, Q_(2c+1) = (P(r) - conj(P(-r))) / 2i, so
+// Q_l comes out conjugate-symmetric bit for bit.
+// Against the GEMM over phasor tables (toeplitz_q_sep) it is faster at every
+// size measured (16^2 x 50 samples: 0.23 -> 0.17 ms; 512^2, 393216 samples,
+// L = 10: 255 -> 1.3 ms, 240 of it the allocation of 9 GB of tables on each
+// call) and closer to 64 bits (2.6e-8 against 1.1e-7), so on 2D standard
+// grids the GEMM is left to grids beyond the transform lengths.
+namespace {
+
+// [sample][slot] = (a_2c, a_(2c+1)) |phi|^2, a_l the Hanning interpolator of
+// hanning_d (computeQ.cmem.cu:125-138)
+__global__ void k_nu_qdata(int m, int nseg, int slots, const float *t, const float *phi_r,
+                           const float *phi_i, float tau, float t0, double2 *wd) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m * slots) return;
+    const int j = i / slots, c = i % slots;
+    double mag = 1.0;
+    if (phi_r) {
+        const double pr = phi_r[j], pi = phi_i[j];
+        mag = pr * pr + pi * pi;
+    }
+    double w[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int l = 2 * c + h;
+        const double arg = (double)t[j] - (double)tau * l - (double)t0;
+        w[h] = l < nseg && fabs(arg) < (double)tau
+                   ? (0.5 + 0.5 * cospi(arg / (double)tau)) * mag : 0.0;
+    }
+    wd[i] = make_double2(w[0], w[1]);
+}
+
+// P[ib][ia][c] (both edges of each axis kept) -> Q_l [iy][ix] without the far
+// edges; cumulative: prefix sums over l
+__global__ __launch_bounds__(256) void k_nu_qout(int Nx, int Ny, int nc, int nseg,
+                                                 int cumulative, const double2 *P, double kcx,
+                                                 double kcy, float *q_r, float *q_i) {
+    const int ix = blockIdx.x * 256 + threadIdx.x, iy = blockIdx.y;
+    if (ix >= 2 * Nx) return;
+    const int nx = 2 * Nx + 1, ny = 2 * Ny + 1;
+    const double2 *a = P + ((size_t)iy * nx + ix) * nc;
+    const double2 *b = P + ((size_t)(ny - 1 - iy) * nx + (nx - 1 - ix)) * nc;
+    const double rev = kcx * (ix - Nx) / Nx + kcy * (iy - Ny) / Ny;
+    double s, c;
+    sincospi(2.0 * (rev - rint(rev)), &s, &c);
+    const double2 e = make_double2(0.5 * c, 0.5 * s);
+    const size_t nq = (size_t)4 * Nx * Ny, o = (size_t)iy * 2 * Nx + ix;
+    double2 run = make_double2(0.0, 0.0);
+    for (int q = 0; q < nc; ++q) {
+        const double2 p = a[q], r = b[q];
+        const double2 v[2] = {cmul(make_double2(p.x + r.x, p.y - r.y), e),
+                              cmul(make_double2(p.y + r.y, r.x - p.x), e)};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int l = 2 * q + h;
+            if (l >= nseg) break;
+            run = cumulative ? make_double2(run.x + v[h].x, run.y + v[h].y) : v[h];
+            q_r[(size_t)l * nq + o] = (float)run.x;
+            q_i[(size_t)l * nq + o] = (float)run.y;
+        }
+    }
+}
+
+}  // namespace
+
+// Geometry of Q on the standard (Nx, Ny) grid; ok = false when it does not fit.
+int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
+                     int Ny, int nseg, NuGeometry *G) {
+    G->ok = false;
+    unsigned h[G_WORDS];
+    IMP_TRY(geo_scan(ctx, m, 0, kx, ky, t, nullptr, nullptr, nullptr, nullptr, h));
+    if (h[G_KFLAG]) return IMP_OK;
+    for (int a = 0; a < 2; ++a) {
+        NuAxis &X = a ? G->B : G->A;
+        const int N = a ? Ny : Nx;
+        if (!plan_axis(2 * N + 1, -1.f, 1.f, 0.f, -1.f, 1.f, dec_f(h[G_MIN + a]),
+                       dec_f(h[G_MAX + a]), &X))
+            return IMP_OK;
+        X.xc = 0.0;
+        X.inv_d = (double)X.L / N;   // exactly, as the grid defines it
+    }
+    G->nz = 1;
+    G->tc = dec_f(h[G_MIN + 2]);
+    G->th = G->wc = G->wh = 0.0;
+    G->a_is_y = false;
+    // all columns in one group
+    G->ok = ((size_t)G->A.n * G->B.nf * sizeof(double2) << log2i((nseg + 1) / 2)) <= NU_MID_BYTES;
+    return IMP_OK;
+}
+
+int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const float *ky,
+            const float *t, const float *phi_r, const float *phi_i, int Nx, int Ny, int nseg,
+            float tau, float t0, bool cumulative, float *q_r, float *q_i) {
+    const hipStream_t st = ctx->stream;
+    const int rec = prof_begin(ctx, "nufft_q");
+    const int cols = (nseg + 1) / 2;
+    NuPass N(ctx, G, m, kx, ky, t);
+    IMP_TRY(N.sort());
+    IMP_TRY(N.layout(cols));
+    const size_t o_p = N.W.take((size_t)G.A.n * G.B.n * cols * sizeof(double2));
+    IMP_TRY(N.build(nullptr, 1, nullptr, 1));
+    if (N.groups != 1) return fail(IMP_EINVAL, "toeplitz_q: %d column groups", N.groups);
+    hipLaunchKernelGGL(k_nu_qdata, dim3(ceil_div((long)m << N.lc, 256)), dim3(256), 0, st, m, nseg,
+                       1 << N.lc, t, phi_r, phi_i, tau, t0, N.at<double2 *>(N.o_wd));
+    IMP_TRY(N.to_mid(cols));
+    IMP_TRY(line_store(ctx, N.lines_b(cols), G.A.n, N.at<double2 *>(o_p), cols,
+                       (size_t)G.A.n * cols));
+    hipLaunchKernelGGL(k_nu_qout, dim3(ceil_div(2 * Nx, 256), 2 * Ny), dim3(256), 0, st, Nx, Ny,
+                       cols, nseg, cumulative ? 1 : 0, N.at<const double2 *>(o_p), G.A.kc, G.B.kc,
+                       q_r, q_i);
     prof_end(ctx, rec);
     IMP_CHECK_LAUNCH();
     return IMP_OK;

@@ -1,5 +1,5 @@
-"""The separable F^H d of large 2D problems (csrc/nufft.hip) against the FP64
-oracle and against the direct kernels.
+"""The separable F^H d of large 2D problems and the 2D Q_l (csrc/nufft.hip)
+against the FP64 oracle and against the direct kernels.
 
 Tolerance: 2e-7 relative L2.  The separable form sums in FP64 and rounds once
 to FP32 (at most 6e-8 per value); its time expansion and its two kernel
@@ -159,3 +159,40 @@ def test_adjoint_separable_repeats_bits_and_matches_direct(ctx):
          None, None, ptr(dr), ptr(di), ptr(sr), ptr(si), ptr(o[0]), ptr(o[1]))
     ctx.synchronize()
     assert rel_l2(a, o[0].get() + 1j * o[1].get()) < DIRECT_TOL
+
+
+@pytest.mark.parametrize("Nx,Ny,L,M,phi,flags", [
+    (8, 8, 0, 40, False, 0), (16, 12, 1, 300, True, 0), (21, 17, 4, 501, False, 1),
+    (32, 33, 7, 2000, True, 1), (64, 48, 12, 3001, False, 0), (24, 32, 31, 1000, False, 0)])
+def test_q_separable(ctx, Nx, Ny, L, M, phi, flags):
+    """Q_l on the 2D standard grid: even and odd segment counts, cumulative
+    sums, odd sizes; exactly conjugate-symmetric."""
+    from impatient import ops
+    from oracle import oracle as orc
+    p = _problem(Nx, Ny, 1, M, seed=7)
+    r = np.random.default_rng(8)
+    ph = (1 + 0.2 * r.standard_normal(M) + 0.2j * r.standard_normal(M)).astype(np.complex64)
+    ph = ph if phi else None
+    t = np.sort(p["t"])
+    got, (n,) = _timer(ctx, lambda: ops.toeplitz_q(ctx, p["kx"], p["ky"], None, t, Nx, Ny, 1, L, ph,
+                                                   flags), "nufft_q")
+    assert n == 1
+    ref = orc.toeplitz_q(p["kx"], p["ky"], None, t, Nx, Ny, 1, L, ph, cumulative=bool(flags & 1))
+    errs = [rel_l2(a, b) for a, b in zip(got, ref)]
+    print(f"worst segment {max(errs):.2e}")
+    assert max(errs) < TOL
+    q = got.reshape(L + 1, 2 * Ny, 2 * Nx)[:, 1:, 1:]
+    assert np.array_equal(q, np.conj(q[:, ::-1, ::-1]))
+
+
+def test_q_beyond_transforms_stays_gemm(ctx):
+    """Samples far beyond the grid's band and non-finite ones keep the table
+    GEMM."""
+    from impatient import ops
+    p = _problem(16, 16, 1, 200)
+    for v in (3e5, np.nan):
+        kx = p["kx"].copy()
+        kx[5] = v
+        _, n = _timer(ctx, lambda: ops.toeplitz_q(ctx, kx, p["ky"], None, np.sort(p["t"]), 16, 16,
+                                                  1, 2), "nufft_q", "k_q_sep")
+        assert n == [0, 1]

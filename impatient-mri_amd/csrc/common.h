@@ -13,7 +13,8 @@
 
 namespace imp {
 
-constexpr size_t HOST_TABLE_WORDS = 4096;   // of imp_ctx::host_tables()
+constexpr size_t HOST_TABLE_WORDS = 2048;   // of a slot of imp_ctx::host_tables()
+constexpr int HOST_TABLES = 32;             // slots
 
 // ---------------------------------------------------------------- errors
 // Thread-local last error; every C entry point records its failure here.
@@ -95,9 +96,10 @@ struct imp_ctx {
     size_t dscratch_n = 0;
     // pinned host words for scalar readback
     double *host_scalars = nullptr;
-    // pinned host words for the separable NUDFT's tables (uploads from it may
-    // still be running when the call that filled it returns; the next such
-    // call synchronises the stream before it writes)
+    // pinned host slots for the separable NUDFT's tables: uploads from them
+    // may still run when the call that filled one returns; table_slot is the
+    // next free one, 0 again whenever the stream has been waited for
+    int table_slot = 0;
     double *host_tables() const { return host_scalars + 64; }
     // FFT twiddle tables: table for length L at offset L (L = 2..2048)
     float2 *twiddle = nullptr;

@@ -150,7 +150,7 @@ extern "C" int imp_ctx_create(int device, imp_ctx **out) {
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->num_cus = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc((void **)&ctx->host_scalars, (64 + HOST_TABLE_WORDS) * sizeof(double),
+        hipHostMalloc((void **)&ctx->host_scalars, (64 + HOST_TABLES * HOST_TABLE_WORDS) * sizeof(double),
                       hipHostMallocDefault) !=
             hipSuccess) {
         (void)hipGetLastError();

@@ -1261,8 +1261,10 @@ size_t adjoint_fixed_bytes(int num_k, int num_x, int ncoils, bool d3) {
 // transforms, behind a fixed part (geometry read-back, sort, ~20 launches).
 constexpr double NUFFT_MIN_PAIRS = 6e8;   // below: the direct kernels win at every size measured
 
+constexpr double DIRECT_FIXED_US = 60.0;
+
 double direct_us(double pairs, int ncoils) {
-    return 60.0 + pairs * (ncoils <= 1 ? 7.9e-4 : ncoils == 2 ? 8.4e-4
+    return DIRECT_FIXED_US + pairs * (ncoils <= 1 ? 7.9e-4 : ncoils == 2 ? 8.4e-4
                            : ncoils <= MF_COLS ? 5.6e-4 : 8.1e-4);
 }
 
@@ -1391,10 +1393,14 @@ int nudft_adjoint_noalloc(imp_ctx *ctx, int num_k, int num_x, int ncoils, const 
                         phi_i, d_r, d_i, s_r, s_i, out_r, out_i);
 }
 
-// F^H d of several images (different sizes, trajectories, coil maps) with
-// one persistent MFMA launch over all of them.  Every job needs 3..32 coils
-// and the same dimensionality.  chunk_scale multiplies the per-job
-// workgroup target (the autotuned knob; 0 = default 8 per CU).
+static int adjoint_batch_direct(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
+                                int chunk_scale, bool d3, int tiles);
+
+// F^H d of several images (different sizes, trajectories, coil maps).  Every
+// job needs 3..32 coils and the same dimensionality.  Large 2D images take the
+// separable form one after another (one geometry read-back for all); the rest
+// share one persistent MFMA launch.  chunk_scale multiplies the per-job
+// workgroup target of that launch (the autotuned knob; 0 = default 8 per CU).
 int nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs, int chunk_scale) {
     if (!ctx || njobs <= 0 || !jobs) return fail(IMP_EINVAL, "nudft_adjoint_batch: bad arguments");
     const bool d3 = jobs[0].kz && jobs[0].z;
@@ -1414,6 +1420,35 @@ int nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs, int 
         if (t != tiles)
             return fail(IMP_EUNSUPPORTED, "nudft_adjoint_batch: jobs need the same coil tile count");
     }
+    std::vector<char> scan(njobs, 0);
+    std::vector<NuGeometry> G(njobs);
+    bool any = false;
+    for (int j = 0; j < njobs && !d3; ++j) {
+        scan[j] = (double)jobs[j].num_k * jobs[j].num_x >= NUFFT_MIN_PAIRS;
+        any = any || scan[j];
+    }
+    std::vector<imp_nudft_job> rest;
+    if (any) IMP_TRY(nufft_geometry_batch(ctx, njobs, jobs, scan, &G));
+    for (int j = 0; j < njobs; ++j) {
+        const imp_nudft_job &b = jobs[j];
+        // the launch's fixed part is shared by the direct jobs
+        if (G[j].ok && nufft_adjoint_us(G[j], b.num_k, b.ncoils) <
+                           direct_us((double)b.num_k * b.num_x, b.ncoils) - DIRECT_FIXED_US)
+            IMP_TRY(nufft_adjoint(ctx, G[j], b.num_k, b.ncoils, b.kx, b.ky, b.t, b.x, b.y, b.fm,
+                                  b.phi_r, b.phi_i, b.d_r, b.d_i, b.s_r, b.s_i, b.out_r,
+                                  b.out_i));
+        else
+            rest.push_back(b);
+    }
+    if (rest.empty()) {
+        IMP_HIP(hipStreamSynchronize(ctx->stream));
+        return IMP_OK;
+    }
+    return adjoint_batch_direct(ctx, (int)rest.size(), rest.data(), chunk_scale, d3, tiles);
+}
+
+static int adjoint_batch_direct(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
+                                int chunk_scale, bool d3, int tiles) {
     const long target = (long)(chunk_scale > 0 ? chunk_scale : 8) * ctx->num_cus;
     // carve one workspace: per job spos, lanes, W, maxbits, bpack, partials
     struct Lay {

@@ -36,6 +36,8 @@ bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double>
 int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
                    const float *x, const float *y, const float *z, const float *fm,
                    NuGeometry *G);
+int nufft_geometry_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
+                         const std::vector<char> &scan, std::vector<NuGeometry> *G);
 // Predicted time of nufft_adjoint in microseconds (for the choice against
 // the direct kernels).
 double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils);

@@ -1466,14 +1466,11 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
 }  // namespace
 
 // Scan of the operands: value ranges, tensor structure of the voxels.  n = 0
-// scans the samples alone.
-static int geo_scan(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
-                    const float *x, const float *y, const float *z, const float *fm,
-                    unsigned (&h)[G_WORDS]) {
+// scans the samples alone.  geo: G_WORDS result words, part: block results.
+static int geo_enqueue(imp_ctx *ctx, unsigned *geo, unsigned *part, int m, int n, const float *kx,
+                       const float *ky, const float *t, const float *x, const float *y,
+                       const float *z, const float *fm) {
     const hipStream_t st = ctx->stream;
-    void *w = nullptr;
-    IMP_TRY(workspace(ctx, WS_NU_GEO, (G_WORDS + 512 * GB_WORDS) * sizeof(unsigned), &w));
-    unsigned *geo = (unsigned *)w, *part = geo + G_WORDS;
     const int kb = std::min(256, ceil_div(m, 1024)), xb = std::min(256, ceil_div(n, 1024));
     hipLaunchKernelGGL(k_geo_scan, dim3(kb + xb), dim3(256), 0, st, m, kx, ky, t, n, x, y, fm, kb,
                        part);
@@ -1482,25 +1479,35 @@ static int geo_scan(imp_ctx *ctx, int m, int n, const float *kx, const float *ky
     if (n)
         hipLaunchKernelGGL(k_geo_check, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, x, y, z, geo);
     IMP_CHECK_LAUNCH();
-    IMP_HIP(hipMemcpyAsync(h, geo, sizeof(h), hipMemcpyDeviceToHost, st));
-    IMP_HIP(hipStreamSynchronize(st));
     return IMP_OK;
 }
 
-// Geometry of an image problem (z null: 2D; else z fastest): axes A and B and
-// the ranges of t and w, or ok = false when the separable evaluation does not
-// apply.  Synchronises (one small read-back).
-int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
-                   const float *x, const float *y, const float *z, const float *fm,
-                   NuGeometry *G) {
+static int geo_buffers(imp_ctx *ctx, int scans, unsigned **geo, unsigned **part) {
+    void *w = nullptr;
+    IMP_TRY(workspace(ctx, WS_NU_GEO,
+                      ((size_t)scans * G_WORDS + 512 * GB_WORDS) * sizeof(unsigned), &w));
+    *geo = (unsigned *)w;
+    *part = *geo + (size_t)scans * G_WORDS;
+    return IMP_OK;
+}
+
+// results of `scans` scans on the host; waits for the stream
+static int geo_read(imp_ctx *ctx, const unsigned *geo, int scans, unsigned *h) {
+    IMP_HIP(hipMemcpyAsync(h, geo, (size_t)scans * G_WORDS * sizeof(unsigned),
+                           hipMemcpyDeviceToHost, ctx->stream));
+    IMP_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->table_slot = 0;   // no table upload is in flight
+    return IMP_OK;
+}
+
+// Axes A and B and the ranges of t and w from a scan, or ok = false when the
+// separable evaluation does not apply.
+static void geo_image(const unsigned *h, int n, bool d3, bool fm, NuGeometry *G) {
     G->ok = false;
-    unsigned h[G_WORDS];
-    IMP_TRY(geo_scan(ctx, m, n, kx, ky, t, x, y, z, fm, h));
     int nA = 0, nz = 0;
     bool a_is_y = false;
-    if (h[G_FLAGS] || h[G_KFLAG] ||
-        !geo_axes(h[G_FCX], h[G_FCY], n, z != nullptr, &a_is_y, &nA, &nz))
-        return IMP_OK;
+    if (h[G_FLAGS] || h[G_KFLAG] || !geo_axes(h[G_FCX], h[G_FCY], n, d3, &a_is_y, &nA, &nz))
+        return;
     const int nB = n / (nA * nz);
     auto lo = [&](int i) { return dec_f(h[G_MIN + i]); };
     auto hi = [&](int i) { return dec_f(h[G_MAX + i]); };
@@ -1509,7 +1516,7 @@ int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky,
                    lo(a), hi(a), &G->A) ||
         !plan_axis(nB, bits_f(h[G_B0]), bits_f(h[G_B1]), bits_f(h[G_DEVB]), lo(3 + b), hi(3 + b),
                    lo(b), hi(b), &G->B))
-        return IMP_OK;
+        return;
     const double tlo = lo(2), thi = hi(2), wlo = fm ? lo(5) : 0.0, whi = fm ? hi(5) : 0.0;
     G->nz = nz;
     G->tc = 0.5 * (tlo + thi);
@@ -1518,6 +1525,39 @@ int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky,
     G->wh = 0.5 * (whi - wlo);
     G->a_is_y = a_is_y;
     G->ok = G->wh * G->th <= NU_MAX_THETA;
+}
+
+// Geometry of an image problem (z null: 2D; else z fastest).  Synchronises
+// (one small read-back).
+int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                   const float *x, const float *y, const float *z, const float *fm,
+                   NuGeometry *G) {
+    unsigned h[G_WORDS], *geo, *part;
+    IMP_TRY(geo_buffers(ctx, 1, &geo, &part));
+    IMP_TRY(geo_enqueue(ctx, geo, part, m, n, kx, ky, t, x, y, z, fm));
+    IMP_TRY(geo_read(ctx, geo, 1, h));
+    geo_image(h, n, z != nullptr, fm != nullptr, G);
+    return IMP_OK;
+}
+
+// The same for several 2D images with one read-back (jobs with scan[j] false
+// are left out).
+int nufft_geometry_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
+                         const std::vector<char> &scan, std::vector<NuGeometry> *G) {
+    unsigned *geo, *part;
+    IMP_TRY(geo_buffers(ctx, njobs, &geo, &part));
+    for (int j = 0; j < njobs; ++j) {
+        const imp_nudft_job &b = jobs[j];
+        if (scan[j])
+            IMP_TRY(geo_enqueue(ctx, geo + (size_t)j * G_WORDS, part, b.num_k, b.num_x, b.kx, b.ky,
+                                b.t, b.x, b.y, nullptr, b.fm));
+    }
+    std::vector<unsigned> h((size_t)njobs * G_WORDS);
+    IMP_TRY(geo_read(ctx, geo, njobs, h.data()));
+    for (int j = 0; j < njobs; ++j)
+        if (scan[j])
+            geo_image(&h[(size_t)j * G_WORDS], jobs[j].num_x, false, jobs[j].fm != nullptr,
+                      &(*G)[j]);
     return IMP_OK;
 }
 
@@ -1683,13 +1723,16 @@ struct NuPass {
         void *p = nullptr;
         IMP_TRY(workspace(ctx, WS_NU, W.off, &p));
         ws = (char *)p;
-        // staged in pinned memory: free, since the geometry read-back of this
-        // call waited for every earlier upload
+        // staged in a slot of the context's pinned memory that no upload reads
         if (tab.size() > HOST_TABLE_WORDS)
             return fail(IMP_EINVAL, "NUDFT: %zu table words", tab.size());
-        std::copy(tab.begin(), tab.end(), ctx->host_tables());
-        IMP_HIP(hipMemcpyAsync(ws + o_tab, ctx->host_tables(), tab.size() * 8,
-                               hipMemcpyHostToDevice, st));
+        if (ctx->table_slot >= HOST_TABLES) {
+            IMP_HIP(hipStreamSynchronize(st));
+            ctx->table_slot = 0;
+        }
+        double *slot = ctx->host_tables() + (size_t)ctx->table_slot++ * HOST_TABLE_WORDS;
+        std::copy(tab.begin(), tab.end(), slot);
+        IMP_HIP(hipMemcpyAsync(ws + o_tab, slot, tab.size() * 8, hipMemcpyHostToDevice, st));
         const int ncells = S.ncA * S.ncB, ntile = S.ntx * S.nty;
         SpCount *cnt = at<SpCount *>(o_cnt);
         hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m, key,
@@ -1916,8 +1959,10 @@ __global__ __launch_bounds__(256) void k_nu_qout(int Nx, int Ny, int nc, int nse
 int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
                      int Ny, int nseg, NuGeometry *G) {
     G->ok = false;
-    unsigned h[G_WORDS];
-    IMP_TRY(geo_scan(ctx, m, 0, kx, ky, t, nullptr, nullptr, nullptr, nullptr, h));
+    unsigned h[G_WORDS], *geo, *part;
+    IMP_TRY(geo_buffers(ctx, 1, &geo, &part));
+    IMP_TRY(geo_enqueue(ctx, geo, part, m, 0, kx, ky, t, nullptr, nullptr, nullptr, nullptr));
+    IMP_TRY(geo_read(ctx, geo, 1, h));
     if (h[G_KFLAG]) return IMP_OK;
     for (int a = 0; a < 2; ++a) {
         NuAxis &X = a ? G->B : G->A;

@@ -196,3 +196,20 @@ def test_q_beyond_transforms_stays_gemm(ctx):
         _, n = _timer(ctx, lambda: ops.toeplitz_q(ctx, kx, p["ky"], None, np.sort(p["t"]), 16, 16,
                                                   1, 2), "nufft_q", "k_q_sep")
         assert n == [0, 1]
+
+
+def test_batch_mixes_separable_and_direct_jobs(ctx):
+    """Large jobs of a batch take the separable form and equal the single call
+    bit for bit; small ones share the direct launch."""
+    from impatient import ops
+    ps = [_problem(48, 48, 5, 3000, seed=1), _problem(200, 187, 6, 60013, seed=2),
+          _problem(64, 40, 3, 2000, seed=3), _problem(192, 192, 8, 70000, seed=4)]
+    jobs = [dict(kx=p["kx"], ky=p["ky"], t=p["t"], x=p["x"], y=p["y"], fm=p["fm"], d=p["d"],
+                 sens=p["s"]) for p in ps]
+    got, n = _timer(ctx, lambda: ops.nudft_adjoint_batch(ctx, jobs), "nufft_adjoint",
+                    "k_nudft_mfma_batch")
+    assert n == [2, 1]
+    for p, g, big in zip(ps, got, (False, True, False, True)):
+        one = ops.nudft_adjoint(ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"],
+                                p["d"], p["s"])
+        assert np.array_equal(g, one) if big else rel_l2(g, one) < DIRECT_TOL

@@ -1274,7 +1274,7 @@ double direct_us(double pairs, int ncoils) {
 // (the geometry is read back).
 int choose_separable(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *kx,
                      const float *ky, const float *t, const float *x, const float *y,
-                     const float *fm, NuGeometry *G) {
+                     const float *fm, bool forward, NuGeometry *G) {
     G->ok = false;
     const double pairs = (double)num_k * num_x;
     if (pairs < NUFFT_MIN_PAIRS || ncoils > 2 * MF_COLS) return IMP_OK;
@@ -1282,13 +1282,17 @@ int choose_separable(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float
     IMP_HIP(hipStreamIsCapturing(ctx->stream, &cap));
     if (cap != hipStreamCaptureStatusNone) return IMP_OK;
     IMP_TRY(nufft_geometry(ctx, num_k, num_x, kx, ky, t, x, y, nullptr, fm, G));
-    if (G->ok && nufft_adjoint_us(*G, num_k, ncoils) >= direct_us(pairs, ncoils)) G->ok = false;
+    const double us = forward ? nufft_forward_us(*G, num_k, ncoils)
+                              : nufft_adjoint_us(*G, num_k, ncoils);
+    if (G->ok && us >= direct_us(pairs, ncoils)) G->ok = false;
     return IMP_OK;
 }
 
-// Workspaces of the direct adjoint of this size, so that a call captured into
-// a graph after calls that took the separable form finds them allocated.
-int reserve_direct(imp_ctx *ctx, int num_k, int num_x, int ncoils) {
+// Workspaces of the direct sum of this size (num_k streamed samples, num_x
+// points; the other way round for the forward operator), so that a call
+// captured into a graph after calls that took the separable form finds them
+// allocated.
+int reserve_direct(imp_ctx *ctx, int num_k, int num_x, int ncoils, bool per_coil) {
     void *p = nullptr;
     IMP_TRY(workspace(ctx, WS_SPOS, spos_bytes(num_k, false), &p));
     IMP_TRY(workspace(ctx, WS_LANES, (size_t)num_x * sizeof(float4), &p));
@@ -1305,7 +1309,8 @@ int reserve_direct(imp_ctx *ctx, int num_k, int num_x, int ncoils) {
     } else {
         const int chunks = pick_chunks(ctx, ceil_div(num_x, NU_THREADS), num_k, 4 * NU_BLK);
         IMP_TRY(workspace(ctx, WS_BPACK, (size_t)num_k * 2 * ncoils * sizeof(float), &p));
-        IMP_TRY(workspace(ctx, WS_PARTIAL, (size_t)chunks * num_x * sizeof(float2), &p));
+        IMP_TRY(workspace(ctx, WS_PARTIAL,
+                          (size_t)chunks * (per_coil ? ncoils : 1) * num_x * sizeof(float2), &p));
     }
     return IMP_OK;
 }
@@ -1321,9 +1326,9 @@ int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
         return fail(IMP_EINVAL, "nudft_adjoint: bad arguments");
     if (!(kz && z)) {
         NuGeometry G;
-        IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, &G));
+        IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, false, &G));
         if (G.ok) {
-            IMP_TRY(reserve_direct(ctx, num_k, num_x, ncoils));
+            IMP_TRY(reserve_direct(ctx, num_k, num_x, ncoils, false));
             return nufft_adjoint(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
                                  d_r, d_i, s_r, s_i, out_r, out_i);
         }
@@ -1586,6 +1591,15 @@ int nudft_forward(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
             IMP_TRY(run_job(ctx, J));
         }
         return IMP_OK;
+    }
+    if (!d3) {
+        NuGeometry G;
+        IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, true, &G));
+        if (G.ok) {
+            IMP_TRY(reserve_direct(ctx, num_x, num_k, ncoils, true));
+            return nufft_forward(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, rho_r, rho_i, s_r,
+                                 s_i, d_r, d_i);
+        }
     }
     const double *spos = nullptr;
     IMP_TRY(build_spos(ctx, num_x, x, y, d3 ? z : nullptr, fm, 1.0 / (2.0 * M_PI), &spos));

@@ -47,6 +47,12 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
                   const float *d_i, const float *s_r, const float *s_i, float *out_r,
                   float *out_i);
 
+double nufft_forward_us(const NuGeometry &G, int m, int ncoils);
+int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
+                  const float *ky, const float *t, const float *x, const float *y,
+                  const float *fm, const float *rho_r, const float *rho_i, const float *s_r,
+                  const float *s_i, float *d_r, float *d_i);
+
 int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
                      int Ny, int nseg, NuGeometry *G);
 int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const float *ky,

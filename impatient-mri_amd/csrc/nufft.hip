@@ -1306,6 +1306,353 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_line_c
     }
 }
 
+// ------------------------------------------------------- forward (voxels -> k)
+// The same separation read the other way round.  With conj(d) = sum conj(S rho)
+// e^{+i(2pi k.r + w t)} every transform keeps the sign of the adjoint:
+//   V_q(r) = conj(S_c rho) e^{i(2pi kc.r + w tc)} i^(l mod 2) vt[l],
+// divided by the kernel's transform and summed onto the k grid one axis at a
+// time; then each sample gathers its NW x NW window of every column.
+
+// i-th output of a transformed line at grid points g = i + j0 mod L
+template <bool UNI>
+__device__ __forceinline__ void fline_out(const LineArgs &P, double2 *base, unsigned el, unsigned c,
+                                          int L, int i, double2 v) {
+    int g = i + P.X.shift;
+    if (g >= L) g -= L;
+    if constexpr (UNI) {
+        for (; g < P.X.nf; g += L) base[(unsigned)g * el + c] = v;
+    } else if (g < P.X.nf) {
+        const double w = P.inw[g];
+        base[(unsigned)g * el + c] = make_double2(v.x * w, v.y * w);
+    }
+}
+
+// One axis, image points -> grid.  FIRST: the points' values are formed here
+// (line = ia, points ib) from img0 = conj(rho) e^{i(...)}, the maps and vt;
+// else read from P.in as in k_line_store.  Nonuniform points are spread onto
+// the line's L cells through LDS: cell p sums the points of its list
+// (P.base[p] .. P.base[p + 1]; ascending, so the sum's order is fixed).
+template <int L, bool UNI, bool FIRST>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_fline(
+    LineArgs P, const int *list, const double *listw, int ncg, const double2 *img0,
+    const float2 *sens, const double *vt, unsigned nvox, double2 *out, size_t out_line,
+    unsigned out_el) {
+    constexpr int E = ln::vals(L), W = ln::lines(L, CO_WG), T = ln::threads(L);
+    constexpr int R0 = ln::radix(L, 0);
+    __shared__ double buf[ln::words(L, W)];
+    const int c = threadIdx.x % W, t = threadIdx.x / W;
+    const int np = (P.nq + W - 1) / W;
+    const int b = (blockIdx.x & ~15) | ((blockIdx.x & 7) << 1) | ((blockIdx.x >> 3) & 1);
+    const int line = b / np, q = (b % np) * W + c;
+    if (line >= P.nlines) return;
+    const bool ok = q < P.nq;
+    const int l = ok ? q / ncg : 0, cc = ok ? q - l * ncg : 0;
+    auto point = [&](int i) {
+        if (!ok) return make_double2(0.0, 0.0);
+        if constexpr (FIRST) {
+            const size_t x = (size_t)line * P.X.n + i;
+            double2 v = img0[x];
+            if (sens) {
+                const float2 s = sens[(size_t)cc * nvox + x];
+                v = make_double2(v.x * s.x + v.y * s.y, v.y * s.x - v.x * s.y);
+            }
+            const double f = vt[(size_t)l * nvox + x];
+            return (l & 1) ? make_double2(-f * v.y, f * v.x) : make_double2(f * v.x, f * v.y);
+        } else {
+            return P.in[(size_t)line * P.in_line + (size_t)i * P.in_el + q];
+        }
+    };
+    double2 v[E];
+    if constexpr (UNI) {
+#pragma unroll
+        for (int i = 0; i < E; ++i) {
+            const unsigned x = bin_index(P.X, L, ln::in_idx<L, 0>(t, i / R0, i % R0));
+            v[i] = make_double2(0.0, 0.0);
+            if (x < (unsigned)P.X.n) {
+                const double2 z = point(x);
+                const double w = P.outw[x];
+                v[i] = make_double2(z.x * w, z.y * w);
+            }
+        }
+    } else {
+        double2 z[E];
+#pragma unroll
+        for (int m = 0; m < E; ++m)
+            z[m] = t + T * m < P.X.n ? point(t + T * m) : make_double2(0.0, 0.0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < E; ++m)
+                if (t + T * m < P.X.n) buf[(t + T * m) * W + c] = h ? z[m].y : z[m].x;
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                const int p = ln::in_idx<L, 0>(t, i / R0, i % R0);
+                double s = 0.0;
+                for (int e = P.base[p]; e < P.base[p + 1]; ++e)
+                    s = fma(listw[e], buf[list[e] * W + c], s);
+                if (h) v[i].y = s;
+                else v[i].x = s;
+            }
+        }
+    }
+    ln::transform<L, W>(v, t, c, buf, P.tw);
+    if (!ok) return;
+    constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
+    double2 *o = out + (size_t)line * out_line + (q - c);
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        fline_out<UNI>(P, o, out_el, c, L, ln::out_idx<L, S>(t, i / R, i % R), v[i]);
+}
+
+// Lists of k_fline's nonuniform axes: cell p of L takes the points within
+// NW/2 cells of it (their positions wrap), weight kb / kb_hat.  One workgroup
+// per axis counts, scans and fills; each cell visits the points in order.
+struct FListTab {
+    NuAxis X;
+    const float *coord;
+    int stride;
+    int *first;       // [L + 1]
+    int *list;        // [n (NW + 1)]
+    double *w;
+};
+__global__ __launch_bounds__(1024) void k_nu_flists(FListTab ta, FListTab tb) {
+    const FListTab &P = blockIdx.x ? tb : ta;
+    const NuAxis &X = P.X;
+    if (X.uniform) return;
+    __shared__ double pos[4096];
+    __shared__ int sm[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < X.n; i += 1024)
+        pos[i] = ((double)P.coord[(size_t)i * P.stride] - X.xc) / X.inv_d * X.L;
+    __syncthreads();
+    // points of cell p: |pos - p| <= NW/2 as the windows of k_nu_axis take it
+    auto visit = [&](int p, auto f) {
+        for (int i = 0; i < X.n; ++i) {
+            const int b = (int)ceil(pos[i] - 0.5 * NW);
+            int k = (p - b) % X.L;
+            if (k < 0) k += X.L;
+            if (k < NW) f(i, b + k);
+        }
+    };
+    int carry = 0;
+    for (int p0 = 0; p0 < X.L; p0 += 1024) {
+        const int p = p0 + threadIdx.x;
+        int n = 0;
+        if (p < X.L) visit(p, [&](int, int) { ++n; });
+        int inc = n;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += o;
+        }
+        if (lane == 63) sm[wave] = inc;
+        __syncthreads();
+        int before = carry, total = 0;
+        for (int w = 0; w < 16; ++w) {
+            if (w < wave) before += sm[w];
+            total += sm[w];
+        }
+        if (p < X.L) {
+            int at = before + inc - n;
+            P.first[p] = at;
+            visit(p, [&](int i, int cell) {
+                P.list[at] = i;
+                P.w[at++] = kb(pos[i] - cell) / kb_hat(pos[i] / X.L);
+            });
+        }
+        carry += total;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) P.first[X.L] = carry;
+}
+
+// img0[ia][ib] = conj(rho) e^{i(2pi kc.r + w tc)}
+__global__ __launch_bounds__(256) void k_nu_img0(int nA, int nB, const float *r_r,
+                                                 const float *r_i, const float *cA,
+                                                 const float *cB, const float *fm, double kcA,
+                                                 double kcB, double tc_2pi, double2 *img0) {
+    __shared__ double2 tile[16][17];
+    const int a0 = blockIdx.x * 16, b0 = blockIdx.y * 16;
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    {
+        const int ia = a0 + tx, ib = b0 + ty;
+        if (ia < nA && ib < nB) {
+            const size_t i = (size_t)ib * nA + ia;
+            const double rev = kcA * cA[i] + kcB * cB[i] + (fm ? tc_2pi * fm[i] : 0.0);
+            double s, c;
+            sincospi(2.0 * (rev - rint(rev)), &s, &c);
+            tile[tx][ty] = cmul(make_double2(r_r[i], -(double)r_i[i]), make_double2(c, s));
+        }
+    }
+    __syncthreads();
+    const int ia = a0 + ty, ib = b0 + tx;
+    if (ia < nA && ib < nB) img0[(size_t)ia * nB + ib] = tile[ty][tx];
+}
+
+// Samples of a tile of TG x TG window starts gather together: GI_S samples
+// per work entry.
+constexpr int TG = 4, GI_S = 16, GI_W = 16;   // GI_W >= NW + TG - 1 cells per row
+struct GiEntry {
+    int tile, s0, n, pad;
+};
+
+__global__ __launch_bounds__(256) void k_gi_list(int m, int ntile, const int *key,
+                                                 GiEntry *entries, int *count) {
+    __shared__ int first[256 + 1];   // first sample of the block's tiles, and one more
+    const int tile = blockIdx.x * 255 + threadIdx.x;
+    int lo = 0, hi = m;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (key[mid] < tile) lo = mid + 1;
+        else hi = mid;
+    }
+    first[threadIdx.x] = lo;
+    __syncthreads();
+    if (threadIdx.x == 255 || tile >= ntile) return;
+    const int n = first[threadIdx.x + 1] - lo, runs = (n + GI_S - 1) / GI_S;
+    if (!runs) return;
+    const int e0 = atomicAdd(count, runs);
+    for (int r = 0; r < runs; ++r)
+        entries[e0 + r] = GiEntry{tile, lo + r * GI_S, min(GI_S, n - r * GI_S), 0};
+}
+
+typedef double dx4 __attribute__((ext_vector_type(4)));
+
+struct GiArgs {
+    int ntx, nfA, nfB, nt, nc, c0, m;
+    const int *perm, *bx, *by;      // sorted
+    const double *wx, *wy;          // [s][NW + 2 (TG - 1)], zeros around the window
+    const double *u;                // [s][nt]
+    const double2 *rot;             // [s] e^{i(wc (t - tc) + 2pi kappa.xc)}
+    const int *count;
+    const GiEntry *entries;
+    const double *grid;             // [gB][gA][nt][nc][2]
+    float *d_r, *d_i;
+};
+
+// One wave per entry: out[sample][column] = sum over the tile's 15 rows x 16
+// cells and nt terms of (wx wy u)[sample] grid[column], a product of 16 x
+// 3840 nt/16 by 3840 nt/16 x 16 matrices on v_mfma_f64_16x16x4_f64 (sample i =
+// lane % 16 and cell k = lane / 16 of A, column j = lane % 16 of B, result row
+// lane / 16 + 4 r).  FP64 MFMA runs at half the FMA rate here, but needs the
+// weights once per lane instead of 16 of them in scalar registers per value.
+template <int CB>
+__global__ __launch_bounds__(64) void k_gather(GiArgs P) {
+    const int lane = threadIdx.x, i = lane & 15, k = lane >> 4;
+    const int ne = *P.count;
+    const int nq2 = P.nt * P.nc * 2;
+    for (int e = blockIdx.x; e < ne; e += gridDim.x) {
+        const GiEntry E = P.entries[e];
+        const int ga = (E.tile % P.ntx) * TG, gb = (E.tile / P.ntx) * TG;
+        const int s = E.s0 + min(i, E.n - 1);
+        constexpr int NX = NW + 2 * (TG - 1);
+        // cell offset of the tile inside the padded window of this sample
+        const double *px = P.wx + (size_t)s * NX + (ga - P.bx[s] + TG - 1);
+        const double *py = P.wy + (size_t)s * NX + (gb - P.by[s] + TG - 1);
+        const double live = i < E.n ? 1.0 : 0.0;
+        double wx[GI_W / 4];
+#pragma unroll
+        for (int h = 0; h < GI_W / 4; ++h)
+            wx[h] = 4 * h + k < NW + TG - 1 ? live * px[4 * h + k] : 0.0;
+        const double *pu = P.u + (size_t)s * P.nt;
+        dx4 acc[CB];
+#pragma unroll
+        for (int b = 0; b < CB; ++b) acc[b] = dx4{0.0, 0.0, 0.0, 0.0};
+        // columns of this lane: 16 values (8 coils, re and im) per block
+        int col[CB];
+#pragma unroll
+        for (int b = 0; b < CB; ++b) col[b] = min(16 * b + i, 2 * P.nc - 1);
+        for (int r = 0; r < NW + TG - 1 && gb + r < P.nfB; ++r) {
+            const double wy = py[r];
+            const double *row = P.grid + ((size_t)(gb + r) * P.nfA + ga) * nq2;
+#pragma unroll
+            for (int h = 0; h < GI_W / 4; ++h) {
+                const double a = wx[h] * wy;
+                // cells past the grid have weight zero: read the last one
+                const int g = min(4 * h + k, P.nfA - 1 - ga);
+                const double *cell = row + (size_t)g * nq2;
+                for (int l = 0; l < P.nt; ++l) {
+                    const double al = a * pu[l];
+#pragma unroll
+                    for (int b = 0; b < CB; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                            al, cell[l * 2 * P.nc + col[b]], acc[b], 0, 0, 0);
+                }
+            }
+        }
+        // row lane / 16 + 4 r is sample r * 4 + k of the entry
+#pragma unroll
+        for (int b = 0; b < CB; ++b) {
+            const int c = 8 * b + (i >> 1);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double mine = acc[b][r], other = __shfl_xor(mine, 1, 64);
+                const int n = 4 * r + k;
+                if (n >= E.n || c >= P.nc) continue;
+                const double2 z = P.rot[E.s0 + n];
+                const size_t o = (size_t)(P.c0 + c) * P.m + P.perm[E.s0 + n];
+                // conj((re + i im) rot)
+                if (i & 1) P.d_i[o] = (float)-(other * z.y + mine * z.x);
+                else P.d_r[o] = (float)(mine * z.x - other * z.y);
+            }
+        }
+    }
+}
+
+// per sorted sample: window starts, both axes' weights (TG - 1 zeros around),
+// time factors, rotation
+__global__ __launch_bounds__(256) void k_gi_prep(int m, const int *perm, const float *kA,
+                                                 const float *kB, const float *t, NuAxis A,
+                                                 NuAxis B, double tc, double tinv, double wc_cyc,
+                                                 const double *coef, const double *poly, int nt,
+                                                 int nleg, int *bx, int *by, double *wx,
+                                                 double *wy, double *u, double2 *rot) {
+    __shared__ double px[PREP_S], py[PREP_S], pt[PREP_S], pl[KB_WORDS];
+    const int s0 = blockIdx.x * PREP_S, ns = min(PREP_S, m - s0);
+    for (int i = threadIdx.x; i < KB_WORDS; i += 256) pl[i] = poly[i];
+    if ((int)threadIdx.x < ns) {
+        const int i = threadIdx.x, j = perm[s0 + i];
+        double p;
+        const int a = window(A, kA[j], &p);
+        px[i] = 2.0 * (p - a - (0.5 * NW - 1)) - 1.0;
+        bx[s0 + i] = a;
+        const int b = window(B, kB[j], &p);
+        py[i] = 2.0 * (p - b - (0.5 * NW - 1)) - 1.0;
+        by[s0 + i] = b;
+        pt[i] = clamp1(((double)t[j] - tc) * tinv);
+        const double rev = ((double)kA[j] - A.kc) * A.xc + ((double)kB[j] - B.kc) * B.xc +
+                           ((double)t[j] - tc) * wc_cyc;
+        double s, c;
+        sincospi(2.0 * (rev - rint(rev)), &s, &c);
+        rot[s0 + i] = make_double2(c, s);
+    }
+    __syncthreads();
+    constexpr int NX = NW + 2 * (TG - 1);
+    for (int e = threadIdx.x; e < ns * NX; e += 256) {
+        const int s = e / NX, g = e - s * NX - (TG - 1);
+        const bool in = g >= 0 && g < NW;
+        wx[(size_t)s0 * NX + e] = in ? kb_cell(pl, g, px[s]) : 0.0;
+        wy[(size_t)s0 * NX + e] = in ? kb_cell(pl, g, py[s]) : 0.0;
+    }
+    for (int e = threadIdx.x; e < ns * nt; e += 256) {
+        const int s = e / nt, l = e - s * nt;
+        u[(size_t)s0 * nt + e] =
+            prolate(coef + (size_t)l * nleg, coef + (size_t)nt * nleg, nleg, l & 1, pt[s]);
+    }
+}
+
+// tile of a sample's window start
+__global__ void k_gi_keys(int m, const float *kA, const float *kB, NuAxis A, NuAxis B, int ntx,
+                          int *key, int *val) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= m) return;
+    double s;
+    key[j] = (window(B, kB[j], &s) / TG) * ntx + window(A, kA[j], &s) / TG;
+    val[j] = j;
+}
+
 // vt[l][ia][ib] = m_l psi_l(w), in (A, B) order; one thread per value
 __global__ __launch_bounds__(256) void k_nu_vt(int nA, int nB, const float *fm, double wc,
                                                double winv, int nt, const double *coef,
@@ -1614,11 +1961,14 @@ struct NuPass {
            const float *t_)
         : ctx(c), G(g), m(m_), kA(g.a_is_y ? ky : kx), kB(g.a_is_y ? kx : ky), t(t_) {}
 
-    // samples sorted by window start (launched before the time expansion is
-    // computed on the host)
-    int sort() {
+    // samples sorted by window start (or by the gather's tiles of starts;
+    // launched before the time expansion is computed on the host)
+    int sort(bool tiles = false) {
         const hipStream_t st = ctx->stream;
-        const int ncells = (G.A.nf - NW + 1) * (G.B.nf - NW + 1), nblk = ceil_div(m, RX_BLOCK);
+        const int gtx = ceil_div(G.A.nf - NW + 1, TG);
+        const int ncells = tiles ? gtx * ceil_div(G.B.nf - NW + 1, TG)
+                                 : (G.A.nf - NW + 1) * (G.B.nf - NW + 1);
+        const int nblk = ceil_div(m, RX_BLOCK);
         Carver c;
         const size_t k0 = c.take((size_t)m * 4), k1 = c.take((size_t)m * 4);
         const size_t v0 = c.take((size_t)m * 4), v1 = c.take((size_t)m * 4);
@@ -1628,8 +1978,12 @@ struct NuPass {
         char *b = (char *)p;
         int *key0 = (int *)(b + k0), *key1 = (int *)(b + k1);
         int *val0 = (int *)(b + v0), *val1 = (int *)(b + v1), *hist = (int *)(b + hi);
-        hipLaunchKernelGGL(k_nu_keys, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, kA, kB, G.A,
-                           G.B, key0, val0);
+        if (tiles)
+            hipLaunchKernelGGL(k_gi_keys, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, kA, kB,
+                               G.A, G.B, gtx, key0, val0);
+        else
+            hipLaunchKernelGGL(k_nu_keys, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, kA, kB,
+                               G.A, G.B, key0, val0);
         for (int shift = 0; shift == 0 || (ncells - 1) >> shift; shift += 8) {
             hipLaunchKernelGGL(k_rx_count, dim3(nblk), dim3(256), 0, st, (const int *)key0, m,
                                shift, hist);
@@ -1646,7 +2000,7 @@ struct NuPass {
 
     // sizes for ncols columns of coils (or other right-hand sides) and the
     // time expansion; the caller then takes its own regions from W
-    int layout(int ncols) {
+    int expand() {
         std::vector<double> mul;
         if (!prolate_expand(G.wh * G.th, tab, mul, &nt, &nleg))
             return fail(IMP_EINVAL, "NUDFT: time expansion of %g", G.wh * G.th);
@@ -1654,6 +2008,21 @@ struct NuPass {
         tab.insert(tab.end(), mul.begin(), mul.end());
         tab_poly = tab.size();
         tab.insert(tab.end(), kb_poly_table(), kb_poly_table() + KB_WORDS);
+        return IMP_OK;
+    }
+    void take_tables() {
+        o_tab = W.take(tab.size() * 8);
+        for (int a = 0; a < 2; ++a) {
+            const NuAxis &X = a ? G.B : G.A;
+            o_tw[a] = W.take((size_t)X.L * sizeof(double2));
+            o_in[a] = W.take((size_t)X.nf * 8);
+            o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
+            o_ob[a] = W.take((size_t)X.n * 4);
+        }
+    }
+
+    int layout(int ncols) {
+        IMP_TRY(expand());
         const NuAxis &A = G.A, &B = G.B;
         cg = std::min(32, 1 << log2i(ncols));
         while (cg > 1 && (size_t)A.n * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
@@ -1697,14 +2066,7 @@ struct NuPass {
         o_ent = W.take((size_t)blocks * S.entry_cap * sizeof(SpEntry));
         o_mul = W.take((size_t)blocks * SP_SLOTS * sizeof(SpMulti));
         o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * 8);
-        o_tab = W.take(tab.size() * 8);
-        for (int a = 0; a < 2; ++a) {
-            const NuAxis &X = a ? B : A;
-            o_tw[a] = W.take((size_t)X.L * sizeof(double2));
-            o_in[a] = W.take((size_t)X.nf * 8);
-            o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
-            o_ob[a] = W.take((size_t)X.n * 4);
-        }
+        take_tables();
         o_grid = W.take((size_t)rb * row_bytes);
         o_mid = W.take((size_t)A.n * B.nf * nt * nc0 * sizeof(double2));
         return IMP_OK;
@@ -1715,11 +2077,11 @@ struct NuPass {
     const double *coef() const { return at<const double *>(o_tab); }
     const double *mul() const { return coef() + tab_mul; }
 
-    // Allocates everything taken from W and fills the tables.  cA, cB: axis
-    // coordinates, sA and sB elements apart (read on nonuniform axes).
-    int build(const float *cA, int sA, const float *cB, int sB) {
+    // Allocates everything taken from W, uploads the expansion and fills the
+    // axis tables.  cA, cB: axis coordinates, sA and sB elements apart (read
+    // on nonuniform axes).
+    int alloc(const float *cA, int sA, const float *cB, int sB) {
         const hipStream_t st = ctx->stream;
-        const dim3 b256(256);
         void *p = nullptr;
         IMP_TRY(workspace(ctx, WS_NU, W.off, &p));
         ws = (char *)p;
@@ -1733,6 +2095,24 @@ struct NuPass {
         double *slot = ctx->host_tables() + (size_t)ctx->table_slot++ * HOST_TABLE_WORDS;
         std::copy(tab.begin(), tab.end(), slot);
         IMP_HIP(hipMemcpyAsync(ws + o_tab, slot, tab.size() * 8, hipMemcpyHostToDevice, st));
+        AxisTab ta[2];
+        int len = 0;
+        for (int a = 0; a < 2; ++a) {
+            const NuAxis &X = a ? G.B : G.A;
+            len = std::max(len, std::max(std::max(X.L, X.nf), X.n));
+            ta[a] = AxisTab{X, a ? cB : cA, a ? sB : sA, at<double2 *>(o_tw[a]),
+                            at<double *>(o_in[a]), at<double *>(o_ow[a]), at<int *>(o_ob[a])};
+        }
+        hipLaunchKernelGGL(k_nu_axis, dim3(ceil_div(len, 256), 2), dim3(256), 0, st, ta[0], ta[1]);
+        IMP_CHECK_LAUNCH();
+        return IMP_OK;
+    }
+
+    // the spread's tables and work lists
+    int build(const float *cA, int sA, const float *cB, int sB) {
+        IMP_TRY(alloc(cA, sA, cB, sB));
+        const hipStream_t st = ctx->stream;
+        const dim3 b256(256);
         const int ncells = S.ncA * S.ncB, ntile = S.ntx * S.nty;
         SpCount *cnt = at<SpCount *>(o_cnt);
         hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m, key,
@@ -1747,15 +2127,6 @@ struct NuPass {
         hipLaunchKernelGGL(k_sp_list, dim3(ceil_div(ntile, 256), blocks), b256, 0, st, S,
                            at<const int *>(o_vis), cnt, at<SpEntry *>(o_ent),
                            at<SpMulti *>(o_mul));
-        AxisTab ta[2];
-        int len = 0;
-        for (int a = 0; a < 2; ++a) {
-            const NuAxis &X = a ? G.B : G.A;
-            len = std::max(len, std::max(std::max(X.L, X.nf), X.n));
-            ta[a] = AxisTab{X, a ? cB : cA, a ? sB : sA, at<double2 *>(o_tw[a]),
-                            at<double *>(o_in[a]), at<double *>(o_ow[a]), at<int *>(o_ob[a])};
-        }
-        hipLaunchKernelGGL(k_nu_axis, dim3(ceil_div(len, 256), 2), b256, 0, st, ta[0], ta[1]);
         IMP_CHECK_LAUNCH();
         return IMP_OK;
     }
@@ -1882,6 +2253,151 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
                        G.tc / (2.0 * M_PI), out_r, out_i);
     prof_end(ctx, rec);
     IMP_CHECK_LAUNCH();
+    return IMP_OK;
+}
+
+// ---------------------------------------------------------------- forward host
+namespace {
+
+int line_forward(imp_ctx *ctx, LineArgs P, int nlines, bool first, const int *list,
+                 const double *listw, int ncg, const double2 *img0, const float2 *sens,
+                 const double *vt, unsigned nvox, double2 *out, size_t out_line,
+                 unsigned out_el) {
+    P.nlines = nlines;
+    return line_switch(P.X.L, [&](auto len) -> int {
+        constexpr int L = decltype(len)::value;
+        const long wgs = ((long)nlines * ceil_div(P.nq, ln::lines(L, CO_WG)) + 15) & ~15L;
+        auto fn = P.X.uniform ? (first ? k_fline<L, true, true> : k_fline<L, true, false>)
+                              : (first ? k_fline<L, false, true> : k_fline<L, false, false>);
+        hipLaunchKernelGGL(fn, dim3((unsigned)wgs), dim3(ln::threads(L) * ln::lines(L, CO_WG)), 0,
+                           ctx->stream, P, list, listw, ncg, img0, sens, vt, nvox, out, out_line,
+                           out_el);
+        IMP_CHECK_LAUNCH();
+        return IMP_OK;
+    });
+}
+
+// k grid of a coil group (bytes)
+constexpr size_t NU_KGRID_BYTES = (size_t)2 << 30;
+
+}  // namespace
+
+double nufft_forward_us(const NuGeometry &G, int m, int ncoils) {
+    const double nt = terms_estimate(G);
+    const double grid = (double)G.A.nf * G.B.nf + (double)G.A.n * G.B.nf;
+    return 250.0 + 4.2e-4 * m * nt * ceil_div(ncoils, 8) + 1.0e-5 * grid * nt * ncoils;
+}
+
+int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
+                  const float *ky, const float *t, const float *x, const float *y,
+                  const float *fm, const float *rho_r, const float *rho_i, const float *s_r,
+                  const float *s_i, float *d_r, float *d_i) {
+    const hipStream_t st = ctx->stream;
+    const dim3 b256(256);
+    const NuAxis &A = G.A, &B = G.B;
+    const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
+    const int nA = A.n, nB = B.n;
+    const size_t nvox = (size_t)nA * nB;
+    const int rec = prof_begin(ctx, "nufft_forward");
+    NuPass N(ctx, G, m, kx, ky, t);
+    IMP_TRY(N.sort(true));
+    IMP_TRY(N.expand());
+    N.take_tables();
+    int cg = std::min(32, ncoils);
+    const size_t col_bytes = (size_t)A.nf * B.nf * N.nt * sizeof(double2);
+    while (cg > 1 && col_bytes * cg > NU_KGRID_BYTES) cg = (cg + 1) / 2;
+    Carver &W = N.W;
+    constexpr int NX = NW + 2 * (TG - 1);
+    const int ntx = ceil_div(A.nf - NW + 1, TG), ntile = ntx * ceil_div(B.nf - NW + 1, TG);
+    const size_t o_bx = W.take((size_t)m * 4), o_by = W.take((size_t)m * 4);
+    const size_t o_wx = W.take((size_t)m * NX * 8), o_wy = W.take((size_t)m * NX * 8);
+    const size_t o_u = W.take((size_t)m * N.nt * 8), o_rot = W.take((size_t)m * sizeof(double2));
+    const size_t o_cnt = W.take(256);
+    const size_t o_ent = W.take(((size_t)ntile + m / GI_S + 1) * sizeof(GiEntry));
+    size_t o_f[2], o_l[2], o_lw[2];
+    for (int a = 0; a < 2; ++a) {
+        const NuAxis &X = a ? B : A;
+        o_f[a] = W.take(((size_t)X.L + 1) * 4);
+        o_l[a] = W.take((size_t)X.n * (NW + 1) * 4);
+        o_lw[a] = W.take((size_t)X.n * (NW + 1) * 8);
+    }
+    const size_t o_vt = W.take((size_t)N.nt * nvox * 8);
+    const size_t o_sens = W.take(s_r ? (size_t)ncoils * nvox * sizeof(float2) : 0);
+    const size_t o_img0 = W.take(nvox * sizeof(double2));
+    const size_t o_mid = W.take((size_t)nA * B.nf * N.nt * cg * sizeof(double2));
+    const size_t o_grid = W.take(col_bytes * cg);
+    IMP_TRY(N.alloc(cA, 1, cB, nA));
+    hipLaunchKernelGGL(k_nu_starts, dim3(1), b256, 0, st, m, N.key, -1, (int *)nullptr,
+                       N.at<int *>(o_cnt), 1);
+    hipLaunchKernelGGL(k_gi_list, dim3(ceil_div(ntile, 255)), b256, 0, st, m, ntile, N.key,
+                       N.at<GiEntry *>(o_ent), N.at<int *>(o_cnt));
+    hipLaunchKernelGGL(k_gi_prep, dim3(ceil_div(m, PREP_S)), b256, 0, st, m, N.perm, N.kA, N.kB,
+                       t, A, B, G.tc, G.th > 0.0 ? 1.0 / G.th : 0.0, G.wc / (2.0 * M_PI),
+                       N.coef(), N.coef() + N.tab_poly, N.nt, N.nleg, N.at<int *>(o_bx),
+                       N.at<int *>(o_by), N.at<double *>(o_wx), N.at<double *>(o_wy),
+                       N.at<double *>(o_u), N.at<double2 *>(o_rot));
+    if (!A.uniform || !B.uniform) {
+        FListTab ft[2];
+        for (int a = 0; a < 2; ++a)
+            ft[a] = FListTab{a ? B : A, a ? cB : cA, a ? nA : 1, N.at<int *>(o_f[a]),
+                             N.at<int *>(o_l[a]), N.at<double *>(o_lw[a])};
+        hipLaunchKernelGGL(k_nu_flists, dim3(2), dim3(1024), 0, st, ft[0], ft[1]);
+    }
+    hipLaunchKernelGGL(k_nu_vt, dim3(ceil_div((long)nvox, 256), N.nt), b256, 0, st, nA, nB, fm,
+                       G.wc, G.wh > 0.0 ? 1.0 / G.wh : 0.0, N.nt, N.coef(), N.mul(), N.nleg,
+                       N.at<double *>(o_vt));
+    if (s_r)
+        hipLaunchKernelGGL(k_nu_sens, dim3(ceil_div(nA, 32), ceil_div(nB, 32), ncoils), b256, 0,
+                           st, nA, nB, s_r, s_i, N.at<float2 *>(o_sens));
+    hipLaunchKernelGGL(k_nu_img0, dim3(ceil_div(nA, 16), ceil_div(nB, 16)), b256, 0, st, nA, nB,
+                       rho_r, rho_i, cA, cB, fm, A.kc, B.kc, G.tc / (2.0 * M_PI),
+                       N.at<double2 *>(o_img0));
+    IMP_CHECK_LAUNCH();
+    for (int c0 = 0; c0 < ncoils; c0 += cg) {
+        const int nc = std::min(cg, ncoils - c0), nq = N.nt * nc;
+        // B axis: lines ia -> mid[gB][ia][q]; A axis: lines gB -> grid[gB][gA][q]
+        LineArgs LB = N.line(1, nullptr, 0, 0, nq);
+        LB.base = N.at<const int *>(o_f[1]);
+        IMP_TRY(line_forward(ctx, LB, nA, true, N.at<const int *>(o_l[1]),
+                             N.at<const double *>(o_lw[1]), nc, N.at<const double2 *>(o_img0),
+                             s_r ? N.at<const float2 *>(o_sens) + (size_t)c0 * nvox : nullptr,
+                             N.at<const double *>(o_vt), (unsigned)nvox, N.at<double2 *>(o_mid),
+                             nq, (unsigned)(nA * nq)));
+        LineArgs LA = N.line(0, N.ws + o_mid, (size_t)nA * nq, nq, nq);
+        LA.base = N.at<const int *>(o_f[0]);
+        IMP_TRY(line_forward(ctx, LA, B.nf, false, N.at<const int *>(o_l[0]),
+                             N.at<const double *>(o_lw[0]), nc, nullptr, nullptr, nullptr, 0u,
+                             N.at<double2 *>(o_grid), (size_t)A.nf * nq, nq));
+        GiArgs P{};
+        P.ntx = ntx;
+        P.nfA = A.nf;
+        P.nfB = B.nf;
+        P.nt = N.nt;
+        P.nc = nc;
+        P.c0 = c0;
+        P.m = m;
+        P.perm = N.perm;
+        P.bx = N.at<const int *>(o_bx);
+        P.by = N.at<const int *>(o_by);
+        P.wx = N.at<const double *>(o_wx);
+        P.wy = N.at<const double *>(o_wy);
+        P.u = N.at<const double *>(o_u);
+        P.rot = N.at<const double2 *>(o_rot);
+        P.count = N.at<const int *>(o_cnt);
+        P.entries = N.at<const GiEntry *>(o_ent);
+        P.grid = N.at<const double *>(o_grid);
+        P.d_r = d_r;
+        P.d_i = d_i;
+        const int cb = ceil_div(nc, 8);
+        auto fn = cb == 1 ? k_gather<1> : cb == 2 ? k_gather<2> : cb == 3 ? k_gather<3>
+                                                                           : k_gather<4>;
+        const int rg = prof_begin(ctx, "k_gather");
+        hipLaunchKernelGGL(fn, dim3(std::min(ntile + m / GI_S + 1, 64 * ctx->num_cus)), dim3(64),
+                           0, st, P);
+        prof_end(ctx, rg);
+        IMP_CHECK_LAUNCH();
+    }
+    prof_end(ctx, rec);
     return IMP_OK;
 }
 

@@ -1,5 +1,5 @@
-"""The separable F^H d of large 2D problems and the 2D Q_l (csrc/nufft.hip)
-against the FP64 oracle and against the direct kernels.
+"""The separable F^H d and F of large 2D problems and the 2D Q_l
+(csrc/nufft.hip) against the FP64 oracle and against the direct kernels.
 
 Tolerance: 2e-7 relative L2.  The separable form sums in FP64 and rounds once
 to FP32 (at most 6e-8 per value); its time expansion and its two kernel
@@ -213,3 +213,72 @@ def test_batch_mixes_separable_and_direct_jobs(ctx):
         one = ops.nudft_adjoint(ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"],
                                 p["d"], p["s"])
         assert np.array_equal(g, one) if big else rel_l2(g, one) < DIRECT_TOL
+
+
+def _check_forward(ctx, p, nc, sens=True, separable=True, tol=TOL):
+    from impatient import ops
+    from oracle import oracle as orc
+    r = np.random.default_rng(12)
+    n = len(p["x"])
+    rho = (r.standard_normal(n) + 1j * r.standard_normal(n)).astype(np.complex64)
+    s = p["s"] if sens else None
+    got, (k,) = _timer(ctx, lambda: ops.nudft_forward(
+        ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"], rho, s, nc),
+        "nufft_forward")
+    assert (k > 0) == separable
+    M = len(p["kx"])
+    idx = np.unique(np.concatenate([[0, M - 1], r.integers(0, M, 60)]))
+    ref = orc.nudft_forward(p["kx"][idx], p["ky"][idx], None, p["t"][idx], p["x"], p["y"], None,
+                            p["fm"], rho, s)
+    err = rel_l2(got[:, idx], ref)
+    print(f"rel_l2 {err:.2e}")
+    assert err < tol
+    return got, rho
+
+
+@pytest.mark.parametrize("Nx,Ny,nc,M", [
+    (128, 192, 1, 60001), (160, 128, 2, 70000), (150, 151, 3, 90001), (192, 197, 8, 80000),
+    (256, 257, 9, 65537), (256, 256, 16, 70000), (300, 287, 17, 60013), (320, 320, 32, 80000)])
+def test_forward_separable(ctx, Nx, Ny, nc, M):
+    _check_forward(ctx, _problem(Nx, Ny, nc, M), nc)
+
+
+@pytest.mark.parametrize("what", ["x_outer", "y_falling", "no_field_map", "no_sens",
+                                  "beyond_nyquist", "wide_time", "clump", "axis_shuffled",
+                                  "points"])
+def test_forward_separable_forms(ctx, what):
+    N, nc, M = 200, 4, 60000
+    kw = dict(beyond_nyquist=dict(kscale=1.7), wide_time=dict(max_hz=600.0),
+              clump=dict(clump=True)).get(what, {})
+    p = _problem(N, N, nc, M, **kw)
+    if what == "x_outer":
+        for k in ("x", "y", "fm"):
+            p[k] = np.ascontiguousarray(p[k].reshape(N, N).T).reshape(-1)
+    if what == "y_falling":
+        p["y"] = -p["y"]
+    if what == "axis_shuffled":
+        o = np.random.default_rng(9).permutation(N)
+        p["x"] = np.ascontiguousarray(p["x"].reshape(N, N)[:, o]).reshape(-1)
+    if what == "no_field_map":
+        p["fm"] = None
+    if what == "points":
+        p["x"] = (p["x"] + np.random.default_rng(2).uniform(-1e-3, 1e-3, N * N)).astype(np.float32)
+    direct = what == "points"
+    _check_forward(ctx, p, 1 if what == "no_sens" else nc, sens=what != "no_sens",
+                   separable=not direct, tol=DIRECT_TOL if direct else TOL)
+
+
+def test_forward_separable_repeats_and_is_the_adjoint(ctx):
+    """Same bits on repeat, and <F x, y> = <x, F^H y> with both separable."""
+    from impatient import ops
+    p = _problem(256, 200, 4, 60000)
+    got, rho = _check_forward(ctx, p, 4)
+    again = ops.nudft_forward(ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"],
+                              rho, p["s"], 4)
+    assert np.array_equal(got, again)
+    back = ops.nudft_adjoint(ctx, p["kx"], p["ky"], None, p["t"], p["x"], p["y"], None, p["fm"],
+                             p["d"], p["s"])
+    a = np.vdot(p["d"].astype(np.complex128), got.astype(np.complex128))
+    b = np.vdot(back.astype(np.complex128), rho.astype(np.complex128))
+    scale = np.linalg.norm(p["d"]) * np.linalg.norm(got)
+    assert abs(a - b) < TOL * scale

@@ -1121,25 +1121,19 @@ int find_stack(imp_ctx *ctx, int num_k, const float *kx, const float *ky, const 
     return IMP_OK;
 }
 
-// Partition length for the separable F^H d, or 0 when the samples are not a
-// stack, the separable form would not save at least half of the phase
-// evaluations, or its partials would exceed STACK_PART_CAP.
+// Whether a stack of partitions of K samples takes the z-separable direct sum:
+// it has to save at least half of the phase evaluations and its partials to
+// stay within STACK_PART_CAP.
 constexpr size_t STACK_PART_CAP = (size_t)8 << 30;
 
-int detect_stack(imp_ctx *ctx, int num_k, int ncoils, int num_x, const float *kx,
-                 const float *ky, const float *kz, const float *t, int *K_out) {
-    *K_out = 0;
-    int K = 0;
-    IMP_TRY(find_stack(ctx, num_k, kx, ky, kz, t, nullptr, nullptr, &K));
-    if (K == 0) return IMP_OK;
+bool stack_pays(imp_ctx *ctx, int num_k, int ncoils, int num_x, int K) {
+    if (K == 0) return false;
     const int P = num_k / K;
     const long groups = ceil_div((long)ncoils * P, 2 * MF_COLS);
-    if (2 * groups > P) return IMP_OK;
+    if (2 * groups > P) return false;
     const long wgs = ceil_div(num_x, MF_WAVE_PTS * (NU_THREADS / 64));
     const int chunks = pick_chunks(ctx, wgs, ceil_div(K, MF_K), 4 * MF_FOLD);
-    if ((size_t)groups * chunks * 64 * num_x * sizeof(float) > STACK_PART_CAP) return IMP_OK;
-    *K_out = K;
-    return IMP_OK;
+    return (size_t)groups * chunks * 64 * num_x * sizeof(float) <= STACK_PART_CAP;
 }
 
 // F^H d of a stack (W = conj(phi) d built, lanes built with the field map).
@@ -1204,16 +1198,14 @@ bool adjoint_args_ok(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float
            d_i && out_r && out_i && !(s_r && !s_i) && !(phi_r && !phi_i);
 }
 
-// F^H d with the scratch of S; stacked trajectories take the separable form
-// only when allow_stack (its detection synchronises with the host).
-int adjoint_impl(imp_ctx *ctx, Scratch &S, bool allow_stack, int num_k, int num_x, int ncoils,
+// F^H d as a direct sum with the scratch of S; K: partition length when the
+// samples are a stack and the z-separable sum is to be used, else 0.
+int adjoint_impl(imp_ctx *ctx, Scratch &S, int K, int num_k, int num_x, int ncoils,
                  const float *kx, const float *ky, const float *kz, const float *t,
                  const float *x, const float *y, const float *z, const float *fm,
                  const float *phi_r, const float *phi_i, const float *d_r, const float *d_i,
                  const float *s_r, const float *s_i, float *out_r, float *out_i) {
     const bool d3 = kz && z;
-    int K = 0;
-    if (d3 && allow_stack) IMP_TRY(detect_stack(ctx, num_k, ncoils, num_x, kx, ky, kz, t, &K));
     const double *spos = nullptr;
     if (K == 0) IMP_TRY(build_spos(ctx, S, num_k, kx, ky, d3 ? kz : nullptr, t, 1.0, &spos));
     void *lanes = nullptr, *W = nullptr;
@@ -1259,13 +1251,14 @@ size_t adjoint_fixed_bytes(int num_k, int num_x, int ncoils, bool d3) {
 // direct kernels cost the same for every geometry; the separable form pays per
 // sample and time term for the spread, and per grid column for the
 // transforms, behind a fixed part (geometry read-back, sort, ~20 launches).
+constexpr double STACK_MIN_US = 400.0;    // direct time of a stack below which it is kept
 constexpr double NUFFT_MIN_PAIRS = 6e8;   // below: the direct kernels win at every size measured
 
 constexpr double DIRECT_FIXED_US = 60.0;
 
 double direct_us(double pairs, int ncoils) {
-    return DIRECT_FIXED_US + pairs * (ncoils <= 1 ? 7.9e-4 : ncoils == 2 ? 8.4e-4
-                           : ncoils <= MF_COLS ? 5.6e-4 : 8.1e-4);
+    return DIRECT_FIXED_US + pairs * (ncoils <= 1 ? 7.9e-7 : ncoils == 2 ? 8.4e-7
+                                      : ncoils <= MF_COLS ? 5.6e-7 : 8.1e-7);
 }
 
 // The separable form evaluates 2D problems of as many coils as one direct
@@ -1324,17 +1317,39 @@ int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
     if (!adjoint_args_ok(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, phi_r, phi_i, d_r, d_i,
                          s_r, s_i, out_r, out_i))
         return fail(IMP_EINVAL, "nudft_adjoint: bad arguments");
-    if (!(kz && z)) {
+    int K = 0;
+    if (kz && z) {
+        IMP_TRY(find_stack(ctx, num_k, kx, ky, kz, t, nullptr, nullptr, &K));
+        bool direct_stack = stack_pays(ctx, num_k, ncoils, num_x, K);
+        if (K > 0) {
+            const int nrhs = ncoils * (num_k / K);
+            NuGeometry G;
+            const double us = direct_stack
+                ? ceil_div(nrhs, 2 * MF_COLS) * direct_us((double)K * num_x, 2 * MF_COLS)
+                : direct_us((double)num_k * num_x, ncoils);
+            // more than 32 coils are refused by the direct sum of a volume
+            if ((direct_stack || ncoils <= 2 * MF_COLS) && us > STACK_MIN_US)
+                IMP_TRY(nufft_geometry(ctx, K, num_x, kx, ky, t, x, y, z, fm, &G));
+            if (G.ok && nufft_stack_us(G, K, nrhs) < us) {
+                const int rc = nufft_stack_adjoint(ctx, G, K, num_k / K, ncoils, kx, ky, kz, t, x,
+                                                   y, z, fm, phi_r, phi_i, d_r, d_i, s_r, s_i,
+                                                   out_r, out_i);
+                if (rc != IMP_ENOMEM) return rc;
+            }
+        }
+        if (!direct_stack) K = 0;
+    } else {
         NuGeometry G;
         IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, false, &G));
         if (G.ok) {
             IMP_TRY(reserve_direct(ctx, num_k, num_x, ncoils, false));
-            return nufft_adjoint(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
-                                 d_r, d_i, s_r, s_i, out_r, out_i);
+            const int rc = nufft_adjoint(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, phi_r, phi_i,
+                                         d_r, d_i, s_r, s_i, out_r, out_i);
+            if (rc != IMP_ENOMEM) return rc;
         }
     }
     Scratch S{ctx};
-    return adjoint_impl(ctx, S, true, num_k, num_x, ncoils, kx, ky, kz, t, x, y, z, fm, phi_r,
+    return adjoint_impl(ctx, S, K, num_k, num_x, ncoils, kx, ky, kz, t, x, y, z, fm, phi_r,
                         phi_i, d_r, d_i, s_r, s_i, out_r, out_i);
 }
 
@@ -1394,7 +1409,7 @@ int nudft_adjoint_noalloc(imp_ctx *ctx, int num_k, int num_x, int ncoils, const 
     void *base = nullptr;
     IMP_TRY(noalloc_scratch(ctx, &base));
     Scratch S{ctx, (char *)base, NOALLOC_SCRATCH_BYTES, 0};
-    return adjoint_impl(ctx, S, false, num_k, num_x, ncoils, kx, ky, kz, t, x, y, z, fm, phi_r,
+    return adjoint_impl(ctx, S, 0, num_k, num_x, ncoils, kx, ky, kz, t, x, y, z, fm, phi_r,
                         phi_i, d_r, d_i, s_r, s_i, out_r, out_i);
 }
 
@@ -1437,13 +1452,13 @@ int nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs, int 
     for (int j = 0; j < njobs; ++j) {
         const imp_nudft_job &b = jobs[j];
         // the launch's fixed part is shared by the direct jobs
+        int rc = IMP_ENOMEM;
         if (G[j].ok && nufft_adjoint_us(G[j], b.num_k, b.ncoils) <
                            direct_us((double)b.num_k * b.num_x, b.ncoils) - DIRECT_FIXED_US)
-            IMP_TRY(nufft_adjoint(ctx, G[j], b.num_k, b.ncoils, b.kx, b.ky, b.t, b.x, b.y, b.fm,
-                                  b.phi_r, b.phi_i, b.d_r, b.d_i, b.s_r, b.s_i, b.out_r,
-                                  b.out_i));
-        else
-            rest.push_back(b);
+            rc = nufft_adjoint(ctx, G[j], b.num_k, b.ncoils, b.kx, b.ky, b.t, b.x, b.y, b.fm,
+                               b.phi_r, b.phi_i, b.d_r, b.d_i, b.s_r, b.s_i, b.out_r, b.out_i);
+        if (rc == IMP_ENOMEM) rest.push_back(b);
+        else IMP_TRY(rc);
     }
     if (rest.empty()) {
         IMP_HIP(hipStreamSynchronize(ctx->stream));
@@ -1597,8 +1612,9 @@ int nudft_forward(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
         IMP_TRY(choose_separable(ctx, num_k, num_x, ncoils, kx, ky, t, x, y, fm, true, &G));
         if (G.ok) {
             IMP_TRY(reserve_direct(ctx, num_x, num_k, ncoils, true));
-            return nufft_forward(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, rho_r, rho_i, s_r,
-                                 s_i, d_r, d_i);
+            const int rc = nufft_forward(ctx, G, num_k, ncoils, kx, ky, t, x, y, fm, rho_r, rho_i,
+                                         s_r, s_i, d_r, d_i);
+            if (rc != IMP_ENOMEM) return rc;
         }
     }
     const double *spos = nullptr;
@@ -2489,9 +2505,11 @@ int toeplitz_q(imp_ctx *ctx, int num_k, const float *kx, const float *ky,
         std::isfinite(t0)) {
         NuGeometry G;
         IMP_TRY(nufft_q_geometry(ctx, num_k, kx, ky, t, Nx, Ny, nseg, &G));
-        if (G.ok)
-            return nufft_q(ctx, G, num_k, kx, ky, t, phi_r, phi_i, Nx, Ny, nseg, tau, t0,
-                           (flags & IMP_Q_CUMULATIVE) != 0, q_r, q_i);
+        if (G.ok) {
+            const int rc = nufft_q(ctx, G, num_k, kx, ky, t, phi_r, phi_i, Nx, Ny, nseg, tau, t0,
+                                   (flags & IMP_Q_CUMULATIVE) != 0, q_r, q_i);
+            if (rc != IMP_ENOMEM) return rc;
+        }
     }
     const double *spos = nullptr;
     IMP_TRY(build_spos(ctx, num_k, kx, ky, d3 ? kz : nullptr, nullptr, 0.0, &spos));

@@ -7,6 +7,9 @@
 
 namespace imp {
 
+// Every operator below returns IMP_ENOMEM before it has written a result when
+// its workspace cannot be had; callers then take the direct path.
+
 // One image axis against the sample coordinate k it pairs with.
 struct NuAxis {
     int n;            // image points
@@ -47,6 +50,15 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
                   const float *d_i, const float *s_r, const float *s_i, float *out_r,
                   float *out_i);
 
+// F^H d of a stack: samples [p K, (p + 1) K) repeat kx, ky, t of the first K
+// at their own kz; G from the first K samples.
+double nufft_stack_us(const NuGeometry &G, int K, int nrhs);
+int nufft_stack_adjoint(imp_ctx *ctx, const NuGeometry &G, int K, int P, int ncoils,
+                        const float *kx, const float *ky, const float *kz, const float *t,
+                        const float *x, const float *y, const float *z, const float *fm,
+                        const float *phi_r, const float *phi_i, const float *d_r,
+                        const float *d_i, const float *s_r, const float *s_i, float *out_r,
+                        float *out_i);
 double nufft_forward_us(const NuGeometry &G, int m, int ncoils);
 int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
                   const float *ky, const float *t, const float *x, const float *y,

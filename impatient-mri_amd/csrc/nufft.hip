@@ -2194,6 +2194,16 @@ struct NuPass {
 
 }  // namespace
 
+// kernel-timer record over a scope (closed on every return)
+namespace {
+struct ProfScope {
+    imp_ctx *ctx;
+    int rec;
+    ProfScope(imp_ctx *c, const char *name) : ctx(c), rec(prof_begin(c, name)) {}
+    ~ProfScope() { prof_end(ctx, rec); }
+};
+}  // namespace
+
 // predicted microseconds of the spread and transforms of ncols columns of nt
 // time terms, without the fixed part
 static double separable_us(const NuAxis &A, const NuAxis &B, int m, double cols) {
@@ -2214,7 +2224,7 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
     const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
     const int nA = G.A.n, nB = G.B.n;
     const size_t nvox = (size_t)nA * nB;
-    const int rec = prof_begin(ctx, "nufft_adjoint");
+    const ProfScope prof(ctx, "nufft_adjoint");
     NuPass N(ctx, G, m, kx, ky, t);
     IMP_TRY(N.sort());
     IMP_TRY(N.layout(ncoils));
@@ -2251,8 +2261,142 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
     hipLaunchKernelGGL(k_nu_out, dim3(ceil_div(nA, 16), ceil_div(nB, 16)), b256, 0, st, nA, nB,
                        parts, N.at<const double2 *>(o_img), cA, cB, fm, G.A.kc, G.B.kc,
                        G.tc / (2.0 * M_PI), out_r, out_i);
-    prof_end(ctx, rec);
     IMP_CHECK_LAUNCH();
+    return IMP_OK;
+}
+
+// ------------------------------------------------------------ stacks (3D F^H d)
+// Samples in P partitions that repeat one 2D trajectory of K samples at kz_p:
+//   out(x, y, z) = sum_l i^(l mod 2) vt[l](w(x, y, z)) sum_(c, p)
+//                  conj(S_c(x, y, z)) e^{i 2pi kz_p z} P_(l, c, p)(x, y),
+// P the separable 2D sums of the C P coil-partition columns over K samples.
+namespace {
+
+// vt[l][voxel] in the voxels' own order
+__global__ __launch_bounds__(256) void k_nu_vt3(int n, const float *fm, double wc, double winv,
+                                                int nt, const double *coef, const double *mul,
+                                                int nleg, double *vt) {
+    const int v = blockIdx.x * 256 + threadIdx.x, l = blockIdx.y;
+    if (v >= n) return;
+    const double s = clamp1(((fm ? (double)fm[v] : 0.0) - wc) * winv);
+    vt[(size_t)l * n + v] =
+        mul[l] * prolate(coef + (size_t)l * nleg, coef + (size_t)nt * nleg, nleg, l & 1, s);
+}
+
+// ez[p][iz] = e^{i 2pi kz_p z}
+__global__ void k_nu_ez(int P, int K, int nz, const float *kz, const float *z, double2 *ez) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= P * nz) return;
+    const double rev = (double)kz[(size_t)(i / nz) * K] * z[i % nz];
+    double s, c;
+    sincospi(2.0 * (rev - rint(rev)), &s, &c);
+    ez[i] = make_double2(c, s);
+}
+
+// The sum over a group's columns at every voxel (one thread each; the voxels
+// of a column read the same P values), added to acc; the last group applies
+// the centre's phase and stores.  ST_C columns' factors conj(S) ez stay in
+// registers over the time terms.
+constexpr int ST_C = 8;
+__global__ __launch_bounds__(256) void k_nu_stack(int n, int nz, int P, int c0, int nc,
+                                                  int nt, const double2 *grid, const double2 *ez,
+                                                  const double *vt, const float *s_r,
+                                                  const float *s_i, double2 *acc, int first,
+                                                  int last, const float *cA, const float *cB,
+                                                  const float *fm, double kcA, double kcB,
+                                                  double tc_2pi, float *out_r, float *out_i) {
+    const int v = blockIdx.x * 256 + threadIdx.x;
+    if (v >= n) return;
+    const int iz = v % nz;
+    const double2 *col = grid + (size_t)(v / nz) * nt * nc;
+    double2 sum = first ? make_double2(0.0, 0.0) : acc[v];
+    for (int cb = 0; cb < nc; cb += ST_C) {
+        double2 f[ST_C];
+#pragma unroll
+        for (int i = 0; i < ST_C; ++i) {
+            const int q = c0 + min(cb + i, nc - 1);
+            f[i] = ez[(q % P) * nz + iz];
+            if (s_r) {
+                const size_t o = (size_t)(q / P) * n + v;
+                f[i] = cmul(f[i], make_double2(s_r[o], -(double)s_i[o]));
+            }
+            if (cb + i >= nc) f[i] = make_double2(0.0, 0.0);
+        }
+        for (int l = 0; l < nt; ++l) {
+            const double2 *p = col + (size_t)l * nc + cb;
+            double2 z = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int i = 0; i < ST_C; ++i) {
+                const double2 g = p[min(i, nc - 1 - cb)];
+                z.x = fma(f[i].x, g.x, fma(-f[i].y, g.y, z.x));
+                z.y = fma(f[i].x, g.y, fma(f[i].y, g.x, z.y));
+            }
+            const double w = vt[(size_t)l * n + v];
+            sum.x = fma(w, (l & 1) ? -z.y : z.x, sum.x);
+            sum.y = fma(w, (l & 1) ? z.x : z.y, sum.y);
+        }
+    }
+    if (!last) {
+        acc[v] = sum;
+        return;
+    }
+    const double rev = kcA * cA[v] + kcB * cB[v] + (fm ? tc_2pi * fm[v] : 0.0);
+    double s, c;
+    sincospi(2.0 * (rev - rint(rev)), &s, &c);
+    const double2 o = cmul(sum, make_double2(c, s));
+    out_r[v] = (float)o.x;
+    out_i[v] = (float)o.y;
+}
+
+}  // namespace
+
+double nufft_stack_us(const NuGeometry &G, int K, int nrhs) {
+    const double nt = terms_estimate(G);
+    const double vox = (double)G.A.n * G.B.n * G.nz;
+    return 300.0 + separable_us(G.A, G.B, K, nt * (nrhs < 32 ? 1 << log2i(nrhs) : nrhs)) +
+           4e-7 * vox * nt * nrhs;
+}
+
+int nufft_stack_adjoint(imp_ctx *ctx, const NuGeometry &G, int K, int P, int ncoils,
+                        const float *kx, const float *ky, const float *kz, const float *t,
+                        const float *x, const float *y, const float *z, const float *fm,
+                        const float *phi_r, const float *phi_i, const float *d_r,
+                        const float *d_i, const float *s_r, const float *s_i, float *out_r,
+                        float *out_i) {
+    const hipStream_t st = ctx->stream;
+    const dim3 b256(256);
+    const ProfScope prof(ctx, "nufft_stack");
+    const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
+    const int nA = G.A.n, nB = G.B.n, nz = G.nz, nrhs = ncoils * P;
+    const int n = nA * nB * nz;
+    NuPass N(ctx, G, K, kx, ky, t);
+    IMP_TRY(N.sort());
+    IMP_TRY(N.layout(nrhs));
+    const size_t o_vt = N.W.take((size_t)N.nt * n * 8);
+    const size_t o_ez = N.W.take((size_t)P * nz * sizeof(double2));
+    const size_t o_acc = N.W.take((size_t)n * sizeof(double2));
+    const size_t o_p = N.W.take((size_t)nA * nB * N.nt * std::min(N.cg, nrhs) * sizeof(double2));
+    IMP_TRY(N.build(cA, nz, cB, nz * nA));
+    hipLaunchKernelGGL(k_nu_vt3, dim3(ceil_div(n, 256), N.nt), b256, 0, st, n, fm, G.wc,
+                       G.wh > 0.0 ? 1.0 / G.wh : 0.0, N.nt, N.coef(), N.mul(), N.nleg,
+                       N.at<double *>(o_vt));
+    hipLaunchKernelGGL(k_nu_ez, dim3(ceil_div(P * nz, 256)), b256, 0, st, P, K, nz, kz, z,
+                       N.at<double2 *>(o_ez));
+    IMP_CHECK_LAUNCH();
+    for (int g = 0; g < N.groups; ++g) {
+        const int c0 = g * N.cg, nc = std::min(N.cg, nrhs - c0), nq = N.nt * nc;
+        hipLaunchKernelGGL(k_nu_data, dim3(ceil_div(K, WD_S)), b256, 0, st, K, c0, nc, 1 << N.lc,
+                           N.kA, N.kB, t, G.A, G.B, G.tc, G.wc / (2.0 * M_PI), phi_r, phi_i, d_r,
+                           d_i, N.at<double2 *>(N.o_wd));
+        IMP_TRY(N.to_mid(nc));
+        IMP_TRY(line_store(ctx, N.lines_b(nc), nA, N.at<double2 *>(o_p), nq, (size_t)nA * nq));
+        hipLaunchKernelGGL(k_nu_stack, dim3(ceil_div(n, 256)), b256, 0, st, n, nz, P, c0, nc,
+                           N.nt, N.at<const double2 *>(o_p), N.at<const double2 *>(o_ez),
+                           N.at<const double *>(o_vt), s_r, s_i, N.at<double2 *>(o_acc), g == 0,
+                           g + 1 == N.groups, cA, cB, fm, G.A.kc, G.B.kc, G.tc / (2.0 * M_PI),
+                           out_r, out_i);
+        IMP_CHECK_LAUNCH();
+    }
     return IMP_OK;
 }
 
@@ -2298,7 +2442,7 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
     const float *cA = G.a_is_y ? y : x, *cB = G.a_is_y ? x : y;
     const int nA = A.n, nB = B.n;
     const size_t nvox = (size_t)nA * nB;
-    const int rec = prof_begin(ctx, "nufft_forward");
+    const ProfScope prof(ctx, "nufft_forward");
     NuPass N(ctx, G, m, kx, ky, t);
     IMP_TRY(N.sort(true));
     IMP_TRY(N.expand());
@@ -2397,7 +2541,6 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
         prof_end(ctx, rg);
         IMP_CHECK_LAUNCH();
     }
-    prof_end(ctx, rec);
     return IMP_OK;
 }
 
@@ -2502,7 +2645,7 @@ int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const flo
             const float *t, const float *phi_r, const float *phi_i, int Nx, int Ny, int nseg,
             float tau, float t0, bool cumulative, float *q_r, float *q_i) {
     const hipStream_t st = ctx->stream;
-    const int rec = prof_begin(ctx, "nufft_q");
+    const ProfScope prof(ctx, "nufft_q");
     const int cols = (nseg + 1) / 2;
     NuPass N(ctx, G, m, kx, ky, t);
     IMP_TRY(N.sort());
@@ -2518,7 +2661,6 @@ int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const flo
     hipLaunchKernelGGL(k_nu_qout, dim3(ceil_div(2 * Nx, 256), 2 * Ny), dim3(256), 0, st, Nx, Ny,
                        cols, nseg, cumulative ? 1 : 0, N.at<const double2 *>(o_p), G.A.kc, G.B.kc,
                        q_r, q_i);
-    prof_end(ctx, rec);
     IMP_CHECK_LAUNCH();
     return IMP_OK;
 }

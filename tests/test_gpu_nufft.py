@@ -282,3 +282,51 @@ def test_forward_separable_repeats_and_is_the_adjoint(ctx):
     b = np.vdot(back.astype(np.complex128), rho.astype(np.complex128))
     scale = np.linalg.norm(p["d"]) * np.linalg.norm(got)
     assert abs(a - b) < TOL * scale
+
+
+def _stack(Nx, Ny, Nz, nc, K, P, seed=4):
+    p = _problem(Nx, Ny, nc, K, seed=seed)
+    r = np.random.default_rng(seed + 1)
+    kz = r.uniform(-Nz / 2, Nz / 2, P).astype(np.float32)
+    vox = lambda a: np.repeat(a, Nz)
+    z = np.tile(((np.arange(Nz) - Nz // 2) / Nz).astype(np.float32), Nx * Ny)
+    q = dict(kx=np.tile(p["kx"], P), ky=np.tile(p["ky"], P), kz=np.repeat(kz, K),
+             t=np.tile(p["t"], P), x=vox(p["x"]), y=vox(p["y"]), z=z)
+    q["fm"] = (vox(p["fm"]) + 200 * z).astype(np.float32)
+    c = lambda *s: (r.standard_normal(s) + 1j * r.standard_normal(s)).astype(np.complex64)
+    q["d"], q["s"], q["phi"] = c(nc, P * K), c(nc, len(z)), c(nc, P * K)
+    return q
+
+
+@pytest.mark.parametrize("Nx,Ny,Nz,nc,K,P,what", [
+    (64, 48, 8, 4, 30000, 16, "plain"), (33, 41, 12, 3, 40001, 33, "phi"),
+    (64, 64, 4, 2, 40000, 34, "no_field_map"), (40, 56, 10, 9, 30000, 20, "y_fast"),
+    (48, 48, 16, 1, 30000, 70, "no_sens"), (48, 48, 12, 4, 30000, 16, "z_slow")])
+def test_adjoint_stack_separable(ctx, Nx, Ny, Nz, nc, K, P, what):
+    """A stack of large partitions: the separable 2D sums of the coil-partition
+    columns, combined over z.  Volumes whose z does not run fastest keep the
+    z-separable direct sum."""
+    from impatient import ops
+    from oracle import oracle as orc
+    q = _stack(Nx, Ny, Nz, nc, K, P)
+    if what in ("y_fast", "z_slow"):   # other voxel orders of [Ny][Nx][Nz]
+        o = (1, 0, 2) if what == "y_fast" else (2, 0, 1)
+        perm = np.transpose(np.arange(Nx * Ny * Nz).reshape(Ny, Nx, Nz), o).reshape(-1)
+        for k in ("x", "y", "z", "fm"):
+            q[k] = np.ascontiguousarray(q[k][perm])
+    if what == "no_field_map":
+        q["fm"] = None
+    phi = q["phi"] if what == "phi" else None
+    s = None if what == "no_sens" else q["s"]
+    got, n = _timer(ctx, lambda: ops.nudft_adjoint(
+        ctx, q["kx"], q["ky"], q["kz"], q["t"], q["x"], q["y"], q["z"], q["fm"], q["d"], s, phi),
+        "nufft_stack", "k_nudft_stack")
+    assert (n[0] > 0, n[1] > 0) == ((False, True) if what == "z_slow" else (True, False))
+    idx = np.unique(np.concatenate([[0, len(q["x"]) - 1],
+                                    np.random.default_rng(1).integers(0, len(q["x"]), 60)]))
+    ref = orc.nudft_adjoint(q["kx"], q["ky"], q["kz"], q["t"], q["x"][idx], q["y"][idx],
+                            q["z"][idx], None if q["fm"] is None else q["fm"][idx], q["d"],
+                            None if s is None else s[:, idx], phi)
+    err = rel_l2(got[idx], ref)
+    print(f"rel_l2 {err:.2e}")
+    assert err < (DIRECT_TOL if what == "z_slow" else TOL)

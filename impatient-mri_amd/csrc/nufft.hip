@@ -41,10 +41,13 @@ namespace {
 
 using fftc::cmul;
 
-constexpr int NW = 12;           // kernel width in cells
+// Kernel width in cells.  One axis at 1.5x is off by 7e-10 (rms over the band;
+// worst 5e-9) at 12 cells, 4e-9 (2.5e-8) at 11, 2.4e-8 (1.4e-7) at 10; the
+// results are stored in FP32, 2.5e-8 rms.  11 costs 1/6 less work than 12.
+constexpr int NW = 11;
 constexpr double NU_SIGMA = 1.5; // oversampling of both grids
-// KB shape for width 12 at 1.5x: pi NW (1 - 1/(2 sigma)), 1% lower (smallest
-// worst-case error over the band, 5e-9, by a scan of the factor)
+// KB shape pi NW (1 - 1/(2 sigma)), 1% lower: the smallest error over the band
+// by a scan of the factor
 constexpr double NU_BETA = 0.99 * M_PI * NW * (1.0 - 1.0 / (2.0 * NU_SIGMA));
 constexpr double NU_TIME_TOL = 1e-8;   // largest error of the time expansion
 constexpr int NU_MAX_TERMS = 48;       // time terms above which the direct kernel runs
@@ -653,9 +656,15 @@ __global__ __launch_bounds__(256) void k_nu_data(int m, int c0, int nc, int slot
 
 // ------------------------------------------------------------------- spread
 // Tile: `T` cells along A on `yg` rows of one row block.  Work entries split
-// a tile's visits (sample, row) into runs of at most the chunk length the
-// count pass settled on; a tile with several runs sums them from slots.
-constexpr int SP_CH0 = 128;        // shortest chunk, visits
+// a tile's visits (sample, row) into runs of the chunk length the count pass
+// settled on; a tile with several runs sums them from slots.  Tiles are split
+// above twice the chunk length, since a slot costs its store and a second read.
+constexpr int SP_CH0 = 64;         // shortest chunk, visits
+constexpr int SP_WAVES = 3072;     // waves in flight: 256 CUs, 4 SIMDs, 3 each
+// Chunks per wave in flight.  2, 4, 8: 539, 507, 514 us for the spread and its
+// second pass on 250 x 234 x 8 coils, 483, 442, 495 on the Q of 512^2.
+constexpr int SP_SHARE = 4;
+constexpr int SP_RUN = 64;         // tiles of a super-block
 constexpr int SP_LEVELS = 12;      // chunk lengths SP_CH0 << level
 constexpr int SP_SLOTS = 8192;     // partial tiles a row block may use
 
@@ -665,19 +674,28 @@ struct SpEntry {
 struct SpMulti {
     int tile, slot, n, pad;
 };
-// Per row block counters: entries, slots, multi-run tiles, slot demand per level
+// Per row block counters: runs of split tiles (each with a slot), whole tiles
+// of more than half a chunk and shorter ones, split tiles; slot demand per level
 struct SpCount {
-    int entries, slots, multis, pad;
+    int heavy, medium, light, multis;
+    int visits, pad[3];     // of the block, in units of SP_CH0
     int need[SP_LEVELS];
 };
 
 struct SpGeom {
     int T, yg, rb;          // tile cells, rows, rows per block (multiple of yg)
     int ntx, nty;           // tiles along A, tile rows per block
+    int bw;                 // tiles along A of a super-block (SP_RUN tiles in all)
+    int ntile;              // tiles per block, whole super-blocks
     int ncA, ncB;           // cells (window starts) per axis
     int nfA, nfB;
-    int entry_cap;          // per row block
+    int entry_cap;          // per row block: SP_SLOTS runs, then whole tiles
 };
+
+// first grid row of local tile row ty of a block
+__device__ __forceinline__ int tile_row(const SpGeom &G, int block, int ty) {
+    return block * G.rb + ty * G.yg;
+}
 
 __device__ __forceinline__ int row_range(const SpGeom &G, const int *start, int gy0, int gx0,
                                          int row, int *s0) {
@@ -690,89 +708,133 @@ __device__ __forceinline__ int row_range(const SpGeom &G, const int *start, int 
     return start[by * G.ncA + hi + 1] - *s0;
 }
 
-__device__ __forceinline__ int tile_visits(const SpGeom &G, const int *start, int block,
-                                           int tile) {
-    const int gy0 = block * G.rb + (tile / G.ntx) * G.yg, gx0 = (tile % G.ntx) * G.T;
-    int n = 0, s0;
-    for (int r = 0; r < NW + G.yg - 1; ++r) n += row_range(G, start, gy0, gx0, r, &s0);
-    return n;
+// Tiles are numbered by super-blocks of SP_RUN (about 16 rows x 64 cells): a
+// sample is visited by tiles of neighbouring rows and columns, so tiles with
+// near numbers read the same samples.  Raster index of tile t of a block, or
+// -1 for the padding of the last super-blocks.
+__device__ __forceinline__ int tile_raster(const SpGeom &G, int t) {
+    const int nbx = (G.ntx + G.bw - 1) / G.bw, sb = t / SP_RUN, in = t % SP_RUN;
+    const int ty = (sb / nbx) * (SP_RUN / G.bw) + in / G.bw, tx = (sb % nbx) * G.bw + in % G.bw;
+    return ty < G.nty && tx < G.ntx ? ty * G.ntx + tx : -1;
 }
 
 __global__ __launch_bounds__(256) void k_sp_count(SpGeom G, const int *start, int *visits,
                                                   SpCount *cnt) {
-    __shared__ int need[SP_LEVELS];
+    __shared__ int need[SP_LEVELS], sum;
     if (threadIdx.x < SP_LEVELS) need[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sum = 0;
     __syncthreads();
-    const int tile = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
-    const int ntile = G.ntx * G.nty;
-    if (tile < ntile) {
-        const int n = tile_visits(G, start, block, tile);
-        visits[(size_t)block * ntile + tile] = n;
-        if (n > SP_CH0) {
+    const int t = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
+    if (t < G.ntile) {
+        const int tile = tile_raster(G, t);
+        int n = -1;
+        if (tile >= 0) {
+            const int gy0 = tile_row(G, block, tile / G.ntx), gx0 = (tile % G.ntx) * G.T;
+            int s0;
+            n = 0;
+            for (int r = 0; r < NW + G.yg - 1; ++r) n += row_range(G, start, gy0, gx0, r, &s0);
+        }
+        visits[(size_t)block * G.ntile + t] = n;
+        atomicAdd(&sum, (max(n, 0) + SP_CH0 - 1) / SP_CH0);
+        if (n > 2 * SP_CH0) {
 #pragma unroll
             for (int k = 0; k < SP_LEVELS; ++k) {
                 const int ch = SP_CH0 << k;
-                if (n > ch) atomicAdd(&need[k], (n + ch - 1) / ch);
+                if (n > 2 * ch) atomicAdd(&need[k], (n + ch - 1) / ch);
             }
         }
     }
     __syncthreads();
     if (threadIdx.x < SP_LEVELS && need[threadIdx.x])
         atomicAdd(&cnt[block].need[threadIdx.x], need[threadIdx.x]);
+    if (threadIdx.x == 0 && sum) atomicAdd(&cnt[block].visits, sum);
 }
 
-// The chunk length is the shortest whose slot demand fits, so it depends on
-// the operands only; which slot a run gets does not change what is summed.
+// The chunk length is the shortest whose slot demand fits and that leaves at
+// most SP_SHARE chunks per wave in flight, so it depends on the operands only; which slot a run gets does not change what is summed.
+// Entries keep the tiles' order within a workgroup's 256 tiles.
 __global__ __launch_bounds__(256) void k_sp_list(SpGeom G, const int *visits, SpCount *cnt,
                                                  SpEntry *entries, SpMulti *multis) {
-    const int tile = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
-    const int ntile = G.ntx * G.nty;
-    if (tile >= ntile) return;
+    __shared__ int wsum[3][4], base[3];
+    const int t = blockIdx.x * 256 + threadIdx.x, block = blockIdx.y;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     SpCount &C = cnt[block];
     int level = 0;
-    while (level < SP_LEVELS && C.need[level] > SP_SLOTS) ++level;
-    const int n = visits[(size_t)block * ntile + tile];
-    const int ch = level < SP_LEVELS ? SP_CH0 << level : 0x7fffffff;
-    const int runs = n > ch ? (n + ch - 1) / ch : 1;
-    const int e0 = atomicAdd(&C.entries, runs);
-    SpEntry *E = entries + (size_t)block * G.entry_cap + e0;
-    if (runs == 1) {
-        E[0] = SpEntry{tile, 0, n, -1};
-        return;
+    while (level < SP_LEVELS &&
+           (C.need[level] > SP_SLOTS || (C.visits >> level) > SP_SHARE * SP_WAVES))
+        ++level;
+    const int n = t < G.ntile ? visits[(size_t)block * G.ntile + t] : -1;
+    const int ch = level < SP_LEVELS ? SP_CH0 << level : 0x3fffffff;
+    const int runs = n > 2 * ch ? (n + ch - 1) / ch : n >= 0 ? 1 : 0;
+    // heavy, medium and light entries before this thread
+    int inc[3] = {runs > 1 ? runs : 0, runs == 1 && n > ch / 2 ? 1 : 0,
+                  runs == 1 && n <= ch / 2 ? 1 : 0};
+    const unsigned long long split = __ballot(runs > 1);
+#pragma unroll
+    for (int h = 0; h < 3; ++h) {
+        const int own = inc[h];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(inc[h], off, 64);
+            if (lane >= off) inc[h] += o;
+        }
+        if (lane == 63) wsum[h][wave] = inc[h];
+        inc[h] -= own;
     }
-    const int s0 = atomicAdd(&C.slots, runs);
-    const int m0 = atomicAdd(&C.multis, 1);
-    multis[(size_t)block * SP_SLOTS + m0] = SpMulti{tile, s0, runs, 0};
-    for (int r = 0; r < runs; ++r) E[r] = SpEntry{tile, r * ch, min(n, (r + 1) * ch), s0 + r};
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        const int h = threadIdx.x;
+        const int sum = wsum[h][0] + wsum[h][1] + wsum[h][2] + wsum[h][3];
+        base[h] = atomicAdd(h == 0 ? &C.heavy : h == 1 ? &C.medium : &C.light, sum);
+    }
+    __syncthreads();
+    SpEntry *E = entries + (size_t)block * G.entry_cap;
+    const int tile = t < G.ntile ? tile_raster(G, t) : -1;
+    const int cls = runs > 1 ? 0 : n > ch / 2 ? 1 : 2;
+    int at = base[cls] + inc[cls];
+    for (int w = 0; w < wave; ++w) at += wsum[cls][w];
+    if (runs == 1) {
+        // medium entries from the front of the whole tiles' part, light ones
+        // from its end
+        E[cls == 1 ? SP_SLOTS + at : G.entry_cap - 1 - at] = SpEntry{tile, 0, n, -1};
+    } else if (runs > 1) {
+        for (int r = 0; r < runs; ++r)
+            E[at + r] = SpEntry{tile, r * ch, min(n, (r + 1) * ch), at + r};
+        int m0 = 0;
+        if (lane == __ffsll((unsigned long long)split) - 1)
+            m0 = atomicAdd(&C.multis, __popcll(split));
+        m0 = __shfl(m0, __ffsll((unsigned long long)split) - 1, 64) +
+             __popcll(split & ((1ull << lane) - 1ull));
+        multis[(size_t)block * SP_SLOTS + m0] = SpMulti{tile, at, runs, 0};
+    }
 }
 
-typedef const __attribute__((address_space(4))) double *cdbl;
 typedef const __attribute__((address_space(4))) int *cint;
 
 struct SpArgs {
     SpGeom G;
-    int r0, block;             // first grid row of the block, its index
+    int block;                 // row block
     int nt, ntp, nc;           // time terms, padded, coils
     int lc, ll;                // log2 of coil slots and time groups in a wave
     const int *start, *perm, *bx;
     const double *wx, *wy, *u;
-    const double *wd;          // [sample][2 slots]
+    const double2 *wd;         // [sample][coil slot]
     const SpCount *cnt;
     const SpEntry *entries;
     const SpMulti *multis;
-    double *part;              // [slot][NL * T][64]
-    double *grid;              // [row in block][nfA][nt * nc][2]
+    double2 *part;             // [slot][NL * T][64]
+    double2 *grid;             // [row in block][nfA][nt][nc]
 };
 
 template <int NL, int T>
 __device__ __forceinline__ void sp_store(const SpArgs &P, int tile, int lane,
-                                         const double (&acc)[NL][T]) {
-    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
-    const int lg = (lane >> (1 + P.lc)) & ((1 << P.ll) - 1), yg = lane >> (1 + P.lc + P.ll);
-    const int row = (tile / P.G.ntx) * P.G.yg + yg, gx0 = (tile % P.G.ntx) * T;
-    if (c >= P.nc || row >= P.G.rb || P.r0 + row >= P.G.nfB) return;
-    double *out = P.grid + (((size_t)row * P.G.nfA + gx0) * P.nt * P.nc + c) * 2 + part;
-    const size_t sx = (size_t)P.nt * P.nc * 2, sl = (size_t)P.nc * 2;
+                                         const double2 (&acc)[NL][T]) {
+    const int c = lane & ((1 << P.lc) - 1), lg = (lane >> P.lc) & ((1 << P.ll) - 1);
+    const int yl = lane >> (P.lc + P.ll);
+    const int row = (tile / P.G.ntx) * P.G.yg + yl, gx0 = (tile % P.G.ntx) * T;
+    if (c >= P.nc || tile_row(P.G, P.block, tile / P.G.ntx) + yl >= P.G.nfB) return;
+    double2 *out = P.grid + ((size_t)row * P.G.nfA + gx0) * P.nt * P.nc + c;
+    const size_t sx = (size_t)P.nt * P.nc, sl = P.nc;
 #pragma unroll
     for (int i = 0; i < T; ++i) {
 #pragma unroll
@@ -783,122 +845,152 @@ __device__ __forceinline__ void sp_store(const SpArgs &P, int tile, int lane,
     }
 }
 
-// One wave sums one entry.  Lanes are (re/im, coil, time group, row); each
-// holds NL time terms x T cells in FP64 registers, so a visit costs NL + 1
-// products and NL T FMAs per lane against one weight load per lane and one
-// set of wave-uniform kernel weights (scalar registers).  Visits are listed
-// 64 at a time (lane v finds its row and sample), then run two at a time from
-// alternating register sets: a set is loaded while the other is consumed.
-// All scalar loads of a set are waited for before the next set's are issued,
-// since scalar loads return in any order.
-template <int NL, int T, bool UNI>
-struct SpSet {
-    double wx[T], wy, w;
-    double u[NL];
-};
-
-template <int NL, int T, bool UNI>
-__global__ __launch_bounds__(64) void k_spread(SpArgs P) {
+// One wave sums one entry.  Lanes are (coil, time group, row); each holds NL
+// time terms x T cells as complex FP64 sums in registers.  Visits go in
+// batches of 64: lane v finds visit v's row and sample, the wave copies the
+// visits' kernel weights and time factors to LDS, then runs over them with the
+// next SP_PF sample weights on their way; a visit costs 2 NL (T + 1) FP64
+// instructions against (T + NL) / 2 broadcast 16-byte LDS reads.
+//
+// The bound is the FP64 rate together with the latency of a visit's operands.
+// Scalar loads for the factors instead (re and im in different lanes) took
+// 528 us per launch on 512^2 x 32 coils; of its variants 588 us had the FP64
+// work taken out and 387 us the loads (640 us with both).  With the factors in
+// LDS: 577 us with one weight on its way, 526 with two, 500 with four; and
+// 468 at a window of 11 cells instead of 12.  250 x 234 x 8 coils: 573 -> 377
+// us; six slices of 128^2..384^2 x 8 coils: 3.26 -> 2.41 ms.  Larger tiles at
+// two waves per SIMD: 628 us (512^2) and 486 (250 x 234).
+constexpr int SP_BATCH = 64, SP_PF = 4;
+template <int NL, int T, bool ROWS>
+__global__ __launch_bounds__(64, NL * T > 24 ? 2 : 3) void k_spread(SpArgs P) {
+    __shared__ double sx[SP_BATCH * T];
+    extern __shared__ double dyn[];      // [SP_BATCH][ntp], then [SP_BATCH][yg] (ROWS)
+    double *su = dyn, *sy = dyn + SP_BATCH * P.ntp;
     const int lane = threadIdx.x;
-    const int wave = blockIdx.x, nwaves = gridDim.x;
-    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
-    const int lg = UNI ? 0 : (lane >> (1 + P.lc)) & ((1 << P.ll) - 1);
-    const int yl = UNI ? 0 : lane >> (1 + P.lc + P.ll);
-    const int slots2 = 2 << P.lc, wdo = 2 * c + part;
-    const int nx = NW + 2 * (T - 1), ny = NW + 2 * (P.G.yg - 1);
-    const int rows = NW + P.G.yg - 1;
-    const int ne = ((cint)(const int *)&P.cnt[P.block])[0];
-    using Set = SpSet<NL, T, UNI>;
+    // workgroups go round the 8 XCDs; each takes SP_RUN entries in a row, whose
+    // samples then stay in that XCD's L2 (gridDim.x is a multiple of 8 SP_RUN)
+    const int wave = (blockIdx.x / (8 * SP_RUN)) * 8 * SP_RUN + (blockIdx.x & 7) * SP_RUN +
+                     ((blockIdx.x >> 3) & (SP_RUN - 1));
+    const int nwaves = gridDim.x;
+    const int c = lane & ((1 << P.lc) - 1), lg = (lane >> P.lc) & ((1 << P.ll) - 1);
+    const int yl = ROWS ? lane >> (P.lc + P.ll) : 0;
+    const int yg = ROWS ? P.G.yg : 1;
+    const int nx = NW + 2 * (T - 1), ny = NW + 2 * (yg - 1);
+    const int rows = NW + yg - 1;
+    // long entries first, so that the launch ends on short ones: runs of split
+    // tiles, then whole tiles by size class
+    const cint pc = (cint)(const int *)&P.cnt[P.block];
+    const int nh = pc[0], nm = nh + pc[1], ne = nm + pc[2];
     for (int e = wave; e < ne; e += nwaves) {
-        const cint ep = (cint)(const int *)(P.entries + (size_t)P.block * P.G.entry_cap + e);
+        const cint ep = (cint)(const int *)(P.entries + (size_t)P.block * P.G.entry_cap +
+                                            (e < nh   ? e
+                                             : e < nm ? SP_SLOTS + e - nh
+                                                      : P.G.entry_cap - 1 - (e - nm)));
         const int tile = ep[0], v0 = ep[1], v1 = ep[2], slot = ep[3];
-        const int gy0 = P.r0 + (tile / P.G.ntx) * P.G.yg, gx0 = (tile % P.G.ntx) * T;
-        double acc[NL][T];
+        const int gy0 = tile_row(P.G, P.block, tile / P.G.ntx), gx0 = (tile % P.G.ntx) * T;
+        double2 acc[NL][T];
 #pragma unroll
         for (int k = 0; k < NL; ++k)
 #pragma unroll
-            for (int i = 0; i < T; ++i) acc[k][i] = 0.0;
-        // lane r holds the sample range of row r
-        int rs = 0, rn = 0;
+            for (int i = 0; i < T; ++i) acc[k][i] = make_double2(0.0, 0.0);
+        // lane r holds the sample range of row r (rows <= 64 - 1 + NW fits: at
+        // most 64 rows per tile are split over the lanes twice)
+        int rs = 0, rn = 0, rs2 = 0, rn2 = 0;
         if (lane < rows) rn = row_range(P.G, P.start, gy0, gx0, lane, &rs);
-        for (int vb = v0; vb < v1; vb += 64) {
-            const int nb = min(64, v1 - vb);
+        if (ROWS && lane + 64 < rows) rn2 = row_range(P.G, P.start, gy0, gx0, lane + 64, &rs2);
+        for (int vb = v0; vb < v1; vb += SP_BATCH) {
+            const int nb = min(SP_BATCH, v1 - vb);
             // visit vb + lane: its row and sample
-            int row = 0, smp = -1, base = 0;
+            int row = 0, smp = 0, base = 0;
             for (int r = 0; r < rows; ++r) {
-                const int n = __builtin_amdgcn_readlane(rn, r);
+                const int n = r < 64 ? __builtin_amdgcn_readlane(rn, r)
+                                     : __builtin_amdgcn_readlane(rn2, r - 64);
+                const int s = r < 64 ? __builtin_amdgcn_readlane(rs, r)
+                                     : __builtin_amdgcn_readlane(rs2, r - 64);
                 const int o = vb + lane - base;
                 if (o >= 0 && o < n) {
                     row = r;
-                    smp = __builtin_amdgcn_readlane(rs, r) + o;
+                    smp = s + o;
                 }
                 base += n;
             }
             int va = 0, vj = 0;
-            smp = max(smp, 0);
             if (lane < nb) {
                 va = P.bx[smp];
                 vj = P.perm[smp];
             }
-            // offset of the tile's first cell in the sample's padded window
-            const int vx = gx0 - va + T - 1;
-            auto load = [&](int i, Set &S) {
-                const int s = __builtin_amdgcn_readlane(smp, i);
-                const int j = __builtin_amdgcn_readlane(vj, i);
-                const int ox = __builtin_amdgcn_readlane(vx, i);
-                // row by = gy0 - (NW - 1) + r: this lane's row takes weight
-                // gy0 + yl - by of the window
-                const int iy = NW - 1 - __builtin_amdgcn_readlane(row, i) + P.G.yg - 1;
-                S.w = P.wd[(size_t)j * slots2 + wdo];
-                const cdbl px = (cdbl)P.wx + ((size_t)s * nx + ox);
-#pragma unroll
-                for (int q = 0; q < T; ++q) S.wx[q] = px[q];
-                if constexpr (UNI) {
-                    S.wy = ((cdbl)P.wy)[(size_t)s * ny + iy];
-#pragma unroll
-                    for (int k = 0; k < NL; ++k) S.u[k] = ((cdbl)P.u)[(size_t)s * P.ntp + k];
-                } else {
-                    S.wy = P.wy[(size_t)s * ny + iy + yl];
-                    const double *pu = P.u + ((size_t)s * P.ntp + lg * NL);
-#pragma unroll
-                    for (int k = 0; k < NL; ++k) S.u[k] = pu[k];
+            // offset of the tile's first cell in the sample's padded window;
+            // row by = gy0 - (NW - 1) + r: tile row y takes weight gy0 + y - by
+            const int ox = gx0 - va + T - 1, oy = NW - 1 - row + yg - 1;
+            __syncthreads();
+            // every lane takes part in the exchanges, also past the last
+            // factor; the visits that pad the batch get factors of zero
+            const int np = (nb + SP_PF - 1) / SP_PF * SP_PF;
+            for (int i0 = 0; i0 < np * T; i0 += 64) {
+                const int i = i0 + lane, v = min(i / T, SP_BATCH - 1), q = i % T;
+                const size_t k = __shfl(smp, v, 64);
+                const int x = __shfl(ox, v, 64), y = ROWS ? 0 : __shfl(oy, v, 64);
+                if (i < np * T) {
+                    double f = 0.0;
+                    if (v < nb) {
+                        f = P.wx[k * nx + x + q];
+                        if (!ROWS) f *= P.wy[k * ny + y];
+                    }
+                    sx[i] = f;
                 }
-            };
-            auto use = [&](const Set &S) {
-                const double v = S.w * S.wy;
-#pragma unroll
-                for (int k = 0; k < NL; ++k) {
-                    const double vu = v * S.u[k];
-#pragma unroll
-                    for (int q = 0; q < T; ++q) acc[k][q] = fma(vu, S.wx[q], acc[k][q]);
+            }
+            for (int i0 = 0; i0 < np * P.ntp; i0 += 64) {
+                const int i = i0 + lane, v = min(i / P.ntp, SP_BATCH - 1);
+                const size_t k = __shfl(smp, v, 64);
+                if (i < np * P.ntp) su[i] = v < nb ? P.u[k * P.ntp + (i - v * P.ntp)] : 0.0;
+            }
+            if (ROWS)
+                for (int i0 = 0; i0 < np * yg; i0 += 64) {
+                    const int i = i0 + lane, v = min(i / yg, SP_BATCH - 1);
+                    const size_t k = __shfl(smp, v, 64);
+                    const int y = __shfl(oy, v, 64);
+                    if (i < np * yg) sy[i] = v < nb ? P.wy[k * ny + y + (i - v * yg)] : 0.0;
                 }
+            __syncthreads();
+            // SP_PF sample weights are on their way; visits past nb take zero
+            auto weight = [&](int i) {
+                return P.wd[((size_t)__builtin_amdgcn_readlane(vj, min(i, nb - 1)) << P.lc) + c];
             };
-            // scalar loads issued so far have arrived
-            auto arrived = [] {
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            Set s0, s1;
-            load(0, s0);
-            // an odd count runs its last visit again with weight zero: one
-            // loop and no copies of the accumulators
-            for (int i = 0; i < nb; i += 2) {
-                arrived();
-                load(min(i + 1, nb - 1), s1);
-                __builtin_amdgcn_sched_barrier(0);
-                use(s0);
-                arrived();
-                if (i + 1 >= nb) s1.wy = 0.0;
-                load(min(i + 2, nb - 1), s0);
-                __builtin_amdgcn_sched_barrier(0);
-                use(s1);
+            double2 w[SP_PF];
+#pragma unroll
+            for (int h = 0; h < SP_PF; ++h) w[h] = weight(h);
+            for (int i0 = 0; i0 < nb; i0 += SP_PF) {
+#pragma unroll
+                for (int h = 0; h < SP_PF; ++h) {
+                    const int i = i0 + h;
+                    double2 v = w[h];
+                    if (i >= nb) v = make_double2(0.0, 0.0);
+                    w[h] = weight(i + SP_PF);
+                    if (ROWS) {
+                        const double y = sy[i * yg + yl];
+                        v.x *= y;
+                        v.y *= y;
+                    }
+                    double wx[T];
+#pragma unroll
+                    for (int q = 0; q < T; ++q) wx[q] = sx[i * T + q];
+                    const double *pu = su + i * P.ntp + lg * NL;
+#pragma unroll
+                    for (int k = 0; k < NL; ++k) {
+                        const double u = pu[k], re = v.x * u, im = v.y * u;
+#pragma unroll
+                        for (int q = 0; q < T; ++q) {
+                            acc[k][q].x = fma(re, wx[q], acc[k][q].x);
+                            acc[k][q].y = fma(im, wx[q], acc[k][q].y);
+                        }
+                    }
+                }
             }
         }
         if (slot < 0) {
             sp_store<NL, T>(P, tile, lane, acc);
         } else {
-            double *o = P.part + (size_t)slot * NL * T * 64 + lane;
+            double2 *o = P.part + (size_t)slot * NL * T * 64 + lane;
 #pragma unroll
             for (int k = 0; k < NL; ++k)
 #pragma unroll
@@ -913,39 +1005,45 @@ template <int NL, int T>
 __global__ __launch_bounds__(256) void k_spread_multi(SpArgs P) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    const int part = lane & 1, c = (lane >> 1) & ((1 << P.lc) - 1);
-    const int lg = (lane >> (1 + P.lc)) & ((1 << P.ll) - 1), yg = lane >> (1 + P.lc + P.ll);
+    const int c = lane & ((1 << P.lc) - 1), lg = (lane >> P.lc) & ((1 << P.ll) - 1);
+    const int yl = lane >> (P.lc + P.ll);
     const int n = P.cnt[P.block].multis * NL;
     for (int e = wave; e < n; e += gridDim.x * 4) {
         const SpMulti M = P.multis[(size_t)P.block * SP_SLOTS + e / NL];
         const int k = e % NL;
-        double acc[T];
+        double2 acc[T];
 #pragma unroll
-        for (int i = 0; i < T; ++i) acc[i] = 0.0;
-        const double *o = P.part + ((size_t)M.slot * NL + k) * T * 64 + lane;
+        for (int i = 0; i < T; ++i) acc[i] = make_double2(0.0, 0.0);
+        const double2 *o = P.part + ((size_t)M.slot * NL + k) * T * 64 + lane;
 #pragma unroll 2
         for (int r = 0; r < M.n; ++r, o += NL * T * 64)
 #pragma unroll
-            for (int i = 0; i < T; ++i) acc[i] += o[i * 64];
-        const int row = (M.tile / P.G.ntx) * P.G.yg + yg, gx0 = (M.tile % P.G.ntx) * T;
+            for (int i = 0; i < T; ++i) {
+                const double2 v = o[i * 64];
+                acc[i].x += v.x;
+                acc[i].y += v.y;
+            }
+        const int row = (M.tile / P.G.ntx) * P.G.yg + yl, gx0 = (M.tile % P.G.ntx) * T;
         const int l = lg * NL + k;
-        if (c >= P.nc || row >= P.G.rb || P.r0 + row >= P.G.nfB || l >= P.nt) continue;
-        double *g = P.grid +
-                    ((((size_t)row * P.G.nfA + gx0) * P.nt + l) * P.nc + c) * 2 + part;
+        if (c >= P.nc || tile_row(P.G, P.block, M.tile / P.G.ntx) + yl >= P.G.nfB || l >= P.nt)
+            continue;
+        double2 *g = P.grid + (((size_t)row * P.G.nfA + gx0) * P.nt + l) * P.nc + c;
 #pragma unroll
         for (int i = 0; i < T; ++i)
-            if (gx0 + i < P.G.nfA) g[(size_t)i * P.nt * P.nc * 2] = acc[i];
+            if (gx0 + i < P.G.nfA) g[(size_t)i * P.nt * P.nc] = acc[i];
     }
 }
 
-// tile shape for nl time terms per lane: about 48 FP64 accumulators
-constexpr int sp_cells(int nl) { return nl >= 13 ? 3 : nl >= 10 ? 4 : nl >= 8 ? 6 : nl == 7 ? 7
-                                        : nl == 6 ? 8 : nl == 5 ? 10 : nl == 4 ? 12 : 16; }
+// cells per tile for nl time terms per lane: about 24 complex accumulators,
+// which leave three waves per SIMD up to 12 time terms
+constexpr int sp_cells(int nl) {
+    return nl >= 9 ? 2 : nl >= 7 ? 3 : nl >= 5 ? 4 : nl == 4 ? 6 : nl == 3 ? 8 : nl == 2 ? 8 : 8;
+}
 
 using SpFn = void (*)(SpArgs);
 template <int NL>
-SpFn sp_pick1(bool uni) {
-    return uni ? (SpFn)k_spread<NL, sp_cells(NL), true> : (SpFn)k_spread<NL, sp_cells(NL), false>;
+SpFn sp_pick1(bool rows) {
+    return rows ? (SpFn)k_spread<NL, sp_cells(NL), true> : (SpFn)k_spread<NL, sp_cells(NL), false>;
 }
 template <int NL>
 SpFn sp_multi1() { return (SpFn)k_spread_multi<NL, sp_cells(NL)>; }
@@ -1949,7 +2047,6 @@ struct NuPass {
     std::vector<double> tab;       // coefficients, recurrence, mul, KB polynomials
     size_t tab_mul = 0, tab_poly = 0;
     int cg = 1, groups = 1, lc = 0, ll = 0, nl = 1, yg = 1, T = 1, ntp = 1, blocks = 1;
-    bool uni = false;
     SpGeom S{};
     Carver W;
     size_t o_bx, o_wx, o_wy, o_u, o_wd, o_vis, o_cnt, o_ent, o_mul, o_part, o_tab, o_start,
@@ -2026,16 +2123,29 @@ struct NuPass {
         const NuAxis &A = G.A, &B = G.B;
         cg = std::min(32, 1 << log2i(ncols));
         while (cg > 1 && (size_t)A.n * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
-        // wave layout: column slots x time groups x rows = 32 lane pairs;
-        // fewer columns when the time terms need more groups
-        while (cg > 1 && ceil_div(nt, 32 / cg) > SP_MAX_NL) cg /= 2;
+        // wave layout: column slots x time groups x rows = 64 lanes; fewer
+        // columns when the time terms need more groups
+        while (cg > 1 && ceil_div(nt, 64 / cg) > SP_MAX_NL) cg /= 2;
         groups = ceil_div(ncols, cg);
         lc = log2i(cg);
-        ll = std::min(5 - lc, log2i(nt));
-        nl = ceil_div(nt, 1 << ll);
-        yg = 1 << (5 - lc - ll);
-        uni = lc == 5;
-        T = sp_switch(nl, [](auto k) { return sp_cells(decltype(k)::value); });
+        // the split of the other lanes with the fewest FP64 instructions per
+        // sample: visits x (2 NL (T + 1) + about 16 for the rest)
+        double best = 0.0;
+        for (int l = 0; l <= std::min(6 - lc, log2i(nt)); ++l) {
+            const int k = ceil_div(nt, 1 << l);
+            if (k > SP_MAX_NL) continue;
+            const int cells = sp_switch(k, [](auto n) { return sp_cells(decltype(n)::value); });
+            const int rows = 1 << (6 - lc - l);
+            const double cost = (double)(NW + rows - 1) / rows * (NW + cells - 1) / cells *
+                                (2 * k * (cells + 1) + 16);
+            if (best == 0.0 || cost < best) {
+                best = cost;
+                ll = l;
+                nl = k;
+                yg = rows;
+                T = cells;
+            }
+        }
         ntp = nl << ll;
         S.T = T;
         S.yg = yg;
@@ -2053,7 +2163,9 @@ struct NuPass {
         blocks = ceil_div(B.nf, rb);
         S.rb = rb;
         S.nty = rb / yg;
-        S.entry_cap = S.ntx * S.nty + SP_SLOTS;
+        S.bw = T >= 6 ? 8 : 16;
+        S.ntile = ceil_div(S.ntx, S.bw) * ceil_div(S.nty, SP_RUN / S.bw) * SP_RUN;
+        S.entry_cap = S.ntile + SP_SLOTS;
         const int ncells = S.ncA * S.ncB;
         o_start = W.take(((size_t)ncells + 1) * 4);
         o_bx = W.take((size_t)m * 4);
@@ -2061,11 +2173,11 @@ struct NuPass {
         o_wy = W.take((size_t)m * (NW + 2 * (yg - 1)) * 8);
         o_u = W.take((size_t)m * ntp * 8);
         o_wd = W.take((size_t)m * (1 << lc) * sizeof(double2));
-        o_vis = W.take((size_t)blocks * S.ntx * S.nty * 4);
+        o_vis = W.take((size_t)blocks * S.ntile * 4);
         o_cnt = W.take((size_t)blocks * sizeof(SpCount));
         o_ent = W.take((size_t)blocks * S.entry_cap * sizeof(SpEntry));
         o_mul = W.take((size_t)blocks * SP_SLOTS * sizeof(SpMulti));
-        o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * 8);
+        o_part = W.take((size_t)SP_SLOTS * nl * T * 64 * sizeof(double2));
         take_tables();
         o_grid = W.take((size_t)rb * row_bytes);
         o_mid = W.take((size_t)A.n * B.nf * nt * nc0 * sizeof(double2));
@@ -2113,7 +2225,7 @@ struct NuPass {
         IMP_TRY(alloc(cA, sA, cB, sB));
         const hipStream_t st = ctx->stream;
         const dim3 b256(256);
-        const int ncells = S.ncA * S.ncB, ntile = S.ntx * S.nty;
+        const int ncells = S.ncA * S.ncB, ntile = S.ntile;
         SpCount *cnt = at<SpCount *>(o_cnt);
         hipLaunchKernelGGL(k_nu_starts, dim3(ceil_div(ncells + 1, 256)), b256, 0, st, m, key,
                            ncells, at<int *>(o_start), (int *)cnt,
@@ -2149,7 +2261,7 @@ struct NuPass {
     int to_mid(int nc) {
         const hipStream_t st = ctx->stream;
         const int nq = nt * nc;
-        SpFn spread = sp_switch(nl, [&](auto k) { return sp_pick1<decltype(k)::value>(uni); });
+        SpFn spread = sp_switch(nl, [&](auto k) { return sp_pick1<decltype(k)::value>(yg > 1); });
         SpFn multi = sp_switch(nl, [](auto k) { return sp_multi1<decltype(k)::value>(); });
         SpArgs P{};
         P.G = S;
@@ -2164,20 +2276,20 @@ struct NuPass {
         P.wx = at<const double *>(o_wx);
         P.wy = at<const double *>(o_wy);
         P.u = at<const double *>(o_u);
-        P.wd = at<const double *>(o_wd);
+        P.wd = at<const double2 *>(o_wd);
         P.cnt = at<const SpCount *>(o_cnt);
         P.entries = at<const SpEntry *>(o_ent);
         P.multis = at<const SpMulti *>(o_mul);
-        P.part = at<double *>(o_part);
-        P.grid = at<double *>(o_grid);
+        P.part = at<double2 *>(o_part);
+        P.grid = at<double2 *>(o_grid);
         LineArgs LA = line(0, ws + o_grid, (size_t)G.A.nf * nq, nq, nq);
         for (int b = 0; b < blocks; ++b) {
-            P.r0 = b * S.rb;
             P.block = b;
             // one-wave workgroups: a wave that ends makes room at once
             const int rec = prof_begin(ctx, "k_spread");
-            hipLaunchKernelGGL(spread, dim3(std::min(S.entry_cap, 64 * ctx->num_cus)), dim3(64),
-                               0, st, P);
+            const int wgs = ceil_div(std::min(S.entry_cap, 64 * ctx->num_cus), 8 * SP_RUN);
+            hipLaunchKernelGGL(spread, dim3(wgs * 8 * SP_RUN), dim3(64),
+                               SP_BATCH * (ntp + (yg > 1 ? yg : 0)) * sizeof(double), st, P);
             prof_end(ctx, rec);
             hipLaunchKernelGGL(multi, dim3(4 * ctx->num_cus), dim3(256), 0, st, P);
             IMP_CHECK_LAUNCH();

@@ -10,12 +10,16 @@ namespace imp {
 // Every operator below returns IMP_ENOMEM before it has written a result when
 // its workspace cannot be had; callers then take the direct path.
 
+// Points c0 + i d: read the transform's bins; nearly so: a first-order step
+// from the bins; any other: interpolate.
+enum { AX_UNIFORM, AX_NEAR, AX_FREE };
+
 // One image axis against the sample coordinate k it pairs with.
 struct NuAxis {
     int n;            // image points
     int L;            // transform length
     int nf;           // spread-grid points (every sample's window fits)
-    int uniform;      // points are c0 + i d: read the bins, else interpolate
+    int kind;         // AX_*
     int flip;         // d < 0
     int shift;        // grid point of bin 0, mod L
     double kc;        // centre of k

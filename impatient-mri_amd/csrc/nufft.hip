@@ -16,9 +16,10 @@
 //           divided out (nonuniform FFT of types 1 and 3: Dutt and Rokhlin
 //           1993, Greengard and Lee 2004, Lee and Greengard 2005);
 //   axes    the image points must form a tensor grid (checked on the device,
-//           bit for bit).  Uniform axes read the FFT's bins; others (for
-//           example (i - N/2)/N rounded to float with N no power of two)
-//           interpolate in the transformed line with the same kernel.
+//           bit for bit).  Uniform axes read the FFT's bins, nearly uniform
+//           ones ((i - N/2)/N rounded to float with N no power of two) take
+//           a first-order step from them, others interpolate in the
+//           transformed line with the same kernel.
 // All sums, grids and transforms are FP64 (half the FP32 rate here), so the
 // result carries the rounding of its final FP32 store only.
 //
@@ -1087,11 +1088,14 @@ __host__ __device__ constexpr int lines(int L, int wg) {
     return n;
 }
 __host__ __device__ constexpr int bits(int n) { return n <= 1 ? 0 : 1 + bits(n / 2); }
+// lengths 12 2^k and 144 2^k: radix-12 stages, then 4 and 2
+__host__ __device__ constexpr int twelves(int L) { return L % 9 ? 1 : 2; }
+__host__ __device__ constexpr int rest(int L) { return L / (L % 9 ? 12 : 144); }
 __host__ __device__ constexpr int stages(int L) {
-    return has3(L) ? 1 + (bits(L / 12) + 1) / 2 : (bits(L) + 2) / 3;
+    return has3(L) ? twelves(L) + (bits(rest(L)) + 1) / 2 : (bits(L) + 2) / 3;
 }
 __host__ __device__ constexpr int radix(int L, int s) {
-    return has3(L) ? (s == 0 ? 12 : (bits(L / 12) - 2 * (s - 1) >= 2 ? 4 : 2))
+    return has3(L) ? (s < twelves(L) ? 12 : (bits(rest(L)) - 2 * (s - twelves(L)) >= 2 ? 4 : 2))
                    : (bits(L) - 3 * s >= 3 ? 8 : 1 << (bits(L) - 3 * s));
 }
 __host__ __device__ constexpr int span(int L, int s) {
@@ -1118,9 +1122,16 @@ __device__ __forceinline__ void butterflies(double2 (&v)[vals(L)], int t, const 
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         if constexpr (NS > 1) {
+            // one twiddle is loaded, the others are its powers (the combining
+            // pass of 512^2 x 32 coils took 1.63 ms with table reads, 0.95
+            // with none)
             const int k = (t + threads(L) * b) % NS, step = (L / (NS * R)) * k;
+            double2 w[R];
+            w[1] = tw[step];
 #pragma unroll
-            for (int r = 1; r < R; ++r) v[b * R + r] = cmul(v[b * R + r], tw[r * step]);
+            for (int r = 2; r < R; ++r) w[r] = cmul(w[r / 2], w[r - r / 2]);
+#pragma unroll
+            for (int r = 1; r < R; ++r) v[b * R + r] = cmul(v[b * R + r], w[r]);
         }
         fftc::dft<R, true>(&v[b * R]);
     }
@@ -1164,8 +1175,9 @@ __device__ __forceinline__ void transform(double2 (&v)[vals(L)], int t, int c, d
 }
 }  // namespace ln
 
-// One axis' tables: twiddles [L], input scale [nf] (nonuniform axes) and
-// output weights: [n] (uniform) or [n][NW] with window starts base[n].
+// One axis' tables: twiddles [L]; input scale [nf] (AX_FREE); output weights
+// [n], followed by the points' offsets [n] from their bins in radians per cell
+// (AX_NEAR), or [n][NW] with window starts base[n] (AX_FREE).
 struct AxisTab {
     NuAxis X;
     const float *coord;
@@ -1184,13 +1196,17 @@ __global__ void k_nu_axis(AxisTab ta, AxisTab tb) {
         sincospi(2.0 * i / X.L, &s, &c);
         P.tw[i] = make_double2(c, s);
     }
-    if (!X.uniform && i < X.nf) P.inw[i] = 1.0 / kb_hat((i - X.j0) / X.L);
+    if (X.kind == AX_FREE && i < X.nf) P.inw[i] = 1.0 / kb_hat((i - X.j0) / X.L);
     if (i >= X.n) return;
-    if (X.uniform) {
-        P.outw[i] = 1.0 / kb_hat((double)(i - X.n / 2) / X.L);
+    // cycles per cell
+    const double u0 = (double)(i - X.n / 2) / X.L;
+    const double u = X.kind == AX_UNIFORM
+                         ? u0 : ((double)P.coord[(size_t)i * P.stride] - X.xc) / X.inv_d;
+    if (X.kind != AX_FREE) {
+        P.outw[i] = 1.0 / kb_hat(u);
+        if (X.kind == AX_NEAR) P.outw[X.n + i] = 2.0 * M_PI * (u - (X.flip ? -u0 : u0));
     } else {
-        // cycles per cell, and the position in the transformed line
-        const double u = ((double)P.coord[(size_t)i * P.stride] - X.xc) / X.inv_d;
+        // the position in the transformed line
         const double p = u * X.L, h = kb_hat(u);
         const int b = (int)ceil(p - 0.5 * NW);
         P.base[i] = b;
@@ -1198,10 +1214,9 @@ __global__ void k_nu_axis(AxisTab ta, AxisTab tb) {
     }
 }
 
-// threads per workgroup: whole 128-byte row segments for the storing pass;
-// the combining pass, whose accumulators leave 3 waves per SIMD, runs
-// smaller ones so that several share a CU
-constexpr int ST_WG = 256, CO_WG = 256;
+// threads per workgroup: several share a CU, also in the combining pass, whose
+// accumulators leave 2 to 3 waves per SIMD
+constexpr int ST_WG = 256;
 
 struct LineArgs {
     const double2 *in;          // element j of line x, column q: in[x in_line + j in_el + q]
@@ -1214,37 +1229,64 @@ struct LineArgs {
     const int *base;
 };
 
-// Loads element i (mod L) of a line: grid points j = i + j0 mod L, folded on
-// uniform axes (there the grid is L-periodic exactly) and scaled on others.
+// Loads the elements in_idx<L, 0> (mod L) of a line: grid points j = i + j0 mod
+// L, folded unless the axis is AX_FREE (there the grid is L-periodic exactly),
+// scaled on AX_FREE axes, times j - j0 for the first-order pass of AX_NEAR.
 // base is wave-uniform and the lane offsets are 32 bits wide (a line's
 // elements span far less than 4 GB): one address register per element.
-template <bool UNI>
-__device__ __forceinline__ double2 line_load(const LineArgs &P, const double2 *base, unsigned c,
-                                             int L, int i) {
-    double2 s = make_double2(0.0, 0.0);
-    int j = i + P.X.shift;
-    if (j >= L) j -= L;
-    if constexpr (UNI) {
-        for (; j < P.X.nf; j += L) {
-            const double2 v = base[(unsigned)j * P.in_el + c];
-            s.x += v.x;
-            s.y += v.y;
+// Every lane loads, from a clamped place, and selects afterwards: loads under
+// a lane's condition are waited for one by one (384-point lines 93 -> 71 us).
+template <int L, int KIND>
+__device__ __forceinline__ void line_load(const LineArgs &P, const double2 *base, int t,
+                                          unsigned q, bool ok, int order,
+                                          double2 (&v)[ln::vals(L)]) {
+    constexpr int E = ln::vals(L), R0 = ln::radix(L, 0);
+    const unsigned cl = ok ? q : 0;
+    const int last = P.X.nf - 1, j0 = (int)P.X.j0;
+    auto at = [&](int i) {
+        const int j = ln::in_idx<L, 0>(t, i / R0, i % R0) + P.X.shift;
+        return j >= L ? j - L : j;
+    };
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const int j = at(i);
+        const double2 x = base[(unsigned)min(j, last) * P.in_el + cl];
+        v[i] = ok && j <= last ? x : make_double2(0.0, 0.0);
+        if constexpr (KIND == AX_FREE) {
+            const double w = P.inw[min(j, last)];
+            v[i] = make_double2(v[i].x * w, v[i].y * w);
         }
-    } else if (j < P.X.nf) {
-        const double2 v = base[(unsigned)j * P.in_el + c];
-        const double w = P.inw[j];
-        s = make_double2(v.x * w, v.y * w);
+        if (KIND == AX_NEAR && order) {
+            const double w = j - j0;
+            v[i] = make_double2(v[i].x * w, v[i].y * w);
+        }
     }
-    return s;
+    if constexpr (KIND != AX_FREE)
+        for (int o = L; o <= last; o += L) {
+#pragma unroll
+            for (int i = 0; i < E; ++i) {
+                const int j = at(i) + o;
+                if (ok && j <= last) {
+                    const double2 x = base[(unsigned)j * P.in_el + cl];
+                    const double w = KIND == AX_NEAR && order ? j - j0 : 1;
+                    v[i].x = fma(x.x, w, v[i].x);
+                    v[i].y = fma(x.y, w, v[i].y);
+                }
+            }
+        }
 }
 
-// bin of an L-point transform -> image index on a uniform axis (or >= n)
+__device__ __forceinline__ double2 times_i(double2 v, double f) {
+    return make_double2(-f * v.y, f * v.x);
+}
+
+// bin of an L-point transform -> image index, not on AX_FREE axes (or >= n)
 __device__ __forceinline__ unsigned bin_index(const NuAxis &X, int L, int i) {
     const int f = i < L / 2 ? i : i - L;
     return (unsigned)((X.flip ? -f : f) + X.n / 2);
 }
 
-// Interpolated values of the thread's outputs o = t + T m (nonuniform axes).
+// Interpolated values of the thread's outputs o = t + T m (AX_FREE axes).
 template <int L, int W>
 __device__ __forceinline__ void line_interp(const LineArgs &P, double2 (&v)[ln::vals(L)], int t,
                                             int c, double *buf, double2 (&o)[ln::vals(L)]) {
@@ -1261,28 +1303,50 @@ __device__ __forceinline__ void line_interp(const LineArgs &P, double2 (&v)[ln::
                     h ? v[b * R + r].y : v[b * R + r].x;
         __syncthreads();
 #pragma unroll
-        for (int m = 0; m < E; ++m) {
-            const int i = t + T * m;
-            double s = 0.0;
-            if (i < P.X.n) {
+        for (int m = 0; m < E; m += 2) {
+            // two outputs' weights are loaded together; not more, and neither
+            // they nor their places are kept from re to im (registers), nor are
+            // the sums put off until the results are used
+            int im = t + T * m;
+            asm volatile("" : "+v"(im));
+            double s[2] = {0.0, 0.0};
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                const int i = min(im + T * g, P.X.n - 1);
                 const int b = P.base[i];
                 const double *w = P.outw + (size_t)i * NW;
-#pragma unroll 2
+#pragma unroll
                 for (int k = 0; k < NW; ++k) {
                     int p = b + k;
                     p += p < 0 ? L : 0;
-                    s = fma(w[k], buf[ln::pad(L, p) * W + c], s);
+                    s[g] = fma(w[k], buf[ln::pad(L, p) * W + c], s[g]);
                 }
             }
-            if (h) o[m].y = s;
-            else o[m].x = s;
+            asm volatile("" : "+v"(s[0]), "+v"(s[1]));
+            if (h) {
+                o[m].y = s[0];
+                o[m + 1].y = s[1];
+            } else {
+                o[m].x = s[0];
+                o[m + 1].x = s[1];
+            }
         }
     }
 }
 
 // One axis of a grid: out[i out_el + line out_line + q].
-template <int L, bool UNI>
-__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG)) void k_line_store(
+//
+// AX_NEAR points lie e off their bins (radians per cell, e j < 6e-5: rounded
+// coordinates): e^{i j (u + e)} = e^{i j u} (1 + i j e) to 2e-9, so a second
+// transform, of j g[j], takes the place of interpolation from a line 1.5 times
+// as long (384^2 x 8 coils, two slices: 1.47 -> 0.79 ms, of which 0.45 were LDS
+// reads for the interpolation; 250 x 234 x 8 coils: 251 -> 136 us).
+//
+// Bound by memory: 512^2 x 32 coils, 768-point lines, 3.1 TB/s (reads alone 127
+// us, writes 87, the transforms 14 of 247 us per launch).
+template <int L, int KIND>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG),
+                             KIND == AX_NEAR ? 2 : 4) void k_line_store(
     LineArgs P, double2 *out, size_t out_line, size_t out_el) {
     constexpr int E = ln::vals(L), W = ln::lines(L, ST_WG), T = ln::threads(L);
     __shared__ double buf[ln::words(L, W)];
@@ -1294,25 +1358,15 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG)) void k_line_s
     const int line = b / np, q = (b % np) * W + c;
     if (line >= P.nlines) return;
     const bool ok = q < P.nq;
-    const double2 *base = P.in + (size_t)line * P.in_line + (q - c);
-    double2 v[E];
-    constexpr int R0 = ln::radix(L, 0);
-#pragma unroll
-    for (int i = 0; i < E; ++i)
-        v[i] = ok ? line_load<UNI>(P, base, c, L, ln::in_idx<L, 0>(t, i / R0, i % R0)) : make_double2(0., 0.);
-    ln::transform<L, W>(v, t, c, buf, P.tw);
+    const double2 *base = P.in + (size_t)line * P.in_line;
     double2 *o = out + (size_t)line * out_line + q;
-    if constexpr (UNI) {
-        constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
-#pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(t, i / R, i % R));
-            if (ok && x < (unsigned)P.X.n) {
-                const double w = P.outw[x];
-                o[x * out_el] = make_double2(v[i].x * w, v[i].y * w);
-            }
-        }
-    } else {
+    constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
+    int tp = t;
+    auto bin = [&](int i) { return bin_index(P.X, L, ln::out_idx<L, S>(tp, i / R, i % R)); };
+    double2 v[E];
+    if constexpr (KIND == AX_FREE) {
+        line_load<L, KIND>(P, base, t, q, ok, 0, v);
+        ln::transform<L, W>(v, t, c, buf, P.tw);
         double2 x[E];
         line_interp<L, W>(P, v, t, c, buf, x);
 #pragma unroll
@@ -1320,86 +1374,140 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG)) void k_line_s
             const int i = t + T * m;
             if (ok && i < P.X.n) o[i * out_el] = x[m];
         }
+        return;
     }
+    double2 d[E];
+    if constexpr (KIND == AX_NEAR) {
+        line_load<L, KIND>(P, base, t, q, ok, 1, d);
+        ln::transform<L, W>(d, t, c, buf, P.tw);
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+            d[i] = times_i(d[i], P.outw[P.X.n + min(bin(i), (unsigned)P.X.n - 1)]);
+    }
+    if constexpr (KIND == AX_NEAR) asm volatile("" : "+v"(tp));   // indices anew: registers
+    line_load<L, KIND>(P, base, tp, q, ok, 0, v);
+    ln::transform<L, W>(v, tp, c, buf, P.tw);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+        const double w = P.outw[min(bin(i), (unsigned)P.X.n - 1)];
+        if constexpr (KIND == AX_NEAR) v[i] = make_double2(v[i].x + d[i].x, v[i].y + d[i].y);
+        v[i] = make_double2(v[i].x * w, v[i].y * w);
+    }
+#pragma unroll
+    for (int i = 0; i < E; ++i)
+        if (ok && bin(i) < (unsigned)P.X.n) o[bin(i) * out_el] = v[i];
 }
 
 // Last axis with the time and coil sums: line = ia, out over ib.
-// partial[split][ia][ib] = sum over the split's columns of
-// i^(l mod 2) vt[l] conj(S_c) P_(l,c).
-template <int L, bool UNI>
-__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_line_combine(
-    LineArgs P, int ncg, int splits, const double *vt, const float2 *sens, unsigned nvox,
-    double2 *partial) {
-    constexpr int E = ln::vals(L), W = ln::lines(L, CO_WG), T = ln::threads(L);
+// partial[split][ia][ib] = sum over the split's coils and time terms of
+// conj(S_c) i^(l mod 2) vt[l] P_(l,c).
+//
+// A workgroup's W columns are 2^lcw coils (up to W of them) times W >> lcw time
+// terms; it steps through its time terms, keeps their sum per coil in
+// registers, and applies conj(S) once at the end.  (One pass over all columns
+// with conj(S) applied to each read the maps nt times, half the kernel's time.)
+// A workgroup with several sets of coils adds them to its partial image.
+//
+// Bound by the latency of a step (load, three exchanges, factors) at three
+// waves per SIMD, which the bounds above keep free of spills: 512^2 x 32 coils
+// 1.62 -> 0.92 ms (2.6 TB/s), 250 x 234 x 8 coils 290 -> 148 us, two slices of
+// 384^2 x 8 coils 1.12 -> 0.55 ms.
+struct CombineArgs {
+    int nc, nt;             // coils, time terms
+    int lcw, ncs, nls;      // log2 of the coils side by side; splits of coils, of time terms
+    const double *vt;
+    const float2 *sens;
+    unsigned nvox;
+    double2 *partial;
+};
+
+template <int L, int KIND>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG), 3) void k_line_combine(
+    LineArgs P, CombineArgs C) {
+    constexpr int E = ln::vals(L), W = ln::lines(L, ST_WG), T = ln::threads(L);
     __shared__ double buf[ln::words(L, W)];
     const int c = threadIdx.x % W, t = threadIdx.x / W;
-    const int np = (P.nq + W - 1) / W;
+    const int splits = C.ncs * C.nls;
     const int line = blockIdx.x / splits, split = blockIdx.x % splits;
-    const int p0 = (int)((long)np * split / splits), p1 = (int)((long)np * (split + 1) / splits);
-    constexpr int R0 = ln::radix(L, 0), S = ln::stages(L) - 1, R = ln::radix(L, S);
-    double2 acc[E];
-#pragma unroll
-    for (int i = 0; i < E; ++i) acc[i] = make_double2(0.0, 0.0);
-    const double *vline = vt + (size_t)line * P.X.n;
-    const float2 *sline = sens ? sens + (size_t)line * P.X.n : nullptr;
+    const int cs = split / C.nls, ls = split % C.nls;
+    const int cw = 1 << C.lcw, g = W >> C.lcw;
+    const int ncp = (C.nc + cw - 1) >> C.lcw, nst = (C.nt + g - 1) / g;
+    const int s0 = nst * ls / C.nls, s1 = nst * (ls + 1) / C.nls;
+    constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
+    const double2 *base = P.in + (size_t)line * P.in_line;
     // offsets within vt and sens stay below 2^32 bytes (checked at launch)
-    auto add = [&](int i, unsigned x, double2 p, unsigned vo, unsigned so, bool odd) {
-        if (sens) {
-            const float2 s = sline[so + x];
-            p = make_double2(p.x * s.x + p.y * s.y, p.y * s.x - p.x * s.y);
-        }
-        const double f = vline[vo + x];
-        acc[i].x = fma(f, odd ? -p.y : p.x, acc[i].x);
-        acc[i].y = fma(f, odd ? p.x : p.y, acc[i].y);
+    const double *vline = C.vt + (size_t)line * P.X.n;
+    double2 *out = C.partial + (size_t)split * C.nvox + (size_t)line * P.X.n;
+    const unsigned nmax = (unsigned)P.X.n - 1;
+    auto index = [&](int tp, int i) -> unsigned {
+        if constexpr (KIND == AX_FREE) return tp + T * i;
+        else return bin_index(P.X, L, ln::out_idx<L, S>(tp, i / R, i % R));
     };
-    for (int p = p0; p < p1; ++p) {
-        // opaque to the optimizer: the LDS and element indices are recomputed
-        // per panel instead of being held in registers across panels (spills)
-        int tp = t;
-        asm volatile("" : "+v"(tp));
-        const int q = p * W + c;
-        const bool ok = q < P.nq;
-        const int l = ok ? q / ncg : 0, cc = ok ? q - l * ncg : 0;
-        const double2 *base = P.in + (size_t)line * P.in_line + p * W;
-        double2 v[E];
+    for (int cp = ncp * cs / C.ncs; cp < ncp * (cs + 1) / C.ncs; ++cp) {
+        const int cc = (cp << C.lcw) + (c & (cw - 1));
+        double2 acc[E];
 #pragma unroll
-        for (int i = 0; i < E; ++i)
-            v[i] = ok ? line_load<UNI>(P, base, c, L, ln::in_idx<L, 0>(tp, i / R0, i % R0))
-                      : make_double2(0., 0.);
-        ln::transform<L, W>(v, tp, c, buf, P.tw);
-        const unsigned vo = (unsigned)l * nvox, so = (unsigned)cc * nvox;
-        if constexpr (UNI) {
+        for (int i = 0; i < E; ++i) acc[i] = make_double2(0.0, 0.0);
+        // steps through the time terms, on AX_NEAR axes twice each (k_line_store)
+        constexpr int ORD = KIND == AX_NEAR ? 2 : 1;
+        for (int s = s0 * ORD; s < s1 * ORD; ++s) {
+            // opaque to the optimizer: the LDS and element indices are recomputed
+            // per step instead of being held in registers across them (spills)
+            int tp = t;
+            asm volatile("" : "+v"(tp));
+            const int order = s % ORD, l = (s / ORD) * g + (c >> C.lcw);
+            const bool ok = cc < C.nc && l < C.nt;
+            double2 v[E];
+            line_load<L, KIND>(P, base, tp, l * C.nc + cc, ok, order, v);
+            ln::transform<L, W>(v, tp, c, buf, P.tw);
+            if constexpr (KIND == AX_FREE) {
+                double2 x[E];
+                line_interp<L, W>(P, v, tp, c, buf, x);
+#pragma unroll
+                for (int i = 0; i < E; ++i) v[i] = x[i];
+            }
+            // columns past the last hold zeros; elements past the image are
+            // summed but not stored
+            const unsigned vo = (ok ? l : 0) * C.nvox;
+            asm volatile("" : "+v"(tp));
 #pragma unroll
             for (int i = 0; i < E; ++i) {
-                const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(tp, i / R, i % R));
-                if (ok && x < (unsigned)P.X.n) add(i, x, v[i], vo, so, l & 1);
+                const unsigned x = min(index(tp, i), nmax);
+                double f = vline[vo + x];
+                double2 p = l & 1 ? make_double2(-v[i].y, v[i].x) : v[i];
+                if (KIND == AX_NEAR && order) p = times_i(p, P.outw[P.X.n + x]);
+                acc[i].x = fma(f, p.x, acc[i].x);
+                acc[i].y = fma(f, p.y, acc[i].y);
+                if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
             }
-        } else {
-            double2 o[E];
-            line_interp<L, W>(P, v, tp, c, buf, o);
-#pragma unroll
-            for (int m = 0; m < E; ++m)
-                if (ok && tp + T * m < P.X.n) add(m, tp + T * m, o[m], vo, so, l & 1);
         }
-    }
-    double2 *out = partial + (size_t)split * nvox + (size_t)line * P.X.n;
+        int te = t;
+        asm volatile("" : "+v"(te));
 #pragma unroll
-    for (int i = 0; i < E; ++i) {
-        double2 a = acc[i];
-#pragma unroll
-        for (int off = W / 2; off > 0; off >>= 1) {
-            a.x += __shfl_xor(a.x, off, 64);
-            a.y += __shfl_xor(a.y, off, 64);
-        }
-        if (c != 0) continue;
-        if constexpr (UNI) {
-            const unsigned x = bin_index(P.X, L, ln::out_idx<L, S>(t, i / R, i % R));
-            if (x < (unsigned)P.X.n) {
-                const double w = P.outw[x];
-                out[x] = make_double2(a.x * w, a.y * w);
+        for (int i = 0; i < E; ++i) {
+            const unsigned x = index(te, i), xl = min(x, nmax);
+            double2 a = acc[i];
+            if (C.sens) {
+                const float2 s =
+                    (C.sens + (size_t)line * P.X.n)[(cc < C.nc ? cc : 0) * C.nvox + xl];
+                a = make_double2(a.x * s.x + a.y * s.y, a.y * s.x - a.x * s.y);
             }
-        } else {
-            if (t + T * i < P.X.n) out[t + T * i] = a;
+#pragma unroll
+            for (int off = W / 2; off > 0; off >>= 1) {
+                a.x += __shfl_xor(a.x, off, 64);
+                a.y += __shfl_xor(a.y, off, 64);
+            }
+            if (KIND != AX_FREE) {
+                const double w = P.outw[xl];
+                a = make_double2(a.x * w, a.y * w);
+            }
+            if (c == 0 && x <= nmax) {
+                if (cp > ncp * cs / C.ncs) {
+                    a.x += out[x].x;
+                    a.y += out[x].y;
+                }
+                out[x] = a;
+            }
         }
     }
 }
@@ -1411,14 +1519,22 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_line_c
 // divided by the kernel's transform and summed onto the k grid one axis at a
 // time; then each sample gathers its NW x NW window of every column.
 
-// i-th output of a transformed line at grid points g = i + j0 mod L
-template <bool UNI>
+// i-th output of a transformed line at grid points g = i + j0 mod L; d: the
+// first-order part of AX_NEAR axes
+template <int KIND>
 __device__ __forceinline__ void fline_out(const LineArgs &P, double2 *base, unsigned el, unsigned c,
-                                          int L, int i, double2 v) {
+                                          int L, int i, double2 v, double2 d) {
     int g = i + P.X.shift;
     if (g >= L) g -= L;
-    if constexpr (UNI) {
-        for (; g < P.X.nf; g += L) base[(unsigned)g * el + c] = v;
+    if constexpr (KIND != AX_FREE) {
+        for (; g < P.X.nf; g += L) {
+            double2 z = v;
+            if constexpr (KIND == AX_NEAR) {
+                const double2 r = times_i(d, g - (int)P.X.j0);
+                z = make_double2(v.x + r.x, v.y + r.y);
+            }
+            base[(unsigned)g * el + c] = z;
+        }
     } else if (g < P.X.nf) {
         const double w = P.inw[g];
         base[(unsigned)g * el + c] = make_double2(v.x * w, v.y * w);
@@ -1427,15 +1543,17 @@ __device__ __forceinline__ void fline_out(const LineArgs &P, double2 *base, unsi
 
 // One axis, image points -> grid.  FIRST: the points' values are formed here
 // (line = ia, points ib) from img0 = conj(rho) e^{i(...)}, the maps and vt;
-// else read from P.in as in k_line_store.  Nonuniform points are spread onto
+// else read from P.in as in k_line_store.  AX_NEAR points take a second
+// transform, of their values times their offsets.  AX_FREE points are spread onto
 // the line's L cells through LDS: cell p sums the points of its list
 // (P.base[p] .. P.base[p + 1]; ascending, so the sum's order is fixed).
-template <int L, bool UNI, bool FIRST>
-__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_fline(
+template <int L, int KIND, bool FIRST>
+__global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG),
+                             KIND == AX_NEAR ? 2 : 3) void k_fline(
     LineArgs P, const int *list, const double *listw, int ncg, const double2 *img0,
     const float2 *sens, const double *vt, unsigned nvox, double2 *out, size_t out_line,
     unsigned out_el) {
-    constexpr int E = ln::vals(L), W = ln::lines(L, CO_WG), T = ln::threads(L);
+    constexpr int E = ln::vals(L), W = ln::lines(L, ST_WG), T = ln::threads(L);
     constexpr int R0 = ln::radix(L, 0);
     __shared__ double buf[ln::words(L, W)];
     const int c = threadIdx.x % W, t = threadIdx.x / W;
@@ -1446,7 +1564,6 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_fline(
     const bool ok = q < P.nq;
     const int l = ok ? q / ncg : 0, cc = ok ? q - l * ncg : 0;
     auto point = [&](int i) {
-        if (!ok) return make_double2(0.0, 0.0);
         if constexpr (FIRST) {
             const size_t x = (size_t)line * P.X.n + i;
             double2 v = img0[x];
@@ -1457,26 +1574,35 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_fline(
             const double f = vt[(size_t)l * nvox + x];
             return (l & 1) ? make_double2(-f * v.y, f * v.x) : make_double2(f * v.x, f * v.y);
         } else {
-            return P.in[(size_t)line * P.in_line + (size_t)i * P.in_el + q];
+            return P.in[(size_t)line * P.in_line + (size_t)i * P.in_el + (ok ? q : q - c)];
         }
     };
-    double2 v[E];
-    if constexpr (UNI) {
+    double2 v[E], d[E];
+    int tp = t;
+    if constexpr (KIND != AX_FREE) {
+        auto bins = [&](bool first_order, double2 (&o)[E]) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) {
-            const unsigned x = bin_index(P.X, L, ln::in_idx<L, 0>(t, i / R0, i % R0));
-            v[i] = make_double2(0.0, 0.0);
-            if (x < (unsigned)P.X.n) {
-                const double2 z = point(x);
-                const double w = P.outw[x];
-                v[i] = make_double2(z.x * w, z.y * w);
+            for (int i = 0; i < E; ++i) {
+                const unsigned x = bin_index(P.X, L, ln::in_idx<L, 0>(tp, i / R0, i % R0));
+                const unsigned xl = min(x, (unsigned)P.X.n - 1);
+                const double2 z = point(xl);
+                double w = P.outw[xl];
+                if (first_order) w *= P.outw[P.X.n + xl];
+                o[i] = ok && x < (unsigned)P.X.n ? make_double2(z.x * w, z.y * w)
+                                                 : make_double2(0.0, 0.0);
             }
+        };
+        if constexpr (KIND == AX_NEAR) {
+            bins(true, d);
+            ln::transform<L, W>(d, tp, c, buf, P.tw);
+            asm volatile("" : "+v"(tp));   // indices anew: registers
         }
+        bins(false, v);
     } else {
         double2 z[E];
 #pragma unroll
         for (int m = 0; m < E; ++m)
-            z[m] = t + T * m < P.X.n ? point(t + T * m) : make_double2(0.0, 0.0);
+            z[m] = point(min(t + T * m, P.X.n - 1));
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             __syncthreads();
@@ -1495,16 +1621,17 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, CO_WG)) void k_fline(
             }
         }
     }
-    ln::transform<L, W>(v, t, c, buf, P.tw);
+    ln::transform<L, W>(v, tp, c, buf, P.tw);
     if (!ok) return;
     constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
     double2 *o = out + (size_t)line * out_line + (q - c);
 #pragma unroll
     for (int i = 0; i < E; ++i)
-        fline_out<UNI>(P, o, out_el, c, L, ln::out_idx<L, S>(t, i / R, i % R), v[i]);
+        fline_out<KIND>(P, o, out_el, c, L, ln::out_idx<L, S>(tp, i / R, i % R), v[i],
+                        KIND == AX_NEAR ? d[i] : v[i]);
 }
 
-// Lists of k_fline's nonuniform axes: cell p of L takes the points within
+// Lists of k_fline's AX_FREE axes: cell p of L takes the points within
 // NW/2 cells of it (their positions wrap), weight kb / kb_hat.  One workgroup
 // per axis counts, scans and fills; each cell visits the points in order.
 struct FListTab {
@@ -1518,7 +1645,7 @@ struct FListTab {
 __global__ __launch_bounds__(1024) void k_nu_flists(FListTab ta, FListTab tb) {
     const FListTab &P = blockIdx.x ? tb : ta;
     const NuAxis &X = P.X;
-    if (X.uniform) return;
+    if (X.kind != AX_FREE) return;
     __shared__ double pos[4096];
     __shared__ int sm[16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1817,7 +1944,8 @@ __global__ __launch_bounds__(256) void k_nu_out(int nA, int nB, int splits,
 }
 
 // --------------------------------------------------------------- dispatching
-constexpr int NU_LENGTHS[] = {96, 128, 192, 256, 384, 512, 768, 1024, 1536, 2048, 3072, 4096};
+constexpr int NU_LENGTHS[] = {96,  128, 144,  192,  256,  288,  384,  512, 576,
+                              768, 1024, 1152, 1536, 2048, 2304, 3072, 4096};
 
 int pick_length(double want) {
     for (int L : NU_LENGTHS)
@@ -1830,14 +1958,19 @@ int line_switch(int L, F f) {
     switch (L) {
         case 96: return f(std::integral_constant<int, 96>{});
         case 128: return f(std::integral_constant<int, 128>{});
+        case 144: return f(std::integral_constant<int, 144>{});
         case 192: return f(std::integral_constant<int, 192>{});
         case 256: return f(std::integral_constant<int, 256>{});
+        case 288: return f(std::integral_constant<int, 288>{});
         case 384: return f(std::integral_constant<int, 384>{});
         case 512: return f(std::integral_constant<int, 512>{});
+        case 576: return f(std::integral_constant<int, 576>{});
         case 768: return f(std::integral_constant<int, 768>{});
         case 1024: return f(std::integral_constant<int, 1024>{});
+        case 1152: return f(std::integral_constant<int, 1152>{});
         case 1536: return f(std::integral_constant<int, 1536>{});
         case 2048: return f(std::integral_constant<int, 2048>{});
+        case 2304: return f(std::integral_constant<int, 2304>{});
         case 3072: return f(std::integral_constant<int, 3072>{});
         case 4096: return f(std::integral_constant<int, 4096>{});
         default: return fail(IMP_EINVAL, "NUDFT: line length %d", L);
@@ -1851,7 +1984,10 @@ int line_store(imp_ctx *ctx, LineArgs P, int nlines, double2 *out, size_t out_li
         constexpr int L = decltype(len)::value;
         // a multiple of 16 for the panel order
         const long wgs = ((long)nlines * ceil_div(P.nq, ln::lines(L, ST_WG)) + 15) & ~15L;
-        hipLaunchKernelGGL((P.X.uniform ? k_line_store<L, true> : k_line_store<L, false>), dim3((unsigned)wgs),
+        auto fn = P.X.kind == AX_UNIFORM ? k_line_store<L, AX_UNIFORM>
+                  : P.X.kind == AX_NEAR  ? k_line_store<L, AX_NEAR>
+                                         : k_line_store<L, AX_FREE>;
+        hipLaunchKernelGGL(fn, dim3((unsigned)wgs),
                            dim3(ln::threads(L) * ln::lines(L, ST_WG)), 0, ctx->stream, P, out, out_line,
                            out_el);
         IMP_CHECK_LAUNCH();
@@ -1859,13 +1995,24 @@ int line_store(imp_ctx *ctx, LineArgs P, int nlines, double2 *out, size_t out_li
     });
 }
 
-int line_combine(imp_ctx *ctx, const LineArgs &P, int nlines, int ncg, int splits,
-                 const double *vt, const float2 *sens, size_t nvox, double2 *partial) {
+// Splits of the combining pass over coils, then over time terms: about 16
+// workgroups per CU in all (4 waves each, 8 to 12 of them resident), at most
+// `most` partial images.
+int line_combine(imp_ctx *ctx, const LineArgs &P, int nlines, int most, CombineArgs C,
+                 int *splits) {
     return line_switch(P.X.L, [&](auto len) -> int {
-        constexpr int L = decltype(len)::value;
-        hipLaunchKernelGGL((P.X.uniform ? k_line_combine<L, true> : k_line_combine<L, false>), dim3((unsigned)(nlines * splits)),
-                           dim3(ln::threads(L) * ln::lines(L, CO_WG)), 0, ctx->stream, P, ncg, splits,
-                           vt, sens, nvox, partial);
+        constexpr int L = decltype(len)::value, W = ln::lines(L, ST_WG);
+        C.lcw = std::min(ln::bits(W), C.nc > 1 ? 32 - __builtin_clz(C.nc - 1) : 0);
+        const int want = std::max(1, std::min(most, 16 * ctx->num_cus / nlines));
+        const int ncp = ceil_div(C.nc, 1 << C.lcw), nst = ceil_div(C.nt, W >> C.lcw);
+        C.ncs = ceil_div(ncp, ceil_div(ncp, want));
+        C.nls = std::min(nst, std::max(1, want / C.ncs));
+        *splits = C.ncs * C.nls;
+        auto fn = P.X.kind == AX_UNIFORM ? k_line_combine<L, AX_UNIFORM>
+                  : P.X.kind == AX_NEAR  ? k_line_combine<L, AX_NEAR>
+                                         : k_line_combine<L, AX_FREE>;
+        hipLaunchKernelGGL(fn, dim3((unsigned)(nlines * *splits)), dim3(ln::threads(L) * W), 0,
+                           ctx->stream, P, C);
         IMP_CHECK_LAUNCH();
         return IMP_OK;
     });
@@ -1880,9 +2027,11 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
     X->kc = 0.5 * ((double)klo + khi);
     const double Kh = 0.5 * ((double)khi - klo);
     const double d = ((double)c1 - c0) / (n - 1);
-    // a coordinate off by dev turns the phase by at most 2 pi Kh dev
-    X->uniform = d != 0.0 && Kh * dev < 1e-10;
-    if (X->uniform) {
+    // A coordinate off by dev turns the phase by at most 2 pi Kh dev: nothing
+    // below 1e-10 turns, and to first order (2e-9 off) up to 1e-5, which takes
+    // in coordinates rounded to FP32 up to about 1000 points.
+    X->kind = d == 0.0 || !(Kh * dev < 1e-5) ? AX_FREE : Kh * dev < 1e-10 ? AX_UNIFORM : AX_NEAR;
+    if (X->kind != AX_FREE) {
         X->L = pick_length(2.0 * NU_SIGMA * (n / 2));   // bins up to n / 2
         if (!X->L) return false;
         X->xc = c0 + (n / 2) * d;
@@ -1899,7 +2048,7 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
     if (!(cells < 4096.0)) return false;
     X->j0 = std::ceil(cells + 0.5 * NW) + 1;
     X->nf = 2 * (int)X->j0 + 1;
-    if (!X->uniform) {
+    if (X->kind == AX_FREE) {
         // at least n: every thread interpolates at most vals(L) outputs
         X->L = pick_length(std::max<double>(NU_SIGMA * X->nf, n));
         if (!X->L) return false;
@@ -2113,7 +2262,7 @@ struct NuPass {
             const NuAxis &X = a ? G.B : G.A;
             o_tw[a] = W.take((size_t)X.L * sizeof(double2));
             o_in[a] = W.take((size_t)X.nf * 8);
-            o_ow[a] = W.take((size_t)X.n * (X.uniform ? 1 : NW) * 8);
+            o_ow[a] = W.take((size_t)X.n * (X.kind == AX_FREE ? NW : 2) * 8);
             o_ob[a] = W.take((size_t)X.n * 4);
         }
     }
@@ -2360,14 +2509,15 @@ int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
                            d_i, N.at<double2 *>(N.o_wd));
         IMP_TRY(N.to_mid(nc));
         const LineArgs LB = N.lines_b(nc);
-        const int panels = line_switch(G.B.L, [&](auto len) -> int {
-            return ceil_div(LB.nq, ln::lines(decltype(len)::value, CO_WG));
-        });
-        const int splits =
-            std::max(1, std::min(std::min(splits_max, panels), 12 * ctx->num_cus / nA));
-        IMP_TRY(line_combine(ctx, LB, nA, nc, splits, N.at<const double *>(o_vt),
-                             s_r ? N.at<const float2 *>(o_sens) + (size_t)c0 * nvox : nullptr,
-                             nvox, N.at<double2 *>(o_img) + (size_t)parts * nvox));
+        CombineArgs C{};
+        C.nc = nc;
+        C.nt = N.nt;
+        C.vt = N.at<const double *>(o_vt);
+        C.sens = s_r ? N.at<const float2 *>(o_sens) + (size_t)c0 * nvox : nullptr;
+        C.nvox = (unsigned)nvox;
+        C.partial = N.at<double2 *>(o_img) + (size_t)parts * nvox;
+        int splits = 0;
+        IMP_TRY(line_combine(ctx, LB, nA, splits_max, C, &splits));
         parts += splits;
     }
     hipLaunchKernelGGL(k_nu_out, dim3(ceil_div(nA, 16), ceil_div(nB, 16)), b256, 0, st, nA, nB,
@@ -2522,10 +2672,13 @@ int line_forward(imp_ctx *ctx, LineArgs P, int nlines, bool first, const int *li
     P.nlines = nlines;
     return line_switch(P.X.L, [&](auto len) -> int {
         constexpr int L = decltype(len)::value;
-        const long wgs = ((long)nlines * ceil_div(P.nq, ln::lines(L, CO_WG)) + 15) & ~15L;
-        auto fn = P.X.uniform ? (first ? k_fline<L, true, true> : k_fline<L, true, false>)
-                              : (first ? k_fline<L, false, true> : k_fline<L, false, false>);
-        hipLaunchKernelGGL(fn, dim3((unsigned)wgs), dim3(ln::threads(L) * ln::lines(L, CO_WG)), 0,
+        const long wgs = ((long)nlines * ceil_div(P.nq, ln::lines(L, ST_WG)) + 15) & ~15L;
+        auto fn = P.X.kind == AX_UNIFORM
+                      ? (first ? k_fline<L, AX_UNIFORM, true> : k_fline<L, AX_UNIFORM, false>)
+                  : P.X.kind == AX_NEAR
+                      ? (first ? k_fline<L, AX_NEAR, true> : k_fline<L, AX_NEAR, false>)
+                      : (first ? k_fline<L, AX_FREE, true> : k_fline<L, AX_FREE, false>);
+        hipLaunchKernelGGL(fn, dim3((unsigned)wgs), dim3(ln::threads(L) * ln::lines(L, ST_WG)), 0,
                            ctx->stream, P, list, listw, ncg, img0, sens, vt, nvox, out, out_line,
                            out_el);
         IMP_CHECK_LAUNCH();
@@ -2592,7 +2745,7 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
                        N.coef(), N.coef() + N.tab_poly, N.nt, N.nleg, N.at<int *>(o_bx),
                        N.at<int *>(o_by), N.at<double *>(o_wx), N.at<double *>(o_wy),
                        N.at<double *>(o_u), N.at<double2 *>(o_rot));
-    if (!A.uniform || !B.uniform) {
+    if (A.kind == AX_FREE || B.kind == AX_FREE) {
         FListTab ft[2];
         for (int a = 0; a < 2; ++a)
             ft[a] = FListTab{a ? B : A, a ? cB : cA, a ? nA : 1, N.at<int *>(o_f[a]),

@@ -50,7 +50,11 @@ constexpr double NU_SIGMA = 1.5; // oversampling of both grids
 // KB shape pi NW (1 - 1/(2 sigma)), 1% lower: the smallest error over the band
 // by a scan of the factor
 constexpr double NU_BETA = 0.99 * M_PI * NW * (1.0 - 1.0 / (2.0 * NU_SIGMA));
-constexpr double NU_TIME_TOL = 1e-8;   // largest error of the time expansion
+// Largest error of the time expansion, at the corner |t|, |w| = their largest:
+// about 27 times the error's rms (the first functions left out reach sqrt(l +
+// 1/2) at the ends), so 5e-8 is 2e-9 rms, a twelfth of the FP32 store's
+// rounding.  1e-8 took one term more of about 12.
+constexpr double NU_TIME_TOL = 5e-8;
 constexpr int NU_MAX_TERMS = 48;       // time terms above which the direct kernel runs
                                        // (16 per lane, 3 groups of a 4-group wave)
 constexpr double NU_MAX_THETA = 40.0;  // half widths of t and w multiplied: 44 terms
@@ -369,8 +373,8 @@ __device__ __forceinline__ double kb(double z) {
 // kb on one cell of a window as a polynomial: a point NW/2 - 1 + g behind the
 // window's last whole cell, g in [0, 1], is NW/2 - 1 + g - c from cell c, and
 // kb there is a polynomial in x = 2 g - 1 (degree KB_DEG, fitted on the host
-// at Chebyshev nodes to 1e-14 of kb(0)).  An eighth of the work of I0.
-constexpr int KB_DEG = 12;
+// at Chebyshev nodes).  A tenth of the work of I0.
+constexpr int KB_DEG = 9;   // off by 7e-11 of the peak (10: 2e-12, 8: 8e-10)
 constexpr int KB_WORDS = NW * (KB_DEG + 1);
 __device__ __forceinline__ double kb_cell(const double *poly, int cell, double x) {
     const double *c = poly + cell * (KB_DEG + 1);

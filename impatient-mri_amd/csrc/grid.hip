@@ -21,7 +21,9 @@
 //     samples stay in index order), so each grid point gathers from
 //     contiguous sample ranges with no atomics on the grid;
 //   - one gather launch grids every coil of a segment at once (each sample's
-//     kernel weight serves all coils);
+//     kernel weight serves all coils); 2D grids of many coils in tiles of
+//     points whose lanes are coils, with the coils innermost up to the sum over
+//     them;
 //   - the DFT of step 2 runs per axis on lines of length G = R P (P the
 //     largest power of two dividing G): R radix-2 FFTs of length P in LDS,
 //     then the R-term combination evaluated only at the n kept outputs, with
@@ -32,6 +34,7 @@
 #include <vector>
 
 #include "common.h"
+#include "fftcore.h"
 #include "toeplitz.h"
 
 namespace imp {
@@ -263,6 +266,22 @@ __global__ void k_grid_data(int m, int ncoils, const int *perm, const float *d_r
                                              : make_float2(0.f, 0.f);
 }
 
+// coil data [m][C] in the samples' own order, 64 samples through LDS (393216
+// samples x 32 coils: 41 us; k_grid_data, in sorted order, 275)
+template <int C>
+__global__ __launch_bounds__(GT) void k_grid_rows(int m, int ncoils, const float *d_r,
+                                                  const float *d_i, float2 *out) {
+    __shared__ float2 tile[C][65];
+    const int j0 = blockIdx.x * 64, j = threadIdx.x & 63, q = threadIdx.x >> 6;
+    for (int c = q; c < C; c += GT / 64)
+        tile[c][j] = c < ncoils && j0 + j < m
+                         ? make_float2(d_r[(size_t)c * m + j0 + j], d_i[(size_t)c * m + j0 + j])
+                         : make_float2(0.f, 0.f);
+    __syncthreads();
+    for (int e = threadIdx.x; e < 64 * C && j0 + e / C < m; e += GT)
+        out[(size_t)j0 * C + e] = tile[e % C][e / C];
+}
+
 // The window of grid point id ([gy][gx][gz], the innermost cell axis
 // fastest): the cells whose samples can lie within W/2 of it.
 struct Window {
@@ -427,6 +446,411 @@ __global__ __launch_bounds__(GT) void k_grid_gather_heavy(GridGeom g, const int 
     }
 }
 
+// Tiles of 2D grid points, C coils side by side, grid[gy][gx][coil].  Lanes are
+// coils x sub-tiles of 4 x 4 points, whose sums stay in registers.  The samples
+// of the cells around the tile (few contiguous ranges) go in batches of 64: lane
+// v computes the kernel weights of sample v at the tile's columns and rows, all
+// lanes then run over the samples with the next TL_PF samples' data on their
+// way.  A tile of more than TL_HEAVY samples is listed (by the first launch, of
+// one wave per tile) and summed by TL_WAVES waves, added in a fixed order; one of
+// more than TL_PART (the centre of a variable-density trajectory) by several
+// such workgroups, whose sums k_grid_tiles_sum adds.
+//
+// One thread per point, as below, evaluates a weight for each pair of point and
+// sample and waits on the sample's 32 coils each time.  512^2 x 32 coils, grid
+// 704^2, 11 segments of 393216 samples: gathers 4.31 ms -> 1.27 ms.  TL_WAVES 4, 8,
+// 16: 2.99, 1.67, 1.33 ms for the listed tiles (before they were parted);
+// TL_HEAVY 128, 256, 512, 1024: 0.64, 0.87, 1.15, 1.54 ms for the others.
+constexpr int TL_PF = 4, TL_HEAVY = 256, TL_WAVES = 16, TL_PART = 2048;
+struct TileList {
+    int4 *entries;    // tile, part, parts, slot
+    int4 *multis;     // tile, parts, first slot
+    int *count;       // entries, slots, multis
+    float2 *slots;    // [slot][16][64]
+};
+template <int C>
+struct Tile {
+    static constexpr int SUB = 64 / C, SX = SUB >= 8 ? 4 : 2, SY = SUB / SX;
+    static constexpr int TX = 4 * SX, TY = 4 * SY;
+};
+
+template <int C>
+__device__ __forceinline__ void tile_store(const GridGeom &g, int gx0, int gy0, int lane,
+                                           const float2 (&v)[4][4], float2 *grid) {
+    const int c = lane & (C - 1), sub = lane / C;
+    gx0 += (sub % Tile<C>::SX) * 4;
+    gy0 += (sub / Tile<C>::SX) * 4;
+#pragma unroll
+    for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+            if (gy0 + y < g.G[1] && gx0 + x < g.G[0])
+                grid[((size_t)(gy0 + y) * g.G[0] + gx0 + x) * C + c] = v[y][x];
+}
+
+template <int C, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_grid_tiles(GridGeom g, const int *start,
+                                                           int nbuck, const float4 *pos,
+                                                           const float2 *w, const int *perm,
+                                                           const float2 *data, int l,
+                                                           float2 *grid, int ntx,
+                                                           TileList H) {
+    using TS = Tile<C>;
+    constexpr int TX = TS::TX, TY = TS::TY;
+    constexpr int FACT = WAVES * 64 * (TX + TY), RED = WAVES > 1 ? WAVES / 2 * 16 * 64 * 2 : 0;
+    __shared__ float4 smem[(FACT > RED ? FACT : RED) / 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    float *wx = (float *)smem + wave * 64 * (TX + TY), *wy = wx + 64 * TX;
+    const int c = lane & (C - 1), sub = lane / C, px = (sub % TS::SX) * 4, py = (sub / TS::SX) * 4;
+    const int r_lo = (int)ceilf(g.half), r_hi = (int)floorf(g.half);
+    const int nrow = TY + r_lo + r_hi, nb = min(l + 1, nbuck - 1) - l + 1;
+    const int count = WAVES > 1 ? H.count[0] : (int)gridDim.x;
+    for (int it = blockIdx.x; it < count; it += gridDim.x) {
+        const int4 E = WAVES > 1 ? H.entries[it] : make_int4(it, 0, 1, 0);
+        const int tile = E.x;
+        const int gx0 = (tile % ntx) * TX, gy0 = (tile / ntx) * TY;
+        // lane r: sample range of cell row r of a time bucket (2 nrow <= 64)
+        int rs = 0, rn = 0;
+        const int cy = gy0 - r_lo + lane % nrow;
+        if (lane < nb * nrow && cy >= 0 && cy < g.G[1]) {
+            const long row = ((long)(l + lane / nrow) * g.G[1] + cy) * g.G[0];
+            rs = start[row + max(0, gx0 - r_lo)];
+            rn = start[row + min(g.G[0] - 1, gx0 + TX - 1 + r_hi) + 1] - rs;
+        }
+        int total = rn;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
+        if (WAVES == 1 && total > TL_HEAVY) {
+            if (lane == 0) {
+                const int parts = (total + TL_PART - 1) / TL_PART;
+                const int e0 = atomicAdd(&H.count[0], parts);
+                const int s0 = parts > 1 ? atomicAdd(&H.count[1], parts) : 0;
+                for (int k = 0; k < parts; ++k) H.entries[e0 + k] = make_int4(tile, k, parts, s0 + k);
+                if (parts > 1) H.multis[atomicAdd(&H.count[2], 1)] = make_int4(tile, parts, s0, 0);
+            }
+            return;
+        }
+        // each batch is summed by itself: no chain of FP32 sums is longer than 64
+        float2 tot[4][4];
+#pragma unroll
+        for (int y = 0; y < 4; ++y)
+#pragma unroll
+            for (int x = 0; x < 4; ++x) tot[y][x] = make_float2(0.f, 0.f);
+        for (int vb = (E.y * WAVES + wave) * 64; vb < total; vb += 64 * WAVES * E.z) {
+            const int n = min(64, total - vb);
+            int smp = 0, base = 0;
+            for (int r = 0; r < nb * nrow; ++r) {
+                const int k = __builtin_amdgcn_readlane(rn, r), o = vb + lane - base;
+                if (o >= 0 && o < k) smp = __builtin_amdgcn_readlane(rs, r) + o;
+                base += k;
+            }
+            // this lane's sample; lanes past the batch hold weights of zero
+            float a = 0.f;
+            int row = 0;
+            if (lane < n) {
+                row = perm[smp];
+                const float4 p = pos[smp];
+                const float2 ww = w[smp];
+                const int l0 = __float_as_int(p.w);
+                a = l == l0 ? ww.x : (l == l0 + 1 ? ww.y : 0.f);
+#pragma unroll
+                for (int q = 0; q < TX; ++q)
+                    wx[lane * TX + q] = kb_weight(p.x, gx0 + q, g.inv_os, g.beta);
+#pragma unroll
+                for (int q = 0; q < TY; ++q)
+                    wy[lane * TY + q] = a * kb_weight(p.y, gy0 + q, g.inv_os, g.beta);
+            } else {
+                for (int q = 0; q < TX; ++q) wx[lane * TX + q] = 0.f;
+                for (int q = 0; q < TY; ++q) wy[lane * TY + q] = 0.f;
+            }
+            // the wave reads its own LDS words only
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            auto load = [&](int i) {
+                return data[(size_t)__builtin_amdgcn_readlane(row, min(i, n - 1)) * C + c];
+            };
+            float2 acc[4][4];
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) acc[y][x] = make_float2(0.f, 0.f);
+            float2 d[TL_PF];
+#pragma unroll
+            for (int h = 0; h < TL_PF; ++h) d[h] = load(h);
+            for (int i0 = 0; i0 < n; i0 += TL_PF) {
+#pragma unroll
+                for (int h = 0; h < TL_PF; ++h) {
+                    const int i = i0 + h;
+                    // samples of weight zero in time are left out (not finite)
+                    const float at = __int_as_float(
+                        __builtin_amdgcn_readlane(__float_as_int(a), min(i, 63)));
+                    float2 v = at != 0.f ? d[h] : make_float2(0.f, 0.f);
+                    d[h] = load(i + TL_PF);
+                    const float4 x4 = *(const float4 *)&wx[i * TX + px];
+                    const float4 y4 = *(const float4 *)&wy[i * TY + py];
+                    const float xs[4] = {x4.x, x4.y, x4.z, x4.w};
+                    const float ys[4] = {y4.x, y4.y, y4.z, y4.w};
+#pragma unroll
+                    for (int y = 0; y < 4; ++y) {
+                        const float vr = v.x * ys[y], vi = v.y * ys[y];
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) {
+                            acc[y][x].x = fmaf(vr, xs[x], acc[y][x].x);
+                            acc[y][x].y = fmaf(vi, xs[x], acc[y][x].y);
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    tot[y][x].x += acc[y][x].x;
+                    tot[y][x].y += acc[y][x].y;
+                }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        if constexpr (WAVES > 1) {
+            float2 *red = (float2 *)smem;
+            for (int h = WAVES / 2; h > 0; h >>= 1) {
+                __syncthreads();
+                if (wave >= h && wave < 2 * h)
+#pragma unroll
+                    for (int k = 0; k < 16; ++k)
+                        red[((wave - h) * 16 + k) * 64 + lane] = tot[k / 4][k % 4];
+                __syncthreads();
+                if (wave < h)
+#pragma unroll
+                    for (int k = 0; k < 16; ++k) {
+                        const float2 v = red[(wave * 16 + k) * 64 + lane];
+                        tot[k / 4][k % 4].x += v.x;
+                        tot[k / 4][k % 4].y += v.y;
+                    }
+            }
+            __syncthreads();
+        }
+        if (wave) continue;
+        if (WAVES > 1 && E.z > 1) {
+#pragma unroll
+            for (int k = 0; k < 16; ++k) H.slots[((size_t)E.w * 16 + k) * 64 + lane] = tot[k / 4][k % 4];
+            continue;
+        }
+        tile_store<C>(g, gx0, gy0, lane, tot, grid);
+    }
+}
+
+// one wave per parted tile: the parts in order
+template <int C>
+__global__ __launch_bounds__(64) void k_grid_tiles_sum(GridGeom g, float2 *grid, int ntx,
+                                                       TileList H) {
+    const int lane = threadIdx.x, n = H.count[2];
+    for (int it = blockIdx.x; it < n; it += gridDim.x) {
+        const int4 M = H.multis[it];
+        float2 tot[4][4];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) tot[k / 4][k % 4] = make_float2(0.f, 0.f);
+        for (int p = 0; p < M.y; ++p)
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const float2 v = H.slots[((size_t)(M.z + p) * 16 + k) * 64 + lane];
+                tot[k / 4][k % 4].x += v.x;
+                tot[k / 4][k % 4].y += v.y;
+            }
+        tile_store<C>(g, (M.x % ntx) * Tile<C>::TX, (M.x / ntx) * Tile<C>::TY, lane, tot, grid);
+    }
+}
+
+// ---- steps 2 and 3 on grids with the coils innermost
+// Lines of G = R 2^LOGP points, R odd: a radix-R stage, then radix 8 with a last
+// 4 or 2 (Stockham: input j + r G/RAD, output (j - k) RAD + k + r NS with k = j
+// mod NS).  The first stage reads global memory, the last writes it, those
+// between exchange through LDS [element][coil].  Bound by memory: 704 x 704 x 32
+// coils, 41 us per axis (5.3 TB/s); k_line_dft, which reads and writes its LDS
+// once per radix-2 stage, 147.
+template <int R>
+struct OddTab {   // cos and sin of 2 pi m / R
+    float c[R] = {}, s[R] = {};
+    constexpr OddTab() {
+        for (int m = 0; m < R; ++m) {
+            const double x = 2.0 * 3.14159265358979323846 * m / R;
+            double tc = 1.0, ts = x, sc = 0.0, ss = 0.0;
+            for (int i = 1; i < 40; ++i) {   // the Taylor series
+                sc += tc;
+                ss += ts;
+                tc *= -x * x / ((2 * i - 1) * (2 * i));
+                ts *= -x * x / ((2 * i) * (2 * i + 1));
+            }
+            c[m] = (float)sc;
+            s[m] = (float)ss;
+        }
+    }
+};
+
+// v[k] <- sum_n v[n] e^{+2 pi i n k / R}, R odd, from the sums and differences
+// of v[m] and v[R - m]
+template <int R>
+__device__ __forceinline__ void dft_odd(float2 *v) {
+    constexpr OddTab<R> tab;
+    constexpr int H = (R - 1) / 2;
+    float2 p[H], d[H];
+#pragma unroll
+    for (int m = 0; m < H; ++m) {
+        const float2 a = v[m + 1], b = v[R - 1 - m];
+        p[m] = make_float2(a.x + b.x, a.y + b.y);
+        d[m] = make_float2(a.x - b.x, a.y - b.y);
+    }
+    const float2 v0 = v[0];
+#pragma unroll
+    for (int m = 0; m < H; ++m) {
+        v[0].x += p[m].x;
+        v[0].y += p[m].y;
+    }
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+        float2 e = v0, o = make_float2(0.f, 0.f);
+#pragma unroll
+        for (int m = 0; m < H; ++m) {
+            const int i = (m + 1) * k % R;
+            e.x = fmaf(tab.c[i], p[m].x, e.x);
+            e.y = fmaf(tab.c[i], p[m].y, e.y);
+            o.x = fmaf(tab.s[i], d[m].x, o.x);
+            o.y = fmaf(tab.s[i], d[m].y, o.y);
+        }
+        v[k] = make_float2(e.x - o.y, e.y + o.x);
+        v[R - k] = make_float2(e.x + o.y, e.y - o.x);
+    }
+}
+
+template <int R, int LOGP>
+struct GridLine {
+    static constexpr int G = R << LOGP, T = G / 8;
+    static constexpr int cols() {   // coils of a workgroup
+        int n = 32;
+        while (n > 1 && (n * T > 1024 || (long)n * G * 8 > 65536)) n /= 2;
+        return n;
+    }
+    static constexpr int C = cols();
+};
+
+template <int G, int T, int RAD, int NS, class LD, class MID, class ST>
+__device__ __forceinline__ void grid_stage(int t, const float2 *tw, LD ld, MID mid, ST st) {
+    constexpr int NB = G / RAD, IT = (NB + T - 1) / T;
+    float2 v[IT][RAD];
+#pragma unroll
+    for (int b = 0; b < IT; ++b) {
+        const int j = t + T * b;
+        if (NB % T && j >= NB) break;
+#pragma unroll
+        for (int r = 0; r < RAD; ++r) v[b][r] = ld(j + r * NB);
+        if constexpr (NS > 1) {
+            const int step = G / (NS * RAD) * (j % NS);
+#pragma unroll
+            for (int r = 1; r < RAD; ++r) v[b][r] = fftc::cmul(v[b][r], tw[r * step]);
+        }
+        if constexpr (RAD == 2 || RAD == 4 || RAD == 8) fftc::dft<RAD, true>(v[b]);
+        else dft_odd<RAD>(v[b]);
+    }
+    mid();
+#pragma unroll
+    for (int b = 0; b < IT; ++b) {
+        const int j = t + T * b, k = NS > 1 ? j % NS : 0;
+        if (NB % T && j >= NB) break;
+#pragma unroll
+        for (int r = 0; r < RAD; ++r) st((j - k) * RAD + k + r * NS, v[b][r]);
+    }
+}
+
+// the power-of-two stages, NS points done
+template <int G, int T, int NS, class LLD, class LST, class GST>
+__device__ __forceinline__ void grid_stages(int t, const float2 *tw, LLD lld, LST lst, GST gst) {
+    constexpr int LEFT = G / NS, RAD = LEFT >= 8 ? 8 : LEFT;
+    if constexpr (RAD == LEFT) {
+        grid_stage<G, T, RAD, NS>(t, tw, lld, [] {}, gst);
+    } else {
+        grid_stage<G, T, RAD, NS>(t, tw, lld, [] { __syncthreads(); }, lst);
+        __syncthreads();
+        grid_stages<G, T, NS * RAD>(t, tw, lld, lst, gst);
+    }
+}
+
+// Element j of line b, coil c at in[(b G + j) cs + c]; kept output i at
+// out[i out_el + b cs + c].
+template <int R, int LOGP>
+__global__ __launch_bounds__((GridLine<R, LOGP>::T * GridLine<R, LOGP>::C)) void k_grid_lines(
+    const float2 *__restrict__ in, float2 *__restrict__ out, int nlines, int nc, int cs,
+    size_t out_el, int n, const float2 *__restrict__ tw, const float *__restrict__ dp) {
+    using GL = GridLine<R, LOGP>;
+    constexpr int G = GL::G, T = GL::T, P = GL::C;
+    __shared__ float2 buf[G * P];
+    __shared__ float2 twl[G];
+    __shared__ float dpl[G];
+    for (int i = threadIdx.x; i < G; i += T * P) {
+        twl[i] = tw[i];
+        dpl[i] = i < n ? dp[i] : 0.f;
+    }
+    const int q = threadIdx.x % P, t = threadIdx.x / P;
+    const int np = (nc + P - 1) / P;
+    // workgroups go round the 8 XCDs: b and b + 8 (one XCD) take adjacent coils
+    const int blk = (blockIdx.x & ~15) | ((blockIdx.x & 7) << 1) | ((blockIdx.x >> 3) & 1);
+    const int line = blk / np, c = (blk % np) * P + q;
+    if (line >= nlines) return;
+    const bool ok = c < nc;
+    const float2 *col = in + (size_t)line * G * cs + (ok ? c : 0);
+    float2 *o = out + (size_t)line * cs + c;
+    auto gld = [&](int i) {
+        const float2 v = col[(unsigned)i * cs];
+        return ok ? v : make_float2(0.f, 0.f);
+    };
+    auto gst = [&](int i, float2 v) {
+        const int x = (i < G / 2 ? i : i - G) + n / 2;
+        if (ok && (unsigned)x < (unsigned)n) {
+            const float f = dpl[x];
+            o[x * out_el] = make_float2(v.x * f, v.y * f);
+        }
+    };
+    auto lld = [&](int i) { return buf[i * P + q]; };
+    auto lst = [&](int i, float2 v) { buf[i * P + q] = v; };
+    constexpr int R0 = R > 1 ? R : 8;
+    grid_stage<G, T, R0, 1>(t, tw, gld, [] {}, lst);
+    __syncthreads();
+    grid_stages<G, T, R0>(t, twl, lld, lst, gst);
+}
+
+// f(R, LOGP) for the line lengths of k_grid_lines; false: another length
+template <class F>
+bool grid_line_switch(int G, F f) {
+    auto pow2 = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        switch (G / R) {
+            case 8:
+                if constexpr (R > 1) f(r, std::integral_constant<int, 3>{});
+                return R > 1;
+            case 16: f(r, std::integral_constant<int, 4>{}); return true;
+            case 32: f(r, std::integral_constant<int, 5>{}); return true;
+            case 64: f(r, std::integral_constant<int, 6>{}); return true;
+            case 128: f(r, std::integral_constant<int, 7>{}); return true;
+            case 256: f(r, std::integral_constant<int, 8>{}); return true;
+            default: return false;
+        }
+    };
+    if (G % 8 || G > 4096) return false;
+    int r = G;
+    while (r % 2 == 0) r /= 2;
+    switch (r) {
+        case 3: return pow2(std::integral_constant<int, 3>{});
+        case 5: return pow2(std::integral_constant<int, 5>{});
+        case 7: return pow2(std::integral_constant<int, 7>{});
+        case 9: return pow2(std::integral_constant<int, 9>{});
+        case 11: return pow2(std::integral_constant<int, 11>{});
+        case 1:
+            if (G == 512) return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 9>{}), true;
+            if (G == 1024) return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 10>{}), true;
+            return pow2(std::integral_constant<int, 1>{});
+        default: return false;
+    }
+}
+
 // Cropped, shifted inverse DFT along the contiguous axis of every line:
 //   out[b][i][a] = dp[i] sum_{g<G} in[b][a][g] e^{+i 2pi g (i - n/2) / G}
 // (dp carries (-1)^(i - n/2) of the shift and 1 / (os C(u_i))), for lines
@@ -563,6 +987,50 @@ __global__ void k_grid_fhd_accum(long nv, int ncoils, const float2 *y, size_t pl
         vi += sr * v.y - si * v.x;
     }
     // the reference's expfm: cos / sin of the float product fm (tau l + t0)
+    const float arg = fm ? fm[i] * tl : 0.f;
+    double sn, cs;
+    sincos((double)arg, &sn, &cs);
+    double2 a = acc[i];
+    a.x += cs * vr - sn * vi;
+    a.y += cs * vi + sn * vr;
+    acc[i] = a;
+}
+
+// The same with the coils innermost, y[i][C]: 64 voxels through LDS, four
+// groups of coils (512^2 x 32 coils: 44 us, 3.0 TB/s; one thread per voxel
+// reading its 256 bytes: 85).
+template <int C>
+__global__ __launch_bounds__(GT) void k_grid_accum_rows(long nv, int ncoils, const float2 *y,
+                                                        const float *s_r, const float *s_i,
+                                                        const float *fm, float tl, double2 *acc) {
+    __shared__ float2 tile[64][C + 1];
+    __shared__ double2 part[4][64];
+    const long i0 = (long)blockIdx.x * 64;
+    for (int e = threadIdx.x; e < 64 * C; e += GT)
+        if (i0 + e / C < nv) tile[e / C][e % C] = y[i0 * C + e];
+    __syncthreads();
+    const int j = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const long i = i0 + j;
+    double vr = 0.0, vi = 0.0;
+    if (i < nv) {
+#pragma unroll
+        for (int k = 0; k < C / 4; ++k) {
+            const int c = q * (C / 4) + k;
+            if (c >= ncoils) break;
+            const float2 v = tile[j][c];
+            const double sr = s_r ? s_r[(size_t)c * nv + i] : 1.0;
+            const double si = s_r ? s_i[(size_t)c * nv + i] : 0.0;
+            vr += sr * v.x + si * v.y;
+            vi += sr * v.y - si * v.x;
+        }
+    }
+    part[q][j] = make_double2(vr, vi);
+    __syncthreads();
+    if (q || i >= nv) return;
+    for (int k = 1; k < 4; ++k) {
+        vr += part[k][j].x;
+        vi += part[k][j].y;
+    }
     const float arg = fm ? fm[i] * tl : 0.f;
     double sn, cs;
     sincos((double)arg, &sn, &cs);
@@ -825,6 +1293,83 @@ void launch_gather(imp_ctx *ctx, const GridGeom &g, const Binned &B, const float
                        nheavy);
 }
 
+bool grid_line_ok(int G) {
+    return grid_line_switch(G, [](auto, auto) {});
+}
+
+// f(CP) for the coil lanes of the tiled form of 2D F^H d.  Whole calls before
+// and after: 64^2 x 4 coils 1.49 -> 1.12 ms, 128^2 x 8 1.57 -> 1.03, 256^2 x 4
+// 1.80 -> 1.18, 256^2 x 16 2.27 -> 1.08, 512^2 x 32 8.60 -> 2.98.  With 2 coils
+// a tile would span more cell rows than there are lanes to hold their ranges.
+template <class F>
+bool tile_switch(int CP, F f) {
+    switch (CP) {
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 8: return f(std::integral_constant<int, 8>{});
+        case 16: return f(std::integral_constant<int, 16>{});
+        case 32: return f(std::integral_constant<int, 32>{});
+        default: return false;
+    }
+}
+
+// Most slots that the parted tiles of C coils can take: a sample lies in the
+// windows of at most `per` tiles, and a parted tile has parts <= 2 total / TL_PART.
+template <int C>
+long tile_slots(const GridGeom &g, int m) {
+    const int w = (int)std::ceil(g.half) + (int)std::floor(g.half);
+    const long per = (long)(1 + ceil_div(w, Tile<C>::TX)) * (1 + ceil_div(w, Tile<C>::TY));
+    return 2 * per * m / TL_PART + 1;
+}
+template <int C>
+long tile_count(const GridGeom &g) {
+    return (long)ceil_div(g.G[0], Tile<C>::TX) * ceil_div(g.G[1], Tile<C>::TY);
+}
+size_t tile_list_bytes(long tiles, long slots) {
+    return (size_t)(tiles + 2 * slots) * sizeof(int4) + (size_t)slots * 16 * 64 * sizeof(float2) +
+           2048;
+}
+TileList tile_list(Carve &cv, long tiles, long slots) {
+    TileList H;
+    H.entries = cv.take<int4>(tiles + slots);
+    H.multis = cv.take<int4>(slots);
+    H.count = cv.take<int>(4);
+    H.slots = cv.take<float2>((size_t)slots * 16 * 64);
+    return H;
+}
+
+// tiles of segment l: one wave each, then the listed ones
+template <int C>
+void launch_tiles(imp_ctx *ctx, const GridGeom &g, const Binned &B, const float2 *data, int l,
+                  float2 *grid, const TileList &H) {
+    const int ntx = ceil_div(g.G[0], Tile<C>::TX);
+    hipLaunchKernelGGL(k_zero_i, dim3(1), dim3(256), 0, ctx->stream, H.count, 4L);
+    hipLaunchKernelGGL((k_grid_tiles<C, 1>), dim3((unsigned)tile_count<C>(g)), dim3(64), 0,
+                       ctx->stream, g, B.start, B.nbuck, B.pos, B.w, B.perm, data, l, grid, ntx, H);
+    hipLaunchKernelGGL((k_grid_tiles<C, TL_WAVES>), dim3(2 * ctx->num_cus), dim3(64 * TL_WAVES), 0,
+                       ctx->stream, g, B.start, B.nbuck, B.pos, B.w, B.perm, data, l, grid, ntx, H);
+    hipLaunchKernelGGL(k_grid_tiles_sum<C>, dim3(ctx->num_cus), dim3(64), 0, ctx->stream, g, grid,
+                       ntx, H);
+}
+
+// coils-innermost grids in and out, along axis 0 (x) of G[1] lines, then y
+int lines_tiled(imp_ctx *ctx, const GridGeom &g, const AxisPlan ax[3], int nc, int cs, float2 *a,
+                float2 *b) {
+    for (int q = 0; q < 2; ++q) {
+        const int nlines = q ? g.n[0] : g.G[1];
+        // axis x: b[ix][gy][c]; axis y: a[iy][ix][c]
+        grid_line_switch(g.G[q], [&](auto r, auto lp) {
+            constexpr int R = decltype(r)::value, LP = decltype(lp)::value;
+            using GL = GridLine<R, LP>;
+            const unsigned wgs = ((unsigned)nlines * ceil_div(nc, GL::C) + 15) & ~15u;
+            hipLaunchKernelGGL((k_grid_lines<R, LP>), dim3(wgs), dim3(GL::T * GL::C), 0,
+                               ctx->stream, q ? b : a, q ? a : b, nlines, nc, cs,
+                               (size_t)nlines * cs, g.n[q], ax[q].tw, ax[q].dp);
+        });
+        IMP_CHECK_LAUNCH();
+    }
+    return IMP_OK;
+}
+
 template <int C>
 void launch_data(imp_ctx *ctx, int m, int ncoils, const int *perm, const float *d_r,
                  const float *d_i, float2 *out) {
@@ -906,7 +1451,18 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
                  : ncoils <= 16 ? 16 : 32;
     const int groups = ceil_div(ncoils, CP);
     const size_t gbytes = (size_t)CP * ncells * sizeof(float2);
-    size_t bytes = binned_bytes(num_k, ncells, nseg) + 2 * ((gbytes + 255) & ~(size_t)255) +
+    bool tiled = !g.d3 && grid_line_ok(g.G[0]) && grid_line_ok(g.G[1]) && nv * CP < INT32_MAX;
+    long tiles = 0, slots = 0;
+    tiled = tiled && tile_switch(CP, [&](auto cp) {
+        constexpr int C = decltype(cp)::value;
+        tiles = tile_count<C>(g);
+        slots = tile_slots<C>(g, num_k);
+        // a lane per cell row of two time buckets
+        return 2 * (Tile<C>::TY + std::ceil(g.half) + std::floor(g.half)) <= 64;
+    });
+    if (!tiled) tiles = slots = 0;
+    size_t bytes = binned_bytes(num_k, ncells, nseg) + tile_list_bytes(tiles, slots) +
+                   2 * ((gbytes + 255) & ~(size_t)255) +
                    (((size_t)ncells * 4 + 255) & ~(size_t)255) + 256 +
                    (((size_t)num_k * CP * 8 + 255) & ~(size_t)255) + nv * 16 + 8192 +
                    axis_bytes(g.G[0], n[0]) + axis_bytes(g.G[1], n[1]) + axis_bytes(g.G[2], n[2]);
@@ -919,6 +1475,7 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
     float2 *bufB = cv.take<float2>((size_t)CP * ncells);
     int *heavy = cv.take<int>(ncells);
     int *nheavy = cv.take<int>(1);
+    const TileList H = tile_list(cv, tiles, slots);
     float2 *data = cv.take<float2>((size_t)num_k * CP);
     double2 *acc = cv.take<double2>(nv);
     AxisPlan ax[3];
@@ -927,7 +1484,13 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
     for (int grp = 0; grp < groups; ++grp) {
         const int c0 = grp * CP, cn = std::min(CP, ncoils - c0);
         const float *dr = d_r + (size_t)c0 * num_k, *di = d_i + (size_t)c0 * num_k;
-        switch (CP) {
+        if (tiled) {
+            tile_switch(CP, [&](auto cp) {
+                hipLaunchKernelGGL(k_grid_rows<decltype(cp)::value>, dim3(ceil_div(num_k, 64)),
+                                   dim3(GT), 0, ctx->stream, num_k, cn, dr, di, data);
+                return true;
+            });
+        } else switch (CP) {
             case 1: launch_data<1>(ctx, num_k, cn, B.perm, dr, di, data); break;
             case 2: launch_data<2>(ctx, num_k, cn, B.perm, dr, di, data); break;
             case 4: launch_data<4>(ctx, num_k, cn, B.perm, dr, di, data); break;
@@ -938,7 +1501,12 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
         IMP_CHECK_LAUNCH();
         for (int l = 0; l < nseg; ++l) {
             const int rec = prof_begin(ctx, "k_grid_gather");
-            switch (CP) {
+            if (tiled) {
+                tile_switch(CP, [&](auto cp) {
+                    launch_tiles<decltype(cp)::value>(ctx, g, B, data, l, bufA, H);
+                    return true;
+                });
+            } else switch (CP) {
                 case 1: launch_gather<1>(ctx, g, B, data, l, bufA, ncells, heavy, nheavy); break;
                 case 2: launch_gather<2>(ctx, g, B, data, l, bufA, ncells, heavy, nheavy); break;
                 case 4: launch_gather<4>(ctx, g, B, data, l, bufA, ncells, heavy, nheavy); break;
@@ -950,14 +1518,28 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
             IMP_CHECK_LAUNCH();
             float2 *res = nullptr;
             const int rec2 = prof_begin(ctx, "k_line_dft");
-            IMP_TRY(transform_planes(ctx, g, ax, cn, bufA, bufB, &res));
+            if (tiled) {
+                IMP_TRY(lines_tiled(ctx, g, ax, cn, CP, bufA, bufB));
+                res = bufA;
+            } else {
+                IMP_TRY(transform_planes(ctx, g, ax, cn, bufA, bufB, &res));
+            }
             prof_end(ctx, rec2);
             // expfm argument fm (tau l + t0) in float (recon.cu:1281-1285)
             const float tl = tau * (float)l + tt[0];
-            hipLaunchKernelGGL(k_grid_fhd_accum, dim3(ceil_div(nv, 256)), dim3(256), 0,
-                               ctx->stream, nv, cn, res, (size_t)nv,
-                               s_r ? s_r + (size_t)c0 * nv : nullptr,
-                               s_i ? s_i + (size_t)c0 * nv : nullptr, fm, tl, acc);
+            const float *sr = s_r ? s_r + (size_t)c0 * nv : nullptr;
+            const float *si = s_i ? s_i + (size_t)c0 * nv : nullptr;
+            if (tiled) {
+                tile_switch(CP, [&](auto cp) {
+                    hipLaunchKernelGGL(k_grid_accum_rows<decltype(cp)::value>,
+                                       dim3(ceil_div(nv, 64)), dim3(GT), 0, ctx->stream, nv, cn,
+                                       res, sr, si, fm, tl, acc);
+                    return true;
+                });
+            } else {
+                hipLaunchKernelGGL(k_grid_fhd_accum, dim3(ceil_div(nv, 256)), dim3(256), 0,
+                                   ctx->stream, nv, cn, res, (size_t)nv, sr, si, fm, tl, acc);
+            }
             IMP_CHECK_LAUNCH();
         }
     }

@@ -102,3 +102,36 @@ def test_gridding_against_direct_at_config3_size(ctx):
           f"{eq_mid:.2e}); Toeplitz apply on the phantom {ea:.2e}; gridded F^H d (os 1.375) vs "
           f"direct time-segmented {ef:.2e}")
     assert eq_mid < 0.01 and ea < 0.01 and ef < 0.03
+
+
+# Both forms sum the same FP32 kernel weights and transform in FP32, in another
+# order: sums of up to about 10^3 terms (a few 1e-7) and some ten rounded
+# stages (1e-7).
+TILES_TOL = 1e-6
+
+
+@pytest.mark.parametrize("N,Nx,ncoils,os_,S", [
+    (32, 32, 8, 1.5, 256), (32, 32, 32, 1.5, 1024), (48, 48, 9, 2.0, 300), (16, 24, 17, 1.0, 128),
+    (64, 64, 33, 1.5, 200), (20, 32, 32, 1.5, 256), (128, 128, 16, 1.5, 700),
+    (64, 64, 32, 1.375, 400), (128, 64, 20, 1.25, 300), (32, 32, 8, 1.75, 256),
+    (64, 64, 12, 1.125, 256), (64, 40, 4, 1.375, 300)])
+def test_fhd_gridding_coil_tiles(ctx, N, Nx, ncoils, os_, S):
+    """Several coils in 2D (tiles of grid points with coil lanes: 4 to 32 of
+    them, full and padded; tiles summed by one wave and by many; grid edges
+    inside a tile; every odd factor of the line transforms) against the sum
+    over groups of 2 coils, which keep one thread per grid point."""
+    from impatient import ops, synth
+    p = synth.make_problem("tiles", N, 1, ncoils, 8, S, 4e-3, 60.0, 2, 3, 11, Nx=Nx)
+    rng = np.random.default_rng(62)
+    d = (rng.standard_normal((ncoils, p.nk)) + 1j * rng.standard_normal((ncoils, p.nk)))
+    d = d.astype(np.complex64)
+
+    def fhd(c0, c1):
+        return ops.fhd_gridding(ctx, p.kx, p.ky, p.kz, p.t, p.Nx, p.Ny, 1, p.fm, d[c0:c1],
+                                p.sens[c0:c1], 3, os_)
+    got = fhd(0, ncoils)
+    ref = sum(fhd(c, min(c + 2, ncoils)).astype(np.complex128) for c in range(0, ncoils, 2))
+    e = rel_l2(got, ref)
+    print(f"F^H d gridding tiles {Nx}x{N}, {ncoils} coils, os {os_}: {e:.2e}")
+    assert e < TILES_TOL
+    assert np.array_equal(got, fhd(0, ncoils))

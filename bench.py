@@ -569,8 +569,8 @@ def main():
             call("imp_toep_apply", h, ptr(dbr), ptr(dbi), ptr(dxr), ptr(dxi))
         ctx.synchronize()
         log(f"Toeplitz plan {t_plan:.3f} s, apply {t_apply:.2f} ms (timer off)")
-        # HBM roofline of the FFT passes: algorithmic bytes per launch (one
-        # segment l, all coils; complex64 = 8 B; the padded grid keeps the
+        # HBM roofline of the FFT passes: algorithmic bytes per segment (all
+        # coils; complex64 = 8 B; the padded grid keeps the
         # N1 x 2N2 rows that hold data; Qf_l of this standard-grid Q_l is
         # real, 4 B per point of the 2x grid)
         half = 2 * nv                                   # N1 x 2 N2 points
@@ -582,7 +582,7 @@ def main():
         passes = {}
         for name, nbytes in pass_bytes.items():
             tot, n = kernel_ms(name)
-            avg = tot / max(n, 1)
+            avg = tot / (3 * (prob.ntime_segs + 1))   # a launch may hold several segments
             passes[name] = {"launches": n, "avg_ms": round(avg, 4),
                             "algorithmic_bytes": nbytes,
                             "gbs": round(nbytes / (avg * 1e-3) / 1e9, 1) if avg > 0 else None}

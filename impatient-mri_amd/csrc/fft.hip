@@ -19,6 +19,7 @@
 #include "fftcore.h"
 #include "toeplitz.h"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -136,10 +137,13 @@ constexpr int col_threads() { return col_lines<L, MODE>() * fftc::threads_per_li
 // zero-padded axis of the 2x grid); HALF_OUT: only outputs i < L/2 are
 // stored (the cropped axis).  blockIdx.y selects the batch (bstride).
 // RQ (MODE 2): the spectrum is real and read from qr instead of qf.
-template <int L, int MODE, bool HALF_IN, bool HALF_OUT, bool RQ = false>
+// SEGS (MODE 2): blockIdx.z is the segment, zstride elements of data and qstride
+// of the spectrum apart (the two offsets cost 1.4% at 1024-point columns, so
+// single segments go without).
+template <int L, int MODE, bool HALF_IN, bool HALF_OUT, bool RQ = false, bool SEGS = false>
 __global__ __launch_bounds__((col_threads<L, MODE>())) void k_fft_cols(
     float2 *data, long bstride, long es, int nlines, const float2 *__restrict__ qf,
-    const float2 *__restrict__ tw, const float *__restrict__ qr) {
+    const float2 *__restrict__ tw, const float *__restrict__ qr, long zstride, long qstride) {
     constexpr int P = col_lines<L, MODE>();
     constexpr int E = fftc::vals_per_thread(L);
     __shared__ float2 buf[fftc::num_stages(L) > 1 ? fftc::line_lds(L) * P : 1];
@@ -160,6 +164,7 @@ __global__ __launch_bounds__((col_threads<L, MODE>())) void k_fft_cols(
     constexpr int T = fftc::threads_per_line(L);
     const long step = (long)T * es;
     float2 *col = data + (long)blockIdx.y * bstride + (ok ? j : 0) + (long)tl * es;
+    if constexpr (SEGS) col += (long)blockIdx.z * zstride;
     auto lld = [&](int, int, int i) { return buf[fftc::lpad(i) * P + c]; };
     auto lst = [&](int, int, int i, float2 v) { buf[fftc::lpad(i) * P + c] = v; };
     // i < L/2 exactly when m < E/2 (known per register)
@@ -179,7 +184,8 @@ __global__ __launch_bounds__((col_threads<L, MODE>())) void k_fft_cols(
         run_fft<L, true>(tl, tw, gld, [] {}, gst, lld, lst);
     } else {
         float2 regs[E];
-        const long qoff = (ok ? j : 0) + (long)tl * es;
+        long qoff = (ok ? j : 0) + (long)tl * es;
+        if constexpr (SEGS) qoff += (long)blockIdx.z * qstride;
         // Qf_l of this thread's elements, fetched before the forward
         // transform so that their latency hides under it (108 -> 93 us per
         // launch at 1024-point columns)
@@ -208,15 +214,21 @@ __global__ __launch_bounds__((col_threads<L, MODE>())) void k_fft_cols(
     }
 }
 
+// centre of segment l, rounded as t0 + tau * l
+__device__ __forceinline__ float seg_tau(float t0, float tau, int l) {
+    return __fadd_rn(t0, __fmul_rn(tau, (float)l));
+}
+
 // ---------------------------------------------------------------- pass A
+// Segments l0 + blockIdx.y, each with its own grid, seg elements apart.
 // Lines (c, o): image line o (N1*N2o lines of nlast = L/2 elements,
 // contiguous), v = S_c * e^{-i 2pi f tau_l} * p, zero-padded to L, forward
 // FFT, written to G1 line ((c*N1 + y)*A + x)*L with y = o / N2o, x = o % N2o.
 template <int L>
 __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_a(
     const float2 *__restrict__ p, const float2 *__restrict__ sens,
-    const float *__restrict__ f, float tau_l, int nimg_lines, int N1, int N2o, int A,
-    int ncoils, float2 *__restrict__ g1, const float2 *__restrict__ tw) {
+    const float *__restrict__ f, float t0, float tau, int l0, int nimg_lines, int N1, int N2o,
+    int A, int ncoils, float2 *__restrict__ g1, long seg, const float2 *__restrict__ tw) {
     constexpr int T = fftc::threads_per_line(L);
     constexpr int E = fftc::vals_per_thread(L);
     constexpr int nlast = L / 2;
@@ -233,7 +245,8 @@ __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_a(
     const float2 *pl = p + o * nlast;
     const float *fl = f + o * nlast;
     const float2 *sl = sens ? sens + (long)c * nvox + o * nlast : nullptr;
-    float2 *dst = g1 + (((long)c * N1 + y) * A + x) * L;
+    float2 *dst = g1 + blockIdx.y * seg + (((long)c * N1 + y) * A + x) * L;
+    const float tau_l = seg_tau(t0, tau, l0 + blockIdx.y);
     float2 *lb = buf + (fftc::num_stages(L) > 1 ? ln * fftc::line_lds(L) : 0);
     run_fft<L, false>(
         tl, tw,
@@ -257,11 +270,11 @@ __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_a(
 // ---------------------------------------------------------------- pass E
 // For one image line and the coils of one coil group: inverse FFT of the G1
 // lines, keep the first nlast elements, sum conj(S_c) * z_c over the group
-// in registers, write partial[group][voxel].
+// in registers, write partial[segment][group][voxel].
 template <int L>
 __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_e(
     const float2 *__restrict__ g1, const float2 *__restrict__ sens, int nimg_lines, int N1,
-    int N2o, int A, int ncoils, int coils_per_group, float2 *__restrict__ partial,
+    int N2o, int A, int ncoils, int coils_per_group, float2 *__restrict__ partial, long seg,
     const float2 *__restrict__ tw) {
     constexpr int T = fftc::threads_per_line(L);
     constexpr int E = fftc::vals_per_thread(L);
@@ -284,7 +297,7 @@ __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_e(
 #pragma unroll
     for (int m = 0; m < E / 2; ++m) acc[m] = make_float2(0.f, 0.f);
     for (int c = c0; c < c1; ++c) {
-        const float2 *src = g1 + (((long)c * N1 + y) * A + x) * L;
+        const float2 *src = g1 + blockIdx.z * seg + (((long)c * N1 + y) * A + x) * L;
         const float2 *sl = sens ? sens + (long)c * nvox + oc * nlast : nullptr;
         run_fft<L, true>(
             tl, tw, [&](int, int, int i) { return ok ? src[i] : make_float2(0.f, 0.f); },
@@ -310,31 +323,35 @@ __global__ __launch_bounds__(fftc::row_threads(L)) void k_toep_pass_e(
     if (!ok) return;
 #pragma unroll
     for (int m = 0; m < E / 2; ++m)
-        partial[(long)group * nvox + oc * nlast + tl + T * m] = acc[m];
+        partial[((long)blockIdx.z * gridDim.y + group) * nvox + oc * nlast + tl + T * m] = acc[m];
 }
 
 // ---------------------------------------------------------------- pass F
-// out (+)= scale * e^{+i 2pi f tau_l} * sum_groups partial[g]
-__global__ void k_toep_pass_f(const float2 *__restrict__ partial, int ngroups, long nvox,
-                              const float *__restrict__ f, float tau_l, float scale,
-                              int accumulate, float2 *__restrict__ out) {
+// out (+)= scale * sum over the segments l0, l0 + 1, ... of
+// e^{+i 2pi f tau_l} * sum_groups partial[segment][g]
+__global__ void k_toep_pass_f(const float2 *__restrict__ partial, int nsegs, int ngroups,
+                              long nvox, const float *__restrict__ f, float t0, float tau, int l0,
+                              float scale, float2 *__restrict__ out) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nvox) return;
-    float2 s = make_float2(0.f, 0.f);
-    for (int g = 0; g < ngroups; ++g) {
-        const float2 v = partial[(long)g * nvox + i];
-        s.x += v.x;
-        s.y += v.y;
+    float2 o = l0 > 0 ? out[i] : make_float2(0.f, 0.f);
+    for (int k = 0; k < nsegs; ++k) {
+        float2 s = make_float2(0.f, 0.f);
+        for (int g = 0; g < ngroups; ++g) {
+            const float2 v = partial[((long)k * ngroups + g) * nvox + i];
+            s.x += v.x;
+            s.y += v.y;
+        }
+        float sn, cs;
+        sincos_rev(frac_near(f[i] * seg_tau(t0, tau, l0 + k)), &sn, &cs);
+        float2 r = make_float2(scale * (s.x * cs - s.y * sn), scale * (s.x * sn + s.y * cs));
+        if (l0 + k > 0) {
+            r.x += o.x;
+            r.y += o.y;
+        }
+        o = r;
     }
-    float sn, cs;
-    sincos_rev(frac_near(f[i] * tau_l), &sn, &cs);
-    float2 r = make_float2(scale * (s.x * cs - s.y * sn), scale * (s.x * sn + s.y * cs));
-    if (accumulate) {
-        const float2 o = out[i];
-        r.x += o.x;
-        r.y += o.y;
-    }
-    out[i] = r;
+    out[i] = o;
 }
 
 // ifftshift of Q_l (split, standard grid) into interleaved Qf: out[m] = Q[(m + M/2) mod M]
@@ -470,11 +487,11 @@ int fft_grid(imp_ctx *ctx, float2 *data, int M1, int M2, int M3, bool inverse) {
             if (inverse)
                 hipLaunchKernelGGL((k_fft_cols<L_, 1, false, false>), grid,
                                    dim3(col_threads<L_, 1>()), 0, ctx->stream, data, (long)M2 * M3,
-                                   (long)M3, M3, nullptr, tw, nullptr);
+                                   (long)M3, M3, nullptr, tw, nullptr, 0L, 0L);
             else
                 hipLaunchKernelGGL((k_fft_cols<L_, 0, false, false>), grid,
                                    dim3(col_threads<L_, 0>()), 0, ctx->stream, data, (long)M2 * M3,
-                                   (long)M3, M3, nullptr, tw, nullptr);
+                                   (long)M3, M3, nullptr, tw, nullptr, 0L, 0L);
         });
         IMP_CHECK_LAUNCH();
     }
@@ -485,10 +502,12 @@ int fft_grid(imp_ctx *ctx, float2 *data, int M1, int M2, int M3, bool inverse) {
         dim3 grid(ceil_div(nlines, col_lines<L_, 0>()), 1);
         if (inverse)
             hipLaunchKernelGGL((k_fft_cols<L_, 1, false, false>), grid, dim3(col_threads<L_, 1>()),
-                               0, ctx->stream, data, 0L, (long)nlines, nlines, nullptr, tw, nullptr);
+                               0, ctx->stream, data, 0L, (long)nlines, nlines, nullptr, tw, nullptr,
+                               0L, 0L);
         else
             hipLaunchKernelGGL((k_fft_cols<L_, 0, false, false>), grid, dim3(col_threads<L_, 0>()),
-                               0, ctx->stream, data, 0L, (long)nlines, nlines, nullptr, tw, nullptr);
+                               0, ctx->stream, data, 0L, (long)nlines, nlines, nullptr, tw, nullptr,
+                               0L, 0L);
     });
     IMP_CHECK_LAUNCH();
     return IMP_OK;
@@ -546,15 +565,16 @@ int toep_apply_normal(imp_ctx *ctx, ToepPlan &P, const float2 *p, float2 *out) {
     const int C = P.ncoils;
     const int cpg = P.coils_per_group;
     const int ngroups = ceil_div(C, cpg);
-    for (int l = 0; l < P.nseg; ++l) {
-        const float tau_l = P.t0 + P.tau * (float)l;
+    const long seg = (long)C * P.N1 * A * Ml;   // elements of a segment's pass buffer
+    for (int l = 0; l < P.nseg; l += P.segs_per_pass) {
+        const int ns = std::min(P.segs_per_pass, P.nseg - l);
         // pass A
         int rec = prof_begin(ctx, "toep_pass_a");
         IMP_L_SWITCH(Ml, {
             const long nlines = (long)C * nimg_lines;
-            hipLaunchKernelGGL((k_toep_pass_a<L_>), dim3(ceil_div(nlines, row_lines<L_>())),
-                               dim3(fftc::row_threads(L_)), 0, ctx->stream, p, P.sens, P.fcyc, tau_l,
-                               nimg_lines, P.N1, N2o, A, C, P.g1, tw_last);
+            hipLaunchKernelGGL((k_toep_pass_a<L_>), dim3(ceil_div(nlines, row_lines<L_>()), ns),
+                               dim3(fftc::row_threads(L_)), 0, ctx->stream, p, P.sens, P.fcyc,
+                               P.t0, P.tau, l, nimg_lines, P.N1, N2o, A, C, P.g1, seg, tw_last);
         });
         prof_end(ctx, rec);
         IMP_CHECK_LAUNCH();
@@ -562,10 +582,10 @@ int toep_apply_normal(imp_ctx *ctx, ToepPlan &P, const float2 *p, float2 *out) {
         if (d3) {
             rec = prof_begin(ctx, "toep_pass_b");
             IMP_L_SWITCH(P.M2, {
-                dim3 grid(ceil_div(P.M3, col_lines<L_, 0>()), C * P.N1);
+                dim3 grid(ceil_div(P.M3, col_lines<L_, 0>()), C * P.N1 * ns);
                 hipLaunchKernelGGL((k_fft_cols<L_, 0, true, false>), grid, dim3(col_threads<L_, 0>()),
                                    0, ctx->stream, P.g1, (long)P.M2 * P.M3, (long)P.M3, P.M3,
-                                   nullptr, tw_x, nullptr);
+                                   nullptr, tw_x, nullptr, 0L, 0L);
             });
             prof_end(ctx, rec);
             IMP_CHECK_LAUNCH();
@@ -577,15 +597,14 @@ int toep_apply_normal(imp_ctx *ctx, ToepPlan &P, const float2 *p, float2 *out) {
             rec = prof_begin(ctx, "toep_pass_c");
             const float *qr = P.qf_real ? P.qfr + (long)l * P.G : nullptr;
             IMP_L_SWITCH(P.M1, {
-                dim3 grid(ceil_div(nl, col_lines<L_, 2>()), C);
-                if (qr)
-                    hipLaunchKernelGGL((k_fft_cols<L_, 2, true, true, true>), grid,
-                                       dim3(col_threads<L_, 2>()), 0, ctx->stream, P.g1,
-                                       (long)P.N1 * nl, (long)nl, nl, nullptr, tw_y, qr);
-                else
-                    hipLaunchKernelGGL((k_fft_cols<L_, 2, true, true>), grid,
-                                       dim3(col_threads<L_, 2>()), 0, ctx->stream, P.g1,
-                                       (long)P.N1 * nl, (long)nl, nl, qf, tw_y, nullptr);
+                dim3 grid(ceil_div(nl, col_lines<L_, 2>()), C, ns);
+                auto fn = ns > 1 ? (qr ? k_fft_cols<L_, 2, true, true, true, true>
+                                       : k_fft_cols<L_, 2, true, true, false, true>)
+                                 : (qr ? k_fft_cols<L_, 2, true, true, true>
+                                       : k_fft_cols<L_, 2, true, true>);
+                hipLaunchKernelGGL(fn, grid, dim3(col_threads<L_, 2>()), 0, ctx->stream, P.g1,
+                                   (long)P.N1 * nl, (long)nl, nl, qr ? nullptr : qf, tw_y, qr,
+                                   seg, P.G);
             });
             prof_end(ctx, rec);
             IMP_CHECK_LAUNCH();
@@ -594,10 +613,10 @@ int toep_apply_normal(imp_ctx *ctx, ToepPlan &P, const float2 *p, float2 *out) {
         if (d3) {
             rec = prof_begin(ctx, "toep_pass_d");
             IMP_L_SWITCH(P.M2, {
-                dim3 grid(ceil_div(P.M3, col_lines<L_, 1>()), C * P.N1);
+                dim3 grid(ceil_div(P.M3, col_lines<L_, 1>()), C * P.N1 * ns);
                 hipLaunchKernelGGL((k_fft_cols<L_, 1, false, true>), grid, dim3(col_threads<L_, 1>()),
                                    0, ctx->stream, P.g1, (long)P.M2 * P.M3, (long)P.M3, P.M3,
-                                   nullptr, tw_x, nullptr);
+                                   nullptr, tw_x, nullptr, 0L, 0L);
             });
             prof_end(ctx, rec);
             IMP_CHECK_LAUNCH();
@@ -605,17 +624,17 @@ int toep_apply_normal(imp_ctx *ctx, ToepPlan &P, const float2 *p, float2 *out) {
         // pass E: inverse last axis, conj(S_c), partial sums over coil groups
         rec = prof_begin(ctx, "toep_pass_e");
         IMP_L_SWITCH(Ml, {
-            dim3 grid(ceil_div(nimg_lines, row_lines<L_>()), ngroups);
+            dim3 grid(ceil_div(nimg_lines, row_lines<L_>()), ngroups, ns);
             hipLaunchKernelGGL((k_toep_pass_e<L_>), grid, dim3(fftc::row_threads(L_)), 0,
                                ctx->stream, P.g1, P.sens, nimg_lines, P.N1, N2o, A, C, cpg,
-                               P.partial, tw_last);
+                               P.partial, seg, tw_last);
         });
         prof_end(ctx, rec);
         IMP_CHECK_LAUNCH();
         // pass F
         rec = prof_begin(ctx, "toep_pass_f");
         hipLaunchKernelGGL(k_toep_pass_f, dim3(ceil_div(nvox, 256)), dim3(256), 0, ctx->stream,
-                           P.partial, ngroups, nvox, P.fcyc, tau_l, scale, l > 0 ? 1 : 0, out);
+                           P.partial, ns, ngroups, nvox, P.fcyc, P.t0, P.tau, l, scale, out);
         prof_end(ctx, rec);
         IMP_CHECK_LAUNCH();
     }

@@ -34,8 +34,9 @@ struct ToepPlan {
     float2 *qf = nullptr;         // [nseg][G]  FFT(ifftshift(Q_l)), offsets -N zeroed
     float *qfr = nullptr;         // [nseg][G]  Re(qf), used when qf_real
     bool qf_real = false;         // qf is real to rounding (conjugate-symmetric Q_l)
-    float2 *g1 = nullptr;         // [ncoils][N1][A][Ml] pass buffer
-    float2 *partial = nullptr;    // [ngroups][nvox]
+    int segs_per_pass = 1;        // segments that go through the passes together
+    float2 *g1 = nullptr;         // [segs_per_pass][ncoils][N1][A][Ml] pass buffer
+    float2 *partial = nullptr;    // [segs_per_pass][ngroups][nvox]
     float2 *sens = nullptr;       // [ncoils][nvox] or null (S = 1)
     float *fcyc = nullptr;        // [nvox] field map in Hz (w / 2pi)
     float *w = nullptr;           // [nvox] TV weight or null (W = I), not owned

@@ -190,7 +190,7 @@ def main(argv=None):
     passes = {}
     for name, nbytes in pass_bytes(nv, nc, d3).items():
         tot, n = kernel_ms(name)
-        avg = tot / max(n, 1)
+        avg = tot / (3 * (L + 1))      # per segment; a launch may hold several
         passes[name] = {"launches": n, "avg_ms": round(avg, 4), "algorithmic_bytes": nbytes,
                         "gbs": round(nbytes / (avg * 1e-3) / 1e9, 1) if avg > 0 else None}
         log(f"{name}: {n} launches, {avg:.4f} ms, {passes[name]['gbs']} GB/s")

@@ -98,6 +98,11 @@ int imp_host_free(imp_ctx *ctx, void *hptr);
  *   fm [num_x] or NULL (0); phi_r/phi_i [ncoils*num_k] or NULL (phi = 1);
  *   d_r/d_i [ncoils*num_k] coil-major; s_r/s_i [ncoils*num_x] or NULL (S = 1);
  *   out_r/out_i [num_x].
+ * Large problems whose voxels form a tensor grid (2D, and stacks of 2D
+ * trajectories) are summed in separable form, in FP64, where that is predicted
+ * to be faster; deciding reads a few words back, which waits for the stream.
+ * Under stream capture, and when the workspace cannot be had, the sums are
+ * direct.
  */
 int imp_nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils,
                       const float *kx, const float *ky, const float *kz,
@@ -170,8 +175,9 @@ int imp_nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
  * flags: IMP_Q_CUMULATIVE reproduces the reference direct path, whose device
  * accumulator is not cleared between segments (computeQ.cmem.cu:190-191,
  * 951-963), i.e. returns prefix sums over l.  On the standard grid the
- * sums are evaluated as a separable GEMM (e^{i 2pi k.r} = e_x e_y e_z per
- * sample, each segment over the samples where a_l != 0); IMP_Q_DIRECT
+ * sums are evaluated in separable form (2D: spreading and line transforms in
+ * FP64; 3D, and samples beyond the band: a GEMM, e^{i 2pi k.r} = e_x e_y e_z
+ * per sample, each segment over the samples where a_l != 0); IMP_Q_DIRECT
  * evaluates every grid point with the per-point kernel instead. */
 #define IMP_Q_CUMULATIVE 0x1
 #define IMP_Q_DIRECT 0x2

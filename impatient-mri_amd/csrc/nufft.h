@@ -63,6 +63,9 @@ int nufft_stack_adjoint(imp_ctx *ctx, const NuGeometry &G, int K, int P, int nco
                         const float *phi_r, const float *phi_i, const float *d_r,
                         const float *d_i, const float *s_r, const float *s_i, float *out_r,
                         float *out_i);
+// coils of a group of F from the bytes per coil of its k grid and
+// half-transformed grid
+int nufft_forward_group(size_t grid_bytes, size_t mid_bytes, int ncoils);
 double nufft_forward_us(const NuGeometry &G, int m, int ncoils);
 int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
                   const float *ky, const float *t, const float *x, const float *y,

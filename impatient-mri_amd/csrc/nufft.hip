@@ -2695,6 +2695,20 @@ constexpr size_t NU_KGRID_BYTES = (size_t)2 << 30;
 
 }  // namespace
 
+// Coils that go through F together: the k grid (A.nf x B.nf) and the
+// half-transformed grid (A.n x B.nf) of a group stay within their limits.  One
+// is not enough: of 2730 x 2730 voxels and samples within +-20 cycles along A
+// and the whole band along B, the half-transformed grid is 36 times the larger.
+// k_fline's element offsets are 32 bits wide; a group within the limits has at
+// most 2^28 elements, and a single coil 4096 x 8205 x 48 (plan_axis and
+// prolate_expand admit no more), below 2^31.
+int nufft_forward_group(size_t grid_bytes, size_t mid_bytes, int ncoils) {
+    int cg = std::min(32, ncoils);
+    while (cg > 1 && (grid_bytes * cg > NU_KGRID_BYTES || mid_bytes * cg > NU_MID_BYTES))
+        cg = (cg + 1) / 2;
+    return cg;
+}
+
 double nufft_forward_us(const NuGeometry &G, int m, int ncoils) {
     const double nt = terms_estimate(G);
     const double grid = (double)G.A.nf * G.B.nf + (double)G.A.n * G.B.nf;
@@ -2716,9 +2730,9 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
     IMP_TRY(N.sort(true));
     IMP_TRY(N.expand());
     N.take_tables();
-    int cg = std::min(32, ncoils);
     const size_t col_bytes = (size_t)A.nf * B.nf * N.nt * sizeof(double2);
-    while (cg > 1 && col_bytes * cg > NU_KGRID_BYTES) cg = (cg + 1) / 2;
+    const size_t mid_bytes = (size_t)nA * B.nf * N.nt * sizeof(double2);
+    const int cg = nufft_forward_group(col_bytes, mid_bytes, ncoils);
     Carver &W = N.W;
     constexpr int NX = NW + 2 * (TG - 1);
     const int ntx = ceil_div(A.nf - NW + 1, TG), ntile = ntx * ceil_div(B.nf - NW + 1, TG);
@@ -2737,7 +2751,7 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
     const size_t o_vt = W.take((size_t)N.nt * nvox * 8);
     const size_t o_sens = W.take(s_r ? (size_t)ncoils * nvox * sizeof(float2) : 0);
     const size_t o_img0 = W.take(nvox * sizeof(double2));
-    const size_t o_mid = W.take((size_t)nA * B.nf * N.nt * cg * sizeof(double2));
+    const size_t o_mid = W.take(mid_bytes * cg);
     const size_t o_grid = W.take(col_bytes * cg);
     IMP_TRY(N.alloc(cA, 1, cB, nA));
     hipLaunchKernelGGL(k_nu_starts, dim3(1), b256, 0, st, m, N.key, -1, (int *)nullptr,

@@ -1,0 +1,43 @@
+"""The separable NUDFT (csrc/nufft.hip) at the ends of what its dispatch
+admits: long and unequal axes, grids far beyond the image's band, many time
+terms and samples.  Tolerance as in test_gpu_nufft.py."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+from test_gpu_nufft import TOL, _timer
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(Nx, Ny, x, y):
+    """Voxel coordinates of the tensor grid, x fastest."""
+    f = lambda a: np.ascontiguousarray(a, np.float32).reshape(-1)
+    return f(np.broadcast_to(x, (Ny, Nx))), f(np.broadcast_to(np.asarray(y)[:, None], (Ny, Nx)))
+
+
+def test_forward_half_transformed_grid_larger_than_32_bits(ctx):
+    """2730 x 2730 voxels, 32 coils, samples in a strip: 75 x 4111 grid cells
+    but 2730 x 4111 half-transformed ones, which for 13 time terms of 32 coils
+    exceed 2^32 elements (the coils go in groups)."""
+    from impatient import ops
+    from oracle import oracle as orc
+    N, nc, M = 2730, 32, 20000
+    r = np.random.default_rng(31)
+    i = np.arange(N) - N // 2
+    x, y = _grid(N, N, i / N, i)            # y in voxels: ky in cycles per voxel
+    kx, ky = r.uniform(-20, 20, M).astype(np.float32), r.uniform(-.5, .5, M).astype(np.float32)
+    t = r.uniform(1e-3, 9e-3, M).astype(np.float32)
+    fm = (2 * np.pi * 150 * np.cos(3 * x) * np.sin(2e-3 * y)).astype(np.float32)
+    rho = (r.standard_normal(N * N) + 1j * r.standard_normal(N * N)).astype(np.complex64)
+    got, (n,) = _timer(ctx, lambda: ops.nudft_forward(ctx, kx, ky, None, t, x, y, None, fm, rho,
+                                                      None, nc), "nufft_forward")
+    assert n == 1
+    idx = np.array([0, 777, 12345, M - 1])
+    ref = orc.nudft_forward(kx[idx], ky[idx], None, t[idx], x, y, None, fm, rho, None)
+    got = np.asarray(got).reshape(nc, M)
+    errs = [rel_l2(g[idx], ref) for g in got]
+    print(f"worst coil {max(errs):.2e}")
+    assert max(errs) < TOL

@@ -2842,12 +2842,12 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
 namespace {
 
 // [sample][slot] = (a_2c, a_(2c+1)) |phi|^2, a_l the Hanning interpolator of
-// hanning_d (computeQ.cmem.cu:125-138)
-__global__ void k_nu_qdata(int m, int nseg, int slots, const float *t, const float *phi_r,
+// hanning_d (computeQ.cmem.cu:125-138); 2^lc slots, m of them may pass 2^31
+__global__ void k_nu_qdata(int m, int nseg, int lc, const float *t, const float *phi_r,
                            const float *phi_i, float tau, float t0, double2 *wd) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m * slots) return;
-    const int j = i / slots, c = i % slots;
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (long)m << lc) return;
+    const int j = (int)(i >> lc), c = (int)(i & ((1 << lc) - 1));
     double mag = 1.0;
     if (phi_r) {
         const double pr = phi_r[j], pi = phi_i[j];
@@ -2937,7 +2937,7 @@ int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const flo
     IMP_TRY(N.build(nullptr, 1, nullptr, 1));
     if (N.groups != 1) return fail(IMP_EINVAL, "toeplitz_q: %d column groups", N.groups);
     hipLaunchKernelGGL(k_nu_qdata, dim3(ceil_div((long)m << N.lc, 256)), dim3(256), 0, st, m, nseg,
-                       1 << N.lc, t, phi_r, phi_i, tau, t0, N.at<double2 *>(N.o_wd));
+                       N.lc, t, phi_r, phi_i, tau, t0, N.at<double2 *>(N.o_wd));
     IMP_TRY(N.to_mid(cols));
     IMP_TRY(line_store(ctx, N.lines_b(cols), G.A.n, N.at<double2 *>(o_p), cols,
                        (size_t)G.A.n * cols));

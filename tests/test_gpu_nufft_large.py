@@ -41,3 +41,25 @@ def test_forward_half_transformed_grid_larger_than_32_bits(ctx):
     errs = [rel_l2(g[idx], ref) for g in got]
     print(f"worst coil {max(errs):.2e}")
     assert max(errs) < TOL
+
+
+def test_q_of_more_weights_than_32_bits(ctx):
+    """2^27 samples x 16 column slots: 2^31 weights.  The samples repeat 2^15
+    of them, so the sums are the oracle's over those times the repetitions."""
+    from impatient import Context, ops
+    from oracle import oracle as orc
+    N, L, M, rep = 8, 16, 1 << 15, 1 << 12
+    r = np.random.default_rng(32)
+    kx, ky = r.uniform(-N / 2, N / 2, (2, M)).astype(np.float32)
+    t = np.sort(r.uniform(1e-3, 9e-3, M)).astype(np.float32)
+    big = Context(0)                        # its 90 GB go with it
+    try:
+        got, (n,) = _timer(big, lambda: ops.toeplitz_q(
+            big, np.tile(kx, rep), np.tile(ky, rep), None, np.tile(t, rep), N, N, 1, L), "nufft_q")
+    finally:
+        big.close()
+    assert n == 1
+    ref = rep * orc.toeplitz_q(kx, ky, None, t, N, N, 1, L)
+    errs = [rel_l2(a, b) for a, b in zip(got, ref)]
+    print(f"worst segment {max(errs):.2e}")
+    assert max(errs) < TOL

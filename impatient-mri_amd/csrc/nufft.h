@@ -40,6 +40,8 @@ struct NuGeometry {
 bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double> &mul, int *nt,
                     int *nleg);
 
+// radix passes of the sort by cell
+int nufft_sort_passes(int ncells);
 int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
                    const float *x, const float *y, const float *z, const float *fm,
                    NuGeometry *G);

@@ -2188,6 +2188,18 @@ double terms_estimate(const NuGeometry &G) {
     return th > 0.0 ? 8.0 + 1.2 * std::pow(th, 0.9) : 1.0;
 }
 
+}  // namespace
+
+// 8-bit digits of the cells' numbers 0..ncells - 1 (at least one: the sort
+// also fills the sample order)
+int nufft_sort_passes(int ncells) {
+    int n = 1;
+    while (n < 4 && (ncells - 1) >> (8 * n)) ++n;
+    return n;
+}
+
+namespace {
+
 // The stages shared by the separable operators: samples sorted by window,
 // tables, work lists; then per group of columns, weights -> spread grid ->
 // mid[ia][gB][q].
@@ -2234,7 +2246,7 @@ struct NuPass {
         else
             hipLaunchKernelGGL(k_nu_keys, dim3(ceil_div(m, 256)), dim3(256), 0, st, m, kA, kB,
                                G.A, G.B, key0, val0);
-        for (int shift = 0; shift == 0 || (ncells - 1) >> shift; shift += 8) {
+        for (int pass = 0, shift = 0; pass < nufft_sort_passes(ncells); ++pass, shift += 8) {
             hipLaunchKernelGGL(k_rx_count, dim3(nblk), dim3(256), 0, st, (const int *)key0, m,
                                shift, hist);
             hipLaunchKernelGGL(k_rx_scatter, dim3(nblk), dim3(256), 0, st, (const int *)key0,

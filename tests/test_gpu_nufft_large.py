@@ -63,3 +63,59 @@ def test_q_of_more_weights_than_32_bits(ctx):
     errs = [rel_l2(a, b) for a, b in zip(got, ref)]
     print(f"worst segment {max(errs):.2e}")
     assert max(errs) < TOL
+
+
+def test_q_of_more_than_2_24_cells(ctx):
+    """Q of 1032 x 1032: 4101 x 4101 window starts, four digits in the sort."""
+    from impatient import ops
+    N, L, M = 1032, 2, 4001
+    r = np.random.default_rng(33)
+    kx, ky = r.uniform(-N / 2, N / 2, (2, M)).astype(np.float32)
+    kx[:4], ky[:4] = N / 2 * np.array([-1, 1, -1, 1]), N / 2 * np.array([-1, -1, 1, 1])
+    t = np.sort(r.uniform(1e-3, 9e-3, M)).astype(np.float32)
+    got, (n,) = _timer(ctx, lambda: ops.toeplitz_q(ctx, kx, ky, None, t, N, N, 1, L), "nufft_q")
+    assert n == 1
+    from oracle import oracle as orc
+    pts = r.integers(0, 2 * N, (2, 200))
+    grid = ((pts[0] - N) / N, (pts[1] - N) / N, None)
+    ref = orc.toeplitz_q(kx, ky, None, t, N, N, 1, L, grid=grid)
+    errs = [rel_l2(a[pts[1] * 2 * N + pts[0]], b) for a, b in zip(got, ref)]
+    print(f"worst segment {max(errs):.2e}")
+    assert max(errs) < TOL
+
+
+def _wide(N, nc, M, kmax, seed):
+    """An N x N image and samples over +-kmax cycles (corners included)."""
+    r = np.random.default_rng(seed)
+    kx, ky = r.uniform(-kmax, kmax, (2, M)).astype(np.float32)
+    kx[:4], ky[:4] = kmax * np.array([-1, 1, -1, 1]), kmax * np.array([-1, -1, 1, 1])
+    t = r.uniform(1e-3, 6e-3, M).astype(np.float32)
+    i = (np.arange(N) - N // 2) / N
+    x, y = _grid(N, N, i, i)
+    fm = (2 * np.pi * 60 * np.cos(4 * x + y)).astype(np.float32)
+    c = lambda *s: (r.standard_normal(s) + 1j * r.standard_normal(s)).astype(np.complex64)
+    return kx, ky, t, x, y, fm, c(nc, M), c(nc, N * N), c(N * N)
+
+
+@pytest.mark.parametrize("kmax,M", [(1400.0, 300000), (2650.0, 600000)])
+def test_samples_far_beyond_the_band(ctx, kmax, M):
+    """256 x 256 voxels with samples over 11 and 20 times the band: 4200^2 and
+    7960^2 grid cells, folded up to 21 times onto the line transforms."""
+    from impatient import ops
+    from oracle import oracle as orc
+    kx, ky, t, x, y, fm, d, s, rho = _wide(256, 2, M, kmax, 34)
+    got, (n,) = _timer(ctx, lambda: ops.nudft_adjoint(ctx, kx, ky, None, t, x, y, None, fm, d, s),
+                       "nufft_adjoint")
+    assert n == 1
+    r = np.random.default_rng(2)
+    idx = np.unique(np.concatenate([[0, len(x) - 1], r.integers(0, len(x), 30)]))
+    ref = orc.nudft_adjoint(kx, ky, None, t, x[idx], y[idx], None, fm[idx], d, s[:, idx])
+    ea = rel_l2(got[idx], ref)
+    got, (n,) = _timer(ctx, lambda: ops.nudft_forward(ctx, kx, ky, None, t, x, y, None, fm, rho,
+                                                      s), "nufft_forward")
+    assert n == 1
+    idx = np.unique(np.concatenate([[0, 1, 2, 3, M - 1], r.integers(0, M, 30)]))
+    ref = orc.nudft_forward(kx[idx], ky[idx], None, t[idx], x, y, None, fm, rho, s)
+    ef = rel_l2(np.asarray(got).reshape(2, M)[:, idx], ref)
+    print(f"adjoint {ea:.2e}, forward {ef:.2e}")
+    assert ea < TOL and ef < TOL

@@ -29,3 +29,12 @@ def test_forward_groups_bound_both_grids():
             assert nA * nfB * nt * cg < 2 ** 32 and nfA * nt * cg < 2 ** 32
     assert group(16 * 783 * 783 * 13, 16 * 512 * 783 * 13, 32) == 16
     assert group(16 * 75 * 4111 * 13, 16 * 2730 * 4111 * 13, 32) == 1
+
+
+def test_sort_passes_cover_every_cell_and_end():
+    """8-bit radix passes: enough digits for the last cell's number, no more,
+    and at most the four of a 32-bit key (plan_axis admits 8195^2 cells)."""
+    passes = _fn("_ZN3imp17nufft_sort_passesEi", C.c_int, C.c_int)
+    for n in (1, 2, 255, 256, 257, 65535, 65536, 65537, 2 ** 24 - 1, 2 ** 24, 2 ** 24 + 1,
+              4101 ** 2, 8195 ** 2, 2 ** 31 - 1):
+        assert passes(n) == max(1, ((n - 1).bit_length() + 7) // 8)

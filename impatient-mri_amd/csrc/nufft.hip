@@ -169,10 +169,12 @@ __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, con
 
 // Axis structure implied by the first changes.  In 3D (nz_known = 0) z runs
 // fastest and its period is where x or y first changes; then the coordinate
-// that changes first is axis A, of nA points.  false: none.
+// that changes first is axis A, of nA points.  false: none.  (Index 0 differs
+// from itself where it is NaN: no periods to divide by.)
 __host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool d3, bool *a_is_y,
                                          int *nA, int *nz) {
     const unsigned f = fcx < fcy ? fcx : fcy;
+    if (f == 0) return false;
     *a_is_y = fcy < fcx;
     *nz = d3 ? (int)f : 1;
     const unsigned slow = *a_is_y ? fcx : fcy;

@@ -119,3 +119,26 @@ def test_samples_far_beyond_the_band(ctx, kmax, M):
     ef = rel_l2(np.asarray(got).reshape(2, M)[:, idx], ref)
     print(f"adjoint {ea:.2e}, forward {ef:.2e}")
     assert ea < TOL and ef < TOL
+
+
+@pytest.mark.parametrize("axes", ["x", "y", "xy"])
+def test_volume_whose_first_voxel_is_not_a_number(ctx, axes):
+    """The periods of a volume's axes are counted from voxel 0: where that is
+    NaN there are none, and the sum stays direct (NaN at that voxel alone)."""
+    from impatient import ops
+    from oracle import oracle as orc
+    from test_gpu_nufft import DIRECT_TOL, _stack
+    q = _stack(48, 40, 8, 4, 30000, 16)
+    for a in axes:
+        q[a] = q[a].copy()
+        q[a][0] = np.nan
+    got, n = _timer(ctx, lambda: ops.nudft_adjoint(
+        ctx, q["kx"], q["ky"], q["kz"], q["t"], q["x"], q["y"], q["z"], q["fm"], q["d"], q["s"]),
+        "nufft_stack", "k_nudft_stack")
+    assert n[0] == 0 and n[1] > 0
+    assert np.isnan(got[0])
+    idx = np.unique(np.concatenate([[1, len(q["x"]) - 1],
+                                    np.random.default_rng(1).integers(1, len(q["x"]), 20)]))
+    ref = orc.nudft_adjoint(q["kx"], q["ky"], q["kz"], q["t"], q["x"][idx], q["y"][idx],
+                            q["z"][idx], q["fm"][idx], q["d"], q["s"][:, idx])
+    assert rel_l2(got[idx], ref) < DIRECT_TOL

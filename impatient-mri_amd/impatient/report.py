@@ -105,6 +105,28 @@ def sparse_reg_timing(ctx, p, timer_on, kernel_ms, log):
     return res
 
 
+def fhd_account(kernel_ms, nk, nv, nz):
+    """Time, path, evaluated pairs and timer records of one F^H d of nk samples
+    and nv voxels (nz planes): the separable evaluation of an image or a stack
+    (one record for all its launches; it visits no pairs), or the direct
+    kernels, or the z-separable sum's group launches and its reduction.
+    Evaluated are the (sample, voxel) pairs whose phase and sin/cos were
+    computed: once per pair for all coils on the direct path; on the
+    z-separable one once per pair of one partition and group launch of 32
+    coil-partition columns."""
+    parts = {k: kernel_ms(k) for k in ("k_nudft_mfma", "k_nudft_valu", "k_nudft_stack",
+                                       "k_reduce_stack", "nufft_adjoint", "nufft_stack")}
+    ms = sum(v[0] for v in parts.values())
+    if parts["nufft_adjoint"][1] or parts["nufft_stack"][1]:
+        path, evaluated = "separable", 0.0
+    elif parts["k_nudft_stack"][1]:
+        path = "stacked (z-separable)"
+        evaluated = float(parts["k_nudft_stack"][1]) * (nk // nz) * nv
+    else:
+        path, evaluated = "direct", float(nk) * nv
+    return ms, path, evaluated, parts
+
+
 def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__.split("\n")[0])
     ap.add_argument("--config", type=int, default=2)
@@ -141,26 +163,10 @@ def main(argv=None):
     ops.nudft_adjoint(ctx, p.kx, p.ky, p.kz, p.t, p.x, p.y, p.z, p.fm, d, p.sens)
     timer_on()
     b = ops.nudft_adjoint(ctx, p.kx, p.ky, p.kz, p.t, p.x, p.y, p.z, p.fm, d, p.sens)
-    # direct kernels, the stacked path's group launches and its reduction, or
-    # the separable evaluation (which visits no pairs)
-    parts = {k: kernel_ms(k) for k in ("k_nudft_mfma", "k_nudft_valu", "k_nudft_stack",
-                                       "k_reduce_stack", "nufft_adjoint")}
-    fhd_ms = sum(v[0] for v in parts.values())
-    stacked = parts["k_nudft_stack"][1] > 0
-    separable = parts["nufft_adjoint"][1] > 0
-    path = "separable" if separable else "stacked (z-separable)" if stacked else "direct"
+    fhd_ms, path, evaluated, parts = fhd_account(kernel_ms, nk, nv, p.Nz)
     pairs = float(nc) * nk * nv
-    # (sample, voxel) pairs whose phase and sin/cos were evaluated: once per
-    # pair for all coils on the direct path; on the stacked path once per
-    # pair of one partition and group launch of 32 coil-partition columns
-    if separable:
-        evaluated = 0.0
-    elif stacked:
-        K = nk // p.Nz
-        evaluated = float(parts["k_nudft_stack"][1]) * K * nv
-    else:
-        evaluated = float(nk) * nv
-    log(f"F^H d ({path}): {fhd_ms:.1f} ms, {pairs / fhd_ms / 1e6:.1f} GSample*vox/s; "
+    gs = round(pairs / fhd_ms / 1e6, 1) if fhd_ms > 0 else None
+    log(f"F^H d ({path}): {fhd_ms:.1f} ms, {gs} GSample*vox/s; "
         + ", ".join(f"{k} {v[1]} x {v[0] / max(v[1], 1):.2f} ms" for k, v in parts.items() if v[1]))
 
     # Q_l and the plan from device arrays (no host round trip of the planes)
@@ -212,7 +218,7 @@ def main(argv=None):
     out = {"config": p.name, "nsamples": nk, "nvox": nv, "ncoils": nc, "segments": L,
            "fhd_path": path, "fhd_ms": round(fhd_ms, 3),
            "fhd_direct_equivalent_pairs": pairs, "fhd_evaluated_phase_pairs": evaluated,
-           "fhd_gsample_vox_s": round(pairs / fhd_ms / 1e6, 1),
+           "fhd_gsample_vox_s": gs,
            "q_s": round(t_q, 4), "toeplitz_plan_s": round(t_plan, 4),
            "toeplitz_passes": passes, "tol": args.tol, "solves": solves}
     if sreg is not None:

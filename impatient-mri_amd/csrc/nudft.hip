@@ -888,11 +888,14 @@ MFn pick_mfma(int tiles, bool d3) {
 constexpr int MFMA_MIN_RHS = 3;
 
 // Chunks so the launch holds enough workgroups to fill the GPU.
-int pick_chunks(imp_ctx *ctx, long wgs, int n_units, int min_units_per_chunk) {
-    const long target = 8L * ctx->num_cus;
+int pick_chunks(int num_cus, long wgs, int n_units, int min_units_per_chunk) {
+    const long target = 8L * num_cus;
     int chunks = 1;
     while (wgs * chunks < target && n_units / (chunks * 2) >= min_units_per_chunk) chunks *= 2;
     return chunks;
+}
+int pick_chunks(imp_ctx *ctx, long wgs, int n_units, int min_units_per_chunk) {
+    return pick_chunks(ctx->num_cus, wgs, n_units, min_units_per_chunk);
 }
 
 enum class Out { Combine, PerRhs, PerRhsCumulative };
@@ -1290,20 +1293,41 @@ size_t adjoint_fixed_bytes(int num_k, int num_x, int ncoils, bool d3) {
 }  // namespace
 
 // ---- direct sum or separable evaluation (nufft.hip) -------------------------
-// Times of both in microseconds on an MI355X, fitted to single calls over
-// 48^2..512^2 voxels x 2e3..4e5 samples x 1..32 coils (within 30%).  The
-// direct kernels cost the same for every geometry; the separable form pays per
-// sample and time term for the spread, and per grid column for the
-// transforms, behind a fixed part (geometry read-back, sort, ~20 launches).
+// Chosen by predicted times (microseconds on an MI355X; the separable forms'
+// are in nufft.hip).  The direct kernels cost the same for every geometry: pairs,
+// operands packed per streamed point and coil, partial sums per chunk.
 constexpr double STACK_MIN_US = 400.0;    // direct time of a stack below which it is kept
 constexpr double NUFFT_MIN_PAIRS = 6e8;   // below: the direct kernels win at every size measured
+constexpr double DIRECT_FIXED_US = 70.0;
 
-constexpr double DIRECT_FIXED_US = 60.0;
-
-double direct_us(double pairs, int ncoils) {
-    return DIRECT_FIXED_US + pairs * (ncoils <= 1 ? 7.9e-7 : ncoils == 2 ? 8.4e-7
-                                      : ncoils <= MF_COLS ? 5.6e-7 : 8.1e-7);
+double direct_us(int n_stream, int n_lane, int ncoils, bool forward, int num_cus) {
+    double us = DIRECT_FIXED_US + (double)n_stream * n_lane *
+                                      (ncoils <= 1 ? 7.7e-7 : ncoils == 2 ? 8.0e-7
+                                       : ncoils <= MF_COLS ? 5.45e-7 : 7.5e-7) +
+                (forward ? 5.7e-5 : 1.73e-4) * n_stream * ncoils;
+    if (ncoils >= MFMA_MIN_RHS) {
+        const long wgs = ceil_div(n_lane, MF_WAVE_PTS * (NU_THREADS / 64));
+        const int chunks = pick_chunks(num_cus, wgs, ceil_div(n_stream, MF_K), 4 * MF_FOLD);
+        us += 33.0 + 1.45e-4 * chunks * ceil_div(ncoils, MF_COLS) * (double)n_lane;
+    }
+    return us;
 }
+
+// The z-separable direct sum of nrhs coil-partition columns (a launch sequence
+// for each 32, less than separate calls: within 8% rms of 159 random stacks),
+// and the direct sum of a volume (a third coordinate: 15% more).
+double stack_us(int K, int num_x, int nrhs, int num_cus) {
+    return 83.0 + ceil_div(nrhs, 2 * MF_COLS) *
+                      (direct_us(K, num_x, 2 * MF_COLS, false, num_cus) - 44.0);
+}
+double volume_us(int num_k, int num_x, int ncoils, int num_cus) {
+    return 1.15 * direct_us(num_k, num_x, ncoils, false, num_cus);
+}
+
+// A tenth in favour of the direct sums: of the 1000 calls timed 642 take the
+// separable form and 18 of them would have been faster directly, by 1.4 at most
+// (without the tenth 677 and 29; of those left direct none loses over 1.5).
+bool separable_pays(double separable, double direct) { return separable < 0.9 * direct; }
 
 // The separable form evaluates 2D problems of as many coils as one direct
 // launch takes; refusals and everything else stay with the direct path.
@@ -1321,7 +1345,9 @@ int choose_separable(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float
     IMP_TRY(nufft_geometry(ctx, num_k, num_x, kx, ky, t, x, y, nullptr, fm, G));
     const double us = forward ? nufft_forward_us(*G, num_k, ncoils)
                               : nufft_adjoint_us(*G, num_k, ncoils);
-    if (G->ok && us >= direct_us(pairs, ncoils)) G->ok = false;
+    const double direct = forward ? direct_us(num_x, num_k, ncoils, true, ctx->num_cus)
+                                  : direct_us(num_k, num_x, ncoils, false, ctx->num_cus);
+    if (G->ok && !separable_pays(us, direct)) G->ok = false;
     return IMP_OK;
 }
 
@@ -1368,13 +1394,12 @@ int nudft_adjoint(imp_ctx *ctx, int num_k, int num_x, int ncoils, const float *k
         if (K > 0) {
             const int nrhs = ncoils * (num_k / K);
             NuGeometry G;
-            const double us = direct_stack
-                ? ceil_div(nrhs, 2 * MF_COLS) * direct_us((double)K * num_x, 2 * MF_COLS)
-                : direct_us((double)num_k * num_x, ncoils);
+            const double us = direct_stack ? stack_us(K, num_x, nrhs, ctx->num_cus)
+                                           : volume_us(num_k, num_x, ncoils, ctx->num_cus);
             // more than 32 coils are refused by the direct sum of a volume
             if ((direct_stack || ncoils <= 2 * MF_COLS) && us > STACK_MIN_US)
                 IMP_TRY(nufft_geometry(ctx, K, num_x, kx, ky, t, x, y, z, fm, &G));
-            if (G.ok && nufft_stack_us(G, K, nrhs) < us) {
+            if (G.ok && separable_pays(nufft_stack_us(G, K, nrhs), us)) {
                 const int rc = nufft_stack_adjoint(ctx, G, K, num_k / K, ncoils, kx, ky, kz, t, x,
                                                    y, z, fm, phi_r, phi_i, d_r, d_i, s_r, s_i,
                                                    out_r, out_i);
@@ -1497,8 +1522,10 @@ int nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs, int 
         const imp_nudft_job &b = jobs[j];
         // the launch's fixed part is shared by the direct jobs
         int rc = IMP_ENOMEM;
-        if (G[j].ok && nufft_adjoint_us(G[j], b.num_k, b.ncoils) <
-                           direct_us((double)b.num_k * b.num_x, b.ncoils) - DIRECT_FIXED_US)
+        if (G[j].ok &&
+            separable_pays(nufft_adjoint_us(G[j], b.num_k, b.ncoils),
+                           direct_us(b.num_k, b.num_x, b.ncoils, false, ctx->num_cus) -
+                               DIRECT_FIXED_US))
             rc = nufft_adjoint(ctx, G[j], b.num_k, b.ncoils, b.kx, b.ky, b.t, b.x, b.y, b.fm,
                                b.phi_r, b.phi_i, b.d_r, b.d_i, b.s_r, b.s_i, b.out_r, b.out_i);
         if (rc == IMP_ENOMEM) rest.push_back(b);

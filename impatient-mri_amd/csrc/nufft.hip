@@ -2183,11 +2183,44 @@ int log2i(int n) {
     return b;
 }
 
-// time terms as the predicted times use them (the exact count follows from
-// prolate_expand; within 2)
-double terms_estimate(const NuGeometry &G) {
+// time terms as the predicted times use them (within 1 of what prolate_expand
+// finds from theta = 0.3 to 40, 2 below)
+int terms_estimate(const NuGeometry &G) {
     const double th = G.wh * G.th;
-    return th > 0.0 ? 8.0 + 1.2 * std::pow(th, 0.9) : 1.0;
+    if (!(th > 0.0)) return 1;
+    const double n = th > 1.0 ? 8.0 + 1.6 * std::pow(th - 1.0, 0.85) : 8.0 + 1.2 * std::log(th);
+    return (int)std::lround(std::min<double>(NU_MAX_TERMS, std::max(2.0, n)));
+}
+
+// Coils (or other columns) of a group: the half-transformed grid within its
+// limit, and column slots x time groups x rows = 64 lanes, so fewer columns
+// when the time terms need more groups.
+int column_group(const NuGeometry &G, int nt, int ncols) {
+    int cg = std::min(32, 1 << log2i(ncols));
+    while (cg > 1 && (size_t)G.A.n * G.B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
+    while (cg > 1 && ceil_div(nt, 64 / cg) > SP_MAX_NL) cg /= 2;
+    return cg;
+}
+
+// The split of the lanes beside 2^lc columns into time groups and rows with the
+// fewest FP64 instructions per sample: visits x (2 NL (T + 1) + about 16 for
+// the rest).
+struct SpreadSplit {
+    int ll = 0, nl = 1, yg = 1, T = 1;
+    double cost = 0.0;
+};
+SpreadSplit spread_split(int nt, int lc) {
+    SpreadSplit best;
+    for (int l = 0; l <= std::min(6 - lc, log2i(nt)); ++l) {
+        const int k = ceil_div(nt, 1 << l);
+        if (k > SP_MAX_NL) continue;
+        const int cells = sp_switch(k, [](auto n) { return sp_cells(decltype(n)::value); });
+        const int rows = 1 << (6 - lc - l);
+        const double cost = (double)(NW + rows - 1) / rows * (NW + cells - 1) / cells *
+                            (2 * k * (cells + 1) + 16);
+        if (best.cost == 0.0 || cost < best.cost) best = SpreadSplit{l, k, rows, cells, cost};
+    }
+    return best;
 }
 
 }  // namespace
@@ -2288,31 +2321,14 @@ struct NuPass {
     int layout(int ncols) {
         IMP_TRY(expand());
         const NuAxis &A = G.A, &B = G.B;
-        cg = std::min(32, 1 << log2i(ncols));
-        while (cg > 1 && (size_t)A.n * B.nf * nt * cg * sizeof(double2) > NU_MID_BYTES) cg /= 2;
-        // wave layout: column slots x time groups x rows = 64 lanes; fewer
-        // columns when the time terms need more groups
-        while (cg > 1 && ceil_div(nt, 64 / cg) > SP_MAX_NL) cg /= 2;
+        cg = column_group(G, nt, ncols);
         groups = ceil_div(ncols, cg);
         lc = log2i(cg);
-        // the split of the other lanes with the fewest FP64 instructions per
-        // sample: visits x (2 NL (T + 1) + about 16 for the rest)
-        double best = 0.0;
-        for (int l = 0; l <= std::min(6 - lc, log2i(nt)); ++l) {
-            const int k = ceil_div(nt, 1 << l);
-            if (k > SP_MAX_NL) continue;
-            const int cells = sp_switch(k, [](auto n) { return sp_cells(decltype(n)::value); });
-            const int rows = 1 << (6 - lc - l);
-            const double cost = (double)(NW + rows - 1) / rows * (NW + cells - 1) / cells *
-                                (2 * k * (cells + 1) + 16);
-            if (best == 0.0 || cost < best) {
-                best = cost;
-                ll = l;
-                nl = k;
-                yg = rows;
-                T = cells;
-            }
-        }
+        const SpreadSplit split = spread_split(nt, lc);
+        ll = split.ll;
+        nl = split.nl;
+        yg = split.yg;
+        T = split.T;
         ntp = nl << ll;
         S.T = T;
         S.yg = yg;
@@ -2483,14 +2499,50 @@ struct ProfScope {
 };
 }  // namespace
 
-// predicted microseconds of the spread and transforms of ncols columns of nt
-// time terms, without the fixed part
-static double separable_us(const NuAxis &A, const NuAxis &B, int m, double cols) {
-    return 3.0e-5 * m * cols + 1.0e-5 * ((double)A.nf * B.nf + (double)A.n * B.nf) * cols;
+// Predicted times.  Each form was timed on 1000 random single calls (12..900
+// points per axis, 4e3..8e5 samples within 0.25 to 5 times the band, dense and
+// even, 1 to 32 coils, 1 to 40 time terms, all axis kinds): the separable
+// adjoint is within 15% rms (0.57 to 1.7 times) of the sum below, F within 13%,
+// the direct sums within 6%.  Prices without the axis kinds, the columns that pad a
+// workgroup and F's nearly empty tiles were 41% and 53% off and sent calls to
+// the form that took up to 2.5 times as long.
+
+// Lines of all columns along an axis, in transformed elements: whole
+// workgroups' columns; AX_NEAR takes two transforms, AX_FREE an interpolation
+// (about three).
+static double line_work(const NuAxis &X, double nlines, double columns) {
+    return nlines * columns * X.L * (X.kind == AX_UNIFORM ? 1 : X.kind == AX_NEAR ? 2 : 3);
+}
+static double padded(int columns, int L) {
+    const int w = ln::lines(L, ST_WG);
+    return (double)ceil_div(columns, w) * w;
+}
+// prolate functions of `points` points: every Legendre degree of each term
+static double expansion_work(const NuGeometry &G, int nt, double points) {
+    return points * nt * (0.75 * G.wh * G.th + 36.0);
+}
+// fixed part, samples and A transform of ncols columns
+static double to_mid_us(const NuGeometry &G, int nt, int m, int ncols) {
+    const int cg = column_group(G, nt, ncols), groups = ceil_div(ncols, cg);
+    const SpreadSplit sp = spread_split(nt, log2i(cg));
+    const double prep = 2 * NW + 2 * (sp.T - 1) + 2 * (sp.yg - 1) + nt +
+                        2.0 * groups * (1 << log2i(cg));
+    const double lines = groups * padded(nt * std::min(cg, ncols), G.A.L);
+    // a group is half a dozen launches of some 8 us
+    return 144.0 + 50.0 * (groups - 1) + m * (2.79e-6 * groups * sp.cost + 1.46e-5 * prep) +
+           1.5e-6 * expansion_work(G, nt, m) + 9.74e-6 * G.A.nf * G.B.nf * (double)nt * ncols +
+           4.16e-6 * line_work(G.A, G.B.nf, lines);
 }
 
 double nufft_adjoint_us(const NuGeometry &G, int m, int ncoils) {
-    return 250.0 + separable_us(G.A, G.B, m, terms_estimate(G) * (1 << log2i(ncoils)));
+    const int nt = terms_estimate(G);
+    const int cg = column_group(G, nt, ncoils), groups = ceil_div(ncoils, cg);
+    // the combining pass holds whole workgroups of coils x time terms
+    const int nc = std::min(cg, ncoils), w = ln::lines(G.B.L, ST_WG);
+    const int cw = std::min(w, 1 << log2i(nc));
+    const double steps = (double)groups * ceil_div(nc, cw) * ceil_div(nt, w / cw) * w;
+    return to_mid_us(G, nt, m, ncoils) + 4.16e-6 * line_work(G.B, G.A.n, steps) +
+           8.7e-7 * expansion_work(G, nt, (double)G.A.n * G.B.n);
 }
 
 int nufft_adjoint(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,
@@ -2631,10 +2683,12 @@ __global__ __launch_bounds__(256) void k_nu_stack(int n, int nz, int P, int c0, 
 }  // namespace
 
 double nufft_stack_us(const NuGeometry &G, int K, int nrhs) {
-    const double nt = terms_estimate(G);
+    const int nt = terms_estimate(G);
+    const int cg = column_group(G, nt, nrhs), groups = ceil_div(nrhs, cg);
     const double vox = (double)G.A.n * G.B.n * G.nz;
-    return 300.0 + separable_us(G.A, G.B, K, nt * (nrhs < 32 ? 1 << log2i(nrhs) : nrhs)) +
-           4e-7 * vox * nt * nrhs;
+    const double lines = groups * padded(nt * std::min(cg, nrhs), G.B.L);
+    return 50.0 + to_mid_us(G, nt, K, nrhs) + 4.16e-6 * line_work(G.B, G.A.n, lines) +
+           8.7e-7 * expansion_work(G, nt, vox) + 4e-7 * vox * nt * nrhs;
 }
 
 int nufft_stack_adjoint(imp_ctx *ctx, const NuGeometry &G, int K, int P, int ncoils,
@@ -2723,10 +2777,31 @@ int nufft_forward_group(size_t grid_bytes, size_t mid_bytes, int ncoils) {
     return cg;
 }
 
+// The gather takes up to GI_S samples of a tile together, so where samples are
+// few per tile it works on almost empty products; k_nu_flists visits every
+// point of an AX_FREE axis for each 1024 cells, in one workgroup.
 double nufft_forward_us(const NuGeometry &G, int m, int ncoils) {
-    const double nt = terms_estimate(G);
-    const double grid = (double)G.A.nf * G.B.nf + (double)G.A.n * G.B.nf;
-    return 250.0 + 4.2e-4 * m * nt * ceil_div(ncoils, 8) + 1.0e-5 * grid * nt * ncoils;
+    const int nt = terms_estimate(G);
+    const NuAxis &A = G.A, &B = G.B;
+    const double grid = (double)A.nf * B.nf * nt * sizeof(double2);
+    const double mid = (double)A.n * B.nf * nt * sizeof(double2);
+    const int cg = nufft_forward_group((size_t)grid, (size_t)mid, ncoils);
+    const double tiles = (double)ceil_div(A.nf - NW + 1, TG) * ceil_div(B.nf - NW + 1, TG);
+    const double entries = tiles * (1.0 - std::exp(-m / tiles)) + (double)m / GI_S;
+    double blocks = 0.0, linesA = 0.0, linesB = 0.0, lists = 0.0;
+    for (int c0 = 0; c0 < ncoils; c0 += cg) {
+        const int nc = std::min(cg, ncoils - c0);
+        blocks += ceil_div(nc, 8);
+        linesA += padded(nt * nc, A.L);
+        linesB += padded(nt * nc, B.L);
+    }
+    for (const NuAxis *X : {&A, &B})
+        if (X->kind == AX_FREE) lists += (double)X->n * ceil_div(X->L, 1024);
+    return 114.0 + 2.09e-3 * entries * nt * blocks + 3.6e-5 * (double)m * ncoils +
+           5.35e-6 * expansion_work(G, nt, m) + 1.17e-5 * A.nf * B.nf * (double)nt * ncoils +
+           0.48 * lists + 2.9e-6 * line_work(A, B.nf, linesA) +
+           6.4e-6 * line_work(B, A.n, linesB) +
+           8.0e-7 * expansion_work(G, nt, (double)A.n * B.n);
 }
 
 int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const float *kx,

@@ -97,7 +97,7 @@ def _wide(N, nc, M, kmax, seed):
     return kx, ky, t, x, y, fm, c(nc, M), c(nc, N * N), c(N * N)
 
 
-@pytest.mark.parametrize("kmax,M", [(1400.0, 300000), (2650.0, 600000)])
+@pytest.mark.parametrize("kmax,M", [(1400.0, 300000), (2650.0, 2000000)])
 def test_samples_far_beyond_the_band(ctx, kmax, M):
     """256 x 256 voxels with samples over 11 and 20 times the band: 4200^2 and
     7960^2 grid cells, folded up to 21 times onto the line transforms."""

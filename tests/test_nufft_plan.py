@@ -38,3 +38,64 @@ def test_sort_passes_cover_every_cell_and_end():
     for n in (1, 2, 255, 256, 257, 65535, 65536, 65537, 2 ** 24 - 1, 2 ** 24, 2 ** 24 + 1,
               4101 ** 2, 8195 ** 2, 2 ** 31 - 1):
         assert passes(n) == max(1, ((n - 1).bit_length() + 7) // 8)
+
+
+class _Axis(C.Structure):   # NuAxis
+    _fields_ = ([(f, C.c_int) for f in ("n", "L", "nf", "kind", "flip", "shift")] +
+                [(f, C.c_double) for f in ("kc", "xc", "inv_d", "j0")])
+
+
+class _Geometry(C.Structure):   # NuGeometry
+    _fields_ = ([("ok", C.c_bool), ("a_is_y", C.c_bool), ("A", _Axis), ("B", _Axis),
+                 ("nz", C.c_int)] + [(f, C.c_double) for f in ("tc", "th", "wc", "wh")])
+
+
+# Single calls timed on an MI355X in both forms (microseconds).  Axes: points,
+# line length, grid cells, kind (0 uniform, 1 rounded, 2 free); half widths of t
+# and w multiplied; coils; samples; direct sum, separable form.
+TIMED = [
+    # sparse samples on large grids, free axes, few coils on long lines
+    ("forward", (527, 4096, 2261, 2), (381, 576, 1653, 0), 9.512, 17, 130640, 18654, 110898),
+    ("forward", (428, 2048, 1289, 2), (568, 3072, 1705, 2), 2.182, 32, 94369, 18815, 48118),
+    ("forward", (514, 2048, 1097, 2), (492, 2048, 1045, 2), 7.223, 12, 40831, 5843, 14033),
+    ("adjoint", (559, 1536, 857, 2), (499, 1152, 767, 2), 7.576, 32, 28657, 6693, 14991),
+    ("forward", (423, 512, 319, 2), (338, 512, 257, 2), 17.866, 9, 13962, 1375, 3061),
+    ("forward", (829, 2048, 1059, 2), (100, 256, 139, 2), 1.572, 4, 11675, 705, 1514),
+    ("forward", (468, 768, 1531, 0), (401, 768, 1529, 0), 19.14, 3, 32385, 3467, 7300),
+    ("adjoint", (91, 144, 53, 1), (17, 96, 39, 1), 0.0, 2, 580170, 1052, 2153),
+    ("adjoint", (542, 1024, 939, 1), (542, 1152, 749, 2), 10.939, 16, 23677, 4057, 8274),
+    ("forward", (191, 192, 125, 2), (235, 256, 151, 2), 18.277, 8, 13799, 494, 1245),
+    # and calls that the separable form does faster
+    ("forward", (60, 96, 107, 0), (204, 384, 379, 0), 0.42, 9, 165741, 1347, 731),
+    ("adjoint", (273, 512, 1083, 1), (336, 2048, 1065, 2), 15.642, 1, 42984, 3142, 899),
+    ("adjoint", (106, 192, 221, 1), (125, 192, 221, 1), 1.283, 4, 183972, 1639, 718),
+    ("adjoint", (441, 768, 745, 0), (549, 1024, 989, 0), 8.643, 3, 68252, 8759, 1421),
+    ("forward", (299, 512, 1327, 0), (773, 1536, 3953, 0), 0.0, 12, 19815, 2971, 914),
+    ("adjoint", (359, 576, 507, 0), (346, 576, 507, 0), 1.957, 16, 50683, 3858, 1007),
+    ("adjoint", (187, 288, 413, 1), (263, 512, 723, 1), 0.901, 12, 133601, 4174, 1207),
+    ("forward", (324, 512, 311, 2), (644, 1024, 605, 2), 0.393, 2, 11166, 2001, 879),
+    ("adjoint", (646, 1536, 1001, 2), (16, 96, 33, 2), 0.616, 8, 722497, 4901, 2493),
+]
+
+
+def test_the_faster_form_is_chosen():
+    """Predicted times against timed calls, of those the ones that prices
+    without axis kinds, padding and empty tiles got wrong by the most: the form
+    timed as the slower is not taken, and each price is within a factor of two."""
+    g = C.POINTER(_Geometry)
+    adj = _fn("_ZN3imp16nufft_adjoint_usERKNS_10NuGeometryEii", C.c_double, g, C.c_int, C.c_int)
+    fwd = _fn("_ZN3imp16nufft_forward_usERKNS_10NuGeometryEii", C.c_double, g, C.c_int, C.c_int)
+    direct = _fn("_ZN3imp9direct_usEiiibi", C.c_double, C.c_int, C.c_int, C.c_int, C.c_bool,
+                 C.c_int)
+    pays = _fn("_ZN3imp14separable_paysEdd", C.c_bool, C.c_double, C.c_double)
+    for op, a, b, theta, nc, m, t_direct, t_sep in TIMED:
+        G = _Geometry(ok=True, nz=1, th=theta, wh=1.0)
+        for X, v in ((G.A, a), (G.B, b)):
+            X.n, X.L, X.nf, X.kind = v
+        n = a[0] * b[0]
+        if op == "adjoint":
+            us, d = adj(C.byref(G), m, nc), direct(m, n, nc, False, 256)
+        else:
+            us, d = fwd(C.byref(G), m, nc), direct(n, m, nc, True, 256)
+        assert 0.5 < us / t_sep < 2 and 0.5 < d / t_direct < 2, (op, a, b, us, d)
+        assert pays(us, d) == (t_sep < t_direct), (op, a, b, us, d)

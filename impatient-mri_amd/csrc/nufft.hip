@@ -30,6 +30,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
+#include <utility>
 #include <vector>
 
 #include "common.h"
@@ -57,7 +59,7 @@ constexpr double NU_BETA = 0.99 * M_PI * NW * (1.0 - 1.0 / (2.0 * NU_SIGMA));
 constexpr double NU_TIME_TOL = 5e-8;
 constexpr int NU_MAX_TERMS = 48;       // time terms above which the direct kernel runs
                                        // (16 per lane, 3 groups of a 4-group wave)
-constexpr double NU_MAX_THETA = 40.0;  // half widths of t and w multiplied: 44 terms
+constexpr double NU_MAX_THETA = 40.0;  // half widths of t and w multiplied: 43 terms
 constexpr int NU_MAX_LEG = 160;        // Legendre coefficients per prolate function
 
 // ------------------------------------------------------------------ geometry
@@ -221,69 +223,104 @@ __global__ void k_geo_check(int n, const float *x, const float *y, const float *
 }
 
 // ------------------------------------------------------- prolate expansion
-// Eigenvectors of a symmetric tridiagonal matrix (diagonal d, off-diagonal
-// e[i] between i and i + 1) by implicit QL with Wilkinson shifts; z gets one
-// row per component.  Sorted ascending.
-bool tridiag_eig(std::vector<double> &d, std::vector<double> e, std::vector<double> &z) {
-    const int n = (int)d.size();
-    z.assign((size_t)n * n, 0.0);
-    for (int i = 0; i < n; ++i) z[(size_t)i * n + i] = 1.0;
-    e.resize(n, 0.0);
-    for (int l = 0; l < n; ++l) {
-        for (int it = 0;; ++it) {
-            int m = l;
-            while (m + 1 < n &&
-                   std::fabs(e[m]) > 1e-17 * (std::fabs(d[m]) + std::fabs(d[m + 1])))
-                ++m;
-            if (m == l) break;
-            if (it > 60) return false;
-            double g = (d[l + 1] - d[l]) / (2.0 * e[l]);
-            double r = std::hypot(g, 1.0);
-            g = d[m] - d[l] + e[l] / (g + std::copysign(r, g));
-            double s = 1.0, c = 1.0, p = 0.0;
-            bool split = false;
-            for (int i = m - 1; i >= l; --i) {
-                double f = s * e[i];
-                const double b = c * e[i];
-                r = std::hypot(f, g);
-                e[i + 1] = r;
-                if (r == 0.0) {   // the matrix splits here
-                    d[i + 1] -= p;
-                    e[m] = 0.0;
-                    split = true;
-                    break;
-                }
-                s = f / r;
-                c = g / r;
-                g = d[i + 1] - p;
-                r = (d[i] - g) * s + 2.0 * c * b;
-                p = s * r;
-                d[i + 1] = g + p;
-                g = c * r - b;
-                for (int k = 0; k < n; ++k) {
-                    f = z[(size_t)k * n + i + 1];
-                    z[(size_t)k * n + i + 1] = s * z[(size_t)k * n + i] + c * f;
-                    z[(size_t)k * n + i] = c * z[(size_t)k * n + i] - s * f;
-                }
-            }
-            if (split) continue;
-            d[l] -= p;
-            e[l] = g;
-            e[m] = 0.0;
+// Unit eigenvectors of a symmetric tridiagonal matrix, one at a time from the
+// lowest eigenvalue up.  The pivots of T - s from the top, p_i, and from the
+// bottom, q_i, hold everything wanted at a shift s: as many p_i are negative as
+// eigenvalues lie below s (Sylvester's law of inertia), and where the two
+// eliminations are joined at row k the vector x with x_k = 1 that solves all
+// rows but k misses that one by g = p_k + q_k - (d_k - s) (Parlett and Dhillon,
+// Linear Algebra Appl. 267, 1997).  So the counts bracket one eigenvalue, and x
+// at the k of the smallest |g| gives the next shift, its Rayleigh quotient s +
+// g / x.x.  Six to nine shifts per vector; the expansions below need about four
+// vectors more than they keep (on the host, 36 us for 11 terms, 130 for 28).
+class LowestEigenvectors {
+  public:
+    // off[i] couples rows i and i + 1
+    LowestEigenvectors(std::vector<double> diag, std::vector<double> off)
+        : d_(std::move(diag)), e_(std::move(off)), n_((int)d_.size()), p_(n_), q_(n_) {
+        double lo = d_[0], hi = d_[0];
+        for (int i = 0; i < n_; ++i) {
+            const double r = (i ? std::fabs(e_[i - 1]) : 0.0) + (i + 1 < n_ ? std::fabs(e_[i]) : 0.0);
+            lo = std::min(lo, d_[i] - r);
+            hi = std::max(hi, d_[i] + r);
         }
+        norm_ = std::max(std::fabs(lo), std::fabs(hi));
+        below_ = lo - 1e-12 * norm_;
+        step_ = (hi - lo) / (n_ * n_);   // eigenvalues grow like squares
     }
-    std::vector<int> o(n);
-    for (int i = 0; i < n; ++i) o[i] = i;
-    std::sort(o.begin(), o.end(), [&](int a, int b) { return d[a] < d[b]; });
-    std::vector<double> d2(n), z2((size_t)n * n);
-    for (int i = 0; i < n; ++i) {
-        d2[i] = d[o[i]];
-        for (int k = 0; k < n; ++k) z2[(size_t)k * n + i] = z[(size_t)k * n + o[i]];
+    // x: the next eigenvector.  false: none left, or no convergence.
+    bool next(std::vector<double> &x) {
+        if (found_ >= n_) return false;
+        double lo = below_, hi = lo + step_;
+        int count = pivots_down(hi);
+        for (int i = 0; count <= found_; ++i, count = pivots_down(hi)) {
+            if (i > 200) return false;
+            lo = hi;
+            step_ *= 2.0;
+            hi = lo + step_;
+        }
+        for (int i = 0; count > found_ + 1; ++i) {
+            if (i > 200) return false;
+            const double mid = 0.5 * (lo + hi);
+            const int c = pivots_down(mid);
+            if (c <= found_) lo = mid;
+            else { hi = mid; count = c; }
+        }
+        double s = 0.5 * (lo + hi), last = norm_;
+        for (int i = 0; i < 100; ++i) {
+            (pivots_down(s) <= found_ ? lo : hi) = s;
+            pivots_up(s);
+            const double g = joined(s, x), len = std::sqrt(std::inner_product(
+                x.begin(), x.end(), x.begin(), 0.0));
+            const double miss = std::fabs(g) / len;
+            if (miss <= 1e-16 * norm_ || (miss < 1e-10 * norm_ && miss > 0.25 * last)) {
+                for (double &v : x) v /= len;
+                step_ = std::max(hi - below_, 1e-6 * norm_);
+                below_ = hi;
+                ++found_;
+                return true;
+            }
+            last = miss;
+            s += g / (len * len);
+            if (!(s > lo && s < hi)) s = 0.5 * (lo + hi);
+        }
+        return false;
     }
-    d.swap(d2);
-    z.swap(z2);
-    return true;
-}
+
+  private:
+    double pivot(double v) const {
+        const double tiny = 1e-30 * norm_;
+        return std::fabs(v) < tiny ? -tiny : v;
+    }
+    int pivots_down(double s) {
+        int negative = 0;
+        for (int i = 0; i < n_; ++i) {
+            p_[i] = pivot(d_[i] - s - (i ? e_[i - 1] * e_[i - 1] / p_[i - 1] : 0.0));
+            negative += p_[i] < 0.0;
+        }
+        return negative;
+    }
+    void pivots_up(double s) {
+        for (int i = n_ - 1; i >= 0; --i)
+            q_[i] = pivot(d_[i] - s - (i + 1 < n_ ? e_[i] * e_[i] / q_[i + 1] : 0.0));
+    }
+    // the joined solution and what it misses its row by
+    double joined(double s, std::vector<double> &x) const {
+        int k = 0;
+        auto miss = [&](int i) { return p_[i] + q_[i] - (d_[i] - s); };
+        for (int i = 1; i < n_; ++i)
+            if (std::fabs(miss(i)) < std::fabs(miss(k))) k = i;
+        x.assign(n_, 1.0);
+        for (int i = k - 1; i >= 0; --i) x[i] = -e_[i] * x[i + 1] / p_[i];
+        for (int i = k + 1; i < n_; ++i) x[i] = -e_[i - 1] * x[i - 1] / q_[i];
+        return miss(k);
+    }
+
+    std::vector<double> d_, e_;
+    int n_, found_ = 0;
+    std::vector<double> p_, q_;
+    double norm_, below_, step_;   // below_: found_ eigenvalues lie under it
+};
 
 }  // namespace
 
@@ -303,43 +340,44 @@ bool prolate_expand(double theta, std::vector<double> &coef, std::vector<double>
     const int K = 2 * (((int)(0.75 * theta) + 36) / 2);   // Legendre degrees, both parities
     const int H = K / 2;
     if (K > NU_MAX_LEG) return false;
-    std::vector<double> z[2];
-    const double c2 = theta * theta;
-    for (int par = 0; par < 2; ++par) {
-        std::vector<double> d(H), e(H, 0.0);
+    auto matrix = [&](int par) {   // of the Legendre coefficients of one parity
+        const double c2 = theta * theta;
+        std::vector<double> d(H), e(H - 1);
         for (int i = 0; i < H; ++i) {
             const double k = 2 * i + par;
             d[i] = k * (k + 1) + (2 * k * (k + 1) - 1) / ((2 * k + 3) * (2 * k - 1)) * c2;
-            e[i] = (k + 2) * (k + 1) / ((2 * k + 3) * std::sqrt((2 * k + 1) * (2 * k + 5))) * c2;
+            if (i + 1 < H)
+                e[i] = (k + 2) * (k + 1) / ((2 * k + 3) * std::sqrt((2 * k + 1) * (2 * k + 5))) * c2;
         }
-        e[H - 1] = 0.0;
-        if (!tridiag_eig(d, e, z[par])) return false;
-    }
-    const int nmax = std::min(NU_MAX_TERMS + 1, K - 8);
-    std::vector<double> m(nmax), at1(nmax);
-    std::vector<double> c((size_t)nmax * H);
-    for (int l = 0; l < nmax; ++l) {
-        const int par = l & 1, col = l / 2;
+        return LowestEigenvectors(std::move(d), std::move(e));
+    };
+    LowestEigenvectors vectors[2] = {matrix(0), matrix(1)};
+    const int most = std::min(NU_MAX_TERMS + 1, K - 8);
+    std::vector<double> m, at1, c, z;
+    for (int l = 0; l < most; ++l) {
+        const int par = l & 1;
+        if (!vectors[par].next(z)) return false;
         double s1 = 0.0, v0 = 0.0, p = 1.0;
         // P_k(0) for even k and P_k'(0) for odd k, by their recurrences:
         // P_(k+2)(0) = -(k+1)/(k+2) P_k(0); P_(k+2)'(0) = -(k+2)/(k+1) P_k'(0)
         for (int i = 0; i < H; ++i) {
             const double k = 2 * i + par;
-            const double a = z[par][(size_t)i * H + col] * std::sqrt(k + 0.5);
-            c[(size_t)l * H + i] = a;
+            const double a = z[i] * std::sqrt(k + 0.5);
+            c.push_back(a);
             s1 += a;
             v0 += a * p;
             p *= par ? -(k + 2) / (k + 1) : -(k + 1) / (k + 2);
         }
-        at1[l] = s1;
+        at1.push_back(s1);
         // int e^{i theta s u} psi(s) ds = mu psi(u), at u = 0 (its derivative
         // for odd l); only the Legendre degree 0 (1) of psi integrates
         const double a0 = c[(size_t)l * H];
-        if (par == 0)
-            m[l] = 2.0 * a0 / v0;
-        else
-            m[l] = theta * (2.0 / 3.0) * a0 / v0;
+        m.push_back((par ? theta * (2.0 / 3.0) : 2.0) * a0 / v0);
+        // past their largest the terms fall faster than any power: those after
+        // one of a thousandth of the tolerance do not matter to the tail
+        if (l > theta && std::fabs(m[l]) * s1 * s1 < 1e-3 * NU_TIME_TOL) break;
     }
+    const int nmax = (int)m.size();
     // tail beyond the kept terms, at the corner where it is largest
     int keep = nmax;
     double tail = 0.0;

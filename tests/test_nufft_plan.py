@@ -2,6 +2,9 @@
 built library without a GPU."""
 import ctypes as C
 
+import numpy as np
+import pytest
+
 from impatient import _lib
 
 
@@ -99,3 +102,43 @@ def test_the_faster_form_is_chosen():
             us, d = fwd(C.byref(G), m, nc), direct(n, m, nc, True, 256)
         assert 0.5 < us / t_sep < 2 and 0.5 < d / t_direct < 2, (op, a, b, us, d)
         assert pays(us, d) == (t_sep < t_direct), (op, a, b, us, d)
+
+
+class _Vector(C.Structure):   # std::vector<double>
+    _fields_ = [("begin", C.c_void_p), ("end", C.c_void_p), ("cap", C.c_void_p)]
+
+    def array(self):
+        n = (self.end - self.begin) // 8
+        return np.ctypeslib.as_array((C.c_double * n).from_address(self.begin)).copy()
+
+
+@pytest.mark.parametrize("theta", [1e-6, 1e-3, 0.1, 1.0, 3.77, 8.0, 12.5, 20.0, 31.0, 40.0])
+def test_time_expansion(theta):
+    """e^{i theta s u} from the expansion's terms over [-1, 1]^2 to the tolerance
+    it is cut at (5e-8 at the corners), its functions orthonormal, and no more
+    of them than that tolerance asks for."""
+    f = _fn("_ZN3imp14prolate_expandEdRSt6vectorIdSaIdEES3_PiS4_", C.c_bool, C.c_double,
+            C.POINTER(_Vector), C.POINTER(_Vector), C.POINTER(C.c_int), C.POINTER(C.c_int))
+    a, b, nt, nleg = _Vector(), _Vector(), C.c_int(), C.c_int()
+    assert f(theta, C.byref(a), C.byref(b), C.byref(nt), C.byref(nleg))
+    nt, nleg = nt.value, nleg.value
+    coef, mul = a.array()[:nt * nleg].reshape(nt, nleg), b.array()
+    assert len(mul) == nt
+
+    def psi(u):
+        out = []
+        for l in range(nt):
+            k = np.zeros(2 * nleg + 1)
+            k[l % 2:l % 2 + 2 * nleg:2] = coef[l]
+            out.append(np.polynomial.legendre.legval(u, k))
+        return np.array(out)
+    s = np.linspace(-1, 1, 101)
+    w = mul * 1j ** (np.arange(nt) % 2)
+    p = psi(s)
+    exact = np.exp(1j * theta * np.outer(s, s))
+    assert np.abs((p.T * w) @ p - exact).max() < 5e-8 + 1e-12
+    if nt > 1:   # one term less would not do
+        assert np.abs((p[:-1].T * w[:-1]) @ p[:-1] - exact).max() > 2e-8
+    x, g = np.polynomial.legendre.leggauss(120)
+    q = psi(x)
+    assert np.abs((q * g) @ q.T - np.eye(nt)).max() < 1e-12

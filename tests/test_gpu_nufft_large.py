@@ -142,3 +142,36 @@ def test_volume_whose_first_voxel_is_not_a_number(ctx, axes):
     ref = orc.nudft_adjoint(q["kx"], q["ky"], q["kz"], q["t"], q["x"][idx], q["y"][idx],
                             q["z"][idx], q["fm"][idx], q["d"], q["s"][:, idx])
     assert rel_l2(got[idx], ref) < DIRECT_TOL
+
+
+def test_large_workspaces_are_given_back():
+    """F of 512 x 512 voxels with samples over ten times the band and 27 time
+    terms needs 34 GB; the context keeps none of it (at most 16 GB stay)."""
+    from impatient import Context, _lib, ops
+    from oracle import oracle as orc
+    lib = _lib.load()
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+    N, M = 512, 2000000
+    kx, ky, t, x, y, fm, _, _, rho = _wide(N, 1, M, 2650.0, 35)
+    fm *= np.float32(1100 / 60)
+    ctx = Context(0)
+    try:
+        ops.nudft_forward(ctx, kx[:64], ky[:64], None, t[:64], x, y, None, fm, rho)
+        before = free()
+        got, (n,) = _timer(ctx, lambda: ops.nudft_forward(ctx, kx, ky, None, t, x, y, None, fm,
+                                                          rho), "nufft_forward")
+        assert n == 1
+        ctx.synchronize()
+        kept = before - free()
+    finally:
+        ctx.close()
+    idx = np.array([0, 1, 2, 3, 99999, M - 1])
+    ref = orc.nudft_forward(kx[idx], ky[idx], None, t[idx], x, y, None, fm, rho, None)
+    e = rel_l2(np.asarray(got).reshape(-1)[idx], ref)
+    print(f"kept {kept / 1e9:.2f} GB, {e:.2e}")
+    assert e < TOL
+    assert kept < 17 << 30

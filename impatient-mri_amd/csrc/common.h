@@ -15,6 +15,7 @@ namespace imp {
 
 constexpr size_t HOST_TABLE_WORDS = 2048;   // of a slot of imp_ctx::host_tables()
 constexpr int HOST_TABLES = 32;             // slots
+constexpr int GEO_HOST_WORDS = 64;          // of imp_ctx::geo_host
 
 // ---------------------------------------------------------------- errors
 // Thread-local last error; every C entry point records its failure here.
@@ -101,6 +102,10 @@ struct imp_ctx {
     // next free one, 0 again whenever the stream has been waited for
     int table_slot = 0;
     double *host_tables() const { return host_scalars + 64; }
+    // pinned, coherent host words that the separable NUDFT's geometry scan writes
+    // itself, and the number of the last scan
+    unsigned *geo_host = nullptr;
+    unsigned geo_seq = 0;
     // FFT twiddle tables: table for length L at offset L (L = 2..2048)
     float2 *twiddle = nullptr;
     // live Toeplitz operators created on this context

@@ -153,11 +153,16 @@ extern "C" int imp_ctx_create(int device, imp_ctx **out) {
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
         hipHostMalloc((void **)&ctx->host_scalars, (64 + HOST_TABLES * HOST_TABLE_WORDS) * sizeof(double),
                       hipHostMallocDefault) !=
-            hipSuccess) {
+            hipSuccess ||
+        hipHostMalloc((void **)&ctx->geo_host, GEO_HOST_WORDS * sizeof(unsigned),
+                      hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
+        if (ctx->host_scalars) (void)hipHostFree(ctx->host_scalars);
+        if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
         delete ctx;
         return fail(IMP_EHIP, "imp_ctx_create: stream / pinned allocation failed");
     }
+    std::fill(ctx->geo_host, ctx->geo_host + GEO_HOST_WORDS, 0u);
     // reduction partials (up to 1024 blocks) with their sums, and the FFT
     // twiddles, made here so that solves never allocate on first use
     if (ensure_dscratch(ctx, 1024 + 16) != IMP_OK || twiddle_table_create(ctx) != IMP_OK) {
@@ -166,6 +171,7 @@ extern "C" int imp_ctx_create(int device, imp_ctx **out) {
         if (ctx->twiddle) (void)hipFree(ctx->twiddle);
         (void)hipStreamDestroy(ctx->stream);
         (void)hipHostFree(ctx->host_scalars);
+        (void)hipHostFree(ctx->geo_host);
         delete ctx;
         return fail(IMP_ENOMEM, "imp_ctx_create: reduction scratch / twiddle table");
     }
@@ -201,6 +207,7 @@ extern "C" int imp_ctx_destroy(imp_ctx *ctx) {
     if (ctx->dscratch) (void)hipFree(ctx->dscratch);
     if (ctx->twiddle) (void)hipFree(ctx->twiddle);
     if (ctx->host_scalars) (void)hipHostFree(ctx->host_scalars);
+    if (ctx->geo_host) (void)hipHostFree(ctx->geo_host);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return IMP_OK;

@@ -28,6 +28,7 @@
 // varies fastest in the voxel index.  Rows gB go through the spread and the
 // A transform in blocks, so the spread grid stays small.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -74,12 +75,14 @@ enum {
     G_DEVB,
     G_A0, G_A1, G_B0, G_B1,   // first and last coordinate of each axis (float bits)
     G_KFLAG,          // a sample value is not finite
+    G_DONE,           // blocks of k_geo_check that have ended
     G_WORDS = 32
 };
 
 __host__ __device__ inline unsigned enc_f(unsigned u) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
+static_assert(G_WORDS < GEO_HOST_WORDS, "the call's number follows the words");
 inline float dec_f(unsigned e) {
     const unsigned u = (e & 0x80000000u) ? (e & 0x7fffffffu) : ~e;
     float f;
@@ -141,8 +144,24 @@ __global__ __launch_bounds__(256) void k_geo_scan(int m, const float *kx, const 
     }
 }
 
+// The result words straight into pinned host memory, then the call's number
+// (one block; host null: not wanted).  A copy and a wait for the stream instead
+// leave the GPU idle for some 30 us more.
+__device__ __forceinline__ void geo_export(const unsigned *geo, unsigned *host, unsigned seq) {
+    if (!host) return;
+    if (threadIdx.x < G_WORDS)
+        __hip_atomic_store(&host[threadIdx.x],
+                           __hip_atomic_load(&geo[threadIdx.x], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(&host[G_WORDS], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, const unsigned *part,
-                                                   unsigned *geo) {
+                                                   unsigned *geo, unsigned *host, unsigned seq) {
     // one wave per result word and block range
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int r = wave; r < 2 * GB_WORDS; r += 4) {
@@ -166,7 +185,10 @@ __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, con
             else if (!ks) geo[q == 6 ? G_FCX : G_FCY] = v;
         }
     }
-    if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = 0u;
+    if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = geo[G_DONE] = 0u;
+    __threadfence();
+    __syncthreads();
+    geo_export(geo, host, seq);
 }
 
 // Axis structure implied by the first changes.  In 3D (nz_known = 0) z runs
@@ -185,41 +207,60 @@ __host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool
            (unsigned)n % slow == 0;
 }
 
-__global__ void k_geo_check(int n, const float *x, const float *y, const float *z,
-                            unsigned *geo) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    bool a_is_y;
+// Whether the voxels form the grid that their first changes imply, bit for bit,
+// and how far its axes are from uniform.  The last block to end exports.
+__global__ __launch_bounds__(256) void k_geo_check(int n, const float *x, const float *y,
+                                                   const float *z, unsigned *geo, unsigned *host,
+                                                   unsigned seq) {
+    bool a_is_y, bad = false;
     int nA, nz;
+    float devA = 0.f, devB = 0.f;
     if (!geo_axes(geo[G_FCX], geo[G_FCY], n, z != nullptr, &a_is_y, &nA, &nz)) {
-        if (i == 0) atomicOr(&geo[G_FLAGS], 2u);
-        return;
+        bad = true;
+    } else {
+        const float *a = a_is_y ? y : x, *b = a_is_y ? x : y;
+        const unsigned sa = nz, sb = sa * nA, nB = n / sb;
+        const float a1 = a[(size_t)(nA - 1) * sa], b1 = b[(size_t)(nB - 1) * sb];
+        const double a0 = a[0], da = nA > 1 ? ((double)a1 - a0) / (nA - 1) : 0.0;
+        const double b0 = b[0], db = nB > 1 ? ((double)b1 - b0) / (nB - 1) : 0.0;
+        for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < (unsigned)n; i += gridDim.x * 256) {
+            const unsigned ia = i / sa % nA, ib = i / sb;
+            bad = bad || a[i] != a[(size_t)ia * sa] || b[i] != b[(size_t)ib * sb];
+            if (z) bad = bad || z[i] != z[i % sa] || !isfinite(z[i]);
+            if (i % sa) continue;
+            if (i < sb)
+                devA = fmaxf(devA, (float)(fabs((double)a[i] - (a0 + ia * da)) * 1.000001));
+            if (i % sb == 0)
+                devB = fmaxf(devB, (float)(fabs((double)b[i] - (b0 + ib * db)) * 1.000001));
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            geo[G_A0] = __float_as_uint(a[0]);
+            geo[G_A1] = __float_as_uint(a1);
+            geo[G_B0] = __float_as_uint(b[0]);
+            geo[G_B1] = __float_as_uint(b1);
+        }
     }
-    const float *a = a_is_y ? y : x, *b = a_is_y ? x : y;
-    const int sa = nz, sb = nz * nA, nB = n / sb;
-    const int ia = (i / sa) % nA, ib = i / sb;
-    bool ok = a[i] == a[(size_t)ia * sa] && b[i] == b[(size_t)ib * sb];
-    if (z) ok = ok && z[i] == z[i % nz] && isfinite(z[i]);
-    if (__ballot(!ok) && !ok) atomicOr(&geo[G_FLAGS], 2u);
-    if (i % sa) return;
-    if (i < sb) {
-        const double a0 = a[0],
-                     d = nA > 1 ? ((double)a[(size_t)(nA - 1) * sa] - a0) / (nA - 1) : 0.0;
-        const float dev = (float)(fabs((double)a[i] - (a0 + ia * d)) * 1.000001);
-        if (dev > 0.f) atomicMax(&geo[G_DEVA], __float_as_uint(dev));
+    // one atomic per wave at most
+    const bool any = __ballot(bad) != 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        devA = fmaxf(devA, __shfl_xor(devA, off, 64));
+        devB = fmaxf(devB, __shfl_xor(devB, off, 64));
     }
-    if (i % sb == 0) {
-        const double b0 = b[0],
-                     d = nB > 1 ? ((double)b[(size_t)(nB - 1) * sb] - b0) / (nB - 1) : 0.0;
-        const float dev = (float)(fabs((double)b[i] - (b0 + ib * d)) * 1.000001);
-        if (dev > 0.f) atomicMax(&geo[G_DEVB], __float_as_uint(dev));
+    if ((threadIdx.x & 63) == 0) {
+        if (any) atomicOr(&geo[G_FLAGS], 2u);
+        if (devA > 0.f) atomicMax(&geo[G_DEVA], __float_as_uint(devA));
+        if (devB > 0.f) atomicMax(&geo[G_DEVB], __float_as_uint(devB));
     }
-    if (i == 0) {
-        geo[G_A0] = __float_as_uint(a[0]);
-        geo[G_A1] = __float_as_uint(a[(size_t)(nA - 1) * sa]);
-        geo[G_B0] = __float_as_uint(b[0]);
-        geo[G_B1] = __float_as_uint(b[(size_t)(nB - 1) * sb]);
-    }
+    if (!host) return;
+    __shared__ unsigned last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(&geo[G_DONE], 1u) + 1 == gridDim.x;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    geo_export(geo, host, seq);
 }
 
 // ------------------------------------------------------- prolate expansion
@@ -2105,17 +2146,20 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
 
 // Scan of the operands: value ranges, tensor structure of the voxels.  n = 0
 // scans the samples alone.  geo: G_WORDS result words, part: block results.
+// The last kernel exports the words to ctx->geo_host under this number (0: not).
 static int geo_enqueue(imp_ctx *ctx, unsigned *geo, unsigned *part, int m, int n, const float *kx,
                        const float *ky, const float *t, const float *x, const float *y,
-                       const float *z, const float *fm) {
+                       const float *z, const float *fm, unsigned seq) {
+    unsigned *host = seq ? ctx->geo_host : nullptr;
     const hipStream_t st = ctx->stream;
     const int kb = std::min(256, ceil_div(m, 1024)), xb = std::min(256, ceil_div(n, 1024));
     hipLaunchKernelGGL(k_geo_scan, dim3(kb + xb), dim3(256), 0, st, m, kx, ky, t, n, x, y, fm, kb,
                        part);
     hipLaunchKernelGGL(k_geo_final, dim3(1), dim3(256), 0, st, kb, xb, (const unsigned *)part,
-                       geo);
+                       geo, n ? nullptr : host, seq);
     if (n)
-        hipLaunchKernelGGL(k_geo_check, dim3(ceil_div(n, 256)), dim3(256), 0, st, n, x, y, z, geo);
+        hipLaunchKernelGGL(k_geo_check, dim3(std::min(ctx->num_cus, ceil_div(n, 256))), dim3(256),
+                           0, st, n, x, y, z, geo, host, seq);
     IMP_CHECK_LAUNCH();
     return IMP_OK;
 }
@@ -2134,6 +2178,31 @@ static int geo_read(imp_ctx *ctx, const unsigned *geo, int scans, unsigned *h) {
     IMP_HIP(hipMemcpyAsync(h, geo, (size_t)scans * G_WORDS * sizeof(unsigned),
                            hipMemcpyDeviceToHost, ctx->stream));
     IMP_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->table_slot = 0;   // no table upload is in flight
+    return IMP_OK;
+}
+
+// One scan with its result exported: the words are here, and all that was
+// queued before them has ended, once the host sees the scan's number.  Watched
+// for about as long as a wake-up takes; then, or where the memory is not seen
+// before the kernel ends, the stream is waited for.
+static int geo_scan(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
+                    const float *x, const float *y, const float *z, const float *fm, unsigned *h) {
+    unsigned *geo, *part;
+    IMP_TRY(geo_buffers(ctx, 1, &geo, &part));
+    if (++ctx->geo_seq == 0) ctx->geo_seq = 1;
+    const unsigned seq = ctx->geo_seq;
+    IMP_TRY(geo_enqueue(ctx, geo, part, m, n, kx, ky, t, x, y, z, fm, seq));
+    const auto seen = [&] {
+        return __atomic_load_n(&ctx->geo_host[G_WORDS], __ATOMIC_ACQUIRE) == seq;
+    };
+    const auto start = std::chrono::steady_clock::now();
+    while (!seen()) {
+        if (std::chrono::steady_clock::now() - start < std::chrono::microseconds(200)) continue;
+        IMP_HIP(hipStreamSynchronize(ctx->stream));
+        if (!seen()) return fail(IMP_EHIP, "NUDFT: the geometry scan left no result");
+    }
+    std::memcpy(h, ctx->geo_host, G_WORDS * sizeof(unsigned));
     ctx->table_slot = 0;   // no table upload is in flight
     return IMP_OK;
 }
@@ -2170,10 +2239,8 @@ static void geo_image(const unsigned *h, int n, bool d3, bool fm, NuGeometry *G)
 int nufft_geometry(imp_ctx *ctx, int m, int n, const float *kx, const float *ky, const float *t,
                    const float *x, const float *y, const float *z, const float *fm,
                    NuGeometry *G) {
-    unsigned h[G_WORDS], *geo, *part;
-    IMP_TRY(geo_buffers(ctx, 1, &geo, &part));
-    IMP_TRY(geo_enqueue(ctx, geo, part, m, n, kx, ky, t, x, y, z, fm));
-    IMP_TRY(geo_read(ctx, geo, 1, h));
+    unsigned h[G_WORDS];
+    IMP_TRY(geo_scan(ctx, m, n, kx, ky, t, x, y, z, fm, h));
     geo_image(h, n, z != nullptr, fm != nullptr, G);
     return IMP_OK;
 }
@@ -2188,7 +2255,7 @@ int nufft_geometry_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
         const imp_nudft_job &b = jobs[j];
         if (scan[j])
             IMP_TRY(geo_enqueue(ctx, geo + (size_t)j * G_WORDS, part, b.num_k, b.num_x, b.kx, b.ky,
-                                b.t, b.x, b.y, nullptr, b.fm));
+                                b.t, b.x, b.y, nullptr, b.fm, 0u));
     }
     std::vector<unsigned> h((size_t)njobs * G_WORDS);
     IMP_TRY(geo_read(ctx, geo, njobs, h.data()));
@@ -3039,10 +3106,8 @@ __global__ __launch_bounds__(256) void k_nu_qout(int Nx, int Ny, int nc, int nse
 int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
                      int Ny, int nseg, NuGeometry *G) {
     G->ok = false;
-    unsigned h[G_WORDS], *geo, *part;
-    IMP_TRY(geo_buffers(ctx, 1, &geo, &part));
-    IMP_TRY(geo_enqueue(ctx, geo, part, m, 0, kx, ky, t, nullptr, nullptr, nullptr, nullptr));
-    IMP_TRY(geo_read(ctx, geo, 1, h));
+    unsigned h[G_WORDS];
+    IMP_TRY(geo_scan(ctx, m, 0, kx, ky, t, nullptr, nullptr, nullptr, nullptr, h));
     if (h[G_KFLAG]) return IMP_OK;
     for (int a = 0; a < 2; ++a) {
         NuAxis &X = a ? G->B : G->A;

@@ -175,3 +175,43 @@ def test_large_workspaces_are_given_back():
     print(f"kept {kept / 1e9:.2f} GB, {e:.2e}")
     assert e < TOL
     assert kept < 17 << 30
+
+
+def test_geometry_scans_behind_queued_work(ctx):
+    """Calls queued without a wait between them, the scans of the later ones
+    behind milliseconds of direct sums, each on other points and a grid of other
+    structure (one not a grid): every result as of the call by itself."""
+    from impatient._lib import call, ptr
+    from test_gpu_nufft import _problem
+    jobs = []
+    for i, (Nx, Ny, move) in enumerate([(160, 160, True), (200, 120, False), (160, 160, True),
+                                        (97, 251, False)]):
+        p = _problem(Nx, Ny, 4, 60000, seed=50 + i)
+        if move:
+            p["x"][777] += np.float32(1e-4)
+        up = lambda v: ctx.to_device(np.ascontiguousarray(v, np.float32).reshape(-1))
+        g = [up(p[k]) for k in ("kx", "ky", "t", "x", "y", "fm")]
+        v = [up(p["d"].real), up(p["d"].imag), up(p["s"].real), up(p["s"].imag)]
+        out = [ctx.alloc((Nx * Ny,)) for _ in range(2)]
+        jobs.append((g, v, out, Nx * Ny))
+
+    def run(j):
+        g, v, out, n = j
+        call("imp_nudft_adjoint", ctx.h, C.c_int(60000), C.c_int(n), C.c_int(4), ptr(g[0]),
+             ptr(g[1]), None, ptr(g[2]), ptr(g[3]), ptr(g[4]), None, ptr(g[5]), None, None,
+             *(ptr(q) for q in (*v, *out)))
+
+    def results():
+        ctx.synchronize()
+        return [np.stack([o.get() for o in j[2]]) for j in jobs]
+    alone = []
+    for j in jobs:
+        run(j)
+        alone.append(results()[len(alone)])
+    for j in jobs:
+        for o in j[2]:
+            o.zero()
+    for j in jobs:
+        run(j)
+    for a, b in zip(alone, results()):
+        assert np.array_equal(a, b)

@@ -451,7 +451,7 @@ __global__ __launch_bounds__(GT) void k_grid_gather_heavy(GridGeom g, const int 
 // of the cells around the tile (few contiguous ranges) go in batches of 64: lane
 // v computes the kernel weights of sample v at the tile's columns and rows, all
 // lanes then run over the samples with the next TL_PF samples' data on their
-// way.  A tile of more than TL_HEAVY samples is listed (by the first launch, of
+// way.  A tile of more than H.heavy samples is listed (by the first launch, of
 // one wave per tile) and summed by TL_WAVES waves, added in a fixed order; one of
 // more than TL_PART (the centre of a variable-density trajectory) by several
 // such workgroups, whose sums k_grid_tiles_sum adds.
@@ -461,12 +461,20 @@ __global__ __launch_bounds__(GT) void k_grid_gather_heavy(GridGeom g, const int 
 // 704^2, 11 segments of 393216 samples: gathers 4.31 ms -> 1.27 ms.  TL_WAVES 4, 8,
 // 16: 2.99, 1.67, 1.33 ms for the listed tiles (before they were parted);
 // TL_HEAVY 128, 256, 512, 1024: 0.64, 0.87, 1.15, 1.54 ms for the others.
-constexpr int TL_PF = 4, TL_HEAVY = 256, TL_WAVES = 16, TL_PART = 2048;
+//
+// Few samples leave few tiles that are long, and the launch waits for the waves
+// that sum 200 of them: up to TL_FEW samples a tile is listed above TL_LOW. Whole
+// calls of 3 coils, 16000 samples, os 1.5, one thread per point / 256 / 64: 64^2
+// 662 / 739 / 530 us, 96^2 682 / 767 / 580. At 64 from 160000 samples on: 0.9 to
+// 1.8 times the time at 256.
+constexpr int TL_PF = 4, TL_HEAVY = 256, TL_LOW = 64, TL_FEW = 40000, TL_WAVES = 16,
+              TL_PART = 2048;
 struct TileList {
     int4 *entries;    // tile, part, parts, slot
     int4 *multis;     // tile, parts, first slot
     int *count;       // entries, slots, multis
     float2 *slots;    // [slot][16][64]
+    int heavy;        // samples above which a tile is listed
 };
 template <int C>
 struct Tile {
@@ -520,7 +528,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_grid_tiles(GridGeom g, const int
         int total = rn;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) total += __shfl_xor(total, off, 64);
-        if (WAVES == 1 && total > TL_HEAVY) {
+        if (WAVES == 1 && total > H.heavy) {
             if (lane == 0) {
                 const int parts = (total + TL_PART - 1) / TL_PART;
                 const int e0 = atomicAdd(&H.count[0], parts);
@@ -1328,8 +1336,9 @@ size_t tile_list_bytes(long tiles, long slots) {
     return (size_t)(tiles + 2 * slots) * sizeof(int4) + (size_t)slots * 16 * 64 * sizeof(float2) +
            2048;
 }
-TileList tile_list(Carve &cv, long tiles, long slots) {
+TileList tile_list(Carve &cv, long tiles, long slots, int m) {
     TileList H;
+    H.heavy = m <= TL_FEW ? TL_LOW : TL_HEAVY;
     H.entries = cv.take<int4>(tiles + slots);
     H.multis = cv.take<int4>(slots);
     H.count = cv.take<int>(4);
@@ -1475,7 +1484,7 @@ int gridding_fhd(imp_ctx *ctx, int num_k, int ncoils, const float *kx, const flo
     float2 *bufB = cv.take<float2>((size_t)CP * ncells);
     int *heavy = cv.take<int>(ncells);
     int *nheavy = cv.take<int>(1);
-    const TileList H = tile_list(cv, tiles, slots);
+    const TileList H = tile_list(cv, tiles, slots, num_k);
     float2 *data = cv.take<float2>((size_t)num_k * CP);
     double2 *acc = cv.take<double2>(nv);
     AxisPlan ax[3];

@@ -76,6 +76,7 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
 
 int nufft_q_geometry(imp_ctx *ctx, int m, const float *kx, const float *ky, const float *t, int Nx,
                      int Ny, int nseg, NuGeometry *G);
+double nufft_q_us(const NuGeometry &G, int m, int nseg);
 int nufft_q(imp_ctx *ctx, const NuGeometry &G, int m, const float *kx, const float *ky,
             const float *t, const float *phi_r, const float *phi_i, int Nx, int Ny, int nseg,
             float tau, float t0, bool cumulative, float *q_r, float *q_i);

@@ -2637,6 +2637,14 @@ static double padded(int columns, int L) {
 static double expansion_work(const NuGeometry &G, int nt, double points) {
     return points * nt * (0.75 * G.wh * G.th + 36.0);
 }
+// The sort's blocks each read every block's digit counts (about 5 TB/s).
+static double sort_us(int m, double ncells) {
+    const double nblk = ceil_div(m, RX_BLOCK);
+    return nufft_sort_passes((int)ncells) * nblk * nblk * (RX_BINS * sizeof(int)) / 5e6;
+}
+static double cells(const NuAxis &A, const NuAxis &B) {
+    return (double)(A.nf - NW + 1) * (B.nf - NW + 1);
+}
 // fixed part, samples and A transform of ncols columns
 static double to_mid_us(const NuGeometry &G, int nt, int m, int ncols) {
     const int cg = column_group(G, nt, ncols), groups = ceil_div(ncols, cg);
@@ -2645,7 +2653,7 @@ static double to_mid_us(const NuGeometry &G, int nt, int m, int ncols) {
                         2.0 * groups * (1 << log2i(cg));
     const double lines = groups * padded(nt * std::min(cg, ncols), G.A.L);
     // a group is half a dozen launches of some 8 us
-    return 144.0 + 50.0 * (groups - 1) + m * (2.79e-6 * groups * sp.cost + 1.46e-5 * prep) +
+    return 144.0 + 50.0 * (groups - 1) + sort_us(m, cells(G.A, G.B)) + m * (2.79e-6 * groups * sp.cost + 1.46e-5 * prep) +
            1.5e-6 * expansion_work(G, nt, m) + 9.74e-6 * G.A.nf * G.B.nf * (double)nt * ncols +
            4.16e-6 * line_work(G.A, G.B.nf, lines);
 }
@@ -2913,7 +2921,7 @@ double nufft_forward_us(const NuGeometry &G, int m, int ncoils) {
     }
     for (const NuAxis *X : {&A, &B})
         if (X->kind == AX_FREE) lists += (double)X->n * ceil_div(X->L, 1024);
-    return 114.0 + 2.09e-3 * entries * nt * blocks + 3.6e-5 * (double)m * ncoils +
+    return 114.0 + sort_us(m, tiles) + 2.09e-3 * entries * nt * blocks + 3.6e-5 * (double)m * ncoils +
            5.35e-6 * expansion_work(G, nt, m) + 1.17e-5 * A.nf * B.nf * (double)nt * ncoils +
            0.48 * lists + 2.9e-6 * line_work(A, B.nf, linesA) +
            6.4e-6 * line_work(B, A.n, linesB) +
@@ -3039,11 +3047,22 @@ int nufft_forward(imp_ctx *ctx, const NuGeometry &G, int m, int ncoils, const fl
 // column's sum is P = Q_2c + i Q_(2c+1), and Q_l(-r) = conj(Q_l(r)) gives
 // Q_2c = (P(r) + conj(P(-r))) / 2, Q_(2c+1) = (P(r) - conj(P(-r))) / 2i, so
 // Q_l comes out conjugate-symmetric bit for bit.
-// Against the GEMM over phasor tables (toeplitz_q_sep) it is faster at every
-// size measured (16^2 x 50 samples: 0.23 -> 0.17 ms; 512^2, 393216 samples,
-// L = 10: 255 -> 1.3 ms, 240 of it the allocation of 9 GB of tables on each
-// call) and closer to 64 bits (2.6e-8 against 1.1e-7), so on 2D standard
-// grids the GEMM is left to grids beyond the transform lengths.
+// Against the GEMM over phasor tables (toeplitz_q_sep) it is closer to 64 bits
+// (2.6e-8 against 1.1e-7) and faster wherever samples are not few for the grid
+// (16^2 x 500 samples, L = 10: 0.27 -> 0.16 ms; 512^2 x 393216, L = 10: 16 -> 1.07
+// ms, and 255 in a process where the 9 GB of tables made on each call came
+// slowly); the GEMM's time is in the samples: 700^2 x 500, L = 31: 0.75 ms
+// against 3.9.  Price within 17% rms of 136 calls, 16^2 to 1300^2, 500 to 10^6
+// samples, L = 3 to 31.
+double nufft_q_us(const NuGeometry &G, int m, int nseg) {
+    const int cols = (nseg + 1) / 2, cg = column_group(G, 1, cols);
+    const SpreadSplit sp = spread_split(1, log2i(cg));
+    const double prep = 2 * NW + 2 * (sp.T - 1) + 2 * (sp.yg - 1) + 1 + 2.0 * cg;
+    return 151.0 + sort_us(m, cells(G.A, G.B)) + m * (2.17e-6 * sp.cost + 1.49e-5 * prep) +
+           1.39e-5 * G.A.nf * G.B.nf * (double)cols +
+           1.32e-5 * (line_work(G.A, G.B.nf, padded(cols, G.A.L)) +
+                      line_work(G.B, G.A.n, padded(cols, G.B.L)));
+}
 namespace {
 
 // [sample][slot] = (a_2c, a_(2c+1)) |phi|^2, a_l the Hanning interpolator of

@@ -142,3 +142,26 @@ def test_time_expansion(theta):
     x, g = np.polynomial.legendre.leggauss(120)
     q = psi(x)
     assert np.abs((q * g) @ q.T - np.eye(nt)).max() < 1e-12
+
+
+def test_q_takes_the_faster_form():
+    """Q_l on the standard grid, calls timed in both forms (N, L, samples;
+    microseconds of the GEMM over tables and of the separable sums): few samples
+    on a large grid are the GEMM's."""
+    us = _fn("_ZN3imp10nufft_q_usERKNS_10NuGeometryEii", C.c_double, C.POINTER(_Geometry), C.c_int,
+             C.c_int)
+    gemm = _fn("_ZN3imp9q_gemm_usEiiii", C.c_double, C.c_int, C.c_int, C.c_int, C.c_int)
+    pays = _fn("_ZN3imp14separable_paysEdd", C.c_bool, C.c_double, C.c_double)
+    lengths = {16: 96, 64: 192, 512: 1536, 700: 2304, 1024: 3072, 1300: 4096}
+    for N, L, m, t_gemm, t_sep in ((1300, 31, 500, 1663, 12058), (1024, 31, 500, 1213, 7111),
+                                   (700, 31, 500, 754, 3885), (1024, 10, 500, 624, 2377),
+                                   (700, 31, 10000, 1759, 3980), (512, 31, 10000, 1067, 1683),
+                                   (512, 10, 393216, 16300, 1070), (64, 3, 10000, 374, 229),
+                                   (16, 10, 500, 270, 158)):
+        G = _Geometry(ok=True, nz=1)
+        for X in (G.A, G.B):
+            X.n, X.L = 2 * N + 1, lengths[N]
+            X.nf = 2 * int(np.ceil(0.49 * X.L + 5.5) + 1) + 1
+        a, b = us(C.byref(G), m, L + 1), gemm(m, N, N, L + 1)
+        assert 0.5 < a / t_sep < 2 and 0.5 < b / t_gemm < 2, (N, L, m, a, b)
+        assert pays(a, b) == (t_sep < t_gemm), (N, L, m, a, b)

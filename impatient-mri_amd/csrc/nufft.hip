@@ -75,7 +75,6 @@ enum {
     G_DEVB,
     G_A0, G_A1, G_B0, G_B1,   // first and last coordinate of each axis (float bits)
     G_KFLAG,          // a sample value is not finite
-    G_DONE,           // blocks of k_geo_check that have ended
     G_WORDS = 32
 };
 
@@ -144,20 +143,21 @@ __global__ __launch_bounds__(256) void k_geo_scan(int m, const float *kx, const 
     }
 }
 
-// The result words straight into pinned host memory, then the call's number
-// (one block; host null: not wanted).  A copy and a wait for the stream instead
-// leave the GPU idle for some 30 us more.
+// The result words straight into pinned host memory, then the call's number (one
+// block).  A copy and a wait for the stream instead take some 10 us more.
 __device__ __forceinline__ void geo_export(const unsigned *geo, unsigned *host, unsigned seq) {
-    if (!host) return;
     if (threadIdx.x < G_WORDS)
-        __hip_atomic_store(&host[threadIdx.x],
-                           __hip_atomic_load(&geo[threadIdx.x], __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&host[threadIdx.x], geo[threadIdx.x], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0)
         __hip_atomic_store(&host[G_WORDS], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// After k_geo_check, in a launch of its own: counting ended blocks there takes
+// a device-wide fence from each of them, which made its 6 us 24.
+__global__ void k_geo_export(const unsigned *geo, unsigned *host, unsigned seq) {
+    geo_export(geo, host, seq);
 }
 
 __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, const unsigned *part,
@@ -185,8 +185,8 @@ __global__ __launch_bounds__(256) void k_geo_final(int kblocks, int xblocks, con
             else if (!ks) geo[q == 6 ? G_FCX : G_FCY] = v;
         }
     }
-    if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = geo[G_DONE] = 0u;
-    __threadfence();
+    if (threadIdx.x == 0) geo[G_DEVA] = geo[G_DEVB] = 0u;
+    if (!host) return;   // the voxels are checked first
     __syncthreads();
     geo_export(geo, host, seq);
 }
@@ -208,10 +208,9 @@ __host__ __device__ inline bool geo_axes(unsigned fcx, unsigned fcy, int n, bool
 }
 
 // Whether the voxels form the grid that their first changes imply, bit for bit,
-// and how far its axes are from uniform.  The last block to end exports.
+// and how far its axes are from uniform.
 __global__ __launch_bounds__(256) void k_geo_check(int n, const float *x, const float *y,
-                                                   const float *z, unsigned *geo, unsigned *host,
-                                                   unsigned seq) {
+                                                   const float *z, unsigned *geo) {
     bool a_is_y, bad = false;
     int nA, nz;
     float devA = 0.f, devB = 0.f;
@@ -252,15 +251,6 @@ __global__ __launch_bounds__(256) void k_geo_check(int n, const float *x, const 
         if (devA > 0.f) atomicMax(&geo[G_DEVA], __float_as_uint(devA));
         if (devB > 0.f) atomicMax(&geo[G_DEVB], __float_as_uint(devB));
     }
-    if (!host) return;
-    __shared__ unsigned last;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(&geo[G_DONE], 1u) + 1 == gridDim.x;
-    __syncthreads();
-    if (!last) return;
-    __threadfence();
-    geo_export(geo, host, seq);
 }
 
 // ------------------------------------------------------- prolate expansion
@@ -2146,7 +2136,7 @@ bool plan_axis(int n, float c0, float c1, float dev, float cmin, float cmax, flo
 
 // Scan of the operands: value ranges, tensor structure of the voxels.  n = 0
 // scans the samples alone.  geo: G_WORDS result words, part: block results.
-// The last kernel exports the words to ctx->geo_host under this number (0: not).
+// The last kernel writes the words to ctx->geo_host under this number (0: not).
 static int geo_enqueue(imp_ctx *ctx, unsigned *geo, unsigned *part, int m, int n, const float *kx,
                        const float *ky, const float *t, const float *x, const float *y,
                        const float *z, const float *fm, unsigned seq) {
@@ -2157,9 +2147,13 @@ static int geo_enqueue(imp_ctx *ctx, unsigned *geo, unsigned *part, int m, int n
                        part);
     hipLaunchKernelGGL(k_geo_final, dim3(1), dim3(256), 0, st, kb, xb, (const unsigned *)part,
                        geo, n ? nullptr : host, seq);
-    if (n)
-        hipLaunchKernelGGL(k_geo_check, dim3(std::min(ctx->num_cus, ceil_div(n, 256))), dim3(256),
-                           0, st, n, x, y, z, geo, host, seq);
+    if (n) {
+        hipLaunchKernelGGL(k_geo_check, dim3(std::min(4 * ctx->num_cus, ceil_div(n, 256))),
+                           dim3(256), 0, st, n, x, y, z, geo);
+        if (host)
+            hipLaunchKernelGGL(k_geo_export, dim3(1), dim3(64), 0, st, (const unsigned *)geo, host,
+                               seq);
+    }
     IMP_CHECK_LAUNCH();
     return IMP_OK;
 }

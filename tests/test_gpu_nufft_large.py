@@ -43,7 +43,7 @@ def test_forward_half_transformed_grid_larger_than_32_bits(ctx):
     assert max(errs) < TOL
 
 
-def test_q_of_more_weights_than_32_bits():
+def test_q_of_more_weights_than_32_bits(ctx):
     """2^27 samples x 16 column slots: 2^31 weights.  The samples repeat 2^15
     of them, so the sums are the oracle's over those times the repetitions (at
     some points of each segment)."""
@@ -147,7 +147,7 @@ def test_volume_whose_first_voxel_is_not_a_number(ctx, axes):
     assert rel_l2(got[idx], ref) < DIRECT_TOL
 
 
-def test_large_workspaces_are_given_back():
+def test_large_workspaces_are_given_back(ctx):
     """F of 512 x 512 voxels with samples over ten times the band and 27 time
     terms needs 34 GB; the context keeps none of it (at most 16 GB stay)."""
     from impatient import Context, _lib, ops
@@ -161,17 +161,17 @@ def test_large_workspaces_are_given_back():
     N, M = 512, 2000000
     kx, ky, t, x, y, fm, _, _, rho = _wide(N, 1, M, 2650.0, 35)
     fm *= np.float32(1100 / 60)
-    ctx = Context(0)
+    own = Context(0)
     try:
-        ops.nudft_forward(ctx, kx[:64], ky[:64], None, t[:64], x, y, None, fm, rho)
+        ops.nudft_forward(own, kx[:64], ky[:64], None, t[:64], x, y, None, fm, rho)
         before = free()
-        got, (n,) = _timer(ctx, lambda: ops.nudft_forward(ctx, kx, ky, None, t, x, y, None, fm,
+        got, (n,) = _timer(own, lambda: ops.nudft_forward(own, kx, ky, None, t, x, y, None, fm,
                                                           rho), "nufft_forward")
         assert n == 1
-        ctx.synchronize()
+        own.synchronize()
         kept = before - free()
     finally:
-        ctx.close()
+        own.close()
     idx = np.array([0, 1, 2, 3, 99999, M - 1])
     ref = orc.nudft_forward(kx[idx], ky[idx], None, t[idx], x, y, None, fm, rho, None)
     e = rel_l2(np.asarray(got).reshape(-1)[idx], ref)

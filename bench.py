@@ -501,10 +501,11 @@ def main():
                                   "transformed grids the separable form streams besides are not "
                                   "counted",
                 "kernel": "separable F^H d (all its launches)", "kernel_ms": round(k_ms, 3),
+                "spread_ms": round(kernel_ms("k_spread")[0] / max(k_n, 1), 3),
                 "limit": "FP64 issue in the spread, then the line transforms' latency"}
 
     result = {
-        "metric": "NUDFT GSample*vox/s (direct field-corrected F^H d); time to rel-residual 1e-5 "
+        "metric": "NUDFT GSample*vox/s (field-corrected F^H d, pairs of a direct sum); time to rel-residual 1e-5 "
                   "(plain CG) reported in recon",
         "value": round(value, 2), "unit": "GSample*vox/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(ms, 3),

@@ -1297,7 +1297,8 @@ size_t adjoint_fixed_bytes(int num_k, int num_x, int ncoils, bool d3) {
 // are in nufft.hip).  The direct kernels cost the same for every geometry: pairs,
 // operands packed per streamed point and coil, partial sums per chunk.
 constexpr double STACK_MIN_US = 400.0;    // direct time of a stack below which it is kept
-constexpr double NUFFT_MIN_PAIRS = 6e8;   // below: the direct kernels win at every size measured
+constexpr double NUFFT_MIN_PAIRS = 6e8;   // below, the scan and the separable form's fixed part
+                                          // (170 us) are most of the direct sum's time
 constexpr double DIRECT_FIXED_US = 70.0;
 
 double direct_us(int n_stream, int n_lane, int ncoils, bool forward, int num_cus) {
@@ -2602,8 +2603,8 @@ int toeplitz_q(imp_ctx *ctx, int num_k, const float *kx, const float *ky,
     IMP_CHECK_LAUNCH();
     const Out mode = (flags & IMP_Q_CUMULATIVE) ? Out::PerRhsCumulative : Out::PerRhs;
     // Standard grid (main_mri.cu:461-500; y outer, x, z inner, r = (x/Nx,
-    // y/Ny, z/Nz)), 3D or beyond the 2D transforms: the separable GEMM unless the direct kernel is asked for
-    // (or tau is degenerate); the direct kernel evaluates the half grid and
+    // y/Ny, z/Nz)) in 3D, beyond the 2D transforms, or of few samples: the
+    // separable GEMM unless the direct kernel is asked for (or tau is degenerate); the direct kernel evaluates the half grid and
     // fills the rest by Hermitian symmetry.
     if (std_grid && !(flags & IMP_Q_DIRECT) && tau > 0.f && std::isfinite(tau) &&
         std::isfinite(t0)) {

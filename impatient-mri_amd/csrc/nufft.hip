@@ -1417,8 +1417,8 @@ __device__ __forceinline__ void line_interp(const LineArgs &P, double2 (&v)[ln::
 // as long (384^2 x 8 coils, two slices: 1.47 -> 0.79 ms, of which 0.45 were LDS
 // reads for the interpolation; 250 x 234 x 8 coils: 251 -> 136 us).
 //
-// Bound by memory: 512^2 x 32 coils, 768-point lines, 3.1 TB/s (reads alone 127
-// us, writes 87, the transforms 14 of 247 us per launch).
+// Bound by memory: 512^2 x 32 coils, 768-point lines, 3.3 TB/s by the counters
+// (reads alone 127 us, writes 87, the transforms 14 of 247 us per launch).
 template <int L, int KIND>
 __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG),
                              KIND == AX_NEAR ? 2 : 4) void k_line_store(
@@ -1485,8 +1485,9 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG),
 //
 // Bound by the latency of a step (load, three exchanges, factors) at three
 // waves per SIMD, which the bounds above keep free of spills: 512^2 x 32 coils
-// 1.62 -> 0.92 ms (2.6 TB/s), 250 x 234 x 8 coils 290 -> 148 us, two slices of
-// 384^2 x 8 coils 1.12 -> 0.55 ms.
+// 1.62 -> 0.92 ms (2.6 TB/s of its input; the counters show twice the bytes, its
+// columns being 64-byte pieces of 128-byte lines), 250 x 234 x 8 coils 290 -> 148
+// us, two slices of 384^2 x 8 coils 1.12 -> 0.55 ms.
 struct CombineArgs {
     int nc, nt;             // coils, time terms
     int lcw, ncs, nls;      // log2 of the coils side by side; splits of coils, of time terms
@@ -1510,7 +1511,8 @@ __global__ __launch_bounds__(ln::threads(L) * ln::lines(L, ST_WG), 3) void k_lin
     const int s0 = nst * ls / C.nls, s1 = nst * (ls + 1) / C.nls;
     constexpr int S = ln::stages(L) - 1, R = ln::radix(L, S);
     const double2 *base = P.in + (size_t)line * P.in_line;
-    // offsets within vt and sens stay below 2^32 bytes (checked at launch)
+    // element offsets within vt and sens are 32 bits wide: at most 48 terms or 32
+    // coils x 4096 x 4096 points, below 2^30
     const double *vline = C.vt + (size_t)line * P.X.n;
     double2 *out = C.partial + (size_t)split * C.nvox + (size_t)line * P.X.n;
     const unsigned nmax = (unsigned)P.X.n - 1;
@@ -1832,12 +1834,14 @@ struct GiArgs {
     float *d_r, *d_i;
 };
 
-// One wave per entry: out[sample][column] = sum over the tile's 15 rows x 16
-// cells and nt terms of (wx wy u)[sample] grid[column], a product of 16 x
-// 3840 nt/16 by 3840 nt/16 x 16 matrices on v_mfma_f64_16x16x4_f64 (sample i =
-// lane % 16 and cell k = lane / 16 of A, column j = lane % 16 of B, result row
-// lane / 16 + 4 r).  FP64 MFMA runs at half the FMA rate here, but needs the
-// weights once per lane instead of 16 of them in scalar registers per value.
+// One wave per entry: out[sample][column] = sum over the tile's NW + TG - 1 = 14
+// rows x GI_W = 16 cells and nt terms of (wx wy u)[sample] grid[column], a
+// product of a 16 x 224 nt by a 224 nt x 16 matrix on v_mfma_f64_16x16x4_f64
+// (sample i = lane % 16 and cell k = lane / 16 of A, column j = lane % 16 of B,
+// result row lane / 16 + 4 r); 121 of the 224 products are of a sample's own
+// window.  FP64 MFMA runs at 37.7 TFLOP/s here against 57.6 of the FMAs, but
+// needs the weights once per lane instead of 16 of them in scalar registers per
+// value.
 template <int CB>
 __global__ __launch_bounds__(64) void k_gather(GiArgs P) {
     const int lane = threadIdx.x, i = lane & 15, k = lane >> 4;
@@ -2278,8 +2282,8 @@ constexpr size_t NU_MID_BYTES = (size_t)3 << 30;
 // What a context keeps of the workspaces from call to call: 4.2 GB serve 512^2 x
 // 32 coils, 12 GB the largest images at 32 coils.  Larger ones (samples far
 // beyond the band, 10^7 samples and more) are freed when the call ends: making
-// them anew took 0.4 ms for 1 to 32 GB in a bare process, but 27 ms per GB in one
-// that held much else.
+// them anew took 0.4 ms for 1 to 32 GB in a bare process, and up to 27 ms per GB
+// in others.
 constexpr size_t NU_KEEP_BYTES = (size_t)16 << 30;
 
 int log2i(int n) {

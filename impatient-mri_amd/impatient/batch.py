@@ -4,7 +4,8 @@ The slices (N x N, N in {128, 256, 384} for the 48-slice workload, 8 coils
 each, spiral trajectories scaled per matrix size, field maps within
 +-150 Hz) go through:
 
-  1. one persistent MFMA launch for all F^H d (imp_nudft_adjoint_batch);
+  1. all F^H d in one call (imp_nudft_adjoint_batch: large slices in separable
+     form, the others in one persistent MFMA launch);
   2. Q_l once per size class (the trajectory is shared within a class) and a
      Toeplitz plan per slice (field map and coils are per slice);
   3. per slice: the learned warm start (network of the size class, trained
@@ -115,7 +116,8 @@ def reconstruct(ctx: Context, slices, tol=1e-5, max_iter=500, model=None, tuner=
     host arrays, copied after the slice's timing ends)."""
     tuner = tuner or Autotuner(ctx)
     t_all = time.perf_counter()
-    # 1. F^H d of every slice in one persistent launch (autotuned chunking)
+    # 1. F^H d of every slice in one call (autotuned chunking of its launch of
+    # the smaller slices)
     jobs = [dict(kx=s.prob.kx, ky=s.prob.ky, t=s.prob.t, x=s.prob.x, y=s.prob.y, fm=s.prob.fm,
                  d=s.d, sens=s.prob.sens) for s in slices]
     key = ("fhd_batch", tuple(sorted({s.prob.Nx for s in slices})), len(slices))
@@ -237,7 +239,7 @@ def reconstruct(ctx: Context, slices, tol=1e-5, max_iter=500, model=None, tuner=
         c.close()
     t_total = time.perf_counter() - t_all
     log(f"batch: {len(slices)} slices in {t_total:.3f} s ({len(slices) / t_total:.1f} slices/s); "
-        f"F^H d {t_fhd * 1e3:.1f} ms (one launch, chunk scale {scale}), Q {t_q * 1e3:.1f} ms, "
+        f"F^H d {t_fhd * 1e3:.1f} ms (one call, chunk scale {scale}), Q {t_q * 1e3:.1f} ms, "
         f"solves {t_solve * 1e3:.1f} ms on {nw} streams")
     return dict(slices=recs, total_s=t_total, fhd_s=t_fhd, q_s=t_q, solve_s=t_solve,
                 streams=nw, nudft_chunk_scale=scale,

@@ -79,7 +79,7 @@ def _fill(host, parts, piece=1 << 22):
 
 
 def nudft_adjoint_batch(ctx: Context, jobs, chunk_scale=0):
-    """F^H d of several 2D images in one persistent launch.  jobs: list of
+    """F^H d of several 2D images in one call.  jobs: list of
     dicts with kx, ky, t, x, y, fm, d [C, M], sens [C, N] (numpy).  Returns
     the list of images."""
     from ._lib import NudftJob

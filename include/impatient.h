@@ -7,7 +7,8 @@
  * printf + exit(1) come back as status codes here.
  *
  * Memory: functions named imp_<op> take DEVICE pointers (HBM-resident
- * operands, asynchronous on the context's HIP stream). The file-level
+ * operands, asynchronous on the context's HIP stream unless their comment says
+ * that they wait for it). The file-level
  * wrappers (imp_toeplitz_computeQ_GPU, imp_toeplitz_computeFH_GPU,
  * imp_toeplitz_recon, imp_bruteForceGpu) take HOST pointers exactly like the
  * reference functions they replace and are synchronous.
@@ -137,7 +138,9 @@ int imp_nudft_adjoint_noalloc(imp_ctx *ctx, int num_k, int num_x, int ncoils,
 /* Replaces ftGpu + parallelFtGpu (kernels/ftGpu.cu:198-604,
  * kernels/parImagingGpu.cu:92-117):
  *   d_c(k) = sum_x S_c(x) rho(x) e^{-i(2pi k.x + fm(x) t_k)}
- *   d_r/d_i [ncoils*num_k] coil-major.  No power-of-two padding is needed. */
+ *   d_r/d_i [ncoils*num_k] coil-major.  No power-of-two padding is needed.
+ * Large 2D problems take the separable form as imp_nudft_adjoint does, and wait
+ * for the stream as it does. */
 int imp_nudft_forward(imp_ctx *ctx, int num_k, int num_x, int ncoils,
                       const float *kx, const float *ky, const float *kz,
                       const float *t,
@@ -148,10 +151,12 @@ int imp_nudft_forward(imp_ctx *ctx, int num_k, int num_x, int ncoils,
                       float *d_r, float *d_i);
 
 /* Batched F^H d: several images (different sizes, trajectories, coil maps;
- * each 3..32 coils, all 2D or all 3D) in one persistent MFMA launch whose
- * flattened grid covers every image's point tiles.  Arguments of each job
- * as for imp_nudft_adjoint.  chunk_scale: workgroups per CU targeted per job
- * (the schedule knob an autotuner sweeps; 0 = 8).  No counterpart in the
+ * each 3..32 coils, all 2D or all 3D): large 2D images in separable form, one
+ * after another behind one read-back of what decides it, the others in one
+ * persistent MFMA launch whose flattened grid covers every image's point tiles.
+ * Waits for the stream.  Arguments of each job as for imp_nudft_adjoint.
+ * chunk_scale: workgroups per CU targeted per job of that launch (the schedule
+ * knob an autotuner sweeps; 0 = 8).  No counterpart in the
  * reference, which loops slices on the host (main_mri.cu:771-904). */
 typedef struct {
     int num_k, num_x, ncoils;
@@ -176,8 +181,9 @@ int imp_nudft_adjoint_batch(imp_ctx *ctx, int njobs, const imp_nudft_job *jobs,
  * accumulator is not cleared between segments (computeQ.cmem.cu:190-191,
  * 951-963), i.e. returns prefix sums over l.  On the standard grid the
  * sums are evaluated in separable form (2D: spreading and line transforms in
- * FP64; 3D, and samples beyond the band: a GEMM, e^{i 2pi k.r} = e_x e_y e_z
- * per sample, each segment over the samples where a_l != 0); IMP_Q_DIRECT
+ * FP64; 3D, samples beyond the band or few for the grid: a GEMM, e^{i 2pi k.r}
+ * = e_x e_y e_z per sample, each segment over the samples where a_l != 0);
+ * either way the call waits for the stream.  IMP_Q_DIRECT
  * evaluates every grid point with the per-point kernel instead. */
 #define IMP_Q_CUMULATIVE 0x1
 #define IMP_Q_DIRECT 0x2

@@ -1333,10 +1333,11 @@ double q_gemm_us(int m, int Nx, int Ny, int nseg) {
            2.26e-5 * nseg * area + 4.0e-4 * m * nseg;
 }
 
-// A tenth in favour of the direct sums: of the 1000 calls timed 642 take the
-// separable form and 18 of them would have been faster directly, by 1.4 at most
-// (without the tenth 677 and 29; of those left direct none loses over 1.5).
-bool separable_pays(double separable, double direct) { return separable < 0.9 * direct; }
+// Where the prices are within 5% the separable form is taken, which is 2 to 10
+// times closer to 64 bits.  Of the 1000 calls timed 700 take it; 34 of them would
+// have been faster directly by more than 2%, 7 by more than 25%, 1.44 times at
+// most (with 0.9, 1.0, 1.1: 642, 676, 713 calls, 14, 25, 41 of them slower).
+bool separable_pays(double separable, double direct) { return separable < 1.05 * direct; }
 
 // The separable form evaluates 2D problems of as many coils as one direct
 // launch takes; refusals and everything else stay with the direct path.
